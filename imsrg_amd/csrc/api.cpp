@@ -45,14 +45,12 @@ struct BatchCache {
   int cnt[10] = {0};
   double *work = nullptr;
   int maxn = 0, maxnch = 0, maxjmax = 0, maxnorb = 0, maxn1pairs = 0, maxncls = 0, maxbin = 0, maxent = 0;
-  long maxn122 = 0;
   void release() {
     if (d_tab) (void)hipFree(d_tab);
     if (d_items) (void)hipFree(d_items);
     if (work) (void)hipFree(work);
     d_tab = nullptr; d_items = nullptr; work = nullptr;
     maxn = maxnch = maxjmax = maxnorb = maxn1pairs = maxncls = maxbin = maxent = 0;
-    maxn122 = 0;
     key.clear();
   }
 };
@@ -145,7 +143,6 @@ struct imsrg_ctx {
   DeviceBasis db;
   double *Xt = nullptr, *Yt = nullptr, *Zbar = nullptr;
   double *scratch = nullptr;
-  double2 *c122 = nullptr;
   double *obpart = nullptr;  // one-body partial sums (nobpart)
   double *diag = nullptr;    // inverse-Pandya diagonal terms (ndiag)
   double *panel = nullptr;   // bf16x3 operand panels of the mixed pp/hh GEMM (allocated on first use)
@@ -172,9 +169,9 @@ struct imsrg_ctx {
   std::string err;
   bool profiling = false;
   // phase events of profiled commutators: a ring of sets recorded without host
-  // synchronisation, read (and summed) by imsrg_hip_phase_times; marks 0..8 on
-  // the main stream, 9, 10, 11 around the pp/hh GEMM and comm122 on the side stream
-  static constexpr int kRing = 32, kMarks = 12;
+  // synchronisation, read (and summed) by imsrg_hip_phase_times; marks 0..6 on
+  // the main stream, 7, 8, 9 around the pp/hh GEMM and comm122 on the side stream
+  static constexpr int kRing = 32, kMarks = 10;
   std::vector<std::array<hipEvent_t, kMarks>> ring;
   int ring_head = 0, ring_count = 0;
   bool ring_side[kRing] = {};  // set recorded with the pp/hh GEMM on the side stream
@@ -273,7 +270,6 @@ static int ctx_init(imsrg_ctx *ctx, const imsrg_basis_desc *b, int device) {
   // cross-coupled channels without ph kets are never written and must read as 0
   HIPCHK(ctx, hipMemset(ctx->Zbar, 0, sizeof(double) * std::max<long>(B.zsize, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->scratch, sizeof(double) * (B.nch + 8)));
-  HIPCHK(ctx, hipMalloc(&ctx->c122, sizeof(double2) * std::max<long>(B.n122, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->obpart, sizeof(double) * std::max(B.nobpart, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->diag, sizeof(double) * std::max(B.ndiag, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->c122w, sizeof(double) * (B.tbsize + 8)));
@@ -331,7 +327,6 @@ extern "C" int imsrg_hip_ctx_destroy(imsrg_ctx *ctx) {
   if (ctx->Yt) (void)hipFree(ctx->Yt);
   if (ctx->Zbar) (void)hipFree(ctx->Zbar);
   if (ctx->scratch) (void)hipFree(ctx->scratch);
-  if (ctx->c122) (void)hipFree(ctx->c122);
   if (ctx->obpart) (void)hipFree(ctx->obpart);
   if (ctx->diag) (void)hipFree(ctx->diag);
   if (ctx->panel) (void)hipFree(ctx->panel);
@@ -1282,16 +1277,16 @@ static int herm_rule(int hx, int hy) { return (hx == hy) ? -1 : 1; }  // src/Com
 // Sums the phase durations of the oldest recorded event set (waits for it).
 static int harvest_oldest(imsrg_ctx *ctx) {
   auto &set = ctx->ring[ctx->ring_head];
-  HIPCHK(ctx, hipEventSynchronize(set[8]));
-  // sequence order of the phases: zero-body, one-body, pp/hh, 122 coefficients,
-  // Pandya, ph GEMM, inverse Pandya, last kernel; reported in the header's order
-  const int map[8] = {0, 1, 3, 2, 4, 5, 6, 7};
-  for (int i = 0; i < 8; ++i) {
+  HIPCHK(ctx, hipEventSynchronize(set[6]));
+  // marks on the main stream: pp/hh, comm122, first launch (Pandya, zero- and
+  // one-body), ph GEMM, inverse Pandya, last launch; reported in the header's order
+  const int map[6] = {3, 2, 4, 5, 6, 7};
+  for (int i = 0; i < 6; ++i) {
     float ms = 0.f;
-    if (i == 2 && ctx->ring_side[ctx->ring_head])
-      HIPCHK(ctx, hipEventElapsedTime(&ms, set[9], set[10]));
-    else if (i == 3 && ctx->ring_side[ctx->ring_head])  // comm122 on the side stream
-      HIPCHK(ctx, hipEventElapsedTime(&ms, set[10], set[11]));
+    if (i == 0 && ctx->ring_side[ctx->ring_head])
+      HIPCHK(ctx, hipEventElapsedTime(&ms, set[7], set[8]));
+    else if (i == 1 && ctx->ring_side[ctx->ring_head])  // comm122 on the side stream
+      HIPCHK(ctx, hipEventElapsedTime(&ms, set[8], set[9]));
     else
       HIPCHK(ctx, hipEventElapsedTime(&ms, set[i], set[i + 1]));
     ctx->phase_sum[map[i]] += ms * 1000.0;
@@ -1312,16 +1307,16 @@ static bool uses_panels(const imsrg_ctx *ctx, int prec) {
 }
 
 static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const int4 *const *items, const int *cnt,
-                          unsigned mask, int prec, int maxn, int maxnch, long maxn122, int maxjmax, int maxnorb,
+                          unsigned mask, int prec, int maxn, int maxnch, int maxjmax, int maxnorb,
                           int maxn1pairs, int maxncls, int maxbin, int maxent) {
   const Tuning &tu = ctx->db.tune;
   // split products take both GEMM families whatever the mixed-precision choices
   const int prec_pphh = gemm_family(prec, tu.mixed_pphh);
   const int prec_ph = gemm_family(prec, tu.mixed_ph);
   hipStream_t s = ctx->stream;
-  // With overlap, the pp/hh GEMM and then comm122's coefficients and W run on
-  // the side stream next to the zero-body, one-body, Pandya, ph GEMM and
-  // inverse Pandya kernels (none of them touches the upper triangle of Z's
+  // With overlap, the pp/hh GEMM and then comm122's W run on the side stream
+  // next to the first launch (zero-body, one-body, Pandya), the ph GEMM and the
+  // inverse Pandya kernel (none of them touches the upper triangle of Z's
   // two-body blocks); the main stream waits for them before the last kernel,
   // which folds, applies W and mirrors.
   const bool overlap = tu.overlap_pphh && (mask & MPPHH);
@@ -1341,49 +1336,41 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   auto fork_side = [&]() -> int {
     HIPCHK(ctx, hipEventRecord(ctx->fork, s));
     HIPCHK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork, 0));
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
+    if (set) HIPCHK(ctx, hipEventRecord((*set)[7], ctx->side));
     HIPCHK(ctx, launch_pphh(pa, items[0], cnt[0], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, ctx->side));
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[10], ctx->side));
-    if (mask & M122) {
-      HIPCHK(ctx, launch_c122_coef(pa, npairs, maxn122, ctx->side));
-      HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, ctx->side));
-    }
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[11], ctx->side));
+    if (set) HIPCHK(ctx, hipEventRecord((*set)[8], ctx->side));
+    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, ctx->side));
+    if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, hipEventRecord(ctx->join, ctx->side));
     return IMSRG_OK;
   };
   if (overlap && !fork_late)
     if (int rc = fork_side()) return rc;
   HIPCHK(ctx, mark(0));
-  HIPCHK(ctx, launch_zerobody(pa, npairs, maxnch, s));
-  HIPCHK(ctx, mark(1));
-  HIPCHK(ctx, launch_onebody(pa, items[5], cnt[5], (mask & M221) ? items[2] : nullptr, (mask & M221) ? cnt[2] : 0,
-                             npairs, maxn1pairs, s));
-  HIPCHK(ctx, mark(2));
   if (overlap) {
   } else if (mask & MPPHH) {
     HIPCHK(ctx, launch_pphh(pa, items[0], cnt[0], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, s));
   } else {
     HIPCHK(ctx, launch_zero_two(pa, items[6], cnt[6], s));
   }
+  HIPCHK(ctx, mark(1));
+  if ((mask & M122) && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, s));
+  HIPCHK(ctx, mark(2));
+  const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
+  const FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
+                      mph ? cnt[3] : 0};
+  HIPCHK(ctx, launch_front(pa, fi, maxnch, s));
   HIPCHK(ctx, mark(3));
-  if ((mask & M122) && !overlap) {
-    HIPCHK(ctx, launch_c122_coef(pa, npairs, maxn122, s));
-    HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, s));
-  }
-  HIPCHK(ctx, mark(4));
-  if (mask & MPH) HIPCHK(ctx, launch_pandya(pa, items[3], cnt[3], maxnch, s));
-  HIPCHK(ctx, mark(5));
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));
   if (fork_late)
     if (int rc = fork_side()) return rc;
-  HIPCHK(ctx, mark(6));
+  HIPCHK(ctx, mark(4));
   if (mask & MPH)
     HIPCHK(ctx, launch_invpandya(pa, items[4], cnt[4], maxjmax, maxnorb, maxnch, maxncls, prec_ph == 1, s));
   if (overlap) HIPCHK(ctx, hipStreamWaitEvent(s, ctx->join, 0));
-  HIPCHK(ctx, mark(7));
-  HIPCHK(ctx, launch_finish(pa, items[6], cnt[6], (mask & MPH) != 0, (mask & M122) != 0, s));
-  HIPCHK(ctx, mark(8));
+  HIPCHK(ctx, mark(5));
+  HIPCHK(ctx, launch_finish(pa, items[6], cnt[6], (mask & MPH) != 0, (mask & M122) != 0, npairs, maxn1pairs, s));
+  HIPCHK(ctx, mark(6));
   if (set) ++ctx->ring_count;
   return IMSRG_OK;
 }
@@ -1392,13 +1379,12 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
 // (the layout of the batched path's per-pair workspaces).
 struct Workspace {
   double *Xt, *Yt, *Zbar, *scratch;
-  double2 *c122;
   double *obpart, *diag, *c122w, *panel;
 };
 // panels: room for the bf16x3 operand panels (last region, used by the mixed
 // pp/hh GEMM only)
 static long workspace_doubles(const BasisDev &B, bool panels) {
-  return 2 * r8(B.xsize + 8) + r8(B.zsize) + r8(B.nch + 8) + 2 * r8(B.n122) + r8(B.nobpart) + r8(B.ndiag) +
+  return 2 * r8(B.xsize + 8) + r8(B.zsize) + r8(B.nch + 8) + r8(B.nobpart) + r8(B.ndiag) +
          r8(B.tbsize + 8) + (panels ? r8(2 * B.pk_size) : 0) + 64;
 }
 static Workspace carve_workspace(const BasisDev &B, double *base) {
@@ -1408,8 +1394,7 @@ static Workspace carve_workspace(const BasisDev &B, double *base) {
   w.Yt = w.Xt + r8(B.xsize + 8);
   w.Zbar = w.Yt + r8(B.xsize + 8);
   w.scratch = w.Zbar + r8(B.zsize);
-  w.c122 = (double2 *)(w.scratch + r8(B.nch + 8));
-  w.obpart = (double *)(w.c122) + 2 * r8(B.n122);
+  w.obpart = w.scratch + r8(B.nch + 8);
   w.diag = w.obpart + r8(B.nobpart);
   w.c122w = w.diag + r8(B.ndiag);
   w.panel = w.c122w + r8(B.tbsize + 8);
@@ -1439,7 +1424,6 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
   pa.p0.Yt = ws ? ws->Yt : ctx->Yt;
   pa.p0.Zbar = ws ? ws->Zbar : ctx->Zbar;
   pa.p0.scratch = ws ? ws->scratch : ctx->scratch;
-  pa.p0.c122 = ws ? ws->c122 : ctx->c122;
   pa.p0.obpart = ws ? ws->obpart : ctx->obpart;
   pa.p0.diag = ws ? ws->diag : ctx->diag;
   pa.p0.panel = ws ? ws->panel : ctx->panel;
@@ -1456,7 +1440,7 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
                  (int)db.wl.mirror.size(), (int)db.wl.pphh64.size(), (int)db.wl.pack.size(),
                  (int)db.wl.c122w.size()};
   if (!ctx->use_graphs || ctx->profiling || ws)
-    return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.n122, db.h.jmax,
+    return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
                           db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin, db.h.c122_maxent);
   // replay a captured launch sequence for this operand set, capturing it on first use
   for (const GraphEntry &g : ctx->graphs)
@@ -1466,7 +1450,7 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
       return IMSRG_OK;
     }
   HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-  const int rc = run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.n122, db.h.jmax,
+  const int rc = run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
                                 db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin, db.h.c122_maxent);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);  // always leave capture mode
@@ -2147,7 +2131,7 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       p.X = X[i]->buf; p.Y = Y[i]->buf; p.Z = Z[i]->buf;
       const Workspace w = carve_workspace(B, bc.work + woff[i]);
       p.Xt = w.Xt; p.Yt = w.Yt; p.Zbar = w.Zbar; p.scratch = w.scratch;
-      p.c122 = w.c122; p.obpart = w.obpart; p.diag = w.diag; p.panel = w.panel; p.c122w = w.c122w;
+      p.obpart = w.obpart; p.diag = w.diag; p.panel = w.panel; p.c122w = w.c122w;
       p.hX = X[i]->herm; p.hY = Y[i]->herm; p.hZ = herm_rule(X[i]->herm, Y[i]->herm);
       p.mask = mask;
     }
@@ -2191,7 +2175,6 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       bc.maxjmax = std::max(bc.maxjmax, ctxs[i]->db.h.jmax);
       bc.maxnorb = std::max(bc.maxnorb, ctxs[i]->db.h.norb);
       bc.maxn1pairs = std::max(bc.maxn1pairs, ctxs[i]->db.h.n1pairs);
-      bc.maxn122 = std::max(bc.maxn122, ctxs[i]->db.h.n122);
       bc.maxncls = std::max(bc.maxncls, ctxs[i]->db.h.ncls);
       bc.maxbin = std::max(bc.maxbin, ctxs[i]->db.h.c122_maxbin);
       bc.maxent = std::max(bc.maxent, ctxs[i]->db.h.c122_maxent);
@@ -2233,7 +2216,7 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
     HIPCHK(c0, hipEventRecord(c->batch_ev, c->stream));
     HIPCHK(c0, hipStreamWaitEvent(c0->stream, c->batch_ev, 0));
   }
-  rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxn122, bc.maxjmax,
+  rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxjmax,
                       bc.maxnorb, bc.maxn1pairs, bc.maxncls, bc.maxbin, bc.maxent);
   if (rc) return rc;
   if (!others.empty()) {

@@ -198,14 +198,17 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
           co[((size_t)i * (hb.jmax + 1) + J) * norb + x] = hb.cmap[(size_t)k * (hb.jmax + 1) + J];
         }
     B.ccorb = dupload(*this, co, err);
-    // kmorb: the same for the standard channels (kmap)
-    for (int i = 0; i < norb; ++i)
-      for (int J = 0; J <= hb.jmax; ++J)
-        for (int x = 0; x < norb; ++x) {
-          const int k = ket_index(norb, std::min(i, x), std::max(i, x));
-          co[((size_t)i * (hb.jmax + 1) + J) * norb + x] = hb.kmap[(size_t)k * (hb.jmax + 1) + J];
-        }
-    B.kmorb = dupload(*this, co, err);
+    // kmorb: standard local indices by orbit pair, J fastest (a channel holds fewer
+    // than 2^14.5 kets: its block is addressed with 32-bit byte offsets)
+    B.kmorb_nx = (hb.jmax + 1 + 7) / 8 * 8;
+    std::vector<unsigned short> km((size_t)norb * norb * B.kmorb_nx, 0xffff);
+    for (int x = 0; x < norb; ++x)
+      for (int y = 0; y < norb; ++y) {
+        const size_t k = (size_t)ket_index(norb, std::min(x, y), std::max(x, y)) * (hb.jmax + 1);
+        for (int J = 0; J <= hb.jmax; ++J)
+          km[((size_t)x * norb + y) * B.kmorb_nx + J] = (unsigned short)hb.kmap[k + J];
+      }
+    B.kmorb = dupload(*this, km, err);
   }
   // (parity, Tz) groups of kets
   std::vector<int> grp_start(7, 0), grp_kets;
@@ -314,18 +317,16 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   }
   for (size_t i = 0; i + 1 < c122_start.size(); ++i)  // kets without partners
     c122_start[i + 1] = std::max(c122_start[i + 1], c122_start[i]);
-  B.n122 = (long)c122_ind.size();
   // comm122 column bins.  The partners of ket (p, q) are kets (a, q) and (p, a)
   // with a in the one-body block of p or q, so the kets of one unordered pair
   // of one-body blocks form a group closed under partners.  Groups are packed
   // into bins of at most kC122Cols kets (first fit, largest first); the W
-  // kernel stages a bin's columns of X2 and Y2 in LDS, and c122_gpos gives each
-  // partner entry's position within its bin.
-  std::vector<int> c122_bcols, c122_boff(1, 0), c122_gpos(c122_ind.size(), 0);
-  // bin entries: c122_bent[c122_beoff[b] ..] the global entry indices of bin b,
-  // column by column; c122_bcend[c122_boff[b] + cp] the end of column cp's
-  // entries within the bin
-  std::vector<int> c122_bent, c122_beoff(1, 0), c122_bcend;
+  // kernel stages a bin's columns of X2 and Y2 in LDS.
+  std::vector<int> c122_bcols, c122_boff(1, 0);
+  std::vector<int4> c122_brec;
+  // bin entries: the records c122_brec[c122_beoff[b] ..] of bin b, column by column;
+  // c122_bcend[c122_boff[b] + cp] the end of column cp's entries within the bin
+  std::vector<int> c122_beoff(1, 0), c122_bcend;
   c122w_items.clear();
   int c122_maxbin = 1, c122_maxent = 4;
   {
@@ -357,17 +358,18 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       for (auto &bn : bins) c122_maxbin = std::max(c122_maxbin, (int)bn.size());
       for (auto &bn : bins) {
         for (size_t t = 0; t < bn.size(); ++t) pos[bn[t]] = (int)t;
-        const int ent0 = (int)c122_bent.size();
+        const int ent0 = (int)c122_brec.size();
         for (int q : bn) {
           c122_bcols.push_back(q);
           for (int e = c122_start[ch_kstart[c] + q]; e < c122_start[ch_kstart[c] + q + 1]; ++e) {
-            c122_gpos[e] = pos[c122_ind[e]];
-            c122_bent.push_back(e);
+            int f[2];
+            std::memcpy(f, &c122_f[e], sizeof(double));
+            c122_brec.push_back(make_int4(c122_ao[e].y * norb + c122_ao[e].x, pos[c122_ind[e]], f[0], f[1]));
           }
-          c122_bcend.push_back((int)c122_bent.size() - ent0);
+          c122_bcend.push_back((int)c122_brec.size() - ent0);
         }
-        c122_beoff.push_back((int)c122_bent.size());
-        c122_maxent = std::max(c122_maxent, (int)c122_bent.size() - ent0);
+        c122_beoff.push_back((int)c122_brec.size());
+        c122_maxent = std::max(c122_maxent, (int)c122_brec.size() - ent0);
         const int bi = (int)c122_boff.size() - 1;
         c122_boff.push_back((int)c122_bcols.size());
         for (int r = 0; r < n; r += kC122Rows) c122w_items.push_back(make_int4(0, c, bi, r / kC122Rows));
@@ -411,15 +413,12 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   B.kpp_w = dupload(*this, kpp_w, err);
   B.khh_start = dupload(*this, khh_start, err); B.khh_loc = dupload(*this, khh_loc, err);
   B.khh_w = dupload(*this, khh_w, err);
-  B.c122_start = dupload(*this, c122_start, err); B.c122_ind = dupload(*this, c122_ind, err);
   B.c122_bcols = dupload(*this, c122_bcols, err); B.c122_boff = dupload(*this, c122_boff, err);
-  B.c122_gpos = dupload(*this, c122_gpos, err);
-  B.c122_bent = dupload(*this, c122_bent, err);
+  B.c122_brec = dupload(*this, c122_brec, err);
   B.c122_beoff = dupload(*this, c122_beoff, err);
   B.c122_bcend = dupload(*this, c122_bcend, err);
   B.c122_maxbin = c122_maxbin;
   B.c122_maxent = c122_maxent;
-  B.c122_ao = dupload(*this, c122_ao, err); B.c122_f = dupload(*this, c122_f, err);
   B.gcore_start = dupload(*this, gcore_start, err); B.gcore_loc = dupload(*this, gcore_loc, err);
   B.gnc_start = dupload(*this, gnc_start, err); B.gnc_loc = dupload(*this, gnc_loc, err);
 
@@ -525,7 +524,8 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
     // so that a kJC-wide J chunk starting at the last pair stays inside the allocation
     long totq = (long)B.d1 * B.d1 * B.d1 * B.d1 * B.d2q * B.d2q + (long)(kJC / 2) * 2 * B.d1 * B.d1;
     void *p = nullptr, *pQ = nullptr;
-    if (hipMalloc(&p, tot * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
+    // 8 more: the Pandya kernel reads the J of one row in aligned groups of four pairs
+    if (hipMalloc(&p, (tot + 8) * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(p);
     if (hipMalloc(&pQ, totq * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(pQ);

@@ -59,7 +59,6 @@ struct BasisDev {
   long opsize;   // doubles per operator buffer (including 8 doubles of zero slack at the end)
   int maxn, maxcc, maxblk;
   int ccjmax_ph;  // largest J of a CC channel with ph kets (-1: none); Zbar is zero above it
-  long n122;           // comm122 partner entries (including the padding to multiples of kC122Blk per ket)
   const IMSRG_G int *j2, *l, *tz2, *cvq;
   const IMSRG_G double *occ;
   const IMSRG_G int *holes;
@@ -69,7 +68,10 @@ struct BasisDev {
   const IMSRG_G int *cmapT;     // cmapT[J*nkets + k] = cmap[k*(jmax+1) + J]
   const IMSRG_G int *kmapT;     // kmapT[J*nkets + k] = kmap[k*(jmax+1) + J]
   const IMSRG_G int *ccorb;     // ccorb[(i*(jmax+1) + J)*norb + x] = cmap of the ket (min(i,x), max(i,x)) at J
-  const IMSRG_G int *kmorb;     // kmorb: the same layout over kmap (standard channels)
+  // kmorb[(x*norb + y)*kmorb_nx + J]: standard local index of the ket of orbits x and y at J, 0xffff
+  // for none; kmorb_nx: jmax + 1 rounded up to a multiple of 8
+  const IMSRG_G unsigned short *kmorb;
+  int kmorb_nx;
   // kets of each (parity, Tz) group g = 2(Tz+1) + parity (the channels 6J + g),
   // ascending global index: grp_kets[grp_start[g] .. grp_start[g+1])
   const IMSRG_G int *grp_start, *grp_kets;
@@ -91,24 +93,17 @@ struct BasisDev {
   const IMSRG_G double *kpp_w;
   const IMSRG_G int *khh_start, *khh_loc;  // M_hh list (weights n_p n_q)
   const IMSRG_G double *khh_w;
-  // comm122 partner lists (CSR): the partners of local ket r of channel ch are
-  // the entries c122_start[ch_kstart[ch] + r] .. c122_start[ch_kstart[ch] + r + 1],
-  // a multiple of kC122Blk (padding: the first partner again with factor 0)
-  const IMSRG_G int *c122_start;
-  const IMSRG_G int *c122_ind;     // local ket index ind2 of the partner
-  const IMSRG_G int2 *c122_ao;     // (a, o): coefficient X1(a, o) * f
-  const IMSRG_G double *c122_f;    // phase / sqrt2 factors, times 2 for kets with p == q
   // comm122 column bins (kets of whole one-body block pairs, closed under
   // partners): bin b holds the channel-local kets c122_bcols[c122_boff[b] ..
-  // c122_boff[b + 1]); c122_gpos[e] is the position of entry e's partner in
-  // its column's bin
+  // c122_boff[b + 1]).  The partner entries of its columns, one after another, each
+  // column's a multiple of kC122Blk (padding: factor 0), are the records
+  // c122_brec[c122_beoff[b] ..] = (index a + o norb of the one-body element,
+  // position of the partner in the bin, the factor f -- phase / sqrt2 factors, times
+  // 2 for kets with p == q -- as low and high word); column cp's entries end at
+  // c122_bcend[c122_boff[b] + cp] within the bin
   const IMSRG_G int *c122_bcols;
   const IMSRG_G int *c122_boff;
-  const IMSRG_G int *c122_gpos;
-  // the bin's partner entries, column by column: global entry indices
-  // c122_bent[c122_beoff[b] ..]; column cp's entries end at c122_bcend[c122_boff[b] + cp]
-  // within the bin
-  const IMSRG_G int *c122_bent;
+  const IMSRG_G int4 *c122_brec;
   const IMSRG_G int *c122_beoff;
   const IMSRG_G int *c122_bcend;
   int c122_maxbin;                 // kets of the largest bin
@@ -163,7 +158,6 @@ struct PairPtrs {
   IMSRG_G double *Z;
   IMSRG_G double *Xt, *Yt, *Zbar; // Pandya workspaces
   IMSRG_G double *scratch;        // >= nch + 8 doubles (zero-body partial sums)
-  IMSRG_G double2 *c122;          // per-call comm122 coefficients (X1(a,o) f, Y1(a,o) f), n122 entries
   IMSRG_G double *obpart;         // per-call one-body partial sums, nobpart entries
   IMSRG_G double *diag;           // per-call inverse-Pandya diagonal terms, one per ket of every channel (ndiag)
   IMSRG_G double *panel;          // per-call bf16x3 panels of the mixed pp/hh GEMM (2 pk_size doubles)

@@ -52,16 +52,6 @@ __device__ __forceinline__ double tbme_norm(const BasisDev &B, const double *two
   return ph * two[B.ch_off[ch] + (long)k * B.ch_n[ch] + i];
 }
 
-// TwoBodyME::GetTBMEmonopole for a scalar operator (src/TwoBodyME.cc:615-682)
-__device__ double tbme_monopole(const BasisDev &B, const double *two, int a, int b, int c, int d) {
-  double nrm = (a == b ? SQRT2_D : 1.0) * (c == d ? SQRT2_D : 1.0);
-  int jmin = abs(B.j2[a] - B.j2[b]) / 2, jmax = (B.j2[a] + B.j2[b]) / 2;
-  double mon = 0.0;
-  for (int J = jmin; J <= jmax; ++J) mon += (2 * J + 1) * tbme_norm(B, two, J, a, b, c, d);
-  mon /= (B.j2[a] + 1) * (B.j2[b] + 1);
-  return nrm * mon;
-}
-
 template <int NV>
 __device__ __forceinline__ void block_reduce(double (&v)[NV]) {
   __shared__ double red[NV][4];
@@ -82,14 +72,12 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV]) {
 
 // ---------------------------------------------------------------------------
 // comm110ss (src/Commutator.cc:564-581) and comm220ss (601-631) -> Z0.
-// Grid (nch + 1, npairs): block 0 clears Z's one-body block and forms the
-// comm110 sum, block 1+ch the comm220 contribution of channel ch; partial
-// sums go to scratch and k_zerobody_final adds them in channel order.
-__global__ __launch_bounds__(256) void k_zerobody(PairArg pa) {
-  PairPtrs P = pa.get(blockIdx.y);
+// Block 0 of a pair clears Z's one-body block and forms the comm110 sum, block
+// 1+ch the comm220 contribution of channel ch; partial sums go to scratch and
+// final_zero adds them in channel order.
+__device__ __forceinline__ void front_zero(const PairPtrs &P, int bid) {
   const BasisDev &B = *P.basis;
   const int norb = B.norb;
-  const int bid = blockIdx.x;
   if (bid > B.nch) return;
   double acc[1] = {0.0};
   const bool skip = (P.hX == P.hY);
@@ -126,38 +114,20 @@ __global__ __launch_bounds__(256) void k_zerobody(PairArg pa) {
   if (threadIdx.x == 0) P.scratch[bid] = acc[0];
 }
 
-__global__ void k_zerobody_final(PairArg pa) {
-  PairPtrs P = pa.get(blockIdx.x);
-  if (threadIdx.x != 0) return;
-  const BasisDev &B = *P.basis;
-  const int nch = B.nch;
+// Z0 from the partial sums: one work-group per pair, the channels' sums staged in
+// LDS (`buf`, nbuf doubles) and added in channel order by one thread.
+__device__ __forceinline__ void final_zero(const PairPtrs &P, double *buf, int nbuf) {
+  const int nch = P.basis->nch;
   double s220 = 0.0;
-  // the channels' partial sums added in channel order (the order fixes the
-  // result), loaded in groups of 16 issued before the group's adds: one thread
-  // waiting on each load in turn took 30 us at emax=10
-  for (int c0 = 0; c0 < nch; c0 += 16) {
-    double v[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = P.scratch[1 + min(c0 + u, nch - 1)];
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if (c0 + u < nch) s220 += v[u];
+  for (int c0 = 0; c0 < nch; c0 += nbuf) {
+    const int m = min(nbuf, nch - c0);
+    for (int c = threadIdx.x; c < m; c += blockDim.x) buf[c] = P.scratch[1 + c0 + c];
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int c = 0; c < m; ++c) s220 += buf[c];
+    __syncthreads();
   }
-  P.Z[0] = (0.0 + P.scratch[0]) + s220;
-}
-
-// comm122 coefficients of this call: x = X1(a,o) f, y = Y1(a,o) f for every
-// partner entry (src/Commutator.cc:857-896).
-__global__ __launch_bounds__(256) void k_c122_coef(PairArg pa, int npairs) {
-  PairPtrs P = pa.get(blockIdx.y);
-  const BasisDev &B = *P.basis;
-  const int norb = B.norb;
-  const double *X1 = P.X + B.one_off, *Y1 = P.Y + B.one_off;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < B.n122; e += (long)gridDim.x * blockDim.x) {
-    const int2 ao = B.c122_ao[e];
-    const double f = B.c122_f[e];
-    P.c122[e] = make_double2(X1at(X1, norb, ao.x, ao.y) * f, X1at(Y1, norb, ao.x, ao.y) * f);
-  }
+  if (threadIdx.x == 0) P.Z[0] = (0.0 + P.scratch[0]) + s220;
 }
 
 // ---------------------------------------------------------------------------
@@ -179,9 +149,7 @@ __device__ __forceinline__ double fold_dot(const double *xr, const double *xs, c
   return m1 + hZ * m2;
 }
 
-__global__ __launch_bounds__(256) void k_onebody(PairArg pa, const int4 *items) {
-  const int4 it = items[blockIdx.x];
-  PairPtrs P = pa.get(it.x);
+__device__ __forceinline__ void front_one(const PairPtrs &P, const int4 &it) {
   const BasisDev &B = *P.basis;
   const int norb = B.norb, i = it.y, j = it.z;
   const double *X1 = P.X + B.one_off, *Y1 = P.Y + B.one_off;
@@ -196,21 +164,28 @@ __global__ __launch_bounds__(256) void k_onebody(PairArg pa, const int4 *items) 
     }
   }
   if (P.mask & M121) {
-    // one task per (hole a, partner b, monopole term)
-    const int ntask = B.nholes * B.maxblk * 4;
+    // one task per (hole a, partner b, monopole term, J): the monopoles'
+    // (2J+1)-weighted elements spread over the lanes, so that a lane waits for one
+    // chain of index loads in place of one per J
+    const int nJ = B.j2[i] + 1;  // at most this many J couple an orbit with i
+    const int ntask = B.nholes * B.maxblk * 4 * nJ;
     for (int t = threadIdx.x; t < ntask; t += blockDim.x) {
-      const int term = t & 3, ib = (t >> 2) % B.maxblk, ia = (t >> 2) / B.maxblk;
+      const int dJ = t % nJ, u = t / nJ;
+      const int term = u & 3, ib = (u >> 2) % B.maxblk, ia = (u >> 2) / B.maxblk;
       const int a = B.holes[ia];
-      if (ib >= B.obstart[a + 1] - B.obstart[a]) continue;
-      const int b = B.oblist[B.obstart[a] + ib];
+      const int o0 = B.obstart[a];
+      if (ib >= B.obstart[a + 1] - o0) continue;
+      const int b = B.oblist[o0 + ib];  // j_b = j_a
       const double nanb = B.occ[a] * (1.0 - B.occ[b]);
       if (fabs(nanb) < 1e-6) continue;
-      double v;
-      if (term == 0) v = (B.j2[b] + 1) * nanb * X1at(X1, norb, a, b) * tbme_monopole(B, Y2, b, i, a, j);
-      else if (term == 1) v = -(B.j2[a] + 1) * nanb * X1at(X1, norb, b, a) * tbme_monopole(B, Y2, a, i, b, j);
-      else if (term == 2) v = -(B.j2[b] + 1) * nanb * X1at(Y1, norb, a, b) * tbme_monopole(B, X2, b, i, a, j);
-      else v = (B.j2[a] + 1) * nanb * X1at(Y1, norb, b, a) * tbme_monopole(B, X2, a, i, b, j);
-      acc[1] += v;
+      const int ja = B.j2[a], ji = B.j2[i], J = abs(ja - ji) / 2 + dJ;
+      if (J > (ja + ji) / 2) continue;
+      const int x = (term & 1) ? a : b, y = (term & 1) ? b : a;  // <x i | y j>
+      double v = (2 * J + 1) * tbme_norm(B, term < 2 ? Y2 : X2, J, x, i, y, j);
+      v *= (x == i ? SQRT2_D : 1.0) * (y == j ? SQRT2_D : 1.0);
+      v *= nanb * ((term & 1) ? X1at(term < 2 ? X1 : Y1, norb, b, a) : X1at(term < 2 ? X1 : Y1, norb, a, b));
+      // (2 j_a + 1) over the monopole's (2 j_a + 1)(2 j_i + 1)
+      acc[1] += ((term == 1 || term == 2) ? -v : v) / (ji + 1);
     }
   }
   block_reduce<3>(acc);
@@ -244,10 +219,8 @@ __device__ __forceinline__ double m221_part(const BasisDev &B, const double *X2,
 // comm221 one-body part in partial sums, one slot per item (it.w):
 //  kind 0 (n_c != 0): n_c M_pp for one (c, J), the block's lanes over the pp list;
 //  kind 1 (1 - n_c != 0): (1 - n_c) M_hh for 4 orbits c of the list cpart
-//  (one per wave), all J, the wave's lanes over the hh list.
-__global__ __launch_bounds__(256) void k_onebody221(PairArg pa, const int4 *items) {
-  const int4 it = items[blockIdx.x];
-  PairPtrs P = pa.get(it.x);
+//  (one per wave), the wave's lanes over J and the hh lists.
+__device__ __forceinline__ void front_221(const PairPtrs &P, const int4 &it) {
   const BasisDev &B = *P.basis;
   const int2 pr = B.pairs1[it.y];
   const int i = pr.x, j = pr.y;
@@ -264,7 +237,8 @@ __global__ __launch_bounds__(256) void k_onebody221(PairArg pa, const int4 *item
       const int Jmin = max(abs(B.j2[c] - B.j2[i]), abs(B.j2[c] - B.j2[j])) / 2;
       const int Jmax = (B.j2[c] + min(B.j2[i], B.j2[j])) / 2;
       double m = 0.0;
-      for (int J = Jmin; J <= Jmax; ++J) m += m221_part(B, X2, Y2, i, j, c, J, false, lane, 64, hZ);
+      // eight J at a time, eight lanes on each one's hh list (a few kets)
+      for (int J = Jmin + (lane >> 3); J <= Jmax; J += 8) m += m221_part(B, X2, Y2, i, j, c, J, false, lane & 7, 8, hZ);
       acc[0] = (1.0 - B.occ[c]) * m;
     }
   }
@@ -275,10 +249,9 @@ __global__ __launch_bounds__(256) void k_onebody221(PairArg pa, const int4 *item
 // Z1(i, j) = comm111 + comm121 + comm221 / (j_i + 1) from the partial sums of
 // one-body pair p, one wave per pair (lane-strided sums and a fixed shuffle
 // tree: the same order every call), and Z1(j, i) = hZ Z1(i, j).
-__global__ __launch_bounds__(256) void k_onebody_final(PairArg pa) {
-  PairPtrs P = pa.get(blockIdx.y);
+__device__ __forceinline__ void final_one(const PairPtrs &P, int blk) {
   const BasisDev &B = *P.basis;
-  const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int p = blk * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (p >= B.n1pairs) return;  // wave-uniform
   const int2 pr = B.pairs1[p];
   const int i = pr.x, j = pr.y, s0 = B.ob_start[p], s1 = B.ob_start[p + 1];
@@ -1338,19 +1311,23 @@ __global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big(PairArg pa, const in
 
 // ---------------------------------------------------------------------------
 // DoPandyaTransformation_SingleChannel_XandY (src/Commutator.cc:1392-1485):
-// Xbar (nk x 2nph) and Ybar^T (nk x 2nph), one element each per thread.
-__global__ __launch_bounds__(256) void k_pandya(PairArg pa, const int4 *items) {
-  extern __shared__ __align__(8) unsigned char lds_raw[];
-  const int4 it = items[blockIdx.x];
-  PairPtrs P = pa.get(it.x);
+// Xbar (nk x 2nph) and Ybar^T (nk x 2nph), one element each per thread,
+//   Xbar(cd; ab) = -(n_a - n_b) sum_J (2J+1) {ja jb J'; jc jd J} X^J_{cb,ad},
+// consecutive threads on consecutive kets cd.  X^J_{cb,ad} is read as hX times the
+// element at row (a,d) and column (c,b): for a hole a the rows (a,d) of consecutive d
+// are neighbours, where the columns are a whole column apart.  The local indices of
+// (c,b) and (a,d) come eight J at a time from 16-byte rows of kmorb, the 6j values two
+// J at a time.  Bound by the address processing of its gathers (texture addresser 79%
+// busy with one load per index and 6j value and the transposed elements): 182 us at
+// emax = 10 before.
+__device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, unsigned char *lds_raw) {
   const BasisDev &B = *P.basis;
   // channel offsets and sizes in LDS: the gather of each J then waits on one
   // LDS read instead of two dependent global loads
-  long *s_choff = (long *)lds_raw;
-  int *s_chn = (int *)(s_choff + B.nch);
+  int4 *s_ch = (int4 *)lds_raw;
   for (int c = threadIdx.x; c < B.nch; c += blockDim.x) {
-    s_choff[c] = B.ch_off[c];
-    s_chn[c] = B.ch_n[c];
+    const long off = B.ch_off[c];
+    s_ch[c] = make_int4((int)(off & 0xffffffff), (int)(off >> 32), B.ch_n[c], 0);
   }
   __syncthreads();
   const int cc = it.y;
@@ -1374,55 +1351,54 @@ __global__ __launch_bounds__(256) void k_pandya(PairArg pa, const int4 *items) {
     if (a == d) normf *= SQRT2_D;
     if (c == b) normf *= SQRT2_D;
     const int ja = B.j2[a], jb = B.j2[b], jc = B.j2[c], jd = B.j2[d];
-    int jmin = max(abs(ja - jd), abs(jc - jb)) / 2;
+    const int jmin = max(abs(ja - jd), abs(jc - jb)) / 2;
     const int jmax = min(ja + jd, jc + jb) / 2;
-    int dJ = 1;
-    if (a == d || c == b) {
-      dJ = 2;
-      jmin += jmin & 1;
-    }
+    const int even = a == d || c == b;  // pairs of equal orbits: even J only
     // index work common to X and Y (GetTBME_J_norm_twoOps, src/TwoBodyME.cc:368-409)
     const int pcb = (B.l[c] + B.l[b]) & 1, pad = (B.l[a] + B.l[d]) & 1;
-    const int tcb = (B.tz2[c] + B.tz2[b]) / 2;
-    const double hY = P.hY;
+    const int g = 2 * ((B.tz2[c] + B.tz2[b]) / 2 + 1) + pcb;
     if (pcb == pad) {
-      // two J per pass, every load of both issued before use; an invalid term
-      // reads a clamped in-bounds element and is weighted by 0.  Local indices of
-      // the kets (c,b) and (a,d) come from the per-orbit rows of b and a, where
-      // the lanes' consecutive c and d read neighbouring entries.
-      const IMSRG_G double *sixt = B.sixj;
-      const int nJ = B.jmax + 1, norb = B.norb;
-      const IMSRG_G int *kb1 = B.kmorb + (long)b * nJ * norb + c;
-      const IMSRG_G int *kb2 = B.kmorb + (long)a * nJ * norb + d;
-      for (int J0 = jmin; J0 <= jmax; J0 += 2 * dJ) {
-        double sj[2], xv[2], yv[2], wv2[2];
-        int i1[2], i2[2], ch[2];
+      const int norb = B.norb, nx = B.kmorb_nx;
+      const double *six = B.sixj + sixj_index(B.d1, B.d2, ja, jb, Jcc, jc, jd, 0);
+      const IMSRG_G uint4 *k1 = (const IMSRG_G uint4 *)B.kmorb + ((b * norb + c) * nx >> 3);
+      const IMSRG_G uint4 *k2 = (const IMSRG_G uint4 *)B.kmorb + ((a * norb + d) * nx >> 3);
+      // the swapped kets' phases (-1)^{(j1+j2)/2+1+J}: sign at J = 0 and whether J alternates
+      const int s0 = (c > b ? (jc + jb) / 2 + 1 : 0) + (a > d ? (ja + jd) / 2 + 1 : 0);
+      const int sj = (c > b) != (a > d);
+      for (int c8 = jmin & ~7; c8 <= jmax; c8 += 8) {
+        union {
+          uint4 v;
+          unsigned short s[8];
+        } i1, i2;
+        i1.v = k1[c8 >> 3];
+        i2.v = k2[c8 >> 3];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int J = min(J0 + u * dJ, jmax);
-          sj[u] = sixt[sixj_index(B.d1, B.d2, ja, jb, Jcc, jc, jd, J)];
-          i1[u] = kb1[J * norb];
-          i2[u] = kb2[J * norb];
-          ch[u] = 6 * J + 2 * (tcb + 1) + pcb;
-        }
+        for (int h = 0; h < 8; h += 4) {
+          if (c8 + h > jmax || c8 + h + 3 < jmin) continue;
+          typedef double d2s __attribute__((ext_vector_type(2), aligned(8)));
+          const d2s w01 = *(const IMSRG_G d2s *)(six + c8 + h), w23 = *(const IMSRG_G d2s *)(six + c8 + h + 2);
+          double xv[4], yv[4], wv[4];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int J = J0 + u * dJ;
-          const bool ok = J <= jmax && fabs(sj[u]) >= 1e-8 && i1[u] >= 0 && i2[u] >= 0;
-          double ph = 1.0;
-          if (c > b) ph *= sgn_parity((jc + jb) / 2 + 1 + J);
-          if (a > d) ph *= sgn_parity((ja + jd) / 2 + 1 + J);
-          const long idx = s_choff[ch[u]] + (long)max(i2[u], 0) * s_chn[ch[u]] + max(i1[u], 0);
-          xv[u] = X2[idx];
-          yv[u] = Y2[idx];
-          wv2[u] = ok ? (2 * J + 1) * sj[u] * ph : 0.0;
-        }
+          for (int u = 0; u < 4; ++u) {
+            const int J = c8 + h + u;
+            const unsigned r = i2.s[h + u], cl = i1.s[h + u];  // 0xffff: no such ket
+            const double w = u == 0 ? w01.x : u == 1 ? w01.y : u == 2 ? w23.x : w23.y;
+            const bool ok = J >= jmin && J <= jmax && !(even & J) && fabs(w) >= 1e-8 && r != 0xffff && cl != 0xffff;
+            wv[u] = ok ? (2 * J + 1) * w * sgn_parity(s0 + sj * J) : 0.0;
+            // an invalid term reads the operator's first element and is weighted by 0
+            const int4 ch = s_ch[ok ? 6 * J + g : 0];
+            const long idx = ok ? (((long)ch.y << 32) | (unsigned)ch.x) + (long)(cl * ch.z + r) : 0;
+            xv[u] = X2[idx];
+            yv[u] = Y2[idx];
+          }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          xbar -= wv2[u] * xv[u];
-          ybar -= wv2[u] * yv[u] * hY;
+          for (int u = 0; u < 4; ++u) {
+            xbar -= wv[u] * xv[u];
+            ybar -= wv[u] * yv[u];
+          }
         }
       }
+      xbar *= P.hX;  // X(cb, ad) = hX X(ad, cb); Ybar^T holds hY Y(cb, ad) = Y(ad, cb)
     }
   }
   const long o = B.cc_xoff[cc] + (long)mp * nk + ik;
@@ -1430,6 +1406,33 @@ __global__ __launch_bounds__(256) void k_pandya(PairArg pa, const int4 *items) {
   P.Yt[o] = ybar * normf;
 }
 
+// First launch of a commutator: the kernels that read only X and Y and write
+// scratch, Z1 or Xbar / Ybar, side by side in one grid (work-group ranges in this
+// order): zero-body channels, one-body pairs, comm221 partial sums, Pandya chunks.
+// Launched one after another they are a chain of four launches of mostly latency
+// before the ph GEMM can start (emax = 6: 6 + 18 + 15 + 15 us and the gaps).
+__global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  int b = blockIdx.x;
+  if (b < f.nzeros) {
+    front_zero(pa.get(b / f.nzero), b % f.nzero);
+    return;
+  }
+  b -= f.nzeros;
+  if (b < f.none) {
+    const int4 it = f.one[b];
+    front_one(pa.get(it.x), it);
+    return;
+  }
+  b -= f.none;
+  if (b < f.n221) {
+    const int4 it = f.ob221[b];
+    front_221(pa.get(it.x), it);
+    return;
+  }
+  const int4 it = f.pandya[b - f.n221];
+  front_pandya(pa.get(it.x), it, lds_raw);
+}
 
 // wave-wide min / max of an int, returned as a wave-uniform (scalar) value
 __device__ __forceinline__ int wave_min(int v) {
@@ -1710,10 +1713,19 @@ __global__ __launch_bounds__(256, 5) void k_invpandya(PairArg pa, const int4 *it
   }
 }
 
+// The last launch's work-groups before its tile pairs: Z0 (block 0 of a pair) and Z1
+// (four one-body pairs each) from the partial sums of the first launch.
+__device__ __forceinline__ void finals(const PairArg &pa, int b, int nfin, double *buf, int nbuf) {
+  const PairPtrs P = pa.get(b / nfin);
+  if (b % nfin == 0) final_zero(P, buf, nbuf);
+  else final_one(P, b % nfin - 1);
+}
+
 // Lower triangle <- hZ * upper triangle; anti-Hermitian diagonal <- 0.
-__global__ __launch_bounds__(256) void k_mirror(PairArg pa, const int4 *items) {
+__global__ __launch_bounds__(256) void k_mirror(PairArg pa, const int4 *items, int nfins, int nfin) {
   __shared__ double t[kTile][kTile + 1];
-  const int4 it = items[blockIdx.x];
+  if ((int)blockIdx.x < nfins) return finals(pa, blockIdx.x, nfin, &t[0][0], kTile * kTile);
+  const int4 it = items[blockIdx.x - nfins];
   if (it.y < 0) return;  // empty item (padding of an XCD run)
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
@@ -1750,8 +1762,9 @@ __device__ __forceinline__ const T &blk_at(const T *base, unsigned idx) {
 }
 
 // W of comm122ss (src/Commutator.cc:908-926) by column bins:
-//   W(r, q) = sum over the partner entries e of ket q of Y2(r, ind_e) x_e - X2(r, ind_e) y_e
-// (x_e, y_e from k_c122_coef).  Every partner of a bin's kets lies in the bin,
+//   W(r, q) = sum over the partner entries e of ket q of Y2(r, ind_e) x_e - X2(r, ind_e) y_e,
+//   x_e = X1(a,o) f, y_e = Y1(a,o) f for the entry's orbits and factor (857-896).
+// Every partner of a bin's kets lies in the bin,
 // so a work-group stages the bin's columns of X2 and Y2 for kC122Rows rows in
 // LDS (each column segment read once, coalesced), together with the bin's
 // partner entries (position in the bin, coefficients); each lane then forms W
@@ -1783,9 +1796,10 @@ __global__ __launch_bounds__(256) void k_c122_w(PairArg pa, const int4 *items, i
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned r = (unsigned)min(R0 + lane, n - 1);
   for (int t = threadIdx.x; t < ne; t += blockDim.x) {
-    const int e = B.c122_bent[eo + t];
-    sp[t] = B.c122_gpos[e];
-    sc[t] = P.c122[e];
+    const int4 rec = B.c122_brec[eo + t];
+    const double f = __hiloint2double(rec.w, rec.z);
+    sp[t] = rec.y;
+    sc[t] = make_double2(P.X[B.one_off + rec.x] * f, P.Y[B.one_off + rec.x] * f);
   }
   for (int t = threadIdx.x; t < nc; t += blockDim.x) se[t] = B.c122_bcend[b0 + t];
   // columns: up to 16 per wave and pass, every load issued before the LDS
@@ -1858,9 +1872,10 @@ __device__ __forceinline__ void blk_st2(double *base, unsigned idx, double2 v) {
 // Z2 then move 16 bytes per lane (address processing per instruction, not
 // bytes, bounds these accesses).
 template <bool FOLD, bool C122>
-__global__ __launch_bounds__(256, 4) void k_finish(PairArg pa, const int4 *items) {
+__global__ __launch_bounds__(256, 4) void k_finish(PairArg pa, const int4 *items, int nfins, int nfin) {
   __shared__ double t[kTile][kTile + 1];  // t[rr][cc]: contribution to upper (R0 + rr, S0 + cc)
-  const int4 it = items[blockIdx.x];
+  if ((int)blockIdx.x < nfins) return finals(pa, blockIdx.x, nfin, &t[0][0], kTile * kTile);
+  const int4 it = items[blockIdx.x - nfins];
   if (it.y < 0) return;  // empty item (padding of an XCD run)
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
@@ -1963,18 +1978,26 @@ __global__ __launch_bounds__(256) void k_zero_two(PairArg pa, const int4 *items)
 }
 
 // ---------------------------------------------------------------------------
-hipError_t launch_zerobody(const PairArg &pa, int npairs, int maxnch, hipStream_t s) {
-  if (npairs <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zerobody, dim3(maxnch + 1, npairs), dim3(256), 0, s, pa);
-  hipLaunchKernelGGL(k_zerobody_final, dim3(npairs), dim3(64), 0, s, pa);
-  return hipGetLastError();
-}
-hipError_t launch_onebody(const PairArg &pa, const int4 *items, int nitems, const int4 *items221, int n221,
-                          int npairs, int maxn1pairs, hipStream_t s) {
-  if (nitems <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_onebody, dim3(nitems), dim3(256), 0, s, pa, items);
-  if (n221 > 0) hipLaunchKernelGGL(k_onebody221, dim3(n221), dim3(256), 0, s, pa, items221);
-  hipLaunchKernelGGL(k_onebody_final, dim3((maxn1pairs + 3) / 4, npairs), dim3(256), 0, s, pa);
+// Above this many Pandya chunks (about 7 residencies of the chip) they get a launch of
+// their own after the others: the one-body work-groups then run beside the pp/hh GEMM's
+// packing, and the chunks are not held up behind them (emax = 10 FP64 2.95 -> 2.91 ms,
+// mixed 2.18 -> 2.15 ms, emax = 12 mixed 10.36 -> 10.25 ms); below it one launch is
+// faster (emax = 8 mixed 492 -> 473 us, emax = 6 mixed 159 -> 146 us).
+constexpr int kFrontSplit = 12288;
+
+hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipStream_t s) {
+  const size_t lds = sizeof(int4) * (size_t)std::max(maxnch, 1);  // the Pandya chunks' channel table
+  FrontItems part[2] = {f, f};
+  if (f.npandya > kFrontSplit) {
+    part[0].npandya = 0;
+    part[1].nzeros = part[1].none = part[1].n221 = 0;
+  } else {
+    part[1].nzeros = part[1].none = part[1].n221 = part[1].npandya = 0;
+  }
+  for (const FrontItems &p : part) {
+    const int n = p.nzeros + p.none + p.n221 + p.npandya;
+    if (n > 0) hipLaunchKernelGGL(k_front, dim3(n), dim3(256), lds, s, pa, p);
+  }
   return hipGetLastError();
 }
 hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const int4 *items64, int nitems64,
@@ -2027,18 +2050,6 @@ hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int 
   }
   return hipGetLastError();
 }
-hipError_t launch_c122_coef(const PairArg &pa, int npairs, long maxn122, hipStream_t s) {
-  if (maxn122 <= 0) return hipSuccess;
-  int cb = (int)std::max<long>(1, std::min<long>((maxn122 + 255) / 256, 4096));
-  hipLaunchKernelGGL(k_c122_coef, dim3(cb, npairs), dim3(256), 0, s, pa, npairs);
-  return hipGetLastError();
-}
-hipError_t launch_pandya(const PairArg &pa, const int4 *items, int nitems, int maxnch, hipStream_t s) {
-  if (nitems <= 0) return hipSuccess;
-  const size_t lds = (sizeof(long) + sizeof(int)) * (size_t)std::max(maxnch, 1);
-  hipLaunchKernelGGL(k_pandya, dim3(nitems), dim3(kChunk), lds, s, pa, items);
-  return hipGetLastError();
-}
 hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, int jmax, int norb, int nch,
                             int ncls, bool zbar_f32, hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
@@ -2050,16 +2061,19 @@ hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, in
     hipLaunchKernelGGL(k_invpandya<double>, dim3(nitems), dim3(kChunk), lds, s, pa, items);
   return hipGetLastError();
 }
-hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, hipStream_t s) {
-  if (nitems <= 0) return hipSuccess;
+hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, int npairs,
+                         int maxn1pairs, hipStream_t s) {
+  const int nfin = 1 + (maxn1pairs + 3) / 4;  // work-groups of final_zero and final_one per pair
+  const int nfins = npairs * nfin;
+  const dim3 grid(nfins + nitems);
   if (fold && c122)
-    hipLaunchKernelGGL((k_finish<true, true>), dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL((k_finish<true, true>), grid, dim3(256), 0, s, pa, items, nfins, nfin);
   else if (fold)
-    hipLaunchKernelGGL((k_finish<true, false>), dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL((k_finish<true, false>), grid, dim3(256), 0, s, pa, items, nfins, nfin);
   else if (c122)
-    hipLaunchKernelGGL((k_finish<false, true>), dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL((k_finish<false, true>), grid, dim3(256), 0, s, pa, items, nfins, nfin);
   else
-    hipLaunchKernelGGL(k_mirror, dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL(k_mirror, grid, dim3(256), 0, s, pa, items, nfins, nfin);
   return hipGetLastError();
 }
 hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, int maxent, hipStream_t s) {

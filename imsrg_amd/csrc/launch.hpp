@@ -12,20 +12,19 @@ namespace imsrg {
 hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, int d2q, hipStream_t s);
 
 // commutator phases; items are device arrays of int4 work items
-hipError_t launch_zerobody(const PairArg &pa, int npairs, int maxnch, hipStream_t s);
-// one-body terms: comm111 + comm121 per pair (items), comm221 in partial sums
-// (items221, none when that term is off), then the sums into Z1
-hipError_t launch_onebody(const PairArg &pa, const int4 *items, int nitems, const int4 *items221, int n221,
-                          int npairs, int maxn1pairs, hipStream_t s);
+// first launch: zero-body channels (nzero work-groups per pair: the largest channel
+// count + 1; nzeros in all), one-body pairs (comm111 + comm121), comm221 partial sums
+// and Pandya chunks side by side; maxnch sizes the Pandya chunks' LDS channel table
+struct FrontItems {
+  const int4 *one, *ob221, *pandya;
+  int nzero, nzeros, none, n221, npandya;
+};
+hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipStream_t s);
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
 // under bf16x3 products (kGemmB3) the pack items first write the operand panels
 // maxn: the largest channel dimension of the pairs (sizes the kernel's LDS index list)
 hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const int4 *items64, int nitems64,
                        const int4 *pack, int npack, int precision, int maxn, hipStream_t s);
-// comm122 partner coefficients of this call (used by launch_finish with c122)
-hipError_t launch_c122_coef(const PairArg &pa, int npairs, long maxn122, hipStream_t s);
-// maxnch: the largest channel count of the pairs (sizes the kernel's LDS channel table)
-hipError_t launch_pandya(const PairArg &pa, const int4 *items, int nitems, int maxnch, hipStream_t s);
 // ph GEMM (head and tail of Zbar) on 128x128 tiles (big) or 64x64 tiles; precision 1
 // (FP32 products) stores Zbar in FP32, the others in FP64
 hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int precision, bool big, hipStream_t s);
@@ -33,12 +32,12 @@ hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int 
 // zbar_f32: Zbar holds FP32 elements (written by the precision-1 ph GEMM)
 hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, int jmax, int norb, int nch,
                             int ncls, bool zbar_f32, hipStream_t s);
-// last phase: with fold, upper += the inverse-Pandya contributions stored at the
+// last launch: with fold, upper += the inverse-Pandya contributions stored at the
 // transposed slots; with c122, Z2 -= W + hZ W^T (comm122ss); then lower triangle
-// <- hZ * upper
-hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, hipStream_t s);
-// comm122's W (two-body layout, P.c122w) from the partner coefficients of this
-// call, by column bins; before launch_finish with c122
+// <- hZ * upper; and Z0 and Z1 from the first launch's partial sums
+hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, int npairs,
+                         int maxn1pairs, hipStream_t s);
+// comm122's W (two-body layout, P.c122w) by column bins; before launch_finish with c122
 hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, int maxent, hipStream_t s);
 hipError_t launch_zero_two(const PairArg &pa, const int4 *items, int nitems, hipStream_t s);
 

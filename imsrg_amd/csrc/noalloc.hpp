@@ -12,7 +12,7 @@ namespace imsrg {
 int noalloc_setup(int device, std::string &err);
 
 // One commutator whose per-call workspaces (Pandya matrices, partial sums,
-// comm122 coefficients) are carved from `ws` (`cap` doubles) instead of the
+// comm122's W) are carved from `ws` (`cap` doubles) instead of the
 // context's own buffers.  Allocates nothing.
 // the device a context lives on; sets the context's error message and returns code
 int ctx_device(const imsrg_ctx *ctx);

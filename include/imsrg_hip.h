@@ -227,7 +227,7 @@ int imsrg_hip_commutator_ss_dev_async(imsrg_ctx *ctx, const imsrg_dop *X, const 
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops).  The same
  * commutator as imsrg_hip_commutator_ss_dev, with every per-call workspace
- * (Pandya matrices, partial sums, comm122 coefficients) carved from one static
+ * (Pandya matrices, partial sums, comm122's W) carved from one static
  * device array of 56 MiB per GPU, held from module load until the process
  * ends; the call allocates nothing.  Bases whose workspaces exceed it (above
  * emax = 6 for the O16 reference) return IMSRG_E_INVALID.  All calls on one
@@ -350,10 +350,10 @@ int imsrg_hip_set_tuning(imsrg_ctx *ctx, const imsrg_tuning *t);
 int imsrg_hip_autotune(imsrg_ctx *ctx, int precision, const char *cache_path, imsrg_tuning *out);
 
 /* Per-phase timing of commutators on ctx (microseconds, HIP events):
- * [0] zero-body, [1] one-body, [2] comm122 (coefficients, and with the pp/hh
- * overlap its upper-triangle pass), [3] pp/hh GEMM, [4] Pandya gather, [5] ph
- * GEMM, [6] inverse Pandya, [7] last kernel (fold of the inverse-Pandya terms,
- * comm122 when not overlapped, mirror).  Enabled by imsrg_hip_set_profiling:
+ * [2] comm122's W, [3] pp/hh GEMM, [4] first launch (Pandya gather with the
+ * zero- and one-body terms beside it), [5] ph GEMM, [6] inverse Pandya, [7] last
+ * launch (fold of the inverse-Pandya terms, comm122, mirror, the sums of the
+ * zero- and one-body parts); [0] and [1], once the zero- and one-body launches, are 0.  Enabled by imsrg_hip_set_profiling:
  * each commutator records HIP events on the stream its phases run on (the
  * pp/hh GEMM's own stream when it overlaps the others) without a host
  * synchronisation; imsrg_hip_phase_times returns the average over the
