@@ -745,6 +745,25 @@ hipError_t launch_white(const BasisDev *bd, const BasisDev &bh, const double *H,
 }
 
 // ---------------------------------------------------------------------------
+// Whether two streams run at the same time: k_meet_wait on one stream waits at most
+// `ticks` of the 100 MHz clock for the flag that k_meet_set raises on the other, and
+// reports in met[1] whether it saw it.
+__global__ void k_meet_wait(int *met, long long ticks) {
+  const long long t0 = wall_clock64();
+  int seen = 0;
+  do {
+    seen = __hip_atomic_load(met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } while (!seen && wall_clock64() - t0 < ticks);
+  met[1] = seen;
+}
+__global__ void k_meet_set(int *met) { __hip_atomic_store(met, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+hipError_t launch_meet(int *met, long long ticks, hipStream_t waiter, hipStream_t setter) {
+  hipLaunchKernelGGL(k_meet_wait, dim3(1), dim3(1), 0, waiter, met, ticks);
+  hipLaunchKernelGGL(k_meet_set, dim3(1), dim3(1), 0, setter, met);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 typedef double dbl4u __attribute__((ext_vector_type(4)));
 // One wave: out[0..255] = D with A-operand = lane id, B-operand = 1;
 //           out[256..511] = D with A-operand = 1, B-operand = lane id.

@@ -75,6 +75,10 @@ hipError_t launch_fill_random(const BasisDev *bd, const BasisDev &bh, double *op
 hipError_t launch_white(const BasisDev *bd, const BasisDev &bh, const double *H, double *Eta, const int4 *gen_items,
                         int ngen, hipStream_t s);
 
+// met[1] = whether work on `setter` ran while `waiter` was busy (met[0] = 0 beforehand;
+// waits at most `ticks` of the 100 MHz clock)
+hipError_t launch_meet(int *met, long long ticks, hipStream_t waiter, hipStream_t setter);
+
 // self-test of the MFMA f64 and f32 lane layouts: out[1024] (see imsrg_hip_selftest_mfma)
 hipError_t launch_mfma_probe(double *out, hipStream_t s);
 // one v_mfma_f32_16x16x32_bf16 on host-given operand slots (a, b: 512 floats, d: 256)
