@@ -500,14 +500,14 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
 // double-buffered in LDS and filled by direct global->LDS copies issued one
 // stage ahead.
 //   D(r,s) = alpha * cph(s) * sum_k w_k [ A(r,ka_k) B(s,kb_k) + h B(r,kb_k) A(s,ka_k) ],  r <= s
-// MODE 0: pp/hh term of comm222_pp_hh_221ss (src/Commutator.cc:1171-1194, 1237-1238):
+// PH false: pp/hh term of comm222_pp_hh_221ss (src/Commutator.cc:1171-1194, 1237-1238):
 //         A = X2, B = Y2 of one channel, k over pp/hh kets with weight w_pp - w_hh,
 //         alpha = hY, h = hZ; the upper triangle of Z2 is written.
-// MODE 1: head of Zbar in comm222_phss (src/Commutator.cc:1789-1799): A = Xbar,
+// PH true, head of Zbar in comm222_phss (src/Commutator.cc:1789-1799): A = Xbar,
 //         B = Ybar^T, h = +1 (Z Hermitian) or -1.
-// MODE 2: tail of Zbar (src/Commutator.cc:1788-1789, 1805): B columns permuted
+// PH true, tail of Zbar (src/Commutator.cc:1788-1789, 1805): B columns permuted
 //         by ab <-> ba with weights hY*phi(ph ket), cph(s) = phi(s), h = +1.
-// MODE 1/2 store Zbar in full: the lower triangle as (head) hZ-sign or (tail)
+// The ph GEMM stores Zbar in full: the lower triangle as (head) hZ-sign or (tail)
 // phi_r phi_s times the upper element, as the reference's folds make it
 // (src/Commutator.cc:1792-1805), written through an LDS transpose.
 // MIXED: operands rounded to FP32 when read from LDS, products on f32
@@ -550,20 +550,20 @@ __device__ __forceinline__ bool tile_wave_live(int R0, int S0, int n, int w) {
 
 // Stores a 128x128 tile from the waves' FP64 accumulators (lane layout of the
 // f32 MFMAs when F32L, else of the f64 16x16x4 MFMA).
-// MODE 0: the upper triangle of D = alpha * acc.
-// MODE 1/2: Zbar in full through LDS transposes of the 64 x kGW wave sub-tiles,
+// PH false: the upper triangle of D = alpha * acc.
+// PH true: Zbar in full through LDS transposes of the 64 x kGW wave sub-tiles,
 // four per round in the buffers tb0..tb3 (each >= 64 (kGW + 1) doubles): the
 // lower triangle as (head) h or (tail) phi_r phi_s times the upper element, as
 // the reference's folds make it (src/Commutator.cc:1792-1805); s_ph holds the
-// tile's row (0) and column (1) phases.
-template <int MODE, bool F32L, typename TD = double>
+// tile's row (0) and column (1) phases in the tail (h = 1) and 1 in the head.
+template <bool PH, bool F32L, typename TD = double>
 __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, int n, int R0, int S0,
                                               double alpha, double h, const signed char (*s_ph)[kTileB],
                                               double *tb0, double *tb1, double *tb2, double *tb3) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = (wv & 1) * 64, wc = (wv >> 1) * kGW;
   const bool wave_live = tile_wave_live(R0, S0, n, wv);
-  if constexpr (MODE == 0) {
+  if constexpr (!PH) {
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
@@ -590,12 +590,7 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const int rr = mi * 16 + (lane & 15), cc = ni * 16 + mfma_col<F32L>(lane, q);
-              double v = alpha * acc[mi][ni][q];
-              if (MODE == 2) {
-                const int col = S0 + wc + cc;
-                v *= (col < n) ? (double)s_ph[1][wc + cc] : 0.0;
-              }
-              Tt[rr][cc] = v;
+              Tt[rr][cc] = alpha * acc[mi][ni][q] * (double)s_ph[1][wc + cc];
             }
       }
       __syncthreads();
@@ -630,7 +625,7 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
             for (int q = 0; q < 4; ++q) {
               ok[q] = row2 + q < n && row2 + q > col2;
               // phases from LDS: row2 + q - S0 and col2 - R0 lie in [0, 128)
-              const double sq = (MODE == 1) ? h : (double)(s_ph[1][min(row2 + q - S0, kTileB - 1)] * s_ph[0][col2 - R0]);
+              const double sq = h * (double)(s_ph[1][min(row2 + q - S0, kTileB - 1)] * s_ph[0][col2 - R0]);
               v[q] = sq * Tt[rr][cc + q];
             }
             float *dp = D + (long)col2 * n + row2;
@@ -664,15 +659,15 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
             if (col2 >= n || row2 >= n) continue;
             const bool lo = row2 > col2, hi = row2 + 1 < n && row2 + 1 > col2;
             // phases from LDS: row2 - S0 and col2 - R0 lie in [0, 128)
-            const double s0 = (MODE == 1) ? h : (double)(s_ph[1][row2 - S0] * s_ph[0][col2 - R0]);
+            const double s0 = h * (double)(s_ph[1][row2 - S0] * s_ph[0][col2 - R0]);
             TD *dp = D + (long)col2 * n + row2;
             if (lo && hi) {
-              const double s1 = (MODE == 1) ? h : (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
+              const double s1 = h * (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
               st_nt2(dp, s0 * Tt[rr][cc], s1 * Tt[rr][cc + 1]);
             } else if (lo) {
               st_nt(dp, s0 * Tt[rr][cc]);
             } else if (hi) {
-              const double s1 = (MODE == 1) ? h : (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
+              const double s1 = h * (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
               st_nt(dp + 1, s1 * Tt[rr][cc + 1]);
             }
           }
@@ -683,8 +678,20 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
   }
 }
 
-template <int MODE, bool MIXED, bool SPLIT = false>
-__device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
+// The work-group's tile of a ph item list whose items are each done twice, head and
+// tail, in one launch: runs of 8 work-groups (one per XCD) alternate between the two
+// halves, so that an item's halves, which read the same panels, run close together on
+// one XCD.  Small bases have fewer tiles than CUs and each tile is a chain of k-stages,
+// so two launches one after the other took twice as long (emax = 5 FP32 53 -> 30 us,
+// emax = 7 FP64 85 -> 61 us); emax = 10 517 -> 472 us FP64, 390 -> 357 us FP32.
+__device__ __forceinline__ int4 ph_item(const int4 *items, int nitems, bool &tail) {
+  const int i = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  tail = (blockIdx.x >> 3) & 1;
+  return i < nitems ? items[i] : make_int4(0, -1, 0, 0);
+}
+
+template <bool PH, bool MIXED, bool SPLIT = false>
+__device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items, int nitems) {
   static_assert(MIXED || !SPLIT, "split products are a mixed-precision mode");
   constexpr int T = kTileB, LD = kTileB + 4;
   // operands stay FP64 in LDS (they arrive by direct global->LDS copies); the
@@ -696,7 +703,8 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
   __shared__ __align__(16) double A0[kTileK][LD], A1[kTileK][LD];
   __shared__ __align__(16) double B0[kTileK][LD], B1[kTileK][LD];
   __shared__ double W0[kTileK], W1[kTileK];
-  const int4 it = items[blockIdx.x];
+  bool tail = false;
+  const int4 it = PH ? ph_item(items, nitems, tail) : items[blockIdx.x];
   if (it.y < 0) return;  // padding item of the XCD-balanced order
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
@@ -707,9 +715,9 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
   const signed char *phi = nullptr, *phph = nullptr;
   double alpha, h;
   // Zbar in FP32 from the FP32-product ph GEMM, in FP64 otherwise
-  using ZT = typename std::conditional<MODE != 0 && MIXED && !SPLIT, float, double>::type;
+  using ZT = typename std::conditional<PH && MIXED && !SPLIT, float, double>::type;
   ZT *D;
-  if constexpr (MODE == 0) {
+  if constexpr (!PH) {
     const int ch = it.y;
     n = B.ch_n[ch];
     const long off = B.ch_off[ch];
@@ -730,21 +738,21 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
     const long xo = B.cc_xoff[cc];
     Am = P.Xt + xo;
     Bm = P.Yt + xo;
-    D = reinterpret_cast<ZT *>(P.Zbar) + B.cc_zoff[cc] + (MODE == 2 ? (long)n * n : 0);
+    D = reinterpret_cast<ZT *>(P.Zbar) + B.cc_zoff[cc] + (tail ? (long)n * n : 0);
     alpha = 1.0;
-    h = (MODE == 1) ? (P.hZ == 1 ? 1.0 : -1.0) : 1.0;
+    h = tail || P.hZ == 1 ? 1.0 : -1.0;
     phi = B.cc_phi + B.cc_kstart[cc];
     phph = B.cc_phph + B.cc_phstart[cc];
   }
   const int R0 = it.z * T, S0 = it.w * T;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // MODE 2: the phases of the tile's 128 rows and 128 columns, staged once for
-  // the epilogue (the prologue's barrier below publishes them)
+  // ph: the phases of the tile's 128 rows and 128 columns (tail; 1 in the head), staged
+  // once for the epilogue (the prologue's barrier below publishes them)
   __shared__ signed char s_ph[2][T];
-  if constexpr (MODE == 2) {
+  if constexpr (PH) {
     if (threadIdx.x < 2 * T) {
       const int sd = threadIdx.x / T, e = threadIdx.x - sd * T;
-      s_ph[sd][e] = phi[min((sd ? S0 : R0) + e, n - 1)];
+      s_ph[sd][e] = tail ? phi[min((sd ? S0 : R0) + e, n - 1)] : 1;
     }
   }
   // 8 waves, each a 64x32 sub-tile: rows wr .. wr+63, columns wc .. wc+31
@@ -765,11 +773,11 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
   // at most one element past the column (inside the arena, or the buffer's
   // slack).  Column indices (wave-uniform) are loaded one stage ahead.
   const int ra = min(R0 + 2 * lane, n - 1), rb = min(S0 + 2 * lane, n - 1);
-  // MODE 0: the channel's column-index list kl[0..nk) is staged in LDS (dynamic
+  // pp/hh: the channel's column-index list kl[0..nk) is staged in LDS (dynamic
   // shared memory of at least nk ints), so index reads never wait behind the
   // global->LDS copies in flight
   extern __shared__ int KLs[];
-  if constexpr (MODE == 0) {
+  if constexpr (!PH) {
     for (int e = threadIdx.x; e < nk; e += blockDim.x) KLs[e] = kl[e];
     __syncthreads();
   }
@@ -778,7 +786,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
     for (int j = 0; j < kGC; ++j) {
       const int kk = min(k0 + wv * kGC + j, K2 - 1);
       const int k = kk < nk ? kk : kk - nk;
-      ki[j] = (MODE == 0) ? KLs[k] : k;
+      ki[j] = PH ? k : KLs[k];
     }
   };
   auto issue_stage = [&](int k0, const int (&ki)[kGC], double (&As)[kTileK][LD], double (&Bs)[kTileK][LD]) {
@@ -787,7 +795,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
       const int kq = wv * kGC + j;
       const int kk = min(k0 + kq, K2 - 1);
       const int ca = ki[j];
-      const int cb = (MODE == 2) ? (ca < nph ? ca + nph : ca - nph) : ca;
+      const int cb = tail ? (ca < nph ? ca + nph : ca - nph) : ca;
       const double *sa = kk < nk ? Am + (long)ca * n : Bm + (long)cb * n;
       const double *sb = kk < nk ? Bm + (long)cb * n : Am + (long)ca * n;
       __builtin_amdgcn_global_load_lds((const IMSRG_G void *)(sa + ra),
@@ -801,9 +809,9 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
   auto load_w = [&](int k0) -> double {
     const int kk = min(k0 + (int)(threadIdx.x & (kTileK - 1)), K2 - 1);
     const int k = kk < nk ? kk : kk - nk;
-    if constexpr (MODE == 0) return kw[k];
-    if constexpr (MODE == 1) return 1.0;
-    return (double)P.hY * (double)phph[k < nph ? k : k - nph];
+    if constexpr (!PH) return kw[k];
+    const double w = (double)P.hY * (double)phph[k < nph ? k : k - nph];
+    return tail ? w : 1.0;
   };
   auto store_w = [&](int k0, double (&Ws)[kTileK], double w) {
     if (threadIdx.x < kTileK) {
@@ -911,7 +919,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items) {
   }
   if constexpr (MIXED) flush_t();  // a last stage without its pair
   static_assert(64 * (kGW + 1) <= kTileK * LD, "transpose tile exceeds the operand buffer");
-  gemm_epilogue<MODE, MIXED, ZT>(acc, D, n, R0, S0, alpha, h, s_ph, &A0[0][0], &A1[0][0], &B0[0][0], &B1[0][0]);
+  gemm_epilogue<PH, MIXED, ZT>(acc, D, n, R0, S0, alpha, h, s_ph, &A0[0][0], &A1[0][0], &B0[0][0], &B1[0][0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -960,12 +968,12 @@ __device__ __forceinline__ void split3x2(double x0, double x1, b2v &p0, b2v &p1,
   p2 = __builtin_convertvector(r2, b2v);
 }
 
-template <int MODE>
-__device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items) {
+__device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items, int nitems) {
   constexpr int T = kTileB, KS = 32;
   __shared__ __align__(16) StageB3 L0, L1;
-  const int4 it = items[blockIdx.x];
-  if (it.y < 0) return;  // padding item of the XCD-balanced order
+  bool tail;
+  const int4 it = ph_item(items, nitems, tail);
+  if (it.y < 0) return;
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
   int n, nk, nph = 0;
@@ -973,7 +981,6 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items) {
   const signed char *phi = nullptr, *phph = nullptr;
   double alpha, h;
   double *D;
-  static_assert(MODE == 1 || MODE == 2, "the ph GEMM's head (1) and tail (2); the pp/hh GEMM packs its panels");
   {
     const int cc = it.y;
     n = B.cc_n[cc];
@@ -982,20 +989,18 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items) {
     const long xo = B.cc_xoff[cc];
     Am = P.Xt + xo;
     Bm = P.Yt + xo;
-    D = P.Zbar + B.cc_zoff[cc] + (MODE == 2 ? (long)n * n : 0);
+    D = P.Zbar + B.cc_zoff[cc] + (tail ? (long)n * n : 0);
     alpha = 1.0;
-    h = (MODE == 1) ? (P.hZ == 1 ? 1.0 : -1.0) : 1.0;
+    h = tail || P.hZ == 1 ? 1.0 : -1.0;
     phi = B.cc_phi + B.cc_kstart[cc];
     phph = B.cc_phph + B.cc_phstart[cc];
   }
   const int R0 = it.z * T, S0 = it.w * T;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   __shared__ signed char s_ph[2][T];
-  if constexpr (MODE == 2) {
-    if (threadIdx.x < 2 * T) {
-      const int sd = threadIdx.x / T, e = threadIdx.x - sd * T;
-      s_ph[sd][e] = phi[min((sd ? S0 : R0) + e, n - 1)];
-    }
+  if (threadIdx.x < 2 * T) {
+    const int sd = threadIdx.x / T, e = threadIdx.x - sd * T;
+    s_ph[sd][e] = tail ? phi[min((sd ? S0 : R0) + e, n - 1)] : 1;
   }
   __syncthreads();  // s_ph
   const int K2 = 2 * nk;
@@ -1024,11 +1029,11 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       ca[j] = k[j];
-      wr[j] = (MODE == 1) ? 1.0 : (double)P.hY * (double)phph[k[j] < nph ? k[j] : k[j] - nph];
+      wr[j] = !tail ? 1.0 : (double)P.hY * (double)phph[k[j] < nph ? k[j] : k[j] - nph];
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int cb = (MODE == 2) ? (ca[j] < nph ? ca[j] + nph : ca[j] - nph) : ca[j];
+      const int cb = tail ? (ca[j] < nph ? ca[j] + nph : ca[j] - nph) : ca[j];
       // A side: A(., ca) for kk < nk, else B(., cb); B side the other one
       const bool first = kk[j] < nk;
       const double *src = (first != (opnd != 0)) ? Am + (long)ca[j] * n : Bm + (long)cb * n;
@@ -1125,7 +1130,7 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items) {
   }
   static_assert(2 * 64 * (kGW + 1) * sizeof(double) <= sizeof(StageB3), "transpose tiles exceed the stage buffer");
   double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<MODE, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<true, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
 }
 
 // ---------------------------------------------------------------------------
@@ -1287,26 +1292,25 @@ __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, co
     }
   }
   double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<0, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
 }
 
-template <int MODE>
-__global__ __launch_bounds__(kGWaves * 64, 2) void k_ph_big_b3(PairArg pa, const int4 *items) {
-  gemm_tile_b3<MODE>(pa, items);
+__global__ __launch_bounds__(kGWaves * 64, 2) void k_ph_big_b3(PairArg pa, const int4 *items, int nitems) {
+  gemm_tile_b3(pa, items, nitems);
 }
 
 __global__ __launch_bounds__(kGWaves * 64, 4) void k_pphh_big_f64(PairArg pa, const int4 *items) {
-  gemm_tile<0, false>(pa, items);
+  gemm_tile<false, false>(pa, items, 0);
 }
 __global__ __launch_bounds__(kGWaves * 64, 4) void k_pphh_big_mixed(PairArg pa, const int4 *items) {
-  gemm_tile<0, true>(pa, items);
+  gemm_tile<false, true>(pa, items, 0);
 }
 __global__ __launch_bounds__(kGWaves * 64, 4) void k_pphh_big_split(PairArg pa, const int4 *items) {
-  gemm_tile<0, true, true>(pa, items);
+  gemm_tile<false, true, true>(pa, items, 0);
 }
-template <int MODE, bool MIXED, bool SPLIT = false>
-__global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big(PairArg pa, const int4 *items) {
-  gemm_tile<MODE, MIXED, SPLIT>(pa, items);
+template <bool MIXED, bool SPLIT = false>
+__global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big(PairArg pa, const int4 *items, int nitems) {
+  gemm_tile<true, MIXED, SPLIT>(pa, items, nitems);
 }
 
 // ---------------------------------------------------------------------------
@@ -2026,19 +2030,15 @@ hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const i
 hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int precision, bool big, hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
   if (big) {
-    if (precision == kGemmB3) {
-      hipLaunchKernelGGL((k_ph_big_b3<1>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-      hipLaunchKernelGGL((k_ph_big_b3<2>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-    } else if (precision == 1) {
-      hipLaunchKernelGGL((k_ph_big<1, true>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-      hipLaunchKernelGGL((k_ph_big<2, true>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-    } else if (precision == 2) {
-      hipLaunchKernelGGL((k_ph_big<1, true, true>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-      hipLaunchKernelGGL((k_ph_big<2, true, true>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-    } else {
-      hipLaunchKernelGGL((k_ph_big<1, false>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-      hipLaunchKernelGGL((k_ph_big<2, false>), dim3(nitems), dim3(kGWaves * 64), 0, s, pa, items);
-    }
+    const dim3 grid((nitems + 7) / 8 * 16), blk(kGWaves * 64);  // head and tail of every item (ph_item)
+    if (precision == kGemmB3)
+      hipLaunchKernelGGL(k_ph_big_b3, grid, blk, 0, s, pa, items, nitems);
+    else if (precision == 1)
+      hipLaunchKernelGGL((k_ph_big<true>), grid, blk, 0, s, pa, items, nitems);
+    else if (precision == 2)
+      hipLaunchKernelGGL((k_ph_big<true, true>), grid, blk, 0, s, pa, items, nitems);
+    else
+      hipLaunchKernelGGL((k_ph_big<false>), grid, blk, 0, s, pa, items, nitems);
     return hipGetLastError();
   }
   if (precision == 1) {
