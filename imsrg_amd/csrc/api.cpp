@@ -2135,16 +2135,13 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
     if (Z[i] == X[i] || Z[i] == Y[i]) return fail(c0, IMSRG_E_INVALID, "Z aliases X or Y");
   }
   BatchCache &bc = c0->batch;
-  // The cached device table holds the operator buffers and each context's
-  // basis tables, so the key names those (and each context by its serial
-  // number, never reused), not the handle addresses a new object may take over.
+  // What is kept from one call to the next depends on the contexts and their work
+  // lists alone (each context by its serial number, never reused): workspaces, work
+  // lists and the table's pointers to basis and workspaces.  The operands of a call are
+  // written into the table by a kernel of the call.
   std::vector<long long> key;
   for (int i = 0; i < npairs; ++i) {
     key.push_back(ctxs[i]->serial);
-    key.push_back((long long)(intptr_t)X[i]->buf);
-    key.push_back((long long)(intptr_t)Y[i]->buf);
-    key.push_back((long long)(intptr_t)Z[i]->buf);
-    key.push_back(X[i]->herm * 4 + Y[i]->herm + 8 * (long long)mask);
     key.push_back(ctxs[i]->lists_gen);  // work lists rebuilt by a new tuning
   }
   if (key != bc.key) {
@@ -2158,17 +2155,14 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
     }
     HIPCHK(c0, hipMalloc(&bc.work, sizeof(double) * std::max<long>(wtot, 1)));
     HIPCHK(c0, hipMemset(bc.work, 0, sizeof(double) * std::max<long>(wtot, 1)));
-    std::vector<PairPtrs> tab(npairs);
+    std::vector<PairPtrs> tab(npairs, PairPtrs{});
     for (int i = 0; i < npairs; ++i) {
       const BasisDev &B = ctxs[i]->db.h;
       PairPtrs &p = tab[i];
       p.basis = ctxs[i]->db.d;
-      p.X = X[i]->buf; p.Y = Y[i]->buf; p.Z = Z[i]->buf;
       const Workspace w = carve_workspace(B, bc.work + woff[i]);
       p.Xt = w.Xt; p.Yt = w.Yt; p.Zbar = w.Zbar; p.scratch = w.scratch;
       p.obpart = w.obpart; p.diag = w.diag; p.panel = w.panel; p.c122w = w.c122w;
-      p.hX = X[i]->herm; p.hY = Y[i]->herm; p.hZ = herm_rule(X[i]->herm, Y[i]->herm);
-      p.mask = mask;
     }
     HIPCHK(c0, hipMalloc(&bc.d_tab, sizeof(PairPtrs) * npairs));
     HIPCHK(c0, hipMemcpy(bc.d_tab, tab.data(), sizeof(PairPtrs) * npairs, hipMemcpyHostToDevice));
@@ -2250,6 +2244,14 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
   for (imsrg_ctx *c : others) {
     HIPCHK(c0, hipEventRecord(c->batch_ev, c->stream));
     HIPCHK(c0, hipStreamWaitEvent(c0->stream, c->batch_ev, 0));
+  }
+  for (int i0 = 0; i0 < npairs; i0 += PairOps::kMax) {
+    PairOps ops;
+    ops.n = std::min(npairs - i0, PairOps::kMax);
+    for (int i = 0; i < ops.n; ++i)
+      ops.op[i] = {X[i0 + i]->buf, Y[i0 + i]->buf, Z[i0 + i]->buf, X[i0 + i]->herm, Y[i0 + i]->herm,
+                   Z[i0 + i]->herm, mask};
+    HIPCHK(c0, launch_set_pairs(bc.d_tab + i0, ops, c0->stream));
   }
   rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxjmax,
                       bc.maxnorb, bc.maxn1pairs, bc.maxncls, bc.maxbin, bc.maxent);

@@ -1982,6 +1982,24 @@ __global__ __launch_bounds__(256) void k_zero_two(PairArg pa, const int4 *items)
 }
 
 // ---------------------------------------------------------------------------
+__global__ __launch_bounds__(64) void k_set_pairs(PairPtrs *tab, PairOps ops) {
+  const int i = threadIdx.x;
+  if (i >= ops.n) return;
+  PairPtrs &p = tab[i];
+  p.X = (const IMSRG_G double *)ops.op[i].X;
+  p.Y = (const IMSRG_G double *)ops.op[i].Y;
+  p.Z = (IMSRG_G double *)ops.op[i].Z;
+  p.hX = ops.op[i].hX;
+  p.hY = ops.op[i].hY;
+  p.hZ = ops.op[i].hZ;
+  p.mask = ops.op[i].mask;
+}
+hipError_t launch_set_pairs(PairPtrs *tab, const PairOps &ops, hipStream_t s) {
+  static_assert(PairOps::kMax <= 64, "one thread per pair");
+  hipLaunchKernelGGL(k_set_pairs, dim3(1), dim3(64), 0, s, tab, ops);
+  return hipGetLastError();
+}
+
 // Above this many Pandya chunks (about 7 residencies of the chip) they get a launch of
 // their own after the others: the one-body work-groups then run beside the pp/hh GEMM's
 // packing, and the chunks are not held up behind them (emax = 10 FP64 2.95 -> 2.91 ms,

@@ -12,6 +12,20 @@ namespace imsrg {
 hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, int d2q, hipStream_t s);
 
 // commutator phases; items are device arrays of int4 work items
+// operands, Hermiticities and terms of up to kMax pairs of a batch, into its device
+// table (a kernel argument: nothing of the call stays in host memory)
+struct PairOps {
+  static constexpr int kMax = 64;
+  struct {
+    const double *X, *Y;
+    double *Z;
+    int hX, hY, hZ;
+    unsigned mask;
+  } op[kMax];
+  int n;
+};
+hipError_t launch_set_pairs(PairPtrs *tab, const PairOps &ops, hipStream_t s);
+
 // first launch: zero-body channels (nzero work-groups per pair: the largest channel
 // count + 1; nzeros in all), one-body pairs (comm111 + comm121), comm221 partial sums
 // and Pandya chunks side by side; maxnch sizes the Pandya chunks' LDS channel table
