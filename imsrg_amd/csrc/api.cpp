@@ -164,7 +164,13 @@ struct imsrg_ctx {
     std::vector<int> blk;  // one-body block of each orbit
   } xf;
   double *norm_dev = nullptr;
-  double *norm_host = nullptr;  // pinned
+  // norm results in coherent host memory, written by the norm kernels: slot i holds the
+  // one- and two-body sums and the number of the call that wrote them
+  struct NormSlot {
+    double sum[2];
+    unsigned long long done;
+  } *norm_host = nullptr;
+  unsigned long long norm_seq = 0;
   int npart = 0;
   std::string err;
   bool profiling = false;
@@ -311,7 +317,8 @@ static int ctx_init(imsrg_ctx *ctx, const imsrg_basis_desc *b, int device) {
   ctx->npart = 2049;  // 2048 two-body chunks and the one-body block
   HIPCHK(ctx, hipMalloc(&ctx->partials, sizeof(double) * ctx->npart));
   HIPCHK(ctx, hipMalloc(&ctx->norm_dev, sizeof(double) * 2));
-  HIPCHK(ctx, hipHostMalloc(&ctx->norm_host, sizeof(double) * 2, hipHostMallocDefault));
+  HIPCHK(ctx, hipHostMalloc((void **)&ctx->norm_host, 2 * sizeof(imsrg_ctx::NormSlot), hipHostMallocCoherent));
+  std::memset(ctx->norm_host, 0, 2 * sizeof(imsrg_ctx::NormSlot));
   ctx->ring.resize(imsrg_ctx::kRing);
   for (auto &set : ctx->ring)
     for (auto &ev : set) HIPCHK(ctx, hipEventCreate(&ev));
@@ -697,24 +704,52 @@ extern "C" int imsrg_hip_op_zero(imsrg_dop *op) {
   return IMSRG_OK;
 }
 
-// norm of op; with axpy_to, axpy_to += axpy_a * op in the same pass over op
-static int op_norm(imsrg_dop *op, double *n1, double *n2, double *n, imsrg_dop *axpy_to = nullptr,
-                   double axpy_a = 0.0) {
-  imsrg_ctx *ctx = op->ctx;
-  if (axpy_to)
-    HIPCHK(ctx, launch_axpy_norm(ctx->db.d, axpy_to->buf, axpy_a, op->buf, ctx->partials, ctx->npart,
-                                 ctx->norm_dev, ctx->stream));
-  else
-    HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, op->buf, ctx->partials, ctx->npart, ctx->norm_dev, ctx->stream));
-  HIPCHK(ctx, hipMemcpyAsync(ctx->norm_host, ctx->norm_dev, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  double a = std::sqrt(ctx->norm_host[0]), b = std::sqrt(ctx->norm_host[1]);
+// Queues the norm sums of op into host slot `slot` (and in the same pass, kAxpy: to +=
+// a op, kCopy: to = op).  norm_wait reads them: it watches the slot, so that no copy and
+// no stream wake-up follows the kernel, and asks the stream now and then, so that a
+// failed launch ends it.
+static int norm_launch(imsrg_ctx *ctx, int slot, const imsrg_dop *op, NormOp what = NormOp::kSum,
+                       imsrg_dop *to = nullptr, double a = 0.0) {
+  imsrg_ctx::NormSlot &h = ctx->norm_host[slot];
+  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, what, to ? to->buf : nullptr, a, op->buf, ctx->partials, ctx->npart,
+                          h.sum, &h.done, ++ctx->norm_seq, ctx->stream));
+  return IMSRG_OK;
+}
+// seq: ctx->norm_seq right after the slot's norm_launch
+static int norm_wait(imsrg_ctx *ctx, int slot, unsigned long long seq, double *n1, double *n2, double *n) {
+  imsrg_ctx::NormSlot &h = ctx->norm_host[slot];
+  for (unsigned spin = 0; __atomic_load_n(&h.done, __ATOMIC_ACQUIRE) != seq; ++spin) {
+    if (spin < 4096 || spin % 256) continue;
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) continue;
+    HIPCHK(ctx, e);
+    if (__atomic_load_n(&h.done, __ATOMIC_ACQUIRE) != seq) return fail(ctx, IMSRG_E_HIP, "the norm kernel left no result");
+    break;
+  }
+  const double a = std::sqrt(h.sum[0]), b = std::sqrt(h.sum[1]);
   if (n1) *n1 = a;
   if (n2) *n2 = b;
   if (n) *n = std::sqrt(a * a + b * b);
-  if (!std::isfinite(ctx->norm_host[0]) || !std::isfinite(ctx->norm_host[1]))
+  if (!std::isfinite(h.sum[0]) || !std::isfinite(h.sum[1]))
     return fail(ctx, IMSRG_E_NONFINITE, "operator holds non-finite values");
   return IMSRG_OK;
+}
+// norm of op; with axpy_to, axpy_to += axpy_a * op in the same pass over op
+static int op_norm(const imsrg_dop *op, double *n1, double *n2, double *n, imsrg_dop *axpy_to = nullptr,
+                   double axpy_a = 0.0) {
+  imsrg_ctx *ctx = op->ctx;
+  if (int rc = norm_launch(ctx, 0, op, axpy_to ? NormOp::kAxpy : NormOp::kSum, axpy_to, axpy_a)) return rc;
+  return norm_wait(ctx, 0, ctx->norm_seq, n1, n2, n);
+}
+// norms of two operators, one wait for both; with copy_to, copy_to = x in the pass over x
+static int op_norms(const imsrg_dop *x, const imsrg_dop *y, double *nx, double *ny, imsrg_dop *copy_to = nullptr) {
+  imsrg_ctx *ctx = x->ctx;
+  if (int rc = norm_launch(ctx, 0, x, copy_to ? NormOp::kCopy : NormOp::kSum, copy_to)) return rc;
+  const unsigned long long sx = ctx->norm_seq;
+  if (int rc = norm_launch(ctx, 1, y)) return rc;
+  const unsigned long long sy = ctx->norm_seq;
+  if (int rc = norm_wait(ctx, 0, sx, nullptr, nullptr, nx)) return rc;
+  return norm_wait(ctx, 1, sy, nullptr, nullptr, ny);
 }
 extern "C" int imsrg_hip_op_norm(imsrg_dop *op, double *n1, double *n2, double *n) {
   if (!op) return IMSRG_E_INVALID;
@@ -732,9 +767,8 @@ extern "C" int imsrg_hip_op_normal_order(imsrg_dop *out, const imsrg_dop *op, in
     return fail(ctx, IMSRG_E_UNSUPPORTED, "normal ordering needs a Hermitian or anti-Hermitian operator");
   // the one-body sum runs only when the two-body norm exceeds 1e-7 (src/Operator.cc:493):
   // the norm stays on the device, where the kernel tests it
-  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, op->buf, ctx->partials, ctx->npart, ctx->norm_dev, ctx->stream));
-  if (out != op) HIPCHK(ctx, hipMemcpyAsync(out->buf, op->buf, sizeof(double) * ctx->db.h.opsize,
-                                            hipMemcpyDeviceToDevice, ctx->stream));
+  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, out != op ? NormOp::kCopy : NormOp::kSum, out->buf, 0.0, op->buf,
+                          ctx->partials, ctx->npart, ctx->norm_dev, nullptr, 0, ctx->stream));
   out->herm = op->herm;
   HIPCHK(ctx, launch_normal_order(ctx->db.d, ctx->db.h, out->buf, sign, op->herm, ctx->norm_dev, ctx->stream));
   return IMSRG_OK;
@@ -1629,23 +1663,28 @@ static int bch_transform(imsrg_ctx *ctx, const imsrg_dop *Op, const imsrg_dop *O
                          const imsrg_bch_opts &o, int *ncomm) {
   int rc;
   if ((rc = ensure_ops(ctx, ctx->tmp, 2))) return rc;
-  imsrg_dop *A = ctx->tmp[0], *Bn = ctx->tmp[1];
   double nx, ny;
-  if ((rc = op_norm(const_cast<imsrg_dop *>(Op), nullptr, nullptr, &nx))) return rc;
-  if ((rc = op_norm(const_cast<imsrg_dop *>(Omega), nullptr, nullptr, &ny))) return rc;
-  if ((rc = imsrg_hip_op_copy(Out, Op))) return rc;
+  if ((rc = op_norms(Op, Omega, &nx, &ny, Out != Op ? Out : nullptr))) return rc;  // Out = Op
+  Out->herm = Op->herm;
   int nc = 0;
   bool converged = true;
   if (nx > o.transform_thr) {
     converged = false;
-    if ((rc = imsrg_hip_op_copy(A, Op))) return rc;
-    imsrg_dop *nested = A, *next = Bn;
+    // Out changes only after the first commutator has read Op.  With graphs on a copy of
+    // Op keeps that commutator's operand buffers the same from call to call, as its
+    // captured graph needs them
+    const imsrg_dop *nested = Op;
+    if (ctx->use_graphs) {
+      if ((rc = imsrg_hip_op_copy(ctx->tmp[0], Op))) return rc;
+      nested = ctx->tmp[0];
+    }
     double fact = 1.0;
     double eps = nx * std::exp(-2 * ny) * o.transform_thr / (2 * ny);
     for (int i = 1; i <= o.max_terms; ++i) {
+      imsrg_dop *next = ctx->tmp[i & 1];
       if ((rc = commutator_dev(ctx, Omega, nested, next, IMSRG_ALL_TERMS, o.precision))) return rc;
       nc++;
-      std::swap(nested, next);
+      nested = next;
       fact /= i;
       eps *= i + 1;
       double nn;  // Out += fact * nested, and the norm of nested, in one pass
@@ -1671,9 +1710,7 @@ static int bch_product(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y, i
   if ((rc = ensure_ops(ctx, ctx->tmp, 3))) return rc;
   if (Out == X || Out == Y) return fail(ctx, IMSRG_E_INVALID, "Out must not alias X or Y");
   double nx, ny;
-  if ((rc = op_norm(const_cast<imsrg_dop *>(X), nullptr, nullptr, &nx))) return rc;
-  if ((rc = op_norm(const_cast<imsrg_dop *>(Y), nullptr, nullptr, &ny))) return rc;
-  if ((rc = imsrg_hip_op_copy(Out, X))) return rc;
+  if ((rc = op_norms(X, Y, &nx, &ny, Out))) return rc;  // Out = X
   if ((rc = imsrg_hip_op_axpy(Out, 1.0, Y))) return rc;
   Out->herm = X->herm;
   imsrg_dop *nested = ctx->tmp[0], *next = ctx->tmp[1];
@@ -2005,16 +2042,14 @@ static int magnus_run(imsrg_ctx *ctx, imsrg_solver *sv, const imsrg_dop *H0, ims
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
   while (!rc && s < smax && step < max_steps) {
-    double ne;
-    if ((rc = op_norm(Eta, nullptr, nullptr, &ne))) break;
+    double ne, no;
+    if ((rc = op_norms(Eta, sv->current, &ne, &no))) break;
     if (eta_norm) eta_norm[step] = ne;
     if (ne < eta_crit) break;
     if (ne > 1e12 || std::fabs(Elast) > 1e9) {
       rc = fail(ctx, IMSRG_E_NONFINITE, "flow diverged (||eta|| > 1e12 or |E0| > 1e9)");
       break;
     }
-    double no;
-    if ((rc = op_norm(sv->current, nullptr, nullptr, &no))) break;
     if (no > omega_norm_max) {  // NewOmega, src/IMSRGSolver.cc:44-84
       if ((rc = imsrg_hip_op_copy(Hsaved, Hs))) break;
       if ((rc = new_omega(sv))) break;

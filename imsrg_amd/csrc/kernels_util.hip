@@ -173,20 +173,41 @@ hipError_t launch_scale(double *y, double a, long n, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Norm partial sums.  Block b < npart-1 covers a slice of the two-body arena
-// (weights (2J+1)^2 of the element's channel); the last block does the
-// one-body part with weights (2 j_p + 1).
-__global__ __launch_bounds__(256) void k_norm_partial(const BasisDev *bd, const double *op, double *part, int nblk2) {
+// One pass over an operator buffer x with the partial sums of its norm: OP 0 the sums
+// alone, OP 1 y += a x beside them (the BCH_Transform step, src/BCH.cc:176-191), OP 2
+// y = x (a copy).  Block b < nblk2 takes the b-th contiguous chunk of the two-body arena
+// and the channels it overlaps, each with its weight (2J+1)^2; the last block the
+// one-body part (weights 2 j_p + 1) and the words around the two parts.  Bound by HBM:
+// a block has four 16-byte loads per thread in flight (one 8-byte load each: the norm
+// 101 us for 293 MB at emax = 10, and a separate device copy about as long again).
+template <int OP>
+__global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y, double a, const double *x,
+                                                   double *part, int nblk2) {
   const BasisDev &B = *bd;
   __shared__ double red[4];
   double acc = 0.0;
+  auto put = [&](long e, double v) {  // one word of y
+    if (OP == 1) {
+      double t = a * v;  // (a x) formed first, then added (Operator operator* then +=)
+      y[e] += t;
+    }
+    if (OP == 2) y[e] = v;
+  };
   if ((int)blockIdx.x == nblk2) {
-    const double *one = op + B.one_off;
-    for (long e = threadIdx.x; e < (long)B.norb * B.norb; e += blockDim.x) acc += one[e] * one[e] * B.w1norm[e];
+    const long n1 = (long)B.norb * B.norb;
+    // the zero-body and padding words around the one-body block and after the two-body arena
+    const long rg[3][2] = {{0, B.one_off}, {B.one_off + n1, B.two_off}, {B.two_off + B.tbsize, B.opsize}};
+    if (OP != 0)
+      for (int g = 0; g < 3; ++g)
+        for (long e = rg[g][0] + threadIdx.x; e < rg[g][1]; e += blockDim.x) put(e, x[e]);
+    for (long e = threadIdx.x; e < n1; e += blockDim.x) {
+      const double v = x[B.one_off + e];
+      acc += v * v * B.w1norm[e];
+      put(B.one_off + e, v);
+    }
   } else {
-    // block b takes the b-th contiguous chunk of the two-body arena and the
-    // channels it overlaps, each with its weight (2J+1)^2
-    const double *two = op + B.two_off;
+    const double *two = x + B.two_off;
+    double *y2 = OP ? y + B.two_off : nullptr;
     const long tb = B.tbsize, chunk = (tb + nblk2 - 1) / nblk2;
     const long c0 = (long)blockIdx.x * chunk, c1 = min(c0 + chunk, tb);
     int lo = 0, hi = B.nch - 1;  // last channel starting at or before c0
@@ -199,61 +220,37 @@ __global__ __launch_bounds__(256) void k_norm_partial(const BasisDev *bd, const 
       const long e0 = max(c0, off), e1 = min(c1, off + nn);
       const double w = (double)((2 * (ch / 6) + 1) * (2 * (ch / 6) + 1));
       double s = 0.0;
-      for (long e = e0 + threadIdx.x; e < e1; e += blockDim.x) s += two[e] * two[e];
-      acc += w * s;
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-// y += a x over the whole operator buffer, and the norm partial sums of x with the
-// blocks of k_norm_partial (the same sums in the same order): one pass over x in
-// place of an axpy and a norm (the BCH_Transform step, src/BCH.cc:176-191)
-__global__ __launch_bounds__(256) void k_axpy_norm(const BasisDev *bd, double *y, double a, const double *x,
-                                                   double *part, int nblk2) {
-  const BasisDev &B = *bd;
-  __shared__ double red[4];
-  double acc = 0.0;
-  if ((int)blockIdx.x == nblk2) {
-    const long n1 = (long)B.norb * B.norb;
-    // the zero-body and padding words around the one-body block and after the two-body arena
-    const long rg[3][2] = {{0, B.one_off}, {B.one_off + n1, B.two_off}, {B.two_off + B.tbsize, B.opsize}};
-    for (int g = 0; g < 3; ++g)
-      for (long e = rg[g][0] + threadIdx.x; e < rg[g][1]; e += blockDim.x) {
-        double t = a * x[e];
-        y[e] += t;
-      }
-    const double *one = x + B.one_off;
-    double *yo = y + B.one_off;
-    for (long e = threadIdx.x; e < n1; e += blockDim.x) {
-      const double v = one[e];
-      acc += v * v * B.w1norm[e];
-      double t = a * v;
-      yo[e] += t;
-    }
-  } else {
-    const double *two = x + B.two_off;
-    double *y2 = y + B.two_off;
-    const long tb = B.tbsize, chunk = (tb + nblk2 - 1) / nblk2;
-    const long c0 = (long)blockIdx.x * chunk, c1 = min(c0 + chunk, tb);
-    int lo = 0, hi = B.nch - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (B.ch_off[mid] <= c0) lo = mid; else hi = mid - 1;
-    }
-    for (int ch = lo; ch < B.nch && B.ch_off[ch] < c1; ++ch) {
-      const long off = B.ch_off[ch], nn = (long)B.ch_n[ch] * B.ch_n[ch];
-      const long e0 = max(c0, off), e1 = min(c1, off + nn);
-      const double w = (double)((2 * (ch / 6) + 1) * (2 * (ch / 6) + 1));
-      double s = 0.0;
-      for (long e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-        const double v = two[e];
-        s += v * v;
-        double t = a * v;
-        y2[e] += t;
+      // pairs of words at even offsets (the arena is 64-byte aligned), clamped into
+      // [e0, e1): a pair across an end counts its inner word only
+      constexpr int U = 4;
+      for (long q = (e0 & ~1L) + 2 * (long)threadIdx.x; q < e1; q += 2 * U * (long)blockDim.x) {
+        double2 v[U], o[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const long e = min(q + 2 * u * (long)blockDim.x, (e1 - 1) & ~1L);
+          v[u] = *reinterpret_cast<const double2 *>(two + e);
+          if (OP == 1) o[u] = *reinterpret_cast<const double2 *>(y2 + e);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const long e = q + 2 * u * (long)blockDim.x;
+          const bool m0 = e < e1 && e >= e0, m1 = e + 1 < e1;
+          if (m0) s += v[u].x * v[u].x;
+          if (m1) s += v[u].y * v[u].y;
+          if (OP == 0) continue;
+          double2 r = v[u];
+          if (OP == 1) {
+            double t0 = a * v[u].x, t1 = a * v[u].y;
+            r.x = o[u].x + t0;
+            r.y = o[u].y + t1;
+          }
+          if (m0 && m1)
+            *reinterpret_cast<double2 *>(y2 + e) = r;
+          else if (m0)
+            y2[e] = r.x;
+          else if (m1)
+            y2[e + 1] = r.y;
+        }
       }
       acc += w * s;
     }
@@ -264,7 +261,11 @@ __global__ __launch_bounds__(256) void k_axpy_norm(const BasisDev *bd, double *y
   if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void k_norm_final(const double *part, int nblk2, double *out) {
+// The norm's two sums into out[0..1]; with seq != 0, out is host memory, and seq goes
+// into *done after them, so that the host can read the sums without a copy and without
+// waiting for the stream.
+__global__ void k_norm_final(const double *part, int nblk2, double *out, unsigned long long *done,
+                             unsigned long long seq) {
   __shared__ double red[256];
   double acc = 0.0;
   for (int i = threadIdx.x; i < nblk2; i += blockDim.x) acc += part[i];
@@ -277,6 +278,10 @@ __global__ void k_norm_final(const double *part, int nblk2, double *out) {
   if (threadIdx.x == 0) {
     out[0] = part[nblk2];
     out[1] = red[0];
+    if (seq) {
+      __threadfence_system();
+      __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -362,19 +367,19 @@ hipError_t launch_normal_order(const BasisDev *bd, const BasisDev &bh, double *o
   return hipGetLastError();
 }
 
-hipError_t launch_axpy_norm(const BasisDev *bd, double *y, double a, const double *x, double *partials, int npart,
-                            double *out, hipStream_t s) {
-  const int nblk2 = npart - 1;
-  hipLaunchKernelGGL(k_axpy_norm, dim3(npart), dim3(256), 0, s, bd, y, a, x, partials, nblk2);
-  hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, out);
-  return hipGetLastError();
-}
-hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, const double *op, double *partials, int npart,
-                       double *out, hipStream_t s) {
-  (void)bh;
-  int nblk2 = npart - 1;
-  hipLaunchKernelGGL(k_norm_partial, dim3(npart), dim3(256), 0, s, bd, op, partials, nblk2);
-  hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, out);
+hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, double a, const double *x,
+                       double *partials, int maxpart, double *out, unsigned long long *done, unsigned long long seq,
+                       hipStream_t s) {
+  // two-body chunks of at least 2048 words, so that small bases do not pay for idle blocks
+  const int nblk2 = (int)std::max<long>(1, std::min<long>(maxpart - 1, (bh.tbsize + 2047) / 2048));
+  const dim3 grid(nblk2 + 1), blk(256);
+  if (op == NormOp::kSum)
+    hipLaunchKernelGGL((k_norm_pass<0>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
+  else if (op == NormOp::kAxpy)
+    hipLaunchKernelGGL((k_norm_pass<1>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
+  else
+    hipLaunchKernelGGL((k_norm_pass<2>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
+  hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, out, done, seq);
   return hipGetLastError();
 }
 

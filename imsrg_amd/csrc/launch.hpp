@@ -65,12 +65,13 @@ hipError_t launch_fill(double *y, double v, long n, hipStream_t s);  // y[i] = v
 // (anti-)Hermitian completion of the one-body part always
 hipError_t launch_normal_order(const BasisDev *bd, const BasisDev &bh, double *op, int sign, int herm,
                                const double *n2sq, hipStream_t s);
-// y += a x over an operator buffer, with the norm sums of x into out[0..1] (as launch_norm)
-hipError_t launch_axpy_norm(const BasisDev *bd, double *y, double a, const double *x, double *partials, int npart,
-                            double *out, hipStream_t s);
-// partial sums of squares; out[0] = one-body, out[1] = two-body (weighted)
-hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, const double *op, double *partials, int npart,
-                       double *out, hipStream_t s);
+// sums of squares of an operator buffer x into out[0] (one-body) and out[1] (two-body,
+// weighted), and in the same pass kAxpy: y += a x, kCopy: y = x over the whole buffer;
+// seq != 0: out and *done are host memory, *done = seq once out holds the sums
+enum class NormOp { kSum, kAxpy, kCopy };
+hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, double a, const double *x,
+                       double *partials, int maxpart, double *out, unsigned long long *done, unsigned long long seq,
+                       hipStream_t s);
 // the basis-change matrices D of every channel (two-body layout, tbsize doubles) from
 // the one-body basis change C (norb x norb, column-major)
 // the Hartree-Fock monopoles W[q] = sum_J (2J+1) V~^J_{ia,jb} of quads[q] = (i, a, j, b)
