@@ -44,13 +44,13 @@ struct BatchCache {
   size_t off[10] = {0};
   int cnt[10] = {0};
   double *work = nullptr;
-  int maxn = 0, maxnch = 0, maxjmax = 0, maxnorb = 0, maxn1pairs = 0, maxncls = 0, maxbin = 0, maxent = 0;
+  int maxn = 0, maxnch = 0, maxjmax = 0, maxnorb = 0, maxn1pairs = 0, maxncls = 0, maxbin = 0;
   void release() {
     if (d_tab) (void)hipFree(d_tab);
     if (d_items) (void)hipFree(d_items);
     if (work) (void)hipFree(work);
     d_tab = nullptr; d_items = nullptr; work = nullptr;
-    maxn = maxnch = maxjmax = maxnorb = maxn1pairs = maxncls = maxbin = maxent = 0;
+    maxn = maxnch = maxjmax = maxnorb = maxn1pairs = maxncls = maxbin = 0;
     key.clear();
   }
 };
@@ -1377,7 +1377,7 @@ static bool uses_panels(const imsrg_ctx *ctx, int prec) {
 
 static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const int4 *const *items, const int *cnt,
                           unsigned mask, int prec, int maxn, int maxnch, int maxjmax, int maxnorb,
-                          int maxn1pairs, int maxncls, int maxbin, int maxent) {
+                          int maxn1pairs, int maxncls, int maxbin) {
   const Tuning &tu = ctx->db.tune;
   // split products take both GEMM families whatever the mixed-precision choices
   const int prec_pphh = gemm_family(prec, tu.mixed_pphh);
@@ -1410,7 +1410,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
     if (set) HIPCHK(ctx, hipEventRecord((*set)[7], ctx->side));
     HIPCHK(ctx, launch_pphh(pa, items[0], cnt[0], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, ctx->side));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[8], ctx->side));
-    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, ctx->side));
+    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, hipEventRecord(ctx->join, ctx->side));
     return IMSRG_OK;
@@ -1424,7 +1424,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
     HIPCHK(ctx, launch_zero_two(pa, items[6], cnt[6], s));
   }
   HIPCHK(ctx, mark(1));
-  if ((mask & M122) && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, maxent, s));
+  if ((mask & M122) && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
   HIPCHK(ctx, mark(2));
   const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
   const FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
@@ -1513,7 +1513,7 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
                  (int)db.wl.c122w.size()};
   if (!ctx->use_graphs || ctx->profiling || ws)
     return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
-                          db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin, db.h.c122_maxent);
+                          db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin);
   // replay a captured launch sequence for this operand set, capturing it on first use
   for (const GraphEntry &g : ctx->graphs)
     if (g.x == X->buf && g.y == Y->buf && g.z == Z->buf && g.hx == X->herm && g.hy == Y->herm && g.mask == mask &&
@@ -1523,7 +1523,7 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
     }
   HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   const int rc = run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
-                                db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin, db.h.c122_maxent);
+                                db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);  // always leave capture mode
   if (rc) {
@@ -2244,7 +2244,6 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       bc.maxn1pairs = std::max(bc.maxn1pairs, ctxs[i]->db.h.n1pairs);
       bc.maxncls = std::max(bc.maxncls, ctxs[i]->db.h.ncls);
       bc.maxbin = std::max(bc.maxbin, ctxs[i]->db.h.c122_maxbin);
-      bc.maxent = std::max(bc.maxent, ctxs[i]->db.h.c122_maxent);
     }
     if (c0->db.tune.pphh_order >= 1) {
       all[0] = xcd_order(groups, kXcd);
@@ -2292,7 +2291,7 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
     HIPCHK(c0, launch_set_pairs(bc.d_tab + i0, ops, c0->stream));
   }
   rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxjmax,
-                      bc.maxnorb, bc.maxn1pairs, bc.maxncls, bc.maxbin, bc.maxent);
+                      bc.maxnorb, bc.maxn1pairs, bc.maxncls, bc.maxbin);
   if (rc) return rc;
   if (!others.empty()) {
     HIPCHK(c0, hipEventRecord(c0->batch_ev, c0->stream));

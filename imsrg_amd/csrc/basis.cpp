@@ -290,8 +290,7 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   hh_start[nch] = (int)hh_loc.size(); k_start[nch] = (int)k_loc.size();
   kpp_start[nch] = (int)kpp_loc.size(); khh_start[nch] = (int)khh_loc.size();
   gcore_start[nch] = (int)gcore_loc.size(); gnc_start[nch] = (int)gnc_loc.size();
-  // comm122 lists in CSR form over the kets of all channels; each ket's list is
-  // padded to a multiple of kC122Blk entries with its first partner and factor 0
+  // comm122 lists in CSR form over the kets of all channels
   std::vector<int> c122_start(ch_kets.size() + 1, 0), c122_ind;
   std::vector<int2> c122_ao;
   std::vector<double> c122_f;
@@ -306,11 +305,6 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
         c122_ao.push_back(make_int2(e.y, e.z));
         c122_f.push_back(p122_f[c][u]);
       }
-      for (size_t v = u - t; v % kC122Blk != 0; ++v) {
-        c122_ind.push_back(p122_e[c][t].x);
-        c122_ao.push_back(make_int2(p122_e[c][t].y, p122_e[c][t].z));
-        c122_f.push_back(0.0);
-      }
       c122_start[ch_kstart[c] + ket + 1] = (int)c122_ind.size();
       t = u;
     }
@@ -320,15 +314,14 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   // comm122 column bins.  The partners of ket (p, q) are kets (a, q) and (p, a)
   // with a in the one-body block of p or q, so the kets of one unordered pair
   // of one-body blocks form a group closed under partners.  Groups are packed
-  // into bins of at most kC122Cols kets (first fit, largest first); the W
-  // kernel stages a bin's columns of X2 and Y2 in LDS.
+  // into bins (first fit, largest first) of as many kets as the largest
+  // group (a multiple of 4), at least 32.
   std::vector<int> c122_bcols, c122_boff(1, 0);
   std::vector<int4> c122_brec;
-  // bin entries: the records c122_brec[c122_beoff[b] ..] of bin b, column by column;
-  // c122_bcend[c122_boff[b] + cp] the end of column cp's entries within the bin
-  std::vector<int> c122_beoff(1, 0), c122_bcend;
+  // bin entries: the records c122_brec[c122_beoff[b] ..] of bin b, column by column
+  std::vector<int> c122_beoff(1, 0);
   c122w_items.clear();
-  int c122_maxbin = 1, c122_maxent = 4;
+  int c122_maxbin = 1;
   {
     std::vector<int> blk(norb);
     for (int o = 0; o < norb; ++o) blk[o] = *std::min_element(hb.ob[o].begin(), hb.ob[o].end());
@@ -346,11 +339,11 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       std::stable_sort(gl.begin(), gl.end(),
                        [](const std::vector<int> &a, const std::vector<int> &b) { return a.size() > b.size(); });
       std::vector<std::vector<int>> bins;
+      const size_t cap = gl.empty() ? 32 : std::max<size_t>(32, (gl[0].size() + 3) / 4 * 4);
       for (auto &g : gl) {
-        // a group larger than the bin capacity (emax > 14) takes a bin of its own
         if ((int)g.size() > kC122MaxCols) return "comm122 ket group larger than the W kernel's LDS";
         size_t t = 0;
-        while (t < bins.size() && bins[t].size() + g.size() > (size_t)kC122Cols) ++t;
+        while (t < bins.size() && bins[t].size() + g.size() > cap) ++t;
         if (t == bins.size()) bins.emplace_back();
         bins[t].insert(bins[t].end(), g.begin(), g.end());
       }
@@ -358,21 +351,20 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       for (auto &bn : bins) c122_maxbin = std::max(c122_maxbin, (int)bn.size());
       for (auto &bn : bins) {
         for (size_t t = 0; t < bn.size(); ++t) pos[bn[t]] = (int)t;
-        const int ent0 = (int)c122_brec.size();
         for (int q : bn) {
           c122_bcols.push_back(q);
           for (int e = c122_start[ch_kstart[c] + q]; e < c122_start[ch_kstart[c] + q + 1]; ++e) {
             int f[2];
             std::memcpy(f, &c122_f[e], sizeof(double));
-            c122_brec.push_back(make_int4(c122_ao[e].y * norb + c122_ao[e].x, pos[c122_ind[e]], f[0], f[1]));
+            c122_brec.push_back(make_int4(c122_ao[e].y * norb + c122_ao[e].x, pos[q] << 16 | pos[c122_ind[e]], f[0], f[1]));
           }
-          c122_bcend.push_back((int)c122_brec.size() - ent0);
         }
         c122_beoff.push_back((int)c122_brec.size());
-        c122_maxent = std::max(c122_maxent, (int)c122_brec.size() - ent0);
         const int bi = (int)c122_boff.size() - 1;
         c122_boff.push_back((int)c122_bcols.size());
-        for (int r = 0; r < n; r += kC122Rows) c122w_items.push_back(make_int4(0, c, bi, r / kC122Rows));
+        const int nsub = (int)bn.size() <= kC122MaxN ? 1 : ((int)bn.size() + 15) / 16;
+        for (int r = 0; r < n; r += kC122Rows)
+          for (int u = 0; u < nsub; ++u) c122w_items.push_back(make_int4(0, c, bi, (u << 16) | (r / kC122Rows)));
       }
       for (auto &bn : bins)  // every partner of a bin's column lies in the bin
         for (int q : bn)
@@ -416,9 +408,7 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   B.c122_bcols = dupload(*this, c122_bcols, err); B.c122_boff = dupload(*this, c122_boff, err);
   B.c122_brec = dupload(*this, c122_brec, err);
   B.c122_beoff = dupload(*this, c122_beoff, err);
-  B.c122_bcend = dupload(*this, c122_bcend, err);
   B.c122_maxbin = c122_maxbin;
-  B.c122_maxent = c122_maxent;
   B.gcore_start = dupload(*this, gcore_start, err); B.gcore_loc = dupload(*this, gcore_loc, err);
   B.gnc_start = dupload(*this, gnc_start, err); B.gnc_loc = dupload(*this, gnc_loc, err);
 

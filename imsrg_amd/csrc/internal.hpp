@@ -27,10 +27,9 @@ constexpr int kGN = kGW / 16;     // 16-column MFMA blocks per wave sub-tile
 constexpr int kGC = kTileK / kGWaves;  // k columns each wave copies into LDS per stage
 constexpr int kChunk = 256;       // elements per work item of the gather kernels
 constexpr int kJC = 8;            // J values per register chunk of the inverse Pandya gather (even)
-constexpr int kC122Blk = 4;       // comm122 partner lists are padded to multiples of this (one load block)
-constexpr int kC122Cols = 32;     // kets (columns) a bin of the comm122 W kernel is filled to
-constexpr int kC122MaxCols = 150; // largest bin (LDS: 16 * 64 bytes per column)
-constexpr int kC122Rows = 64;     // rows of one W-kernel work item
+constexpr int kC122MaxN = 64;     // columns of a comm122 bin formed at once (a larger bin takes one item per 16)
+constexpr int kC122MaxCols = 150; // largest bin (LDS: 1 KiB of coefficients per ket)
+constexpr int kC122Rows = 128;    // rows of one comm122 W item (256: 221 against 210 us at emax = 10)
 constexpr int kF32Flush = 4;      // MFMA k-steps (of 4) summed in FP32 before the FP64 flush (mixed, 64x64 tiles)
 
 // GEMM kernel families passed to launch_pphh / launch_ph_gemm: 0 FP64,
@@ -95,19 +94,15 @@ struct BasisDev {
   const IMSRG_G double *khh_w;
   // comm122 column bins (kets of whole one-body block pairs, closed under
   // partners): bin b holds the channel-local kets c122_bcols[c122_boff[b] ..
-  // c122_boff[b + 1]).  The partner entries of its columns, one after another, each
-  // column's a multiple of kC122Blk (padding: factor 0), are the records
-  // c122_brec[c122_beoff[b] ..] = (index a + o norb of the one-body element,
-  // position of the partner in the bin, the factor f -- phase / sqrt2 factors, times
-  // 2 for kets with p == q -- as low and high word); column cp's entries end at
-  // c122_bcend[c122_boff[b] + cp] within the bin
+  // c122_boff[b + 1]).  The partner entries of its columns, one after another, are the
+  // records c122_brec[c122_beoff[b] ..] = (index a + o norb of the one-body element,
+  // column << 16 | position of the partner, both in the bin, the factor f -- phase /
+  // sqrt2 factors, times 2 for kets with p == q -- as low and high word)
   const IMSRG_G int *c122_bcols;
   const IMSRG_G int *c122_boff;
   const IMSRG_G int4 *c122_brec;
   const IMSRG_G int *c122_beoff;
-  const IMSRG_G int *c122_bcend;
   int c122_maxbin;                 // kets of the largest bin
-  int c122_maxent;                 // partner entries of the largest bin
   // cross-coupled channels
   const IMSRG_G int *cc_n, *cc_nph, *cc_kstart, *cc_kets, *cc_phstart, *cc_ph;
   const IMSRG_G signed char *cc_phi;  // (-1)^{(j_p+j_q)} per CC ket

@@ -1768,90 +1768,92 @@ __device__ __forceinline__ const T &blk_at(const T *base, unsigned idx) {
 // W of comm122ss (src/Commutator.cc:908-926) by column bins:
 //   W(r, q) = sum over the partner entries e of ket q of Y2(r, ind_e) x_e - X2(r, ind_e) y_e,
 //   x_e = X1(a,o) f, y_e = Y1(a,o) f for the entry's orbits and factor (857-896).
-// Every partner of a bin's kets lies in the bin,
-// so a work-group stages the bin's columns of X2 and Y2 for kC122Rows rows in
-// LDS (each column segment read once, coalesced), together with the bin's
-// partner entries (position in the bin, coefficients); each lane then forms W
-// for one row of every column of the bin, reading only LDS, and W is stored in
-// the two-body layout.
-__host__ __device__ inline size_t c122w_lds_bytes(int maxbin, int maxent) {
-  return 2 * sizeof(double) * kC122Rows * (size_t)maxbin + (sizeof(double2) + sizeof(int)) * (size_t)maxent +
+// Every partner of a bin's kets lies in the bin, so W of the bin's columns is the product
+//   W = [Y2 X2](rows, bin) [Cx; -Cy]
+// with the coefficient matrices Cx, Cy over the bin, built in LDS from the partner
+// entries once per work-group (LDS adds; only the ket itself appears twice in a column,
+// and a sum of two does not depend on their order).  The
+// products run on f64 16x16x4 MFMAs whose A operands come straight from global memory
+// (a load takes 16 rows of 4 columns), so X2 and Y2 are read once, with no pass through
+// LDS and no barrier between the loads and their use.  Bound by HBM: X2 and Y2 read, W
+// written.  Staging the columns in LDS and mixing them there took 258 us at emax = 10 and
+// 1412 us at emax = 12 (3.4 and 2.4 TB/s): few work-groups fitted in a CU, each waiting
+// for its own staging.  Now 210 and 950 us (4.2 and 3.6 TB/s).
+__host__ __device__ inline int c122w_cols(int nc) { return nc <= kC122MaxN ? (nc + 15) & ~15 : 16; }
+inline size_t c122w_lds_bytes(int maxbin) {
+  const size_t k4 = (size_t)((maxbin + 3) & ~3), full = maxbin <= kC122MaxN ? k4 * c122w_cols(maxbin) : kC122MaxN * kC122MaxN;
+  return 16 * std::max(full, 16 * k4) +  // both matrices of a whole bin, or of 16 columns of a larger one
          sizeof(int) * (size_t)maxbin;
 }
-__global__ __launch_bounds__(256) void k_c122_w(PairArg pa, const int4 *items, int maxbin, int maxent) {
-  static_assert(kC122Rows == 64, "one row per lane of a wave");
+__global__ __launch_bounds__(256, 4) void k_c122_w(PairArg pa, const int4 *items) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  double(*sx)[kC122Rows] = reinterpret_cast<double(*)[kC122Rows]>(lds_raw);  // [maxbin][kC122Rows]
-  double(*sy)[kC122Rows] = sx + maxbin;
-  double2 *sc = reinterpret_cast<double2 *>(sy + maxbin);  // [maxent] coefficients (x_e, y_e)
-  int *sp = reinterpret_cast<int *>(sc + maxent);          // [maxent] partner position in the bin
-  int *se = sp + maxent;                                   // [maxbin] end of each column's entries
+  constexpr int KF = kC122MaxN / 4;  // A fragments (4 columns each) held at once
   const int4 it = items[blockIdx.x];
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
   const int ch = it.y, n = B.ch_n[ch];
   const int b0 = B.c122_boff[it.z], nc = B.c122_boff[it.z + 1] - b0;
   const int eo = B.c122_beoff[it.z], ne = B.c122_beoff[it.z + 1] - eo;
-  const IMSRG_G int *cols = B.c122_bcols + b0;
-  const int R0 = it.w * kC122Rows;
+  const int R0 = (it.w & 0xffff) * kC122Rows;
+  // this item's columns: all of the bin's, or 16 of a bin of more than kC122MaxN
+  const int ns = c122w_cols(nc), n0 = (it.w >> 16) * 16, nn = min(nc - n0, ns), k4 = (nc + 3) & ~3;
+  double *cx = reinterpret_cast<double *>(lds_raw);  // [k4][ns]: coefficients of Y2
+  double *cy = cx + k4 * ns;                         // [k4][ns]: of X2
+  int *sq = reinterpret_cast<int *>(cy + k4 * ns);  // [nc] the bin's kets
+  for (int t = threadIdx.x; t < 2 * k4 * ns; t += blockDim.x) cx[t] = 0.0;
+  for (int t = threadIdx.x; t < nc; t += blockDim.x) sq[t] = B.c122_bcols[b0 + t];
+  __syncthreads();
+  for (int t = threadIdx.x; t < ne; t += blockDim.x) {
+    const int4 rec = B.c122_brec[eo + t];
+    const int c = (rec.y >> 16) - n0;
+    if (c < 0 || c >= nn) continue;
+    const double f = __hiloint2double(rec.w, rec.z);
+    const int at = (rec.y & 0xffff) * ns + c;
+    atomicAdd(&cx[at], P.X[B.one_off + rec.x] * f);
+    atomicAdd(&cy[at], -(P.Y[B.one_off + rec.x] * f));
+  }
+  __syncthreads();
   const long off = B.ch_off[ch];
   const double *X2 = P.X + B.two_off + off, *Y2 = P.Y + B.two_off + off;
   double *W = P.c122w + off;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const unsigned r = (unsigned)min(R0 + lane, n - 1);
-  for (int t = threadIdx.x; t < ne; t += blockDim.x) {
-    const int4 rec = B.c122_brec[eo + t];
-    const double f = __hiloint2double(rec.w, rec.z);
-    sp[t] = rec.y;
-    sc[t] = make_double2(P.X[B.one_off + rec.x] * f, P.Y[B.one_off + rec.x] * f);
-  }
-  for (int t = threadIdx.x; t < nc; t += blockDim.x) se[t] = B.c122_bcend[b0 + t];
-  // columns: up to 16 per wave and pass, every load issued before the LDS
-  // writes (a loop that wrote each column before loading the next waited for
-  // each load in turn)
-  for (int cb = 0; cb < nc; cb += 64) {
-    double xr[16], yr[16];
+  const int m = lane & 15, kq = lane >> 4;
+  for (int r0 = R0 + 16 * wv; r0 < min(R0 + kC122Rows, n); r0 += 64) {
+    const int row = min(r0 + m, n - 1);
+    dbl4 acc[kC122MaxN / 16];
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int c = min(cb + wv + 4 * m, nc - 1);
-      const unsigned q = (unsigned)cols[c];
-      xr[m] = blk_at(X2, q * n + r);
-      yr[m] = blk_at(Y2, q * n + r);
-    }
+    for (int j = 0; j < kC122MaxN / 16; ++j) acc[j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < k4; k0 += kC122MaxN) {  // once unless the bin is larger
+      double ax[KF], ay[KF];
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int c = cb + wv + 4 * m;
-      if (c < nc) {
-        sx[c][lane] = xr[m];
-        sy[c][lane] = yr[m];
-      }
-    }
-  }
-  __syncthreads();
-  const bool row_ok = R0 + lane < n;
-  static_assert(kC122Blk == 4, "partner blocks of four entries");
-  for (int cp = wv; cp < nc; cp += 4) {
-    const int q = cols[cp];
-    const int ea = cp ? se[cp - 1] : 0, eb = se[cp];
-    double w = 0.0;
-    for (int t = ea; t < eb; t += 4) {  // a column's list is a multiple of four entries
-      int pp[4];
-      double2 cf[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        pp[m] = sp[t + m];
-        cf[m] = sc[t + m];
-      }
-      double yv[4], xv[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        yv[m] = sy[pp[m]][lane];
-        xv[m] = sx[pp[m]][lane];
+      for (int ks = 0; ks < KF; ++ks) {
+        if (k0 + 4 * ks >= k4) break;  // uniform
+        const unsigned q = (unsigned)sq[min(k0 + 4 * ks + kq, nc - 1)];  // past nc: coefficients 0
+        ay[ks] = blk_at(Y2, q * n + row);
+        ax[ks] = blk_at(X2, q * n + row);
       }
 #pragma unroll
-      for (int m = 0; m < 4; ++m) w += yv[m] * cf[m].x - xv[m] * cf[m].y;
+      for (int j = 0; j < kC122MaxN / 16; ++j) {
+        if (16 * j >= nn) break;
+#pragma unroll
+        for (int ks = 0; ks < KF; ++ks) {
+          if (k0 + 4 * ks >= k4) break;
+          const int c = (k0 + 4 * ks + kq) * ns + 16 * j + m;
+          // D^T blocks: lane l, register q holds row (l & 15), column 4 q + (l >> 4)
+          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(cx[c], ay[ks], acc[j], 0, 0, 0);
+          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(cy[c], ax[ks], acc[j], 0, 0, 0);
+        }
+      }
     }
-    if (row_ok) blk_at(W, (unsigned)q * n + r) = w;
+#pragma unroll
+    for (int j = 0; j < kC122MaxN / 16; ++j) {
+      if (16 * j >= nn) break;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = 16 * j + 4 * q + kq;
+        if (c < nn && r0 + m < n) blk_at(W, (unsigned)sq[n0 + c] * n + row) = acc[j][q];
+      }
+    }
   }
 }
 
@@ -2094,11 +2096,11 @@ hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool 
     hipLaunchKernelGGL(k_mirror, grid, dim3(256), 0, s, pa, items, nfins, nfin);
   return hipGetLastError();
 }
-hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, int maxent, hipStream_t s) {
+hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
-  const size_t lds = c122w_lds_bytes(maxbin, maxent);
+  const size_t lds = c122w_lds_bytes(maxbin);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_c122_w, dim3(nitems), dim3(256), lds, s, pa, items, maxbin, maxent);
+  hipLaunchKernelGGL(k_c122_w, dim3(nitems), dim3(256), lds, s, pa, items);
   return hipGetLastError();
 }
 hipError_t launch_zero_two(const PairArg &pa, const int4 *items, int nitems, hipStream_t s) {

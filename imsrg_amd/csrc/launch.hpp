@@ -52,7 +52,7 @@ hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, in
 hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, int npairs,
                          int maxn1pairs, hipStream_t s);
 // comm122's W (two-body layout, P.c122w) by column bins; before launch_finish with c122
-hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, int maxent, hipStream_t s);
+hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int maxbin, hipStream_t s);
 hipError_t launch_zero_two(const PairArg &pa, const int4 *items, int nitems, hipStream_t s);
 
 // operator arithmetic
