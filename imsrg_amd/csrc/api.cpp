@@ -41,16 +41,18 @@ struct BatchCache {
   std::vector<long long> key;
   PairPtrs *d_tab = nullptr;
   int4 *d_items = nullptr;
-  size_t off[10] = {0};
-  int cnt[10] = {0};
+  size_t off[11] = {0};
+  int cnt[11] = {0};
   double *work = nullptr;
-  int maxn = 0, maxnch = 0, maxjmax = 0, maxnorb = 0, maxn1pairs = 0, maxncls = 0, maxbin = 0;
+  int maxn = 0, maxnch = 0, maxn1pairs = 0, maxbin = 0;
+  size_t invp_lds[2] = {0, 0};
   void release() {
     if (d_tab) (void)hipFree(d_tab);
     if (d_items) (void)hipFree(d_items);
     if (work) (void)hipFree(work);
     d_tab = nullptr; d_items = nullptr; work = nullptr;
-    maxn = maxnch = maxjmax = maxnorb = maxn1pairs = maxncls = maxbin = 0;
+    maxn = maxnch = maxn1pairs = maxbin = 0;
+    invp_lds[0] = invp_lds[1] = 0;
     key.clear();
   }
 };
@@ -1376,8 +1378,8 @@ static bool uses_panels(const imsrg_ctx *ctx, int prec) {
 }
 
 static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const int4 *const *items, const int *cnt,
-                          unsigned mask, int prec, int maxn, int maxnch, int maxjmax, int maxnorb,
-                          int maxn1pairs, int maxncls, int maxbin) {
+                          unsigned mask, int prec, int maxn, int maxnch, int maxn1pairs, int maxbin,
+                          const size_t *invp_lds) {
   const Tuning &tu = ctx->db.tune;
   // split products take both GEMM families whatever the mixed-precision choices
   const int prec_pphh = gemm_family(prec, tu.mixed_pphh);
@@ -1434,8 +1436,10 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));
   if (fork_late) HIPCHK(ctx, hipEventRecord(ctx->fork, s));
   HIPCHK(ctx, mark(4));
-  if (mask & MPH)
-    HIPCHK(ctx, launch_invpandya(pa, items[4], cnt[4], maxjmax, maxnorb, maxnch, maxncls, prec_ph == 1, s));
+  if (mask & MPH) {
+    const int f = prec_ph == 1 ? 10 : 4;  // FP32 Zbar: twice the elements per item
+    HIPCHK(ctx, launch_invpandya(pa, items[f], cnt[f], invp_lds[prec_ph == 1], prec_ph == 1, s));
+  }
   if (overlap) {
     if (int rc = side_work()) return rc;
     HIPCHK(ctx, hipStreamWaitEvent(s, ctx->join, 0));
@@ -1505,15 +1509,16 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
   pa.p0.hZ = herm_rule(X->herm, Y->herm);
   pa.p0.mask = mask;
   Z->herm = pa.p0.hZ;
-  const int4 *items[10] = {db.d_pphh, db.d_ph,     db.d_ob221,  db.d_pandya, db.d_invp,
-                           db.d_one,  db.d_mirror, db.d_pphh64, db.d_pack,   db.d_c122w};
-  int cnt[10] = {(int)db.wl.pphh.size(),   (int)db.wl.ph.size(),   (int)db.wl.ob221.size(),
+  const int4 *items[11] = {db.d_pphh, db.d_ph,     db.d_ob221,  db.d_pandya, db.d_invp,  db.d_one,
+                           db.d_mirror, db.d_pphh64, db.d_pack,   db.d_c122w,  db.d_invp32};
+  const size_t invp_lds[2] = {db.invp_lds(false), db.invp_lds(true)};
+  int cnt[11] = {(int)db.wl.pphh.size(),   (int)db.wl.ph.size(),   (int)db.wl.ob221.size(),
                  (int)db.wl.pandya.size(), (int)db.wl.invp.size(),  (int)db.wl.one.size(),
                  (int)db.wl.mirror.size(), (int)db.wl.pphh64.size(), (int)db.wl.pack.size(),
-                 (int)db.wl.c122w.size()};
+                 (int)db.wl.c122w.size(),  (int)db.wl.invp32.size()};
   if (!ctx->use_graphs || ctx->profiling || ws)
-    return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
-                          db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin);
+    return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.n1pairs,
+                          db.h.c122_maxbin, invp_lds);
   // replay a captured launch sequence for this operand set, capturing it on first use
   for (const GraphEntry &g : ctx->graphs)
     if (g.x == X->buf && g.y == Y->buf && g.z == Z->buf && g.hx == X->herm && g.hy == Y->herm && g.mask == mask &&
@@ -1522,8 +1527,8 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
       return IMSRG_OK;
     }
   HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-  const int rc = run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.jmax,
-                                db.h.norb, db.h.n1pairs, db.h.ncls, db.h.c122_maxbin);
+  const int rc = run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.n1pairs,
+                                db.h.c122_maxbin, invp_lds);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);  // always leave capture mode
   if (rc) {
@@ -2205,12 +2210,12 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
     HIPCHK(c0, hipMalloc(&bc.d_tab, sizeof(PairPtrs) * npairs));
     HIPCHK(c0, hipMemcpy(bc.d_tab, tab.data(), sizeof(PairPtrs) * npairs, hipMemcpyHostToDevice));
     // concatenated lists; pp/hh tiles of all pairs go through the XCD-balanced order
-    std::vector<int4> all[10];
+    std::vector<int4> all[11];
     std::vector<TileGroup> groups;
     for (int i = 0; i < npairs; ++i) {
       const WorkLists &wl = ctxs[i]->db.wl;
-      const std::vector<int4> *src[10] = {&wl.pphh, &wl.ph,     &wl.ob221,  &wl.pandya, &wl.invp,
-                                          &wl.one,  &wl.mirror, &wl.pphh64, &wl.pack,   &wl.c122w};
+      const std::vector<int4> *src[11] = {&wl.pphh,   &wl.ph,     &wl.ob221, &wl.pandya, &wl.invp,  &wl.one,
+                                          &wl.mirror, &wl.pphh64, &wl.pack,  &wl.c122w,  &wl.invp32};
       {  // ph tiles in the tile size of the first context, whose kernels run the batch
         const int tile = c0->db.tune.ph_big ? kTileB : kTile;
         const DeviceBasis &dbi = ctxs[i]->db;
@@ -2222,7 +2227,7 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
             for (int sb = rb; sb < nt; ++sb) all[1].push_back(make_int4(i, c, rb, sb));
         }
       }
-      for (int t = 2; t < 10; ++t)
+      for (int t = 2; t < 11; ++t)
         for (int4 w : *src[t]) {
           w.x = i;
           all[t].push_back(w);
@@ -2239,10 +2244,8 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       for (auto &kv : gm) groups.push_back(kv.second);
       bc.maxn = std::max(bc.maxn, ctxs[i]->db.h.maxn);
       bc.maxnch = std::max(bc.maxnch, ctxs[i]->db.h.nch);
-      bc.maxjmax = std::max(bc.maxjmax, ctxs[i]->db.h.jmax);
-      bc.maxnorb = std::max(bc.maxnorb, ctxs[i]->db.h.norb);
       bc.maxn1pairs = std::max(bc.maxn1pairs, ctxs[i]->db.h.n1pairs);
-      bc.maxncls = std::max(bc.maxncls, ctxs[i]->db.h.ncls);
+      for (int v = 0; v < 2; ++v) bc.invp_lds[v] = std::max(bc.invp_lds[v], ctxs[i]->db.invp_lds(v != 0));
       bc.maxbin = std::max(bc.maxbin, ctxs[i]->db.h.c122_maxbin);
     }
     if (c0->db.tune.pphh_order >= 1) {
@@ -2254,13 +2257,13 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       for (auto &g : groups) all[0].insert(all[0].end(), g.tiles.begin(), g.tiles.end());
     }
     size_t tot = 0;
-    for (int t = 0; t < 10; ++t) {
+    for (int t = 0; t < 11; ++t) {
       bc.off[t] = tot;
       bc.cnt[t] = (int)all[t].size();
       tot += all[t].size();
     }
     HIPCHK(c0, hipMalloc(&bc.d_items, sizeof(int4) * std::max<size_t>(tot, 1)));
-    for (int t = 0; t < 10; ++t)
+    for (int t = 0; t < 11; ++t)
       if (!all[t].empty())
         HIPCHK(c0, hipMemcpy(bc.d_items + bc.off[t], all[t].data(), sizeof(int4) * all[t].size(),
                              hipMemcpyHostToDevice));
@@ -2270,8 +2273,8 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
   PairArg pa;
   std::memset(&pa.p0, 0, sizeof(pa.p0));
   pa.tab = bc.d_tab;
-  const int4 *items[10];
-  for (int t = 0; t < 10; ++t) items[t] = bc.d_items + bc.off[t];
+  const int4 *items[11];
+  for (int t = 0; t < 11; ++t) items[t] = bc.d_items + bc.off[t];
   // The batch runs on c0's stream.  Work queued on the other contexts' streams
   // (uploads, copies, axpy, generators of X_i / Y_i) finishes before it starts,
   // and their later work (downloads, norms of Z_i) waits for it to end.
@@ -2290,8 +2293,8 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
                    Z[i0 + i]->herm, mask};
     HIPCHK(c0, launch_set_pairs(bc.d_tab + i0, ops, c0->stream));
   }
-  rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxjmax,
-                      bc.maxnorb, bc.maxn1pairs, bc.maxncls, bc.maxbin);
+  rc = run_commutator(c0, pa, npairs, items, bc.cnt, mask, prec, bc.maxn, bc.maxnch, bc.maxn1pairs,
+                      bc.maxbin, bc.invp_lds);
   if (rc) return rc;
   if (!others.empty()) {
     HIPCHK(c0, hipEventRecord(c0->batch_ev, c0->stream));

@@ -171,6 +171,9 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   B.j2 = dupload(*this, hb.j2, err); B.l = dupload(*this, hb.l, err); B.tz2 = dupload(*this, hb.tz2, err);
   B.cvq = dupload(*this, hb.cvq, err); B.occ = dupload(*this, hb.occ, err);
   B.holes = dupload(*this, hb.holes, err);
+  std::vector<int> orbcode((norb + 3) & ~3, 0);
+  for (int o = 0; o < norb; ++o) orbcode[o] = hb.j2[o] | (hb.l[o] & 1) << 16 | (hb.tz2[o] > 0) << 17;
+  B.orbcode = dupload(*this, orbcode, err);
   std::vector<int> obstart(norb + 1, 0), oblist;
   for (int i = 0; i < norb; ++i) {
     obstart[i] = (int)oblist.size();
@@ -188,16 +191,6 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
     for (int k = 0; k < hb.nkets; ++k)
       for (int J = 0; J <= hb.jmax; ++J) cT[(size_t)J * hb.nkets + k] = hb.kmap[(size_t)k * (hb.jmax + 1) + J];
     B.kmapT = dupload(*this, cT, err);
-    // ccorb[(i (jmax+1) + J) norb + x]: cross-coupled local index of the ket of
-    // orbits i and x in channel J (of its parity and |tz_i - tz_x|/2), or -1
-    std::vector<int> co((size_t)norb * (hb.jmax + 1) * norb);
-    for (int i = 0; i < norb; ++i)
-      for (int J = 0; J <= hb.jmax; ++J)
-        for (int x = 0; x < norb; ++x) {
-          const int k = ket_index(norb, std::min(i, x), std::max(i, x));
-          co[((size_t)i * (hb.jmax + 1) + J) * norb + x] = hb.cmap[(size_t)k * (hb.jmax + 1) + J];
-        }
-    B.ccorb = dupload(*this, co, err);
     // kmorb: standard local indices by orbit pair, J fastest (a channel holds fewer
     // than 2^14.5 kets: its block is addressed with 32-bit byte offsets)
     B.kmorb_nx = (hb.jmax + 1 + 7) / 8 * 8;
@@ -222,6 +215,15 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   }
   grp_start[6] = (int)grp_kets.size();
   B.grp_start = dupload(*this, grp_start, err); B.grp_kets = dupload(*this, grp_kets, err);
+  std::vector<int> grp_first((size_t)6 * (norb + 1));
+  for (int g = 0; g < 6; ++g) {
+    int e = grp_start[g];
+    for (int k = 0; k <= norb; ++k) {
+      while (e < grp_start[g + 1] && hb.kp[grp_kets[e]] < k) ++e;
+      grp_first[(size_t)g * (norb + 1) + k] = e - grp_start[g];
+    }
+  }
+  B.grp_first = dupload(*this, grp_first, err);
 
   // ---- standard channels ----
   std::vector<int> ch_n(nch), ch_kstart(nch + 1), ch_kets;
@@ -509,33 +511,45 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   // ---- 6j table on the device ----
   {
     long tot = (long)B.d1 * B.d1 * B.d2 * B.d1 * B.d1 * B.d2;
-    B.d2q = (B.d2 + 1) & ~1;
-    // the gather copy: padded J3 range, plus kJC / 2 (jj4, jj5) blocks of J3 pairs
-    // so that a kJC-wide J chunk starting at the last pair stays inside the allocation
-    long totq = (long)B.d1 * B.d1 * B.d1 * B.d1 * B.d2q * B.d2q + (long)(kJC / 2) * 2 * B.d1 * B.d1;
     void *p = nullptr, *pQ = nullptr;
+    // the inverse Pandya copy: rows of up to 3 J' past the last
     // 8 more: the Pandya kernel reads the J of one row in aligned groups of four pairs
     if (hipMalloc(&p, (tot + 8) * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(p);
-    if (hipMalloc(&pQ, totq * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
+    if (hipMalloc(&pQ, (tot + 4 * B.d2) * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(pQ);
-    if (hipMemset(pQ, 0, totq * sizeof(double)) != hipSuccess) return "hipMemset failed for the 6j table";
-    if (launch_sixj_table((double *)p, (double *)pQ, B.d1, B.d2, B.d2q, 0) != hipSuccess)
+    if (hipMemset((double *)pQ + tot, 0, 4 * B.d2 * sizeof(double)) != hipSuccess)
+      return "hipMemset failed for the 6j table";
+    if (launch_sixj_table((double *)p, (double *)pQ, B.d1, B.d2, 0) != hipSuccess)
       return "6j table kernel failed";
     if (hipDeviceSynchronize() != hipSuccess) return "6j table kernel failed";
     B.sixj = (const double *)p;
     B.sixjQ = (const double *)pQ;
   }
 
-  // ---- (j_k, j_l) class lists of the ket groups (inverse Pandya ket order) ----
+  // ---- inverse Pandya: class lists of the ket groups, cross-coupled kets by orbit, items ----
   {
-    const int ncls = B.d1 * B.d1;
-    std::vector<int> cls_start(6 * ncls + 1, 0), cls_e;
+    const int nJ = hb.jmax + 1, d1 = B.d1, ncls = d1 * (d1 + 1) / 2;
+    std::vector<int> cls_j, cls_of((size_t)d1 * d1), cls_start(6 * ncls + 1, 0), cls_e;
+    for (int a = 0; a < d1; ++a)
+      for (int b = a; b < d1; ++b) {
+        cls_of[a * d1 + b] = cls_of[b * d1 + a] = (int)cls_j.size();
+        cls_j.push_back((2 * a + 1) << 16 | (2 * b + 1));
+      }
+    std::vector<int> before((size_t)(hb.nkets + 6) * ncls, 0);
+    std::vector<int2> rec;
     for (int g = 0; g < 6; ++g) {
+      const int ng = grp_start[g + 1] - grp_start[g];
       std::vector<std::vector<int>> per(ncls);
-      for (int e = 0; e < grp_start[g + 1] - grp_start[g]; ++e) {
+      std::vector<int> cnt(ncls, 0);
+      int *row = &before[(size_t)(grp_start[g] + g) * ncls];
+      for (int e = 0; e < ng; ++e) {
         const int kk = grp_kets[grp_start[g] + e];
-        per[((hb.j2[hb.kp[kk]] - 1) / 2) * B.d1 + (hb.j2[hb.kq[kk]] - 1) / 2].push_back(e);
+        const int c = cls_of[(hb.j2[hb.kp[kk]] - 1) / 2 * d1 + (hb.j2[hb.kq[kk]] - 1) / 2];
+        per[c].push_back(kk);
+        ++cnt[c];
+        row += ncls;
+        std::copy(cnt.begin(), cnt.end(), row);
       }
       for (int c = 0; c < ncls; ++c) {
         cls_start[g * ncls + c] = (int)cls_e.size();
@@ -543,19 +557,153 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       }
     }
     cls_start[6 * ncls] = (int)cls_e.size();
+    std::vector<int> ckm((size_t)(nJ + 16) * hb.nkets, -1);
+    for (size_t t = 0; t < cls_e.size(); ++t) {
+      const int kk = cls_e[t], k = hb.kp[kk], l = hb.kq[kk];
+      const bool sw = hb.j2[k] > hb.j2[l];
+      rec.push_back(sw ? make_int2(l << 16 | k, 1) : make_int2(k << 16 | l, 0));
+      for (int J = 0; J < nJ; ++J) ckm[(size_t)J * hb.nkets + t] = hb.kmap[(size_t)kk * nJ + J];
+    }
     B.ncls = ncls;
+    B.cls_j = dupload(*this, cls_j, err);
     B.cls_start = dupload(*this, cls_start, err);
-    B.cls_e = dupload(*this, cls_e, err);
-    // per class entry: the ket and its orbits' quantum numbers in one record
-    std::vector<int4> rec(cls_e.size());
-    for (int g = 0; g < 6; ++g)
-      for (int t = cls_start[g * ncls]; t < cls_start[(g + 1) * ncls]; ++t) {
-        const int kk = grp_kets[grp_start[g] + cls_e[t]];
-        const int k = hb.kp[kk], l = hb.kq[kk];
-        rec[t] = make_int4(kk, (k << 16) | l, (hb.j2[k] << 16) | hb.j2[l],
-                           (hb.l[k] << 24) | (hb.l[l] << 16) | ((hb.tz2[k] + 1) << 8) | (hb.tz2[l] + 1));
-      }
+    B.cls_before = dupload(*this, before, err);
     B.cls_rec = dupload(*this, rec, err);
+    B.cls_kmap = dupload(*this, ckm, err);
+
+    const int nJp = B.ccjmax_ph + 1, nt = 4 * nJp, norb4 = (norb + 3) & ~3;
+    B.ccnt = nt;
+    std::vector<unsigned short> ccnt((size_t)norb * (norb + 1) * nt, 0), crank((size_t)norb * (nJp + 1) * norb4, 0xFFFF);
+    std::vector<int> crow((size_t)norb * nt, 0), cstart((size_t)norb * nt, 0), ccols;
+    for (int o = 0; o < norb; ++o) {
+      unsigned short *c0 = ccnt.data() + (size_t)o * (norb + 1) * nt;
+      for (int x = 0; x < norb; ++x, c0 += nt) {
+        std::copy(c0, c0 + nt, c0 + nt);
+        const int ts = 2 * (std::abs(hb.tz2[o] - hb.tz2[x]) / 2) + ((hb.l[o] + hb.l[x]) & 1);
+        const int lo = std::abs(hb.j2[o] - hb.j2[x]) / 2, hi = std::min((hb.j2[o] + hb.j2[x]) / 2, nJp - 1);
+        for (int J = lo; J <= hi; ++J) crank[((size_t)o * (nJp + 1) + J) * norb4 + x] = c0[nt + 4 * J + ts]++;
+      }
+      for (int t = 0; t < nt; ++t) {
+        const int J = t >> 2, c = 6 * J + 2 * (((t >> 1) & 1) + 1) + (t & 1);
+        cstart[(size_t)o * nt + t] = (int)ccols.size();
+        bool first = true;
+        for (int x = 0; x < norb; ++x) {
+          if ((((hb.l[o] + hb.l[x]) & 1) | 2 * (std::abs(hb.tz2[o] - hb.tz2[x]) / 2)) != (t & 3)) continue;
+          if (std::abs(hb.j2[o] - hb.j2[x]) > 2 * J || hb.j2[o] + hb.j2[x] < 2 * J) continue;
+          const int loc = hb.cmap[(size_t)ket_index(norb, std::min(o, x), std::max(o, x)) * nJ + J];
+          if (x >= o && first) {
+            crow[(size_t)o * nt + t] = loc;
+            first = false;
+          }
+          ccols.push_back(loc + (x > o ? cc_n[c] : 0));
+        }
+      }
+    }
+    for (int o = 0; o < norb; ++o)
+      for (int t = 0; t < nt; ++t)
+        B.cc_run = std::max(B.cc_run, ccnt[((size_t)o * (norb + 1) + norb) * nt + t] - ccnt[((size_t)o * (norb + 1) + o) * nt + t]);
+    B.cc_cnt = dupload(*this, ccnt, err);
+    B.cc_rank = dupload(*this, crank, err);
+    B.cc_row = dupload(*this, crow, err);
+    B.cc_cstart = dupload(*this, cstart, err);
+    B.cc_cols = dupload(*this, ccols, err);
+
+    // Items (pair, i | j << 16, k0 | k1 << 16, first ket | group << 28) of the bra (ij) and its
+    // kets whose smaller orbit k is in [k0, k1), such that the elements of Zbar they need fit
+    // in LDS, kInvpLds bytes with the tables (a range of one orbit may exceed them).  All items of one j = bra's second orbit run on one XCD,
+    // by ascending i: the work-groups of bras (i, j), (i + 1, j), ... read neighbouring
+    // rows of the same columns of Zbar.
+    int maxquad = 0, maxchunk = 0;
+    std::vector<int> bra_g(hb.nkets), bra_e(hb.nkets);
+    for (int g = 0; g < 6; ++g)
+      for (int e = grp_start[g]; e < grp_start[g + 1]; ++e) {
+        bra_g[grp_kets[e]] = g;
+        bra_e[grp_kets[e]] = e - grp_start[g];
+      }
+    // result quads of the kets [e0, e1) of the bra (ij); jquads: quads of J of its class c
+    std::vector<int> jquads((size_t)d1 * d1 * ncls);
+    for (int a = 0; a < d1; ++a)
+      for (int b = 0; b < d1; ++b)
+        for (int c = 0; c < ncls; ++c) {
+          const int ja = cls_j[c] >> 16, jb = cls_j[c] & 0xFFFF;
+          const int nj = std::min(2 * a + 2 * b + 2, ja + jb) / 2 - std::max(2 * std::abs(a - b), std::abs(ja - jb)) / 2 + 1;
+          jquads[((size_t)a * d1 + b) * ncls + c] = (std::max(nj, 0) + 3) / 4;
+        }
+    auto quads = [&](int i, int j, int g, int e0, int e1) {
+      const int *b0 = &before[(size_t)(grp_start[g] + g + e0) * ncls], *b1 = &before[(size_t)(grp_start[g] + g + e1) * ncls];
+      const int *nj = &jquads[((size_t)((hb.j2[i] - 1) / 2) * d1 + (hb.j2[j] - 1) / 2) * ncls];
+      int nq = 3;
+      for (int c = 0; c < ncls; ++c) nq += ((b1[c] - b0[c] + 3) >> 2) * nj[c];
+      return nq;
+    };
+    int allquads = 0;
+    for (int k = 0; k < hb.nkets; ++k) {
+      const int g = bra_g[k];
+      allquads = std::max(allquads, quads(hb.kp[k], hb.kq[k], g, bra_e[k], grp_start[g + 1] - grp_start[g]));
+    }
+    for (int v = 0; v < 2; ++v) {
+      const double es = v ? sizeof(float) : sizeof(double);  // and 2 bytes per chunk, one chunk more per block
+      const long cap = std::max(2048L, (long)((kInvpLds - InvpLds(nJ, nt, norb, ncls, allquads, 2 * nt).M - es) /
+                                              (es + 2.0 / 64)));
+      long maxel = 1;
+      std::vector<TileGroup> groups;
+      for (int j = 0; j < norb; ++j) {
+        TileGroup G;
+        for (int i = 0; i <= j; ++i) {
+          const int kb = ket_index(norb, i, j), g = bra_g[kb];
+          const unsigned short *ci = &ccnt[(size_t)i * (norb + 1) * nt], *cj = &ccnt[(size_t)j * (norb + 1) * nt];
+          const bool same = hb.tz2[i] == hb.tz2[j];
+          // elements of the kets with k in [k0, k1): rows x >= k0 of the columns y in [k0, k1) and
+          // rows x in [k0, k1) of the columns y >= k1; sets of the other Tz (same) have none
+          auto need = [&](int k0, int k1) {
+            const unsigned short *i0 = ci + (size_t)k0 * nt, *i1 = ci + (size_t)k1 * nt, *in = ci + (size_t)norb * nt;
+            const unsigned short *j0 = cj + (size_t)k0 * nt, *j1 = cj + (size_t)k1 * nt, *jn = cj + (size_t)norb * nt;
+            int tot = 0;
+            for (int t = 0; t < nt; ++t)
+              tot += (same && (t & 2)) ? 0 : (j1[t] - j0[t]) * (in[t] - i0[t]) + (jn[t] - j1[t]) * (i1[t] - i0[t]);
+            return (long)tot;
+          };
+          auto chunks = [&](int k0, int k1) {  // of 64 elements
+            int tot = 0;
+            for (int t = 0; t < nt; ++t) {
+              if (same && (t & 2)) continue;
+              const int W = ci[norb * nt + t] - ci[k0 * nt + t], w = ci[k1 * nt + t] - ci[k0 * nt + t];
+              const int s = cj[k1 * nt + t] - cj[k0 * nt + t], r = cj[norb * nt + t] - cj[k1 * nt + t];
+              tot += (s * W + 63) / 64 + (r * w + 63) / 64;
+            }
+            return tot;
+          };
+          for (int k0 = i; k0 < norb;) {
+            int k1 = norb;
+            long el = need(k0, k1);
+            if (el > cap) {  // the largest k1 that fits, at least k0 + 1
+              int lo = k0 + 1, hi = norb - 1;
+              while (lo < hi) {
+                const int mid = (lo + hi + 1) / 2;
+                if (need(k0, mid) <= cap) lo = mid; else hi = mid - 1;
+              }
+              k1 = lo;
+              el = need(k0, k1);
+            }
+            const int *gf = &grp_first[(size_t)g * (norb + 1)];
+            const int kets = gf[k1] - std::max(gf[k0], bra_e[kb]);
+            if (kets > 0) {
+              G.tiles.push_back(make_int4(0, i | j << 16, k0 | k1 << 16, std::max(gf[k0], bra_e[kb]) | g << 28));
+              G.cost += el + 4 * kets + 512;
+              maxel = std::max(maxel, el);
+              maxquad = std::max(maxquad, quads(i, j, g, gf[k1] - kets, gf[k1]));
+              maxchunk = std::max(maxchunk, chunks(k0, k1));
+            }
+            k0 = k1;
+          }
+        }
+        groups.push_back(G);
+      }
+      invp_items[v] = xcd_order(groups, kXcd);
+      invp_maxel[v] = maxel;
+    }
+    B.invp_nquad = maxquad;
+    B.invp_nchunk = maxchunk;
   }
 
   // ---- work lists ----
@@ -685,18 +833,8 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
       for (size_t j = bound[x]; j < bound[x + 1]; ++j) v[8 * (j - bound[x]) + x] = L[j];
     wl.mirror.swap(v);
   }
-  // inverse Pandya by orbit quadruple: one item (pair, group g, bra b, 0) per
-  // bra ket, whose work-group loops over the group kets e >= b; longest first
-  {
-    std::vector<std::pair<int, int4>> ts;
-    for (int g = 0; g < 6; ++g) {
-      const int gs = grp_start[g], ng = grp_start[g + 1] - gs;
-      for (int b = 0; b < ng; ++b) ts.push_back({ng - b, make_int4(0, g, b, 0)});
-    }
-    std::stable_sort(ts.begin(), ts.end(),
-                     [](const std::pair<int, int4> &x, const std::pair<int, int4> &y) { return x.first > y.first; });
-    for (auto &x : ts) wl.invp.push_back(x.second);
-  }
+  wl.invp = invp_items[0];
+  wl.invp32 = invp_items[1];
   for (int c = 0; c < nch; ++c) {
     const int nk = cc_n[c], nph = cc_nph[c];
     if (nk == 0 || nph == 0) continue;
@@ -727,11 +865,16 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
     return (int4 *)p;
   };
   d_pphh = up(wl.pphh); d_pphh64 = up(wl.pphh64); d_ph = up(wl.ph); d_pack = up(wl.pack);
-  d_pandya = up(wl.pandya); d_invp = up(wl.invp);
+  d_pandya = up(wl.pandya); d_invp = up(wl.invp); d_invp32 = up(wl.invp32);
   d_one = up(wl.one); d_mirror = up(wl.mirror); d_gen = up(wl.gen); d_ob221 = up(wl.ob221);
   d_c122w = up(wl.c122w);
   if (err.empty()) tune = t;
   return err;
+}
+
+size_t DeviceBasis::invp_lds(bool zbar_f32) const {
+  const InvpLds L(h.jmax + 1, h.ccnt, h.norb, h.ncls, h.invp_nquad, h.invp_nchunk);
+  return L.M + (invp_maxel[zbar_f32] + 1) * (zbar_f32 ? sizeof(float) : sizeof(double));
 }
 
 void DeviceBasis::release() {

@@ -63,7 +63,8 @@ struct WorkLists {
   std::vector<int4> pack;    // (pair, ch, k octet, 256-row block): bf16x3 panels of the 128x128-tile channels
   std::vector<int4> ph;      // (pair, cc, rb, sb), rb <= sb, tiles of 128 (ph_big) or 64
   std::vector<int4> pandya;  // (pair, cc, start, 0)
-  std::vector<int4> invp;    // (pair, group, bra, first ket) of the (parity, Tz) ket groups
+  std::vector<int4> invp;    // (pair, i | j << 16, k0 | k1 << 16, first ket | group << 28), FP64 Zbar; .y = -1: empty
+  std::vector<int4> invp32;  // the same with FP32 Zbar, twice the elements per item
   std::vector<int4> one;     // (pair, i, j, index of the one-body pair)
   std::vector<int4> ob221;   // (pair, one-body pair, kind/c/J, partial-sum slot) of the comm221 one-body part
   std::vector<int4> mirror;  // (pair, ch, rb, sb), rb < sb  and diagonal tiles; ch = -1: empty item
@@ -81,12 +82,15 @@ struct DeviceBasis {
   Tuning tune;
   int4 *d_pphh = nullptr, *d_pphh64 = nullptr, *d_ph = nullptr, *d_pandya = nullptr, *d_pack = nullptr,
        *d_invp = nullptr, *d_one = nullptr, *d_mirror = nullptr, *d_gen = nullptr, *d_ob221 = nullptr,
-       *d_c122w = nullptr;
+       *d_c122w = nullptr, *d_invp32 = nullptr;
   // host tables the work lists are built from
   std::vector<int> ch_n, k_start, cc_n, cc_nph, grp_start, grp_kets, gen_ok;
   std::vector<int> ch_kstart, c122_start;
   std::vector<int2> pairs1;
   std::vector<int4> c122w_items;  // the W kernel's items (basis only, not tuned)
+  std::vector<int4> invp_items[2];  // inverse Pandya items with FP64 and FP32 Zbar, and
+  long invp_maxel[2] = {1, 1};      // the most elements of Zbar that one of them holds
+  size_t invp_lds(bool zbar_f32) const;  // LDS bytes of the inverse Pandya kernel on this basis
   std::vector<int4> ob221;
   std::string upload(const HostBasis &hb, int emax6j);  // builds tables, lists, 6j table
   std::string build_lists(const Tuning &t);             // (re)builds and uploads the work lists

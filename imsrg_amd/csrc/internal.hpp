@@ -26,7 +26,8 @@ constexpr int kGW = 32;           // columns of a wave's sub-tile in the 128x128
 constexpr int kGN = kGW / 16;     // 16-column MFMA blocks per wave sub-tile
 constexpr int kGC = kTileK / kGWaves;  // k columns each wave copies into LDS per stage
 constexpr int kChunk = 256;       // elements per work item of the gather kernels
-constexpr int kJC = 8;            // J values per register chunk of the inverse Pandya gather (even)
+constexpr int kLdsUnit = 1280;    // LDS allocation unit in bytes, 128 of them in a CU
+constexpr int kInvpLds = 42 * kLdsUnit;  // LDS of an inverse Pandya work-group: three in a CU
 constexpr int kC122MaxN = 64;     // columns of a comm122 bin formed at once (a larger bin takes one item per 16)
 constexpr int kC122MaxCols = 150; // largest bin (LDS: 1 KiB of coefficients per ket)
 constexpr int kC122Rows = 128;    // rows of one comm122 W item (256: 221 against 210 us at emax = 10)
@@ -59,6 +60,7 @@ struct BasisDev {
   int maxn, maxcc, maxblk;
   int ccjmax_ph;  // largest J of a CC channel with ph kets (-1: none); Zbar is zero above it
   const IMSRG_G int *j2, *l, *tz2, *cvq;
+  const IMSRG_G int *orbcode;   // j2 | (l & 1) << 16 | (tz2 > 0) << 17, norb4 = norb rounded up to 4 entries
   const IMSRG_G double *occ;
   const IMSRG_G int *holes;
   const IMSRG_G int *obstart, *oblist;  // one-body block of each orbit
@@ -66,7 +68,14 @@ struct BasisDev {
   const IMSRG_G int *kmap, *cmap;
   const IMSRG_G int *cmapT;     // cmapT[J*nkets + k] = cmap[k*(jmax+1) + J]
   const IMSRG_G int *kmapT;     // kmapT[J*nkets + k] = kmap[k*(jmax+1) + J]
-  const IMSRG_G int *ccorb;     // ccorb[(i*(jmax+1) + J)*norb + x] = cmap of the ket (min(i,x), max(i,x)) at J
+  // the cross-coupled kets of one orbit o, by t = 4J + 2|tz_o - tz_x|/2 + parity for J <= ccjmax_ph
+  // (ccnt = 4 (ccjmax_ph + 1) such sets), in the order of the other orbit x:
+  const IMSRG_G unsigned short *cc_cnt;   // cc_cnt[(o*(norb+1) + k)*ccnt + t]: orbits x < k of set t
+  const IMSRG_G unsigned short *cc_rank;  // cc_rank[(o*(ccjmax_ph+2) + J)*norb4 + x]: position of x, or 0xFFFF
+  const IMSRG_G int *cc_row;    // cc_row[o*ccnt + t]: local index of the first ket (o, x >= o), the others follow
+  const IMSRG_G int *cc_cstart; // cc_cols[cc_cstart[o*ccnt + t] ..]: columns of Zbar, the local index of
+  const IMSRG_G int *cc_cols;   //   ket (x, o), plus the channel's size (its tail) for x > o
+  int ccnt, cc_run;             // cc_run: most kets of one channel with the same first orbit
   // kmorb[(x*norb + y)*kmorb_nx + J]: standard local index of the ket of orbits x and y at J, 0xffff
   // for none; kmorb_nx: jmax + 1 rounded up to a multiple of 8
   const IMSRG_G unsigned short *kmorb;
@@ -74,6 +83,7 @@ struct BasisDev {
   // kets of each (parity, Tz) group g = 2(Tz+1) + parity (the channels 6J + g),
   // ascending global index: grp_kets[grp_start[g] .. grp_start[g+1])
   const IMSRG_G int *grp_start, *grp_kets;
+  const IMSRG_G int *grp_first;  // grp_first[g*(norb+1) + k]: first ket of group g with an orbit p >= k
   // standard channels
   const IMSRG_G long *ch_off;
   const IMSRG_G int *ch_n, *ch_kstart, *ch_kets;
@@ -109,13 +119,14 @@ struct BasisDev {
   const IMSRG_G signed char *cc_phph; // cc_phi of the ket at each position of the cc_ph lists
   const IMSRG_G long *cc_xoff, *cc_zoff;
   long xsize, zsize;
-  // kets of each (parity, Tz) group g by (j_k, j_l) class c = ((j2k-1)/2) d1 + (j2l-1)/2: the group
-  // indices e, ascending, in cls_e[cls_start[g ncls + c] .. cls_start[g ncls + c + 1]), ncls = d1 * d1
-  const IMSRG_G int *cls_start, *cls_e;
-  // per cls_e entry, the ket and its orbits in one record: (ket, k << 16 | l,
-  // j2k << 16 | j2l, l_k << 24 | l_l << 16 | (tz2k + 1) << 8 | (tz2l + 1))
-  const IMSRG_G int4 *cls_rec;
+  // kets of each (parity, Tz) group g by the class c of their unordered pair of j, ja <= jb
+  // (cls_j[c] = ja << 16 | jb, as 2j): positions cls_start[g ncls + c] .. of the lists below,
+  // ascending kets; cls_before[(grp_start[g] + g + e) ncls + c]: those among the first e kets
+  const IMSRG_G int *cls_j, *cls_start, *cls_before;
+  const IMSRG_G int2 *cls_rec;  // (a << 16 | b, 1 if the ket is (b, a)): its orbits of ja and jb
+  const IMSRG_G int *cls_kmap;  // cls_kmap[J nkets + position]: local index at J or -1, J <= jmax + 16
   int ncls;
+  int invp_nquad, invp_nchunk;  // most result quads and 64-element chunks of an inverse Pandya item
   const IMSRG_G int2 *pairs1;   // one-body pairs (i<=j, same (l,j2,tz2) block)
   // partial sums of the one-body part: slots ob_start[p] .. ob_start[p+1]-1 of pair p
   // (the first: comm111 + comm121, the others: comm221 items); cpart: orbits with 1 - n_c != 0
@@ -125,10 +136,7 @@ struct BasisDev {
   const IMSRG_G double *w1norm; // norb*norb one-body norm weights
   const IMSRG_G double *sixj;   // dense 6j table, layout of SixJCache_112112
   const IMSRG_G double *sixjQ;  // (2 J6 + 1) times the values (0 where |6j| < 1e-8), layout
-                                // [jj1][jj2][J6][J3/2][jj4][jj5][J3%2] (sixjQ_index):
-                                // lanes of one (jj1, jj2, J6, J3 pair) that differ in jj4, jj5 read
-                                // neighbouring 16-byte entries; d2q = d2 rounded up to even
-  int d2q;
+                                // [jj1][jj2][jj4][jj5][J6][J3] (sixjQ_index)
   // generator lists: per channel, core-core kets and (non-core)-(non-core) kets
   const IMSRG_G int *gcore_start, *gcore_loc, *gnc_start, *gnc_loc;
 };
@@ -170,11 +178,29 @@ struct PairArg {
   }
 };
 
+// LDS layout of the inverse Pandya kernel, in bytes
+struct InvpLds {
+  int set, q, z, cls, row, cf, pre, tab, blk, chunk, M;
+  __host__ __device__ InvpLds(int nJ, int nt, int norb, int ncls, int nquad, int nchunk) {
+    set = 0;                       // int4[nt]: columns in [k0, k1), orbits < k0 of j's and of i's set
+    q = set + 16 * nt;             // int4[2 nt]: offset, rows, columns, first entry of cc_cols of the blocks
+    z = q + 32 * nt;               // int4[nt]: offset of the first row's elements (low, high), CC channel size
+    cls = z + 16 * nt;             // int4[2 ncls]: the classes' kets and J (first ncls) and J' and weights
+    row = cls + 32 * ncls;         // long[nJ + 16]: byte offset of the bra's row of the channel 6J + g, or -1
+    cf = row + 8 * (nJ + 16);      // int[2 nt + 2]: first chunk of each block, then all elements
+    pre = cf + 4 * (2 * nt + 2);   // int[ncls + 1]: first result quad of each class
+    tab = (pre + 4 * (ncls + 1) + 15) & ~15;    // ushort2[(nt / 4 + 1) norb4]: column offset and row of (J', orbit)
+    blk = tab + (nt + 4) * ((norb + 3) & ~3);   // unsigned[nquad]: class << 20 | J quad << 15 | ket quad of the results
+    chunk = blk + 4 * nquad;       // ushort[nchunk]: block of each chunk
+    M = (chunk + 2 * nchunk + 15) & ~15;
+  }
+};
+
 __host__ __device__ inline int ket_index(int norb, int p, int q) { return p * (2 * norb - 1 - p) / 2 + q; }
 __host__ __device__ inline int sgn_parity(int x) { return (x & 1) ? -1 : 1; }
-__host__ __device__ inline long sixjQ_index(int d1, int d2q, int jj1, int jj2, int J3, int jj4, int jj5, int J6) {
-  return ((((((long)((jj1 - 1) >> 1) * d1 + ((jj2 - 1) >> 1)) * d2q + J6) * (d2q >> 1) + (J3 >> 1)) * d1 +
-           ((jj4 - 1) >> 1)) * d1 + ((jj5 - 1) >> 1)) * 2 + (J3 & 1);
+__host__ __device__ inline long sixjQ_index(int d1, int d2, int jj1, int jj2, int J3, int jj4, int jj5, int J6) {
+  return (((((long)((jj1 - 1) >> 1) * d1 + ((jj2 - 1) >> 1)) * d1 + ((jj4 - 1) >> 1)) * d1 + ((jj5 - 1) >> 1)) * d2 +
+          J6) * d2 + J3;
 }
 __host__ __device__ inline long sixj_index(int d1, int d2, int jj1, int jj2, int J3, int jj4, int jj5, int J6) {
   return (((((long)((jj1 - 1) >> 1) * d1 + ((jj2 - 1) >> 1)) * d2 + J3) * d1 + ((jj4 - 1) >> 1)) * d1 +

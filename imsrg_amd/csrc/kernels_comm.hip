@@ -507,9 +507,13 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
 //         B = Ybar^T, h = +1 (Z Hermitian) or -1.
 // PH true, tail of Zbar (src/Commutator.cc:1788-1789, 1805): B columns permuted
 //         by ab <-> ba with weights hY*phi(ph ket), cph(s) = phi(s), h = +1.
-// The ph GEMM stores Zbar in full: the lower triangle as (head) hZ-sign or (tail)
-// phi_r phi_s times the upper element, as the reference's folds make it
-// (src/Commutator.cc:1792-1805), written through an LDS transpose.
+// The ph GEMM stores the upper triangle of Zbar and, of the lower one, the elements whose
+// two kets have the same first orbit (all that the inverse Pandya reads): they lie within
+// cc_run of the diagonal, so that sub-tiles further off leave their mirror image out.  The
+// lower elements are (head) hZ-sign or (tail) phi_r phi_s times the upper ones, as the
+// reference's folds make them (src/Commutator.cc:1792-1805), written through an LDS
+// transpose.  Without the others the ph GEMM takes 420 us at emax = 10 (FP64; 472 with them) and
+// 335 us with FP32 products (355).
 // MIXED: operands rounded to FP32 when read from LDS, products on f32
 // 16x16x4 MFMA, FP32 partial sums over two stages (32 k) added into the FP64
 // accumulators.
@@ -551,14 +555,14 @@ __device__ __forceinline__ bool tile_wave_live(int R0, int S0, int n, int w) {
 // Stores a 128x128 tile from the waves' FP64 accumulators (lane layout of the
 // f32 MFMAs when F32L, else of the f64 16x16x4 MFMA).
 // PH false: the upper triangle of D = alpha * acc.
-// PH true: Zbar in full through LDS transposes of the 64 x kGW wave sub-tiles,
+// PH true: Zbar (the lower triangle near the diagonal) through LDS transposes of the 64 x kGW wave sub-tiles,
 // four per round in the buffers tb0..tb3 (each >= 64 (kGW + 1) doubles): the
 // lower triangle as (head) h or (tail) phi_r phi_s times the upper element, as
 // the reference's folds make it (src/Commutator.cc:1792-1805); s_ph holds the
 // tile's row (0) and column (1) phases in the tail (h = 1) and 1 in the head.
 template <bool PH, bool F32L, typename TD = double>
 __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, int n, int R0, int S0,
-                                              double alpha, double h, const signed char (*s_ph)[kTileB],
+                                              double alpha, double h, int run, const signed char (*s_ph)[kTileB],
                                               double *tb0, double *tb1, double *tb2, double *tb3) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = (wv & 1) * 64, wc = (wv >> 1) * kGW;
@@ -615,28 +619,6 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
                 if (row + q < n && row + q <= col) st_nt(dp + q, Tt[rr + q][cc]);
             }
           }
-          for (int e = threadIdx.x; e < 16 * kGW; e += blockDim.x) {
-            const int cc = 4 * (e & (kGW / 4 - 1)), rr = e / (kGW / 4);
-            const int row2 = S1 + cc, col2 = R1 + rr;
-            if (col2 >= n || row2 >= n) continue;
-            double v[4];
-            bool ok[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              ok[q] = row2 + q < n && row2 + q > col2;
-              // phases from LDS: row2 + q - S0 and col2 - R0 lie in [0, 128)
-              const double sq = h * (double)(s_ph[1][min(row2 + q - S0, kTileB - 1)] * s_ph[0][col2 - R0]);
-              v[q] = sq * Tt[rr][cc + q];
-            }
-            float *dp = D + (long)col2 * n + row2;
-            if (ok[0] && ok[1] && ok[2] && ok[3]) {
-              st_nt4(dp, v[0], v[1], v[2], v[3]);
-            } else {
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                if (ok[q]) st_nt(dp + q, v[q]);
-            }
-          }
         } else {
           // Two rows per thread and one 16-byte store where both are written (store
           // instructions, not bytes, bound this epilogue); R1 and S1 are even.
@@ -651,26 +633,15 @@ __device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, 
             else
               st_nt(dp, Tt[rr][cc]);
           }
-          // mirrored elements (S1 + cc, R1 + rr) = sym * upper (R1 + rr, S1 + cc),
-          // consecutive threads on consecutive row pairs S1 + cc
-          for (int e = threadIdx.x; e < 32 * kGW; e += blockDim.x) {
-            const int cc = 2 * (e & (kGW / 2 - 1)), rr = e / (kGW / 2);
-            const int row2 = S1 + cc, col2 = R1 + rr;
-            if (col2 >= n || row2 >= n) continue;
-            const bool lo = row2 > col2, hi = row2 + 1 < n && row2 + 1 > col2;
-            // phases from LDS: row2 - S0 and col2 - R0 lie in [0, 128)
-            const double s0 = h * (double)(s_ph[1][row2 - S0] * s_ph[0][col2 - R0]);
-            TD *dp = D + (long)col2 * n + row2;
-            if (lo && hi) {
-              const double s1 = h * (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
-              st_nt2(dp, s0 * Tt[rr][cc], s1 * Tt[rr][cc + 1]);
-            } else if (lo) {
-              st_nt(dp, s0 * Tt[rr][cc]);
-            } else if (hi) {
-              const double s1 = h * (double)(s_ph[1][row2 + 1 - S0] * s_ph[0][col2 - R0]);
-              st_nt(dp + 1, s1 * Tt[rr][cc + 1]);
-            }
-          }
+        }
+        // mirrored elements (S1 + cc, R1 + rr) = sym * upper (R1 + rr, S1 + cc), near the diagonal
+        if (S1 - (R1 + 63) >= run) continue;
+        for (int e = threadIdx.x; e < 64 * kGW; e += blockDim.x) {
+          const int cc = e & (kGW - 1), rr = e / kGW;
+          const int row2 = S1 + cc, col2 = R1 + rr;
+          if (col2 >= n || row2 >= n || row2 <= col2) continue;
+          // phases from LDS: row2 - S0 and col2 - R0 lie in [0, 128)
+          st_nt(D + (long)col2 * n + row2, h * (double)(s_ph[1][row2 - S0] * s_ph[0][col2 - R0]) * Tt[rr][cc]);
         }
       }
       __syncthreads();
@@ -919,7 +890,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items, int nit
   }
   if constexpr (MIXED) flush_t();  // a last stage without its pair
   static_assert(64 * (kGW + 1) <= kTileK * LD, "transpose tile exceeds the operand buffer");
-  gemm_epilogue<PH, MIXED, ZT>(acc, D, n, R0, S0, alpha, h, s_ph, &A0[0][0], &A1[0][0], &B0[0][0], &B1[0][0]);
+  gemm_epilogue<PH, MIXED, ZT>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, &A0[0][0], &A1[0][0], &B0[0][0], &B1[0][0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1130,7 +1101,7 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items, int 
   }
   static_assert(2 * 64 * (kGW + 1) * sizeof(double) <= sizeof(StageB3), "transpose tiles exceed the stage buffer");
   double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<true, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<true, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
 }
 
 // ---------------------------------------------------------------------------
@@ -1292,7 +1263,7 @@ __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, co
     }
   }
   double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
 }
 
 __global__ __launch_bounds__(kGWaves * 64, 2) void k_ph_big_b3(PairArg pa, const int4 *items, int nitems) {
@@ -1438,282 +1409,335 @@ __global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
   front_pandya(pa.get(it.x), it, lds_raw);
 }
 
-// wave-wide min / max of an int, returned as a wave-uniform (scalar) value
-__device__ __forceinline__ int wave_min(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-  return __builtin_amdgcn_readfirstlane(v);
-}
-__device__ __forceinline__ int wave_max(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return __builtin_amdgcn_readfirstlane(v);
+// AddInversePandyaTransformation (src/Commutator.cc:1501-1616), by bra.
+//   Z^J_{ij,kl} += f(J) [ sum_J' (2J'+1) {ji jj J; jk jl J'} M^{J'}(l, k)
+//                        - (-1)^{(jk+jl)/2 - J} sum_J' (2J'+1) {jj ji J; jk jl J'} M^{J'}(k, l) ] / norm
+// with M^{J'}(x, y) = Zbar^{J'}[(ix), (yj)] of the bra (ij); i <= k <= l, so that the rows
+// (i, x) of a column follow one another in x.  f(J) stands for the second sum where k = l
+// or i = j (1 - (-1)^{(jk+jl)/2 - J}, with (-1)^{(ji+jj+jk+jl)/2} for i = j).
+// One work-group per bra, or per range [k0, k1) of its kets' k where the bra's M exceeds
+// kInvpM bytes.  It
+//  * lays out M in LDS by sets t = (J', parity and |tz| of (i, x)), each in two blocks: the
+//    columns y in [k0, k1) with the rows x >= k0, then the columns y >= k1 with the rows x in
+//    [k0, k1); and a table over (J', orbit) of the orbit's column offset and row;
+//  * copies M in chunks of 64 elements of one block, each read once;
+//  * takes the kets 16 at a time by class (ja <= jb, the unordered j of k and l): the class's
+//    weights W(J, J') times the gathered M(J', ket) on the FP64 matrix units, 16 J at once.
+//    A ket with jk > jl is its class's with both sums exchanged, which is the factor
+//    -(-1)^{(jk+jl)/2 - J} on the result.
+// sixjQ holds the weights (2J'+1) {...}, with zeros where the reference skips |6j| < 1e-8.
+// CC channels without ph kets (Zbar = 0, not written by the ph GEMM) are read as zeros.
+// TZ is the element type of Zbar: float after the FP32-product ph GEMM, double otherwise;
+// the sums are FP64.  Every upper element (ij <= kl, or ij < kl for anti-Hermitian Z) of
+// every channel is produced exactly once and stored at its transposed slot (row ib of
+// channel J, written for this bra only); k_finish adds it to the upper triangle, the
+// diagonal is kept apart.
+// A lane per ket that gathered its elements from memory (the kernel before this one) read
+// the lines again for each class with a ket in them, 3.4 GB at emax = 10 where 0.4 GB are
+// needed, and was bound by that: 594 us at emax = 10 FP64, 531 us with FP32 Zbar, 2310 us at
+// emax = 12 with FP32 Zbar.  Now 395, 342 and 1360 us; 0.6 GB read.  What bounds it now is
+// instruction issue and latency, in about equal parts of the tables, the copies and the
+// results: 24 waves per CU, 45% of the cycles with a vector instruction issued.  Tried:
+// 16x16x4 matrix instructions on blocks of 16 J x 16 kets (a class of a bra has 13 kets and
+// 3.4 J on average): 590 us.
+constexpr int kInvpU = 8;    // chunks in flight per wave
+constexpr int kInvpW = 2;    // steps of 4 J' whose weights are loaded a block ahead
+
+// inclusive prefix sum over the wave
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
 }
 
-// AddInversePandyaTransformation (src/Commutator.cc:1501-1616), by orbit quadruple.
-// One work-group per bra ket (ij) of a (parity, Tz) group; its lanes take the
-// group's kets (kl) = e >= (ij) in (j_k, j_l) class order, so that the lanes of
-// a wave mostly share their J and J' ranges (one lane per ket, in chunks of the
-// work-group size).  The cross-coupled elements Zbar^{J'}[(il),(kj)] (direct) and
-// Zbar^{J'}[(jl),(ki)] (exchange) do not depend on the standard-channel J, so
-// each is loaded once and recoupled into every J of the quadruple (register
-// chunks of kJC values):
-//   commij(J) = -sum_J' (2J'+1) {ji jj J; jk jl J'} Zbar^{J'}[il, kj]
-//   commji(J) = -sum_J' (2J'+1) {jj ji J; jk jl J'} Zbar^{J'}[jl, ki]
-//   Z^J_{ij,kl} += -(commij - (-1)^{(jk+jl)/2 - J} commji) / norm
-// The 6j copy sixjQ holds the weights (2J'+1) {...}, with zeros where the
-// reference skips |6j| < 1e-8.  Every J of a chunk is accumulated unmasked: a J
-// outside the lane's triangles has a zero 6j, and the accumulators of J values
-// the lane does not own (odd J of a (p,p) ket, J past the range) are never
-// stored.  CC channels without ph kets (Zbar = 0, not written by the ph GEMM)
-// are skipped.  TZ is the element type of Zbar: float after the FP32-product ph
-// GEMM, double otherwise; the sums are FP64.  The cross-coupled local indices of
-// the kets (i,x) and (j,x), the CC channel sizes/offsets and the bra's
-// standard-channel data are staged in LDS once per work-group.  Every upper
-// element (ij <= kl, or ij < kl for anti-Hermitian Z) of every channel is
-// produced exactly once and stored at its transposed slot (row ib of channel J,
-// written by this work-group only, so the L2 merges the lanes' scattered
-// stores); k_finish adds it to the upper triangle, the diagonal is kept apart.
-__host__ __device__ inline size_t invp_lds_bytes(int jmax, int norb, int nch, int ncls) {
-  const size_t nJ = (size_t)jmax + 1;
-  return 8 * (size_t)nch + 8 * nJ + 4 * (size_t)nch + 4 * nJ * (2 * (size_t)norb + 3) + 4 * (2 * (size_t)ncls + 1);
+// element at a 32-bit byte offset of a (wave-uniform) base
+template <class T>
+__device__ __forceinline__ T ld_at(const IMSRG_G void *base, unsigned off) {
+  return *(const IMSRG_G T *)((const IMSRG_G char *)base + off);
 }
 
-template <typename TZ>
-__global__ __launch_bounds__(256, 5) void k_invpandya(PairArg pa, const int4 *items) {
+template <typename TZ, int kT>
+__global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *items) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int4 it = items[blockIdx.x];
+  if (it.y < 0) return;  // padding item of the XCD-balanced order
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
-  const int g = it.y, b = it.z;
+  const int i = it.y & 0xFFFF, j = it.y >> 16, k0 = it.z & 0xFFFF, k1 = it.z >> 16, g = it.w >> 28;
+  const int nk = B.nkets, norb = B.norb, nJ = B.jmax + 1, nt = B.ccnt, nJp = nt >> 2, ncls = B.ncls;
+  const int d1 = B.d1, d2 = B.d2;
+  const int norb4 = (norb + 3) & ~3;  // entries of a table row
+  const InvpLds L(nJ, nt, norb, ncls, B.invp_nquad, B.invp_nchunk);
+  int4 *s_set = (int4 *)(lds_raw + L.set), *s_q = (int4 *)(lds_raw + L.q), *s_z = (int4 *)(lds_raw + L.z);
+  int4 *s_cls = (int4 *)(lds_raw + L.cls), *s_cls2 = s_cls + ncls;
+  long *s_row = (long *)(lds_raw + L.row);
+  int *s_cf = (int *)(lds_raw + L.cf), *s_pre = (int *)(lds_raw + L.pre);
+  unsigned *tabw = (unsigned *)(lds_raw + L.tab);
+  const unsigned short *tab = (const unsigned short *)tabw;
+  unsigned *s_blk = (unsigned *)(lds_raw + L.blk);
+  unsigned short *s_chunk = (unsigned short *)(lds_raw + L.chunk);
+  TZ *M = (TZ *)(lds_raw + L.M);
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int nw = kT / 64;
+  // the kets elo .. ehi of the group; a range that starts at the bra's own orbit starts at
+  // the bra, or after it (anti-Hermitian Z)
+  const int elo = (it.w & 0xFFFFFFF) + (k0 == i && P.hZ != 1 ? 1 : 0), ehi = B.grp_first[g * (norb + 1) + k1];
   const int gs = B.grp_start[g];
-  const int nk = B.nkets, norb = B.norb, nJ = B.jmax + 1, nch = B.nch;
-  long *s_zoff = (long *)lds_raw;      // [nch] CC channel offsets in Zbar
-  long *s_choff = s_zoff + nch;        // [nJ]  offsets of the standard channels 6J + g
-  int *s_ccn = (int *)(s_choff + nJ);  // [nch] CC channel sizes
-  int *s_chn = s_ccn + nch;            // [nJ]  sizes of the standard channels 6J + g
-  int *s_ib = s_chn + nJ;              // [nJ]  local index of the bra in channel 6J + g
-  int *s_chks = s_ib + nJ;             // [nJ]  first ket (all-channel index) of channel 6J + g
-  int *Ti = s_chks + nJ;               // [nJ * norb] CC local index of ket (i,x) in channel J'
-  int *Tj = Ti + nJ * norb;            // [nJ * norb] CC local index of ket (j,x) in channel J'
-  const int ncls = B.ncls;
-  int *s_us = Tj + nJ * norb;          // [ncls] first position of class c with e >= emin
-  int *s_pre = s_us + ncls;            // [ncls + 1] positions of the classes in the bra's ket order
-  const int kb = B.grp_kets[gs + b];
-  const int emin = (P.hZ == 1) ? b : b + 1;
-  const int i = B.kp[kb], j = B.kq[kb];
-  // a CC channel without ph kets has Zbar = 0, which the ph GEMM does not write:
-  // offset -1 marks it, and its terms are skipped
-  for (int c = threadIdx.x; c < nch; c += blockDim.x) {
-    s_zoff[c] = B.cc_nph[c] > 0 ? B.cc_zoff[c] : -1;
-    s_ccn[c] = B.cc_n[c];
+  const int oi = B.orbcode[i], oj = B.orbcode[j], ji = oi & 0xFFFF, jj = oj & 0xFFFF;
+  const bool same = i == j;
+  // the table as it is in memory, four orbits per thread: their positions in j's and in i's set
+  // at J', or 0xFFFF
+  const IMSRG_G uint2 *rkj = (const IMSRG_G uint2 *)(B.cc_rank + (long)j * (nJp + 1) * norb4);
+  const IMSRG_G uint2 *rki = (const IMSRG_G uint2 *)(B.cc_rank + (long)i * (nJp + 1) * norb4);
+  const int ntab = (nJp + 1) * norb4 >> 2;
+  for (int e0 = threadIdx.x; e0 < ntab; e0 += 2 * kT) {
+    const int e1 = min(e0 + kT, ntab - 1);
+    const uint2 y0 = rkj[e0], x0 = rki[e0], y1 = rkj[e1], x1 = rki[e1];
+    uint4 *d = (uint4 *)tabw;
+    d[e0] = make_uint4((y0.x & 0xFFFF) | x0.x << 16, y0.x >> 16 | (x0.x & 0xFFFF0000), (y0.y & 0xFFFF) | x0.y << 16,
+                       y0.y >> 16 | (x0.y & 0xFFFF0000));
+    if (e0 + kT < ntab)
+      d[e1] = make_uint4((y1.x & 0xFFFF) | x1.x << 16, y1.x >> 16 | (x1.x & 0xFFFF0000), (y1.y & 0xFFFF) | x1.y << 16,
+                         y1.y >> 16 | (x1.y & 0xFFFF0000));
   }
-  for (int J = threadIdx.x; J < nJ; J += blockDim.x) {
-    s_choff[J] = B.ch_off[6 * J + g];
-    s_chn[J] = B.ch_n[6 * J + g];
-    s_ib[J] = B.kmapT[(long)J * nk + kb];
-    s_chks[J] = B.ch_kstart[6 * J + g];
-  }
-  // the bra's rows of the per-orbit cross-coupled index table: contiguous reads
-  const IMSRG_G int *ci = B.ccorb + (long)i * nJ * norb, *cj = B.ccorb + (long)j * nJ * norb;
-  for (int e = threadIdx.x; e < nJ * norb; e += blockDim.x) {
-    Ti[e] = ci[e];
-    Tj[e] = cj[e];
-  }
-  // kets e >= emin taken class by class: the lanes of a wave then mostly share
-  // j_k and j_l, hence their J and J' ranges
-  for (int c = threadIdx.x; c < ncls; c += blockDim.x) {
-    int lo = B.cls_start[g * ncls + c];
-    const int end = B.cls_start[g * ncls + c + 1];
-    int hi = end;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (B.cls_e[mid] < emin) lo = mid + 1; else hi = mid;
+  if (wv == 0) {
+    for (int t = lane; t < nt; t += 64) {
+      const IMSRG_G unsigned short *ci = B.cc_cnt + (long)i * (norb + 1) * nt + t;
+      const IMSRG_G unsigned short *cj = B.cc_cnt + (long)j * (norb + 1) * nt + t;
+      const int ci0 = ci[k0 * nt], cj0 = cj[k0 * nt], cii = ci[i * nt];
+      int W = ci[norb * nt] - ci0, w = ci[k1 * nt] - ci0;
+      const int ns = cj[k1 * nt] - cj0, ny = cj[norb * nt] - cj0;
+      if ((t & 2) && !((oi ^ oj) >> 17)) W = w = 0;  // kets of the other Tz
+      const int cc = 6 * (t >> 2) + 2 * (((t >> 1) & 1) + 1) + (t & 1), cst = B.cc_cstart[j * nt + t] + cj0;
+      const long zo = B.cc_nph[cc] > 0 ? B.cc_zoff[cc] + B.cc_row[i * nt + t] + ci0 - cii : -1;
+      s_set[t] = make_int4(ns, cj0, ci0, 0);
+      s_q[2 * t] = make_int4(0, W, ns, cst);
+      s_q[2 * t + 1] = make_int4(0, w, ny - ns, cst + ns);
+      s_z[t] = make_int4((int)(zo & 0xFFFFFFFF), (int)(zo >> 32), B.cc_n[cc], 0);
     }
-    s_us[c] = lo;
-    s_pre[c + 1] = end - lo;
+  } else if (wv == 1) {
+    const long kb = ket_index(norb, i, j);
+    for (int J = lane; J < nJ + 16; J += 64) {
+      const int ib = J < nJ ? B.kmapT[J * (long)nk + kb] : -1;
+      s_row[J] = ib < 0 ? -1 : 8 * (B.ch_off[6 * J + g] + (long)ib * B.ch_n[6 * J + g]);
+    }
+  } else if (wv < 4) {
+    for (int c = threadIdx.x - 128; c < ncls; c += 128) {
+      const IMSRG_G int *bf = B.cls_before + (long)(gs + g) * ncls + c;
+      const int lo = bf[(long)elo * ncls], cnt = elo < ehi ? bf[(long)ehi * ncls] - lo : 0;
+      const int jab = B.cls_j[c], ja = jab >> 16, jb = jab & 0xFFFF;
+      const int Jlo = max(abs(ji - jj), abs(ja - jb)) / 2, nj = min(ji + jj, ja + jb) / 2 - Jlo + 1;
+      const int Dlo = max(abs(ji - jb), abs(jj - ja)) / 2, nD = min(min(ji + jb, jj + ja) / 2, nJp - 1) - Dlo + 1;
+      const int Xlo = max(abs(jj - jb), abs(ji - ja)) / 2, nX = min(min(jj + jb, ji + ja) / 2, nJp - 1) - Xlo + 1;
+      s_cls[c] = make_int4(B.cls_start[g * ncls + c] + lo, cnt, Jlo | (ja + jb) / 2 << 16, (max(nj, 0) + 3) >> 2);
+      // the two sums' rows of weights at J' = 0, first J', and steps of 4 J'
+      s_cls2[c] = make_int4((int)(sixjQ_index(d1, d2, ji, jj, 0, ja, jb, 0) / d2),
+                            (int)(sixjQ_index(d1, d2, jj, ji, 0, ja, jb, 0) / d2), Dlo | Xlo << 16,
+                            (max(max(nD, same ? 0 : nX), 0) + 3) >> 2);
+    }
   }
   __syncthreads();
-  // inclusive prefix sum of s_pre[1..ncls] by the first wave, 64 classes per pass
-  if (threadIdx.x < 64) {
-    if (threadIdx.x == 0) s_pre[0] = 0;
-    int carry = 0;
+  // prefix sums: element offsets and chunks of the blocks (wave 0), result quads of the classes
+  // (wave 1)
+  if (wv == 0) {
+    int sum = 0;  // chunks << 17 | elements
+    for (int q0 = 0; q0 < 2 * nt; q0 += 64) {
+      const int q = q0 + lane;
+      const int va = q < 2 * nt ? s_q[q].y * s_q[q].z : 0, v = ((va + 63) >> 6) << 17 | va;
+      const int p = sum + wave_scan(v);
+      if (q < 2 * nt) {
+        s_q[q].x = (p - v) & 0x1FFFF;
+        s_cf[q] = (p - v) >> 17;
+      }
+      sum = __builtin_amdgcn_readlane(p, 63);
+    }
+    if (lane == 0) {
+      s_cf[2 * nt] = sum >> 17;
+      s_cf[2 * nt + 1] = sum & 0x1FFFF;
+    }
+  } else if (wv == 1) {
+    int sum = 0;
     for (int c0 = 0; c0 < ncls; c0 += 64) {
-      const int c = c0 + (int)threadIdx.x;
-      int v = c < ncls ? s_pre[c + 1] : 0;
-      for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, 64);
-        if ((int)threadIdx.x >= o) v += u;
-      }
-      if (c < ncls) s_pre[c + 1] = v + carry;
-      carry += __shfl(v, 63, 64);
+      const int c = c0 + lane;
+      const int v = c < ncls ? ((s_cls[c].y + 3) >> 2) * s_cls[c].w : 0;
+      const int p = sum + wave_scan(v);
+      if (c < ncls) s_pre[c] = p - v;
+      sum = __builtin_amdgcn_readlane(p, 63);
     }
+    if (lane == 0) s_pre[ncls] = sum;
   }
   __syncthreads();
-  const int total = s_pre[ncls];
-  const int jji = B.j2[i], jjj = B.j2[j];
-  const int li = B.l[i], tzi = B.tz2[i];
-  const int d2q = B.d2q;
-  const double hf = (P.hZ == 1) ? 1.0 : -1.0;
-  const TZ *Zb = reinterpret_cast<const TZ *>(P.Zbar);  // FP32 after the FP32-product ph GEMM
-  double *Ztwo = P.Z + B.two_off;
-  const IMSRG_G double *sixq = B.sixjQ;  // held in registers: the stores below could alias B
-  const IMSRG_G int *kmapT = B.kmapT;
-  for (int q0 = 0; q0 < total; q0 += blockDim.x) {
-    const int q = q0 + threadIdx.x;
-    const bool active = q < total;
-    int clo = 0, chi = ncls;  // class of position q: s_pre[clo] <= q < s_pre[chi]
-    while (chi - clo > 1) {
-      const int mid = (clo + chi) >> 1;
-      if (s_pre[mid] <= q) clo = mid; else chi = mid;
-    }
-    const int4 rc = B.cls_rec[active ? s_us[clo] + q - s_pre[clo] : 0];
-    const int kk = active ? rc.x : kb;
-    const int k = active ? rc.y >> 16 : i, l = active ? rc.y & 0xFFFF : j;  // i <= k <= l
-    const int jjk = active ? rc.z >> 16 : jji, jjl = active ? rc.z & 0xFFFF : jjj;
-    const int lk = active ? rc.w >> 24 : B.l[i], ll = active ? (rc.w >> 16) & 0xFF : B.l[j];
-    const int tzk = active ? ((rc.w >> 8) & 0xFF) - 1 : B.tz2[i], tzl = active ? (rc.w & 0xFF) - 1 : B.tz2[j];
-    const bool pauli = (i == j) || (k == l);  // kets (p,p) exist for even J only
-    int Jlo = max(abs(jji - jjj), abs(jjk - jjl)) / 2, Jhi = min(jji + jjj, jjk + jjl) / 2;
-    if (pauli) {
-      Jlo += Jlo & 1;
-      Jhi -= Jhi & 1;
-    }
-    const bool live = active && Jlo <= Jhi;
-    if (!live) {
-      Jlo = 1 << 20;
-      Jhi = -1;
-    }
-    const int wlo = wave_min(Jlo), whi = wave_max(Jhi);
-    if (wlo > whi) continue;  // wave-uniform: no lane of this wave has a channel
-    // direct term: CC channels of (i,l) for J' in tri(ji,jl) ∩ tri(jk,jj)
-    const int jpz = B.ccjmax_ph;  // Zbar is zero for J' above it
-    int Dlo = max(abs(jji - jjl), abs(jjk - jjj)) / 2, Dhi = min(min(jji + jjl, jjk + jjj) / 2, jpz);
-    if (!live) {
-      Dlo = 1 << 20;
-      Dhi = -1;
-    }
-    const int dlo = wave_min(Dlo), dhi = wave_max(Dhi);
-    // exchange term: CC channels of (i,k) for J' in tri(jj,jl) ∩ tri(jk,ji)
-    const bool exch = live && k != l && i != j;
-    int Xlo = max(abs(jjj - jjl), abs(jjk - jji)) / 2, Xhi = min(min(jjj + jjl, jjk + jji) / 2, jpz);
-    if (!exch) {
-      Xlo = 1 << 20;
-      Xhi = -1;
-    }
-    const int xlo = wave_min(Xlo), xhi = wave_max(Xhi);
-    const int pd = (li + ll) & 1, td = abs(tzi - tzl) / 2;
-    const int px = (li + lk) & 1, tx = abs(tzi - tzk) / 2;
-    // 6j entries of J' and the J pair (c0, c0+1) sit at s6 + J' * s6J + (c0/2) * s6P; the next
-    // pair (c0+2, c0+3) one pair stride further
-    const long s6P = 2L * B.d1 * B.d1, s6J = s6P * (d2q >> 1);
-    const long s6d = sixjQ_index(B.d1, d2q, jji, jjj, 0, jjk, jjl, 0);
-    const long s6x = sixjQ_index(B.d1, d2q, jjj, jji, 0, jjk, jjl, 0);
-    // tail element T(ik, lj) = phi_ik phi_lj T(lj, ik), phi_pq = (-1)^{(j_p+j_q)/2};
-    // head H(ik, lj) = hZ-sign H(lj, ik)
-    const double symx = (l > j) ? (double)sgn_parity((jji + jjk) / 2 + (jjl + jjj) / 2) : hf;
-    const int dbra = (i == j), dket = (k == l);
-    const double nrm = (dbra == dket) ? 1.0 + dbra : SQRT2_D;
-    const double pij = sgn_parity((jji + jjj + jjk + jjl) / 2);
-    // J chunks start at even J so that each pair of 6j values is one aligned 16-byte load
-    for (int c0 = wlo & ~1; c0 <= whi; c0 += kJC) {
-      unsigned vm = 0;  // lane's valid J of this chunk
-#pragma unroll
-      for (int t = 0; t < kJC; ++t) {
-        const int J = c0 + t;
-        if (J >= Jlo && J <= Jhi && !(pauli && (J & 1))) vm |= 1u << t;
-      }
-      // acc(J) = sum_J' w_d z_d - (-1)^{(jk+jl)/2 - J} sum_J' w_x z_x, i.e. -(commij - sign commji)
-      // before the special cases k == l, i == j (no exchange sum; factor applied below)
-      double acc[kJC];
-#pragma unroll
-      for (int t = 0; t < kJC; ++t) acc[t] = 0.0;
-      // symx times -(-1)^{(jk+jl)/2 - J} at J = c0
-      const double fx = symx * -(double)sgn_parity((jjk + jjl) / 2 - c0);
-      // two J' per step, the loads of both (Zbar element, three 16-byte 6j pairs each)
-      // issued before the first use; a J' outside the lane's range loads from a
-      // valid address and adds nothing
-      for (int Jp0 = dlo; Jp0 <= dhi; Jp0 += 2) {
-        if (Jp0 + 1 < Dlo || Jp0 > Dhi) continue;
-        bool v[2];
-        double z[2];
-        double2 w[2][kJC / 2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int Jp = min(Jp0 + u, dhi);
-          const int cc = 6 * Jp + 2 * (td + 1) + pd;
-          const int nkc = s_ccn[cc];
-          const long zo = s_zoff[cc];
-          v[u] = Jp0 + u <= dhi && Jp >= Dlo && Jp <= Dhi && zo >= 0;
-          const int il = Ti[Jp * norb + l];
-          const int kj = Tj[Jp * norb + k] + (k > j ? nkc : 0);
-          z[u] = Zb[v[u] ? zo + (long)kj * nkc + il : 0];
-          const double *s6 = sixq + s6d + (long)Jp * s6J + (long)(c0 >> 1) * s6P;
-#pragma unroll
-          for (int hh = 0; hh < kJC / 2; ++hh) w[u][hh] = *(const double2 *)(s6 + hh * s6P);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const double zz = v[u] ? z[u] : 0.0;
-#pragma unroll
-          for (int hh = 0; hh < kJC / 2; ++hh) {
-            acc[2 * hh] += w[u][hh].x * zz;
-            acc[2 * hh + 1] += w[u][hh].y * zz;
-          }
-        }
-      }
-      for (int Jp0 = xlo; Jp0 <= xhi; Jp0 += 2) {
-        if (Jp0 + 1 < Xlo || Jp0 > Xhi) continue;
-        bool v[2];
-        double z[2];
-        double2 w[2][kJC / 2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int Jp = min(Jp0 + u, xhi);
-          const int cc = 6 * Jp + 2 * (tx + 1) + px;
-          const int nkc = s_ccn[cc];
-          const long zo = s_zoff[cc];
-          v[u] = Jp0 + u <= xhi && Jp >= Xlo && Jp <= Xhi && zo >= 0;
-          const int ik = Ti[Jp * norb + k];
-          const int lj = Tj[Jp * norb + l];
-          z[u] = Zb[v[u] ? zo + (long)((l > j ? nkc : 0) + ik) * nkc + lj : 0];
-          const double *s6 = sixq + s6x + (long)Jp * s6J + (long)(c0 >> 1) * s6P;
-#pragma unroll
-          for (int hh = 0; hh < kJC / 2; ++hh) w[u][hh] = *(const double2 *)(s6 + hh * s6P);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const double zz = v[u] ? fx * z[u] : 0.0;
-#pragma unroll
-          for (int hh = 0; hh < kJC / 2; ++hh) {
-            acc[2 * hh] += w[u][hh].x * zz;
-            acc[2 * hh + 1] -= w[u][hh].y * zz;
-          }
-        }
-      }
-      // the ket's local indices in the chunk's channels, all loaded and waited for
-      // before the first store: loads and stores share one counter, so a load
-      // still in flight behind a store would cost a wait for that store
-      int ikv[kJC];
-#pragma unroll
-      for (int t = 0; t < kJC; ++t) ikv[t] = ((vm >> t) & 1) ? kmapT[(long)(c0 + t) * nk + kk] : -1;
-      __builtin_amdgcn_s_waitcnt(0);
-#pragma unroll
-      for (int t = 0; t < kJC; ++t) {
-        if (!((vm >> t) & 1)) continue;
-        const int J = c0 + t;
-        // commji = commij for k == l, pij commij for i == j (no exchange sum then)
-        const double s = sgn_parity((jjk + jjl) / 2 - J);
-        const double f = (k == l) ? 1.0 - s : (i == j) ? 1.0 - s * pij : 1.0;
-        const double z = acc[t] * f / nrm;
-        const int n = s_chn[J];
-        const int ib = s_ib[J], ik = ikv[t];
-        if (ik == ib)  // diagonal: kept apart (the pp/hh GEMM may still be writing Z's diagonal)
-          P.diag[s_chks[J] + max(ib, 0)] = z;
-        else
-          Ztwo[s_choff[J] + (long)ib * n + ik] = z;
+  const int nquad = s_pre[ncls], nblk = (nquad + 3) >> 2, nchunk = s_cf[2 * nt];
+  const unsigned mz = s_cf[2 * nt + 1];  // the element past M: zero
+  if (nblk == 0) return;
+  // the table in its final form (each thread its own entries): column offset and row in M,
+  // 0xFFFF -- past any element -- where there is none
+  for (int e = threadIdx.x; e < ntab; e += kT) {
+    const int Jp = (int)(((float)(4 * e) + 2.0f) * __builtin_amdgcn_rcpf((float)norb4)), o4 = 4 * e - Jp * norb4;
+    const int4 oc = *(const IMSRG_G int4 *)(B.orbcode + o4);
+    uint4 *d = (uint4 *)tabw + e;
+    const uint4 v4 = *d;
+    auto fin = [&](unsigned v, int oo) -> unsigned {
+      const int tx = ((oo ^ oi) >> 16) & 3, ty = ((oo ^ oj) >> 16) & 3;
+      const unsigned ry = v & 0xFFFF, rx = v >> 16;
+      const int Jc = min(Jp, nJp - 1);
+      const int4 st = s_set[4 * Jc + ty];
+      const int yr = (int)ry - st.y, part = yr >= st.x;
+      const int4 q = s_q[2 * (4 * Jc + ty) + part];
+      const unsigned off = ry == 0xFFFF ? ry : (unsigned)(q.x + (yr - (part ? st.x : 0)) * q.y) & 0xFFFF;
+      return off | (rx == 0xFFFF ? rx : rx - s_set[4 * Jc + tx].z) << 16;
+    };
+    if (nJp > 0) *d = make_uint4(fin(v4.x, oc.x), fin(v4.y, oc.y), fin(v4.z, oc.z), fin(v4.w, oc.w));
+  }
+  for (int q = threadIdx.x; q < 2 * nt; q += kT)
+    for (int c = s_cf[q]; c < s_cf[q + 1]; ++c) s_chunk[c] = (unsigned short)q;
+  for (int c = threadIdx.x; c < ncls; c += kT) {
+    const int njb = s_cls[c].w;
+    int jq = 0, kq = 0;
+    for (int q = s_pre[c]; q < s_pre[c + 1]; ++q) {
+      s_blk[q] = c << 20 | jq << 15 | kq;
+      if (++jq == njb) {
+        jq = 0;
+        ++kq;
       }
     }
+    if (s_pre[c] < nquad && s_pre[c + 1] == nquad)  // the last block's quads of no ket
+      for (int q = nquad; q < 4 * nblk; ++q) s_blk[q] = c << 20 | 0x7FFF;
+  }
+  if (threadIdx.x == 0) M[mz] = TZ(0);
+  __syncthreads();
+  // M from Zbar, kInvpU chunks of a wave at once: the columns' indices, then the elements
+  for (int c0 = wv; c0 < nchunk; c0 += nw * kInvpU) {
+    int col[kInvpU], row[kInvpU], dst[kInvpU], tq[kInvpU];
+    TZ z[kInvpU];
+#pragma unroll
+    for (int u = 0; u < kInvpU; ++u) {
+      const int c = min(c0 + u * nw, nchunk - 1);
+      const int q = s_chunk[c];
+      const int4 a = s_q[q];
+      const int m = (c - s_cf[q]) * 64 + lane;
+      // m / width: the float quotient is within 1/2 width of the true one (m < 2^16)
+      const int yr = (int)(((float)m + 0.5f) * __builtin_amdgcn_rcpf((float)a.y));
+      const bool ok = c0 + u * nw < nchunk && yr < a.z;
+      row[u] = m - yr * a.y;
+      dst[u] = ok ? a.x + m : -1;
+      tq[u] = q >> 1;
+      col[u] = ld_at<int>(B.cc_cols, 4u * (a.w + (ok ? yr : 0)));
+    }
+#pragma unroll
+    for (int u = 0; u < kInvpU; ++u) {
+      const int4 h = s_z[tq[u]];
+      const long zo = (((long)h.y << 32) | (unsigned)h.x) + row[u] + (long)((unsigned long)(unsigned)col[u] * (unsigned)h.z);
+      const TZ *Zb = reinterpret_cast<const TZ *>(P.Zbar);
+      z[u] = Zb[dst[u] >= 0 && h.y >= 0 ? zo : 0];
+      if (h.y < 0) z[u] = TZ(0);
+    }
+#pragma unroll
+    for (int u = 0; u < kInvpU; ++u)
+      if (dst[u] >= 0) M[dst[u]] = z[u];
+  }
+  __syncthreads();
+  // The results, four quads (4 J x 4 kets of one class) at a time on the 4x4x4 matrix units:
+  // lane 16 r + 4 b + m holds row m of the weights of quad b at J' r of a step, the element of
+  // its ket m there, and its result of J r and ket m.  The kets' records, their channel indices
+  // and the weights of the first kInvpW steps of block bk + nw are loaded before block bk is
+  // formed: loaded where they are used they cost most of the time.
+  const int rl = lane >> 4, ml = lane & 3;
+  struct Blk {
+    int Jl, jh;        // the lane's J as a result, (ja + jb) / 2
+    int pd, px, ns;    // the lane's first J' in the two sums; steps of 4 J'
+    int cd, cx, JA;    // rows of weights at J' = 0, the lane's J as a row of the weights
+    bool active;
+    int2 rec;
+    int ik;
+    double wd[kInvpW], wx[kInvpW];
+  };
+  // held in registers: the stores below could alias B
+  const IMSRG_G double *sixq = B.sixjQ;
+  const IMSRG_G int2 *crec = B.cls_rec;
+  const IMSRG_G int *ckm = B.cls_kmap;
+  IMSRG_G char *Ztwo = (IMSRG_G char *)(P.Z + B.two_off);
+  auto load = [&](int bk) -> Blk {
+    Blk k;
+    const unsigned q = s_blk[4 * bk + ((lane >> 2) & 3)];
+    const int c = q >> 20;
+    const int4 c1 = s_cls[c], c2 = s_cls2[c];
+    const int J0 = (c1.z & 0xFFFF) + (q >> 15 & 31) * 4, p = (q & 0x7FFF) * 4 + ml;
+    k.Jl = J0 + rl;
+    k.jh = c1.z >> 16;
+    k.active = p < c1.y;
+    const int pos = c1.x + (k.active ? p : 0);
+    k.rec = ld_at<int2>(crec, 8u * pos);
+    k.ik = ld_at<int>(ckm, (k.Jl * nk + pos) * 4u);
+    k.pd = (c2.z & 0xFFFF) + rl;
+    k.px = (c2.z >> 16) + rl;
+    k.ns = c2.w;
+    k.cd = c2.x;
+    k.cx = c2.y;
+    k.JA = min(J0 + ml, d2 - 1);
+#pragma unroll
+    for (int u = 0; u < kInvpW; ++u) {  // past the quad's last step: row 0
+      k.wd[u] = sixq[(long)(u < k.ns ? k.cd + min(k.pd + 4 * u, nJp) : 0) * d2 + k.JA];
+      k.wx[u] = sixq[(long)(u < k.ns ? k.cx + min(k.px + 4 * u, nJp) : 0) * d2 + k.JA];
+    }
+    return k;
+  };
+  const int brec = ji > jj ? j << 16 | i : i << 16 | j;
+  auto form = [&](const Blk &k) {
+    const bool sw = k.rec.y != 0;
+    const int oa = k.rec.x >> 16, ob = k.rec.x & 0xFFFF;
+    const bool dket = oa == ob;
+    // first sum: the direct elements M(l, k) of k = oa and l = ob; second: the exchange
+    // elements M(k, l), none for k = l.  i = j has the first only, with the true k and l.
+    const bool flip = same && sw;
+    const int xd = flip ? oa : ob, yd = flip ? ob : oa;
+    const unsigned none = dket ? 0xFFFF : 0;
+    const double sx = (k.jh - k.JA) & 1 ? 1.0 : -1.0;
+    const int ns = max(max(__builtin_amdgcn_readlane(k.ns, 0), __builtin_amdgcn_readlane(k.ns, 4)),
+                       max(__builtin_amdgcn_readlane(k.ns, 8), __builtin_amdgcn_readlane(k.ns, 12)));
+    double acc = 0.0;
+    auto step = [&](int u, double wd, double wx) {
+      const int td = min(k.pd + 4 * u, nJp) * norb4, tx = min(k.px + 4 * u, nJp) * norb4;
+      const unsigned ed = min((unsigned)tab[2 * (td + yd)] + tab[2 * (td + xd) + 1], mz);
+      const unsigned ex = min((unsigned)tab[2 * (tx + ob)] + tab[2 * (tx + oa) + 1] + none, mz);
+      const double zd = M[ed], zx = M[ex];
+      acc = __builtin_amdgcn_mfma_f64_4x4x4f64(wd, zd, acc, 0, 0, 0);
+      if (!same) acc = __builtin_amdgcn_mfma_f64_4x4x4f64(sx * wx, zx, acc, 0, 0, 0);
+    };
+#pragma unroll
+    for (int u = 0; u < kInvpW; ++u)
+      if (u < ns) step(u, k.wd[u], k.wx[u]);
+    for (int u = kInvpW; u < ns; ++u)
+      step(u, sixq[(long)(k.cd + min(k.pd + 4 * u, nJp)) * d2 + k.JA], sixq[(long)(k.cx + min(k.px + 4 * u, nJp)) * d2 + k.JA]);
+    const bool odd = (k.jh - k.Jl) & 1;
+    double f;
+    if (same) {
+      const bool oddp = odd != (((ji + jj) / 2 + k.jh) & 1);
+      f = dket ? (odd ? 1.0 : 0.0) : oddp ? SQRT2_D : 0.0;
+    } else {
+      f = dket ? (odd ? SQRT2_D : 0.0) : sw && !odd ? -1.0 : 1.0;
+    }
+    const long row = s_row[k.Jl];
+    if (!k.active || k.ik < 0 || row < 0) return;
+    if (k.rec.x == brec)  // diagonal: kept apart (the pp/hh GEMM may still be writing Z's diagonal)
+      P.diag[B.ch_kstart[6 * k.Jl + g] + k.ik] = acc * f;
+    else
+      *(IMSRG_G double *)(Ztwo + (row + 8L * k.ik)) = acc * f;
+  };
+  // two blocks per turn, so that neither is copied (a copy would wait for its loads)
+  Blk ka = load(min(wv, nblk - 1));
+  for (int bk = wv; bk < nblk; bk += 2 * nw) {
+    const Blk kb2 = load(min(bk + nw, nblk - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    form(ka);
+    if (bk + nw >= nblk) break;
+    ka = load(min(bk + 2 * nw, nblk - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    form(kb2);
   }
 }
 
@@ -2070,15 +2094,23 @@ hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int 
   }
   return hipGetLastError();
 }
-hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, int jmax, int norb, int nch,
-                            int ncls, bool zbar_f32, hipStream_t s) {
+hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, size_t lds, bool zbar_f32,
+                            hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
-  const size_t lds = invp_lds_bytes(jmax, norb, nch, ncls);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  if (zbar_f32)
-    hipLaunchKernelGGL(k_invpandya<float>, dim3(nitems), dim3(kChunk), lds, s, pa, items);
+  // 256 threads where seven and more work-groups fit in a CU: 512 take longer on small items
+  // (emax = 5, FP32 Zbar: 23.7 against 19.2 us) and less on large ones (emax = 10, FP64: 438
+  // against 529 us), of which few fit
+  const bool small = lds <= 18 * kLdsUnit;
+  const dim3 grid(nitems), blk(small ? 256 : 512);
+  if (zbar_f32 && small)
+    hipLaunchKernelGGL((k_invpandya<float, 256>), grid, blk, lds, s, pa, items);
+  else if (zbar_f32)
+    hipLaunchKernelGGL((k_invpandya<float, 512>), grid, blk, lds, s, pa, items);
+  else if (small)
+    hipLaunchKernelGGL((k_invpandya<double, 256>), grid, blk, lds, s, pa, items);
   else
-    hipLaunchKernelGGL(k_invpandya<double>, dim3(nitems), dim3(kChunk), lds, s, pa, items);
+    hipLaunchKernelGGL((k_invpandya<double, 512>), grid, blk, lds, s, pa, items);
   return hipGetLastError();
 }
 hipError_t launch_finish(const PairArg &pa, const int4 *items, int nitems, bool fold, bool c122, int npairs,

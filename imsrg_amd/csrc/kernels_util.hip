@@ -110,7 +110,7 @@ __device__ double sixj_dd(const dd *F, int a, int b, int c, int d, int e, int f)
 }
 
 __global__ __launch_bounds__(256) void k_sixj_table(const dd *F, double *table, double *tableQ, int d1, int d2,
-                                                   int d2q, long total) {
+                                                   long total) {
   for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
     long r = idx;
     const int J6 = r % d2; r /= d2;
@@ -124,12 +124,12 @@ __global__ __launch_bounds__(256) void k_sixj_table(const dd *F, double *table, 
     // the inverse Pandya copy holds the weights (2 J6 + 1) {...}, and 0 where
     // |6j| < 1e-8, the values whose terms the reference skips (src/Commutator.cc:1564-1572,
     // 1593-1604)
-    tableQ[sixjQ_index(d1, d2q, 2 * i1 + 1, 2 * i2 + 1, J3, 2 * i4 + 1, 2 * i5 + 1, J6)] =
+    tableQ[sixjQ_index(d1, d2, 2 * i1 + 1, 2 * i2 + 1, J3, 2 * i4 + 1, 2 * i5 + 1, J6)] =
         fabs(v) >= 1e-8 ? (2 * J6 + 1) * v : 0.0;
   }
 }
 
-hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, int d2q, hipStream_t s) {
+hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, hipStream_t s) {
   if (4 * (d1 - 1) + 4 > kNFact - 4) return hipErrorInvalidValue;
   dd *F = nullptr;
   hipError_t e = hipMalloc(&F, sizeof(dd) * kNFact);
@@ -137,7 +137,7 @@ hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, int 
   hipLaunchKernelGGL(k_factorials, dim3(1), dim3(64), 0, s, F);
   long total = (long)d1 * d1 * d2 * d1 * d1 * d2;
   int blocks = (int)std::min<long>((total + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_sixj_table, dim3(blocks), dim3(256), 0, s, F, table, tableQ, d1, d2, d2q, total);
+  hipLaunchKernelGGL(k_sixj_table, dim3(blocks), dim3(256), 0, s, F, table, tableQ, d1, d2, total);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   e = hipStreamSynchronize(s);

@@ -9,7 +9,7 @@ namespace imsrg {
 // dense 6j table {jj1 jj2 J3; jj4 jj5 J6} (double-double Racah): `table` in the layout of
 // SixJCache_112112, `tableQ` in the sixjQ_index layout as the weights (2 J6 + 1) {6j},
 // 0 in place of |6j| < 1e-8 (padding entries are left untouched)
-hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, int d2q, hipStream_t s);
+hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, hipStream_t s);
 
 // commutator phases; items are device arrays of int4 work items
 // operands, Hermiticities and terms of up to kMax pairs of a batch, into its device
@@ -42,10 +42,10 @@ hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const i
 // ph GEMM (head and tail of Zbar) on 128x128 tiles (big) or 64x64 tiles; precision 1
 // (FP32 products) stores Zbar in FP32, the others in FP64
 hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int precision, bool big, hipStream_t s);
-// jmax, norb, nch, ncls: the largest of the pairs (they size the kernel's LDS tables);
-// zbar_f32: Zbar holds FP32 elements (written by the precision-1 ph GEMM)
-hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, int jmax, int norb, int nch,
-                            int ncls, bool zbar_f32, hipStream_t s);
+// lds: DeviceBasis::invp_lds, the largest of the pairs; zbar_f32: Zbar holds FP32 elements
+// (written by the precision-1 ph GEMM)
+hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, size_t lds, bool zbar_f32,
+                            hipStream_t s);
 // last launch: with fold, upper += the inverse-Pandya contributions stored at the
 // transposed slots; with c122, Z2 -= W + hZ W^T (comm122ss); then lower triangle
 // <- hZ * upper; and Z0 and Z1 from the first launch's partial sums
