@@ -1430,7 +1430,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   HIPCHK(ctx, mark(2));
   const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
   const FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
-                      mph ? cnt[3] : 0};
+                      mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big};
   HIPCHK(ctx, launch_front(pa, fi, maxnch, s));
   HIPCHK(ctx, mark(3));
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));

@@ -445,7 +445,8 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
     cc_nph[c] = (int)(hh.size() + ph.size());
     cc_xoff[c] = xo;
     cc_zoff[c] = zo;
-    xo += (long)nk * 2 * cc_nph[c];
+    // room for FP32 columns of a multiple of 4 elements, channels 16-byte aligned
+    xo += ((long)std::max(nk, (nk + 3) / 4 * 2) * 2 * cc_nph[c] + 1) & ~1L;
     zo += (long)nk * 2 * nk;
   }
   cc_kstart[nch] = (int)cc_kets.size();

@@ -511,9 +511,8 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
 // two kets have the same first orbit (all that the inverse Pandya reads): they lie within
 // cc_run of the diagonal, so that sub-tiles further off leave their mirror image out.  The
 // lower elements are (head) hZ-sign or (tail) phi_r phi_s times the upper ones, as the
-// reference's folds make them (src/Commutator.cc:1792-1805), written through an LDS
-// transpose.  Without the others the ph GEMM takes 420 us at emax = 10 (FP64; 472 with them) and
-// 335 us with FP32 products (355).
+// reference's folds make them (src/Commutator.cc:1792-1805).  Without the others the ph
+// GEMM took 420 us at emax = 10 (FP64; 472 with them) and 335 us with FP32 products (355).
 // MIXED: operands rounded to FP32 when read from LDS, products on f32
 // 16x16x4 MFMA, FP32 partial sums over two stages (32 k) added into the FP64
 // accumulators.
@@ -521,28 +520,12 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
 // with ah = fl32(a), al = fl32(a - ah), and a product takes three f32 MFMAs,
 // ah*bh + ah*bl + al*bh (the dropped al*bl is 2^-48 of it); the FP32 partial
 // sums are flushed into FP64 after every 4 k.
-// Non-temporal stores of Zbar: the inverse Pandya gather reads it only after
-// the whole ph GEMM, so keeping its lines out of the L2 spares that gather
-// the write-back of dirty lines (inverse Pandya 880 -> 835 us, ph GEMM
-// 398 -> 437 us: a net 1% on the overlapped commutator).  The last kernel's
-// stores of Z use them too (Z is read again only by a later call).
+// Non-temporal stores: the last kernel's of Z, which is read again only by a later call.
 __device__ __forceinline__ void st_nt(double *p, double v) { __builtin_nontemporal_store(v, p); }
 __device__ __forceinline__ void st_nt2(double *p, double a, double b) {
   typedef double d2v __attribute__((ext_vector_type(2)));
   const d2v v = {a, b};
   __builtin_nontemporal_store(v, reinterpret_cast<d2v *>(p));
-}
-// FP32 Zbar (the FP32-product ph GEMM): the values rounded once, when stored
-__device__ __forceinline__ void st_nt(float *p, double v) { __builtin_nontemporal_store((float)v, p); }
-__device__ __forceinline__ void st_nt2(float *p, double a, double b) {
-  typedef float f2s __attribute__((ext_vector_type(2), aligned(4)));
-  const f2s v = {(float)a, (float)b};
-  __builtin_nontemporal_store(v, reinterpret_cast<f2s *>(p));
-}
-__device__ __forceinline__ void st_nt4(float *p, double a, double b, double c, double d) {
-  typedef float f4s __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned rows
-  const f4s v = {(float)a, (float)b, (float)c, (float)d};
-  __builtin_nontemporal_store(v, reinterpret_cast<f4s *>(p));
 }
 
 // A wave of a 128x128 tile owns the 64 x kGW sub-tile at rows (w & 1) * 64,
@@ -552,101 +535,42 @@ __device__ __forceinline__ bool tile_wave_live(int R0, int S0, int n, int w) {
   return R0 + (w & 1) * 64 < n && S0 + (w >> 1) * kGW < n && R0 + (w & 1) * 64 <= S0 + (w >> 1) * kGW + kGW - 1;
 }
 
-// Stores a 128x128 tile from the waves' FP64 accumulators (lane layout of the
-// f32 MFMAs when F32L, else of the f64 16x16x4 MFMA).
+// Stores a wave's sub-tile of a 128x128 tile from its FP64 accumulators (lane layout of the
+// f32 MFMAs when F32L, else of the f64 16x16x4 MFMA): 16 consecutive rows of four columns
+// per store instruction.
 // PH false: the upper triangle of D = alpha * acc.
-// PH true: Zbar (the lower triangle near the diagonal) through LDS transposes of the 64 x kGW wave sub-tiles,
-// four per round in the buffers tb0..tb3 (each >= 64 (kGW + 1) doubles): the
-// lower triangle as (head) h or (tail) phi_r phi_s times the upper element, as
-// the reference's folds make it (src/Commutator.cc:1792-1805); s_ph holds the
-// tile's row (0) and column (1) phases in the tail (h = 1) and 1 in the head.
-template <bool PH, bool F32L, typename TD = double>
-__device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], TD *D, int n, int R0, int S0,
-                                              double alpha, double h, int run, const signed char (*s_ph)[kTileB],
-                                              double *tb0, double *tb1, double *tb2, double *tb3) {
+// PH true: Zbar, the upper triangle and the elements next to the diagonal in the lower one
+// (less than run from it); s_ph holds the tile's row (0) and column (1) phases in the
+// tail (h = 1) and 1 in the head.
+// The elements used to go through LDS (the lower triangle was stored in full, transposed
+// there) and to memory by non-temporal stores.  Stored at once, the waves wait for no other,
+// and plain stores, whose lines the L2 completes from two instructions, are the faster ones
+// here: ph GEMM at emax = 10 FP64 420 -> 395 us (435 with non-temporal stores), emax = 7 61 -> 56.
+template <bool PH, bool F32L>
+__device__ __forceinline__ void gemm_epilogue(const dbl4 (&acc)[4][kGN], double *D, int n, int R0, int S0,
+                                              double alpha, double h, int run, const signed char (*s_ph)[kTileB]) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = (wv & 1) * 64, wc = (wv >> 1) * kGW;
-  const bool wave_live = tile_wave_live(R0, S0, n, wv);
-  if constexpr (!PH) {
+  const bool near = PH && S0 + wc - (R0 + wr + 63) < run;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+  for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
-      for (int ni = 0; ni < kGN; ++ni)
+    for (int ni = 0; ni < kGN; ++ni)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int row = R0 + wr + mi * 16 + (lane & 15);
-          const int col = S0 + wc + ni * 16 + mfma_col<F32L>(lane, q);
-          if (row < n && col < n && row <= col) D[(long)col * n + row] = alpha * acc[mi][ni][q];
-        }
-  } else {
-    static_assert(kGWaves == 8, "two rounds of four sub-tiles");
-    auto Tb = [&](int j) {
-      double *p = j == 0 ? tb0 : j == 1 ? tb1 : j == 2 ? tb2 : tb3;
-      return reinterpret_cast<double(*)[kGW + 1]>(p);
-    };
-    for (int rd = 0; rd < 2; ++rd) {
-      if ((wv >> 2) == rd && wave_live) {
-        double(*Tt)[kGW + 1] = Tb(wv & 3);
-#pragma unroll
-        for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-          for (int ni = 0; ni < kGN; ++ni)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int rr = mi * 16 + (lane & 15), cc = ni * 16 + mfma_col<F32L>(lane, q);
-              Tt[rr][cc] = alpha * acc[mi][ni][q] * (double)s_ph[1][wc + cc];
-            }
-      }
-      __syncthreads();
-      for (int j = 0; j < 4; ++j) {
-        const int w = 4 * rd + j;
-        if (!tile_wave_live(R0, S0, n, w)) continue;  // block-uniform
-        double(*Tt)[kGW + 1] = Tb(j);
-        const int R1 = R0 + (w & 1) * 64, S1 = S0 + (w >> 1) * kGW;
-        if constexpr (std::is_same<TD, float>::value) {
-          // FP32 Zbar: four rows per thread and one 16-byte store where all four
-          // are written; R1 and S1 are multiples of 4
-          for (int e = threadIdx.x; e < 16 * kGW; e += blockDim.x) {
-            const int rr = 4 * (e & 15), cc = e >> 4;
-            const int row = R1 + rr, col = S1 + cc;
-            if (col >= n || row >= n || row > col) continue;
-            float *dp = D + (long)col * n + row;
-            if (row + 3 < n && row + 3 <= col) {
-              st_nt4(dp, Tt[rr][cc], Tt[rr + 1][cc], Tt[rr + 2][cc], Tt[rr + 3][cc]);
-            } else {
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                if (row + q < n && row + q <= col) st_nt(dp + q, Tt[rr + q][cc]);
-            }
-          }
+      for (int q = 0; q < 4; ++q) {
+        const int rr = wr + mi * 16 + (lane & 15), cc = wc + ni * 16 + mfma_col<F32L>(lane, q);
+        const int row = R0 + rr, col = S0 + cc;
+        if (row >= n || col >= n || row > col) continue;
+        if constexpr (!PH) {
+          D[(long)col * n + row] = alpha * acc[mi][ni][q];
         } else {
-          // Two rows per thread and one 16-byte store where both are written (store
-          // instructions, not bytes, bound this epilogue); R1 and S1 are even.
-          // upper elements (R1 + rr, S1 + cc), consecutive threads on consecutive row pairs
-          for (int e = threadIdx.x; e < 32 * kGW; e += blockDim.x) {
-            const int rr = 2 * (e & 31), cc = e >> 5;
-            const int row = R1 + rr, col = S1 + cc;
-            if (col >= n || row >= n || row > col) continue;
-            TD *dp = D + (long)col * n + row;
-            if (row + 1 < n && row + 1 <= col)
-              st_nt2(dp, Tt[rr][cc], Tt[rr + 1][cc]);
-            else
-              st_nt(dp, Tt[rr][cc]);
-          }
-        }
-        // mirrored elements (S1 + cc, R1 + rr) = sym * upper (R1 + rr, S1 + cc), near the diagonal
-        if (S1 - (R1 + 63) >= run) continue;
-        for (int e = threadIdx.x; e < 64 * kGW; e += blockDim.x) {
-          const int cc = e & (kGW - 1), rr = e / kGW;
-          const int row2 = S1 + cc, col2 = R1 + rr;
-          if (col2 >= n || row2 >= n || row2 <= col2) continue;
-          // phases from LDS: row2 - S0 and col2 - R0 lie in [0, 128)
-          st_nt(D + (long)col2 * n + row2, h * (double)(s_ph[1][row2 - S0] * s_ph[0][col2 - R0]) * Tt[rr][cc]);
+          const double v = acc[mi][ni][q] * (double)s_ph[1][cc];
+          D[(long)col * n + row] = v;
+          // the lower element: h phi_r phi_c times the upper one
+          if (near && col != row && col - row < run)
+            D[(long)row * n + col] = h * (double)(s_ph[1][cc] * s_ph[0][rr]) * v;
         }
       }
-      __syncthreads();
-    }
-  }
 }
 
 // The work-group's tile of a ph item list whose items are each done twice, head and
@@ -685,9 +609,8 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items, int nit
   const double *kw = nullptr;
   const signed char *phi = nullptr, *phph = nullptr;
   double alpha, h;
-  // Zbar in FP32 from the FP32-product ph GEMM, in FP64 otherwise
-  using ZT = typename std::conditional<PH && MIXED && !SPLIT, float, double>::type;
-  ZT *D;
+  static_assert(!PH || MIXED == SPLIT, "the ph GEMM with FP32 products is k_ph_big_f32");
+  double *D;
   if constexpr (!PH) {
     const int ch = it.y;
     n = B.ch_n[ch];
@@ -709,7 +632,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items, int nit
     const long xo = B.cc_xoff[cc];
     Am = P.Xt + xo;
     Bm = P.Yt + xo;
-    D = reinterpret_cast<ZT *>(P.Zbar) + B.cc_zoff[cc] + (tail ? (long)n * n : 0);
+    D = P.Zbar + B.cc_zoff[cc] + (tail ? (long)n * n : 0);
     alpha = 1.0;
     h = tail || P.hZ == 1 ? 1.0 : -1.0;
     phi = B.cc_phi + B.cc_kstart[cc];
@@ -889,8 +812,7 @@ __device__ __forceinline__ void gemm_tile(PairArg pa, const int4 *items, int nit
     if (k0 + kTileK < K2) stage(k0 + kTileK, A1, B1, W1, A0, B0, W0, true);
   }
   if constexpr (MIXED) flush_t();  // a last stage without its pair
-  static_assert(64 * (kGW + 1) <= kTileK * LD, "transpose tile exceeds the operand buffer");
-  gemm_epilogue<PH, MIXED, ZT>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, &A0[0][0], &A1[0][0], &B0[0][0], &B1[0][0]);
+  gemm_epilogue<PH, MIXED>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph);
 }
 
 // ---------------------------------------------------------------------------
@@ -1099,9 +1021,7 @@ __device__ __forceinline__ void gemm_tile_b3(PairArg pa, const int4 *items, int 
       __syncthreads();
     }
   }
-  static_assert(2 * 64 * (kGW + 1) * sizeof(double) <= sizeof(StageB3), "transpose tiles exceed the stage buffer");
-  double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<true, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<true, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph);
 }
 
 // ---------------------------------------------------------------------------
@@ -1262,8 +1182,7 @@ __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, co
       __syncthreads();
     }
   }
-  double *t0 = reinterpret_cast<double *>(&L0[0][0][0][0]), *t2 = reinterpret_cast<double *>(&L1[0][0][0][0]);
-  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph, t0, t0 + 64 * (kGW + 1), t2, t2 + 64 * (kGW + 1));
+  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph);
 }
 
 __global__ __launch_bounds__(kGWaves * 64, 2) void k_ph_big_b3(PairArg pa, const int4 *items, int nitems) {
@@ -1279,9 +1198,160 @@ __global__ __launch_bounds__(kGWaves * 64, 4) void k_pphh_big_mixed(PairArg pa, 
 __global__ __launch_bounds__(kGWaves * 64, 4) void k_pphh_big_split(PairArg pa, const int4 *items) {
   gemm_tile<false, true, true>(pa, items, 0);
 }
-template <bool MIXED, bool SPLIT = false>
+template <bool SPLIT>
 __global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big(PairArg pa, const int4 *items, int nitems) {
-  gemm_tile<true, MIXED, SPLIT>(pa, items, nitems);
+  gemm_tile<true, SPLIT, SPLIT>(pa, items, nitems);
+}
+
+// The ph GEMM with FP32 products (gemm_tile's PH = true, MIXED, without SPLIT) on Xbar and
+// Ybar^T that the Pandya transformation has stored in FP32.  All its weights are +-1, so that
+// rounding the operands there gives the same values as rounding the weighted ones here.
+// A stage holds 32 k: with FP64 operands it held 16 in the same LDS, each behind its own
+// barrier and with half the time for the copies to arrive.  A 16-byte copy of a wave fills a
+// slot of two columns k and k + 4, and slots are 2 x 128 + 16 elements apart: the four k that
+// a wave reads at once then lie in different banks and all its reads of a stage are at fixed
+// distances from one address.  The FP32 sums are flushed every 32 k.
+// emax = 10: 335 -> 254 us, emax = 12: 1461 -> 1145 us (66 -> 85 TF/s on the sub-tiles with
+// results), emax = 5: 29 -> 23 us; 26 and 101 us of the first two are the epilogue's.  A tile
+// has some 7 stages only, so that its start and its stores take a third of its time.
+constexpr int kF32K = 32;
+__global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big_f32(PairArg pa, const int4 *items, int nitems) {
+  constexpr int T = kTileB, SL = 2 * T + 16, NS = kF32K / 2;  // slots of two columns
+  __shared__ __align__(16) float A0[NS * SL], A1[NS * SL], B0[NS * SL], B1[NS * SL];
+  __shared__ signed char s_ph[2][T];
+  bool tail;
+  const int4 it = ph_item(items, nitems, tail);
+  if (it.y < 0) return;  // padding item of the XCD-balanced order
+  PairPtrs P = pa.get(it.x);
+  const BasisDev &B = *P.basis;
+  const int cc = it.y, n = B.cc_n[cc], ld = (n + 3) & ~3, nph = B.cc_nph[cc], nk = 2 * nph, K2 = 2 * nk;
+  const IMSRG_G float *Am = (const IMSRG_G float *)(P.Xt + B.cc_xoff[cc]), *Bm = (const IMSRG_G float *)(P.Yt + B.cc_xoff[cc]);
+  float *D = reinterpret_cast<float *>(P.Zbar) + B.cc_zoff[cc] + (tail ? (long)n * n : 0);
+  const bool hneg = !tail && P.hZ != 1;
+  const signed char *phi = B.cc_phi + B.cc_kstart[cc], *phph = B.cc_phph + B.cc_phstart[cc];
+  const int R0 = it.z * T, S0 = it.w * T;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (threadIdx.x < 2 * T) {
+    const int sd = threadIdx.x / T, e = threadIdx.x - sd * T;
+    s_ph[sd][e] = tail ? phi[min((sd ? S0 : R0) + e, n - 1)] : 1;
+  }
+  const int wr = (wv & 1) * 64, wc = (wv >> 1) * kGW;
+  const bool wave_live = tile_wave_live(R0, S0, n, wv);
+  // copies: lanes 0..31 column k, 32..63 column k + 4 of a slot; four rows per lane, whole
+  // quads of a column (its rows n .. ld - 1 and the clamped ones reach no stored result)
+  const int ra = min(R0 + 4 * (lane & 31), ld - 4), rb = min(S0 + 4 * (lane & 31), ld - 4);
+  auto column = [&](int kk, const IMSRG_G float *&a, const IMSRG_G float *&b) {
+    const int ca = kk < nk ? kk : kk - nk, cb = tail ? (ca < nph ? ca + nph : ca - nph) : ca;
+    const IMSRG_G float *x = Am + (long)ca * ld, *y = Bm + (long)cb * ld;
+    a = kk < nk ? x : y;
+    b = kk < nk ? y : x;
+  };
+  auto issue = [&](int k0, float *As, float *Bs) {
+#pragma unroll
+    for (int j = 0; j < NS / kGWaves; ++j) {
+      const int sl = NS / kGWaves * wv + j, k1 = k0 + 8 * (sl >> 2) + (sl & 3);
+      const IMSRG_G float *a1, *b1, *a2, *b2;  // wave-uniform; the lanes choose
+      column(min(k1, K2 - 1), a1, b1);
+      column(min(k1 + 4, K2 - 1), a2, b2);
+      __builtin_amdgcn_global_load_lds((const IMSRG_G void *)((lane < 32 ? a1 : a2) + ra),
+                                       (__attribute__((address_space(3))) void *)&As[sl * SL], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const IMSRG_G void *)((lane < 32 ? b1 : b2) + rb),
+                                       (__attribute__((address_space(3))) void *)&Bs[sl * SL], 16, 0, 0);
+    }
+  };
+  // signs of the weights of a stage's k, one bit each: (tail) hY phi of the ph ket, (head) the
+  // sign of the second half of the k
+  auto load_w = [&](int k0) -> signed char {
+    const int kk = min(k0 + (lane & (kF32K - 1)), K2 - 1), k = kk < nk ? kk : kk - nk;
+    return phph[k < nph ? k : k - nph];
+  };
+  auto sign_bits = [&](int k0, signed char w) -> unsigned {
+    const bool neg = tail ? (P.hY == 1) != (w > 0) : hneg && k0 + (lane & (kF32K - 1)) >= nk;
+    return (unsigned)__ballot(neg);
+  };
+  dbl4 acc[4][kGN];
+  flt4 t[4][kGN];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < kGN; ++b) {
+      acc[a][b] = dbl4{0.0, 0.0, 0.0, 0.0};
+      t[a][b] = flt4{0.f, 0.f, 0.f, 0.f};
+    }
+  const int kl = lane >> 4, pa0 = kl * SL + wr + (lane & 15), pb0 = kl * SL + wc + (lane & 15);
+  auto step = [&](const float *Ap, const float *Bp, unsigned sg) {
+    const unsigned neg = (sg >> kl) << 31;
+    float am[4], bm[kGN];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) am[m] = Ap[16 * m];
+#pragma unroll
+    for (int m = 0; m < kGN; ++m) bm[m] = __uint_as_float(__float_as_uint(Bp[16 * m]) ^ neg);
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < kGN; ++ni)
+        t[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(am[mi], bm[ni], t[mi][ni], 0, 0, 0);
+  };
+  auto stage = [&](int k0, unsigned sg, const float *As, const float *Bs, float *An, float *Bn) -> unsigned {
+    const signed char w_next = load_w(k0 + kF32K);
+    if (k0 + kF32K < K2) issue(k0 + kF32K, An, Bn);
+    if (wave_live) {
+      const int steps = min(kF32K, K2 - k0) >> 2;  // K2 is a multiple of 4
+      // not unrolled: more reads ahead than one step's do not fit in the registers
+#pragma unroll 1
+      for (int ks = 0; ks < steps; ks += 2) {
+        const float *Ap = As + pa0 + ks * 2 * SL, *Bp = Bs + pb0 + ks * 2 * SL;
+        step(Ap, Bp, sg >> (4 * ks));
+        if (ks + 1 < steps) step(Ap + T, Bp + T, sg >> (4 * ks + 4));
+      }
+#pragma unroll
+      for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < kGN; ++ni) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[mi][ni][q] += (double)t[mi][ni][q];
+          t[mi][ni] = flt4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    const unsigned next = sign_bits(k0 + kF32K, w_next);
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's copies of the next stage have landed
+    __syncthreads();
+    return next;
+  };
+  issue(0, A0, B0);  // K2 > 0: channels with ph kets only
+  unsigned sg = sign_bits(0, load_w(0));
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  for (int k0 = 0; k0 < K2; k0 += 2 * kF32K) {
+    sg = stage(k0, sg, A0, B0, A1, B1);
+    if (k0 + kF32K < K2) sg = stage(k0 + kF32K, sg, A1, B1, A0, B0);
+  }
+  typedef float f4s __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned columns
+  // four consecutive rows of a column per lane: one 16-byte store where all four are stored
+  const bool near = S0 + wc - (R0 + wr + 63) < B.cc_run;
+  const int run = B.cc_run;
+  const double h = hneg ? -1.0 : 1.0;
+#pragma unroll
+  for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < kGN; ++ni) {
+      const int rr = wr + 16 * mi + 4 * kl, c = wc + 16 * ni + (lane & 15), row = R0 + rr, col = S0 + c;
+      if (row >= n || col >= n || row > col) continue;
+      const double sc = s_ph[1][c];
+      float *dp = D + (long)col * n + row;
+      const dbl4 v = acc[mi][ni];
+      if (row + 3 < n && row + 3 <= col)
+        *reinterpret_cast<f4s *>(dp) = f4s{(float)(sc * v[0]), (float)(sc * v[1]), (float)(sc * v[2]), (float)(sc * v[3])};
+      else
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (row + q < n && row + q <= col) dp[q] = (float)(sc * v[q]);
+      if (near)  // the lower elements next to the diagonal: h phi_r phi_c times the upper ones
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (row + q < n && row + q < col && col - row - q < run)
+            D[(long)(row + q) * n + col] = (float)(h * (double)(s_ph[1][c] * s_ph[0][rr + q]) * (sc * v[q]));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1295,7 +1365,7 @@ __global__ __launch_bounds__(kGWaves * 64, 4) void k_ph_big(PairArg pa, const in
 // J at a time.  Bound by the address processing of its gathers (texture addresser 79%
 // busy with one load per index and 6j value and the transposed elements): 182 us at
 // emax = 10 before.
-__device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, unsigned char *lds_raw) {
+__device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, bool f32, unsigned char *lds_raw) {
   const BasisDev &B = *P.basis;
   // channel offsets and sizes in LDS: the gather of each J then waits on one
   // LDS read instead of two dependent global loads
@@ -1376,6 +1446,12 @@ __device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, 
       xbar *= P.hX;  // X(cb, ad) = hX X(ad, cb); Ybar^T holds hY Y(cb, ad) = Y(ad, cb)
     }
   }
+  if (f32) {  // rounded once, as k_ph_big_f32 would; columns of a multiple of 4 elements
+    const long o = (long)mp * ((nk + 3) & ~3) + ik;
+    ((IMSRG_G float *)(P.Xt + B.cc_xoff[cc]))[o] = (float)(xbar * normf * nanb);
+    ((IMSRG_G float *)(P.Yt + B.cc_xoff[cc]))[o] = (float)(ybar * normf);
+    return;
+  }
   const long o = B.cc_xoff[cc] + (long)mp * nk + ik;
   P.Xt[o] = xbar * normf * nanb;
   P.Yt[o] = ybar * normf;
@@ -1406,7 +1482,7 @@ __global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
     return;
   }
   const int4 it = f.pandya[b - f.n221];
-  front_pandya(pa.get(it.x), it, lds_raw);
+  front_pandya(pa.get(it.x), it, f.xbar_f32, lds_raw);
 }
 
 // AddInversePandyaTransformation (src/Commutator.cc:1501-1616), by bra.
@@ -2078,9 +2154,9 @@ hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int 
     if (precision == kGemmB3)
       hipLaunchKernelGGL(k_ph_big_b3, grid, blk, 0, s, pa, items, nitems);
     else if (precision == 1)
-      hipLaunchKernelGGL((k_ph_big<true>), grid, blk, 0, s, pa, items, nitems);
+      hipLaunchKernelGGL(k_ph_big_f32, grid, blk, 0, s, pa, items, nitems);
     else if (precision == 2)
-      hipLaunchKernelGGL((k_ph_big<true, true>), grid, blk, 0, s, pa, items, nitems);
+      hipLaunchKernelGGL((k_ph_big<true>), grid, blk, 0, s, pa, items, nitems);
     else
       hipLaunchKernelGGL((k_ph_big<false>), grid, blk, 0, s, pa, items, nitems);
     return hipGetLastError();

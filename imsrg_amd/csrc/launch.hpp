@@ -32,6 +32,7 @@ hipError_t launch_set_pairs(PairPtrs *tab, const PairOps &ops, hipStream_t s);
 struct FrontItems {
   const int4 *one, *ob221, *pandya;
   int nzero, nzeros, none, n221, npandya;
+  bool xbar_f32;  // Xbar and Ybar in FP32 (the ph GEMM on 128x128 tiles with FP32 products reads them so)
 };
 hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipStream_t s);
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
