@@ -160,8 +160,8 @@ struct imsrg_ctx {
     bool built = false, usable = false;
     XformDev d{};
     std::vector<void *> allocs;
-    int2 *right = nullptr, *left = nullptr;
-    int nright = 0, nleft = 0, R = 64, kc = 4;
+    int2 *items = nullptr;
+    int nitems = 0;
     long dg_size = 0;
     std::vector<int> blk;  // one-body block of each orbit
   } xf;
@@ -796,64 +796,54 @@ static int xform_tables(imsrg_ctx *ctx) {
   const int norb = hb.norb;
   xf.blk.assign(norb, -1);
   for (int o = 0; o < norb; ++o) xf.blk[o] = hb.ob[o].front();  // the block's first orbit names it
-  std::vector<int> g_start{0}, g_kets, g_ch, k_start(hb.nch + 1, 0), k_grp, k_pos;
+  std::vector<int> g_start{0}, g_kets, g_ch, c_start(hb.nch + 1, 0);
   std::vector<long> g_doff;
-  std::vector<int2> right, left;
   long doff = 0;
-  int maxm = 0, maxn = 0;
+  int maxm = 0;
   for (int c = 0; c < hb.nch; ++c) {
     const auto &kets = hb.ch[c].kets;
     const int n = (int)kets.size();
-    k_start[c] = (int)k_grp.size();
-    maxn = std::max(maxn, n);
+    c_start[c] = (int)g_ch.size();
     std::map<std::pair<int, int>, std::vector<int>> groups;
     for (int i = 0; i < n; ++i) {
       const int bp = xf.blk[hb.kp[kets[i]]], bq = xf.blk[hb.kq[kets[i]]];
       groups[{std::min(bp, bq), std::max(bp, bq)}].push_back(i);
     }
-    k_grp.resize(k_start[c] + n);
-    k_pos.resize(k_start[c] + n);
     for (const auto &kv : groups) {
-      const int G = (int)g_ch.size(), m = (int)kv.second.size();
+      const int m = (int)kv.second.size();
       g_ch.push_back(c);
       g_doff.push_back(doff);
-      doff += (long)m * m;
+      doff += 64L * ((m + 3) / 4) * ((m + 15) / 16);
       maxm = std::max(maxm, m);
-      for (int pos = 0; pos < m; ++pos) {
-        g_kets.push_back(kv.second[pos]);
-        k_grp[k_start[c] + kv.second[pos]] = G;
-        k_pos[k_start[c] + kv.second[pos]] = pos;
-      }
+      g_kets.insert(g_kets.end(), kv.second.begin(), kv.second.end());
       g_start.push_back((int)g_kets.size());
     }
   }
-  k_start[hb.nch] = (int)k_grp.size();
+  c_start[hb.nch] = (int)g_ch.size();
   xf.built = true;
-  // LDS of one work-group stays within 64 KiB; beyond that the dense path runs
-  xf.R = maxm <= 48 ? 64 : 32;
-  xf.kc = maxn <= 2048 ? 4 : maxn <= 4096 ? 2 : 1;
-  if (sizeof(double) * ((size_t)maxm * xf.R + (size_t)maxm * maxm) > 65536 || (size_t)maxn * 8 * xf.kc > 65536)
-    return IMSRG_OK;
-  for (int G = 0; G < (int)g_ch.size(); ++G)
-    for (int r0 = 0; r0 < (int)hb.ch[g_ch[G]].kets.size(); r0 += xf.R) right.push_back(make_int2(G, r0));
-  for (int c = 0; c < hb.nch; ++c)
-    for (int b0 = 0; b0 < (int)hb.ch[c].kets.size(); b0 += xf.kc) left.push_back(make_int2(c, b0));
+  if (maxm > kXfMaxM) return IMSRG_OK;  // beyond a work-group's registers: the dense path
+  // a channel's items on one XCD, whose L2 puts the lines together that several groups write
+  std::vector<TileGroup> runs(hb.nch);
+  for (int G = 0; G < (int)g_ch.size(); ++G) {
+    TileGroup &t = runs[g_ch[G]];
+    const int n = (int)hb.ch[g_ch[G]].kets.size();
+    for (int r0 = 0; r0 < n; r0 += kXfRows) t.tiles.push_back(make_int4(0, G, r0, 0));
+    t.cost += (long)n * (g_start[G + 1] - g_start[G] + 4);
+  }
+  std::vector<int2> items;
+  for (const int4 &w : xcd_order(runs, kXcd)) items.push_back(make_int2(w.y, w.z));
   hipError_t e = hipSuccess;
   XformDev &d = xf.d;
   d.g_start = xf_upload(ctx, g_start, e);
   d.g_kets = xf_upload(ctx, g_kets, e);
   d.g_ch = xf_upload(ctx, g_ch, e);
   d.g_doff = xf_upload(ctx, g_doff, e);
-  d.k_start = xf_upload(ctx, k_start, e);
-  d.k_grp = xf_upload(ctx, k_grp, e);
-  d.k_pos = xf_upload(ctx, k_pos, e);
-  xf.right = xf_upload(ctx, right, e);
-  xf.left = xf_upload(ctx, left, e);
+  d.c_start = xf_upload(ctx, c_start, e);
+  xf.items = xf_upload(ctx, items, e);
   if (e != hipSuccess) return fail(ctx, IMSRG_E_HIP, std::string("basis transformation tables: ") + hipGetErrorString(e));
   d.ngroups = (int)g_ch.size();
   d.maxm = maxm;
-  xf.nright = (int)right.size();
-  xf.nleft = (int)left.size();
+  xf.nitems = (int)items.size();
   xf.dg_size = doff;
   xf.usable = true;
   return IMSRG_OK;
@@ -900,8 +890,8 @@ extern "C" int imsrg_hip_op_transform_basis(imsrg_dop *out, const imsrg_dop *op,
                                      hipMemcpyDeviceToDevice, ctx->stream));
     }
     out->herm = op->herm;
-    HIPCHK(ctx, launch_xform_blocks(ctx->db.d, B, ctx->xf.d, Cd, op->buf, out->buf, T, Dg, T1, ctx->xf.right,
-                                    ctx->xf.nright, ctx->xf.R, ctx->xf.left, ctx->xf.nleft, ctx->xf.kc, ctx->stream));
+    HIPCHK(ctx, launch_xform_blocks(ctx->db.d, B, ctx->xf.d, Cd, op->buf, out->buf, T, Dg, T1, ctx->xf.items,
+                                    ctx->xf.nitems, op->herm, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return IMSRG_OK;
   }

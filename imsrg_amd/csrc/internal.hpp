@@ -31,6 +31,8 @@ constexpr int kInvpLds = 42 * kLdsUnit;  // LDS of an inverse Pandya work-group:
 constexpr int kC122MaxN = 64;     // columns of a comm122 bin formed at once (a larger bin takes one item per 16)
 constexpr int kC122MaxCols = 150; // largest bin (LDS: 1 KiB of coefficients per ket)
 constexpr int kC122Rows = 128;    // rows of one comm122 W item (256: 221 against 210 us at emax = 10)
+constexpr int kXfRows = 128;      // rows of one item of the basis transformation's passes
+constexpr int kXfMaxM = 80;       // kets of its largest group (their fragments are held in registers)
 constexpr int kF32Flush = 4;      // MFMA k-steps (of 4) summed in FP32 before the FP64 flush (mixed, 64x64 tiles)
 
 // GEMM kernel families passed to launch_pphh / launch_ph_gemm: 0 FP64,
@@ -147,10 +149,8 @@ struct XformDev {
   const IMSRG_G int *g_start;   // ngroups + 1: group g holds g_kets[g_start[g] .. g_start[g+1])
   const IMSRG_G int *g_kets;    // channel-local ket indices, ascending within a group
   const IMSRG_G int *g_ch;      // channel of each group
-  const IMSRG_G long *g_doff;   // offset of each group's m x m block of D (column-major)
-  const IMSRG_G int *k_start;   // per channel: where its kets start in k_grp / k_pos
-  const IMSRG_G int *k_grp;     // group of each channel ket
-  const IMSRG_G int *k_pos;     // its position inside the group
+  const IMSRG_G long *g_doff;   // offset of each group's fragments of D
+  const IMSRG_G int *c_start;   // channel c's groups are c_start[c] .. c_start[c+1] - 1
   int ngroups, maxm;
 };
 

@@ -463,90 +463,97 @@ hipError_t launch_hf_mono(const BasisDev *bd, const double *op, const int4 *quad
 // a channel take their orbits from the same pair of one-body blocks, so after
 // grouping each channel's kets by that pair, D is block diagonal with groups of at
 // most (block size)^2 kets, and V' = D^T V D is two passes over the channel:
-//   T  = V D     column a of T mixes the columns of V in a's group   (k_xf_right)
-//   V' = D^T T   row a of V' mixes the rows of T in a's group        (k_xf_left)
-// Every element of V, T and V' is read or written once from HBM.
+//   T  = V D                              column a of T mixes the columns of V in a's group
+//   V' = D^T T = (T^T D)^T                row a of V' mixes the rows of T in a's group
+// and the second is the first on T^T, which k_xf_pass<false> stores: U(a, r) = T(r, a), with
+// its rows a in the order of the groups (X.g_kets), so that both passes read and the first
+// writes runs of consecutive elements.  The second stores V'(a, b) at column b of V' (as
+// V'(b, a), herm times it), at the rows' places, scattered over the column; without
+// Hermiticity at its own place.
+// Every element of V, U and V' is read or written once from HBM.  Both passes are products
+// with small matrices and run on the FP64 matrix units; D is kept as their operand: the 64
+// values of fragment (16 columns c, 4 rows k) of a group lie together, lane l's D(4k + l/16,
+// 16c + l%16), zero past the group.  Bound by HBM: two passes of two-body size, read and
+// written, 293 MB each at emax = 10.  There the first takes 178 us (368 with V and D staged
+// in LDS and vector sums) and the second 269 us (700 with a row of V' per thread on four
+// columns of T in LDS, its D column from the L2; 571 on the matrix units like that).
+typedef double xfd4 __attribute__((ext_vector_type(4)));
 
-// D blocks, one work-group per group g: Dg[doff[g] + r + c m] = D(kets r, c of g)
-// (the formula of k_hf_D).
+// D blocks, one work-group per group g (the formula of k_hf_D).
 __global__ __launch_bounds__(256) void k_xf_D(const BasisDev *bd, XformDev X, const double *C, double *Dg) {
   const BasisDev &B = *bd;
   const int g = blockIdx.x, s = X.g_start[g], m = X.g_start[g + 1] - s, ch = X.g_ch[g], J = ch / 6;
   const long N = B.norb;
   const int *kets = B.ch_kets + B.ch_kstart[ch];
-  for (int e = threadIdx.x; e < m * m; e += blockDim.x) {
-    const int r = e % m, c = e / m;
-    const int ki = kets[X.g_kets[s + r]], ka = kets[X.g_kets[s + c]];
-    const int p = B.kp[ki], q = B.kq[ki], pp = B.kp[ka], qq = B.kq[ka];
-    double d = C[p + pp * N] * C[q + qq * N];
-    if (p != q) {
-      const double ph = (((B.j2[p] + B.j2[q]) / 2 + 1 + J) & 1) ? -1.0 : 1.0;
-      double x = C[q + pp * N] * C[p + qq * N];
-      d += ph * x;
+  const int nks = (m + 3) >> 2, nel = 64 * nks * ((m + 15) >> 4);
+  for (int e = threadIdx.x; e < nel; e += blockDim.x) {
+    const int f = e >> 6, r = 4 * (f % nks) + ((e >> 4) & 3), c = 16 * (f / nks) + (e & 15);
+    double d = 0.0;
+    if (r < m && c < m) {
+      const int ki = kets[X.g_kets[s + r]], ka = kets[X.g_kets[s + c]];
+      const int p = B.kp[ki], q = B.kq[ki], pp = B.kp[ka], qq = B.kq[ka];
+      d = C[p + pp * N] * C[q + qq * N];
+      if (p != q) {
+        const double ph = (((B.j2[p] + B.j2[q]) / 2 + 1 + J) & 1) ? -1.0 : 1.0;
+        double x = C[q + pp * N] * C[p + qq * N];
+        d += ph * x;
+      }
+      if (p == q) d *= 1.4142135623730951;
+      if (pp == qq) d /= 1.4142135623730951;
     }
-    if (p == q) d *= 1.4142135623730951;
-    if (pp == qq) d /= 1.4142135623730951;
     Dg[X.g_doff[g] + e] = d;
   }
 }
 
-// T = V D on one item (group g, rows r0 .. r0+R-1 of its channel): V's rows in
-// the group's columns and the group's D block staged in LDS, then each of the
-// R x m outputs is a dot product of length m.
-__global__ __launch_bounds__(256) void k_xf_right(const BasisDev *bd, XformDev X, const double *V, const double *Dg,
-                                                  double *T, const int2 *items, int R) {
-  extern __shared__ double lds[];
+// One pass on one item (group g, rows r0 .. r0 + kXfRows - 1 of the input): D's fragments in
+// LDS, 16 rows of the input's columns of the group per wave straight into the other operand.
+template <bool SECOND>
+__global__ __launch_bounds__(256) void k_xf_pass(const BasisDev *bd, XformDev X, const double *V, const double *Dg,
+                                                 double *out, const int2 *items, double herm) {
+  extern __shared__ __align__(16) double lds[];
   const BasisDev &B = *bd;
   const int2 it = items[blockIdx.x];
+  if (it.x < 0) return;  // empty item (padding of an XCD run)
   const int g = it.x, r0 = it.y, s = X.g_start[g], m = X.g_start[g + 1] - s, ch = X.g_ch[g];
-  const int n = B.ch_n[ch];
+  const int n = B.ch_n[ch], nks = (m + 3) >> 2, nc = (m + 15) >> 4;
   const long off = B.ch_off[ch];
-  double *Vs = lds, *Ds = lds + (long)X.maxm * R;
-  for (int e = threadIdx.x; e < m * R; e += blockDim.x) {
-    const int k = e / R, row = e - k * R;
-    Vs[e] = (r0 + row < n) ? V[off + (long)X.g_kets[s + k] * n + r0 + row] : 0.0;
-  }
-  for (int e = threadIdx.x; e < m * m; e += blockDim.x) Ds[e] = Dg[X.g_doff[g] + e];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const double *Vc = V + off;
+  double *oc = out + off;
+  const int cs = X.g_start[X.c_start[ch]];  // the channel's first entry of g_kets
+  int *ket = (int *)(lds + 64 * nks * nc);  // the group's kets, past it the last one
+  for (int e = threadIdx.x; e < 16 * nc; e += blockDim.x) ket[e] = X.g_kets[s + min(e, m - 1)];
+  for (int e = threadIdx.x; e < 64 * nks * nc; e += blockDim.x) lds[e] = Dg[X.g_doff[g] + e];
   __syncthreads();
-  const int row = threadIdx.x % R, lanes = blockDim.x / R;
-  if (r0 + row >= n) return;
-  for (int c = threadIdx.x / R; c < m; c += lanes) {
-    double acc = 0.0;
-    for (int k = 0; k < m; ++k) acc += Vs[k * R + row] * Ds[c * m + k];
-    T[off + (long)X.g_kets[s + c] * n + r0 + row] = acc;
-  }
-}
-
-// V' = D^T T on one item (channel ch, columns b0 .. b0+kc-1): the columns of T
-// staged in LDS (ket-major, kc values per ket), then row a of each column is the
-// dot product of a's D column with the rows of T in a's group.
-__global__ __launch_bounds__(256) void k_xf_left(const BasisDev *bd, XformDev X, const double *T, const double *Dg,
-                                                 double *Vout, const int2 *items, int kc) {
-  extern __shared__ double lds[];
-  const BasisDev &B = *bd;
-  const int2 it = items[blockIdx.x];
-  const int ch = it.x, b0 = it.y, n = B.ch_n[ch];
-  const int nb = min(kc, n - b0);
-  const long off = B.ch_off[ch];
-  for (int e = threadIdx.x; e < n * nb; e += blockDim.x) {
-    const int bb = e / n, i = e - bb * n;
-    lds[i * kc + bb] = T[off + (long)(b0 + bb) * n + i];
-  }
-  __syncthreads();
-  const int kbase = X.k_start[ch];
-  for (int a = threadIdx.x; a < n; a += blockDim.x) {
-    const int g = X.k_grp[kbase + a], c = X.k_pos[kbase + a];
-    const int s = X.g_start[g], m = X.g_start[g + 1] - s;
-    const double *Dc = Dg + X.g_doff[g] + (long)c * m;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int k = 0; k < m; ++k) {
-      const double d = Dc[k];
-      const double *t = lds + X.g_kets[s + k] * kc;
-      for (int bb = 0; bb < 4; ++bb)
-        if (bb < nb) acc[bb] += d * t[bb];
+  for (int rb = r0 + 16 * wv; rb < min(n, r0 + kXfRows); rb += 64) {
+    const int row = rb + (lane & 15);
+    const double *v = Vc + min(row, n - 1);
+    double a[kXfMaxM / 4];
+#pragma unroll
+    for (int k = 0; k < kXfMaxM / 4; ++k)
+      if (k < nks) a[k] = v[(long)ket[4 * k + (lane >> 4)] * n];
+    const double f = herm != 0.0 ? herm : 1.0;
+    const int to = SECOND ? X.g_kets[cs + min(row, n - 1)] : 0;  // the row's place in V'
+    for (int c = 0; c < nc; ++c) {
+      xfd4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < kXfMaxM / 4; ++k)
+        if (k < nks) {
+          const double d = lds[(c * nks + k) * 64 + lane];
+          acc = SECOND ? __builtin_amdgcn_mfma_f64_16x16x4f64(d, a[k], acc, 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], d, acc, 0, 0, 0);
+        }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (SECOND) {  // column 4 q + lane / 16, row lane % 16
+          const int col = 16 * c + 4 * q + (lane >> 4);
+          if (col < m && row < n) oc[herm != 0.0 ? (long)ket[col] * n + to : (long)to * n + ket[col]] = f * acc[q];
+        } else {                 // row 4 q + lane / 16, column lane % 16
+          const int col = 16 * c + (lane & 15), rr = rb + 4 * q + (lane >> 4);
+          if (col < m && rr < n) oc[(long)rr * n + s - cs + col] = acc[q];
+        }
+      }
     }
-    for (int bb = 0; bb < 4; ++bb)
-      if (bb < nb) Vout[off + (long)(b0 + bb) * n + a] = acc[bb];
   }
 }
 
@@ -573,14 +580,13 @@ __global__ __launch_bounds__(256) void k_xf_one(const BasisDev *bd, const double
 
 hipError_t launch_xform_blocks(const BasisDev *bd, const BasisDev &bh, const XformDev &X, const double *C,
                                const double *op, double *out, double *T, double *Dg, double *one_tmp,
-                               const int2 *right_items, int nright, int R, const int2 *left_items, int nleft, int kc,
-                               hipStream_t s) {
+                               const int2 *items, int nitems, int herm, hipStream_t s) {
   if (X.ngroups > 0) {
     hipLaunchKernelGGL(k_xf_D, dim3(X.ngroups), dim3(256), 0, s, bd, X, C, Dg);
-    const size_t lr = sizeof(double) * ((size_t)X.maxm * R + (size_t)X.maxm * X.maxm);
-    hipLaunchKernelGGL(k_xf_right, dim3(nright), dim3(256), lr, s, bd, X, op + bh.two_off, Dg, T, right_items, R);
-    const size_t ll = sizeof(double) * (size_t)bh.maxn * kc;
-    hipLaunchKernelGGL(k_xf_left, dim3(nleft), dim3(256), ll, s, bd, X, T, Dg, out + bh.two_off, left_items, kc);
+    const size_t nc = (X.maxm + 15) / 16, lds = 512 * ((X.maxm + 3) / 4) * nc + 64 * nc;
+    hipLaunchKernelGGL(k_xf_pass<false>, dim3(nitems), dim3(256), lds, s, bd, X, op + bh.two_off, Dg, T, items, 1.0);
+    hipLaunchKernelGGL(k_xf_pass<true>, dim3(nitems), dim3(256), lds, s, bd, X, T, Dg, out + bh.two_off, items,
+                       (double)herm);
   }
   const int n1 = bh.norb * bh.norb;
   if (n1 > 0) {
