@@ -41,8 +41,8 @@ struct BatchCache {
   std::vector<long long> key;
   PairPtrs *d_tab = nullptr;
   int4 *d_items = nullptr;
-  size_t off[11] = {0};
-  int cnt[11] = {0};
+  size_t off[12] = {0};
+  int cnt[12] = {0};
   double *work = nullptr;
   int maxn = 0, maxnch = 0, maxn1pairs = 0, maxbin = 0;
   size_t invp_lds[2] = {0, 0};
@@ -178,11 +178,12 @@ struct imsrg_ctx {
   bool profiling = false;
   // phase events of profiled commutators: a ring of sets recorded without host
   // synchronisation, read (and summed) by imsrg_hip_phase_times; marks 0..6 on
-  // the main stream, 7, 8, 9 around the pp/hh GEMM and comm122 on the side stream
-  static constexpr int kRing = 32, kMarks = 10;
+  // the main stream, 7, 8, 9 around the pp/hh GEMM and comm122 on the side stream (9, 10
+  // around comm122 on the main one)
+  static constexpr int kRing = 32, kMarks = 11;
   std::vector<std::array<hipEvent_t, kMarks>> ring;
   int ring_head = 0, ring_count = 0;
-  bool ring_side[kRing] = {};  // set recorded with the pp/hh GEMM on the side stream
+  int ring_side[kRing] = {};  // 1: the pp/hh GEMM and comm122 on the side stream, 2: comm122 on the main one
   double phase_sum[8] = {0};
   int phase_n = 0;
   imsrg_dop *stage[3] = {nullptr, nullptr, nullptr};
@@ -1342,14 +1343,14 @@ static int harvest_oldest(imsrg_ctx *ctx) {
   // marks on the main stream: pp/hh, comm122, first launch (Pandya, zero- and
   // one-body), ph GEMM, inverse Pandya, last launch; reported in the header's order
   const int map[6] = {3, 2, 4, 5, 6, 7};
+  const int side = ctx->ring_side[ctx->ring_head];
   for (int i = 0; i < 6; ++i) {
     float ms = 0.f;
-    if (i == 0 && ctx->ring_side[ctx->ring_head])
-      HIPCHK(ctx, hipEventElapsedTime(&ms, set[7], set[8]));
-    else if (i == 1 && ctx->ring_side[ctx->ring_head])  // comm122 on the side stream
-      HIPCHK(ctx, hipEventElapsedTime(&ms, set[8], set[9]));
-    else
-      HIPCHK(ctx, hipEventElapsedTime(&ms, set[i], set[i + 1]));
+    int a = i, b = i + 1;
+    if (side && i == 0) a = 7, b = 8;
+    if (side && i == 1) a = side == 2 ? 9 : 8, b = side == 2 ? 10 : 9;
+    if (side == 2 && i == 4) b = 9;
+    HIPCHK(ctx, hipEventElapsedTime(&ms, set[a], set[b]));
     ctx->phase_sum[map[i]] += ms * 1000.0;
   }
   ++ctx->phase_n;
@@ -1375,7 +1376,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   const int prec_pphh = gemm_family(prec, tu.mixed_pphh);
   const int prec_ph = gemm_family(prec, tu.mixed_ph);
   hipStream_t s = ctx->stream;
-  // With overlap, the pp/hh GEMM and then comm122's W run on the side stream
+  // With overlap, the pp/hh GEMM and then (mostly) comm122's W run on the side stream
   // next to the first launch (zero-body, one-body, Pandya), the ph GEMM and the
   // inverse Pandya kernel (none of them touches the upper triangle of Z's
   // two-body blocks); the main stream waits for them before the last kernel,
@@ -1384,6 +1385,12 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so
   // that the pp/hh GEMM shares the GPU with the inverse Pandya gather only
   const bool fork_late = overlap && tu.overlap_pphh == 2;
+  const int big = prec_pphh == kGemmB3 ? 11 : 0;  // the bf16x3 GEMM's order of the 128x128 tiles
+  // comm122's W on the main stream, after the inverse Pandya kernel, where the bf16x3 GEMM
+  // takes longer than the main stream's kernels: that GEMM leaves the memory idle.  emax = 10
+  // (1539 tiles) 1801 -> 1759 us, emax = 12 (5387) 8.22 -> 8.08 ms; emax = 9 (700) 805 -> 812,
+  // FP64 emax = 10 2630 -> 2638 us, where the FP64 GEMM's waves leave no room beside them.
+  const bool c122_main = overlap && prec_pphh == kGemmB3 && cnt[big] > 1024;
   // profiling: this commutator's phase events go to the next free set of the ring
   std::array<hipEvent_t, imsrg_ctx::kMarks> *set = nullptr;
   if (ctx->profiling) {
@@ -1391,7 +1398,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
       if (int rc = harvest_oldest(ctx)) return rc;
     const int slot = (ctx->ring_head + ctx->ring_count) % imsrg_ctx::kRing;
     set = &ctx->ring[slot];
-    ctx->ring_side[slot] = overlap;
+    ctx->ring_side[slot] = c122_main ? 2 : overlap ? 1 : 0;
   }
   auto mark = [&](int i) -> hipError_t { return set ? hipEventRecord((*set)[i], s) : hipSuccess; };
   // The side stream starts where the fork event was recorded.  Its calls come after the
@@ -1400,10 +1407,10 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   auto side_work = [&]() -> int {
     HIPCHK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork, 0));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[7], ctx->side));
-    HIPCHK(ctx, launch_pphh(pa, items[0], cnt[0], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, ctx->side));
+    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, ctx->side));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[8], ctx->side));
-    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
+    if ((mask & M122) && !c122_main) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
+    if (set && !c122_main) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, hipEventRecord(ctx->join, ctx->side));
     return IMSRG_OK;
   };
@@ -1411,7 +1418,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   HIPCHK(ctx, mark(0));
   if (overlap) {
   } else if (mask & MPPHH) {
-    HIPCHK(ctx, launch_pphh(pa, items[0], cnt[0], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, s));
+    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, s));
   } else {
     HIPCHK(ctx, launch_zero_two(pa, items[6], cnt[6], s));
   }
@@ -1429,6 +1436,11 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   if (mask & MPH) {
     const int f = prec_ph == 1 ? 10 : 4;  // FP32 Zbar: twice the elements per item
     HIPCHK(ctx, launch_invpandya(pa, items[f], cnt[f], invp_lds[prec_ph == 1], prec_ph == 1, s));
+  }
+  if (c122_main) {
+    HIPCHK(ctx, mark(9));
+    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
+    HIPCHK(ctx, mark(10));
   }
   if (overlap) {
     if (int rc = side_work()) return rc;
@@ -1499,13 +1511,13 @@ static int commutator_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y
   pa.p0.hZ = herm_rule(X->herm, Y->herm);
   pa.p0.mask = mask;
   Z->herm = pa.p0.hZ;
-  const int4 *items[11] = {db.d_pphh, db.d_ph,     db.d_ob221,  db.d_pandya, db.d_invp,  db.d_one,
-                           db.d_mirror, db.d_pphh64, db.d_pack,   db.d_c122w,  db.d_invp32};
+  const int4 *items[12] = {db.d_pphh,   db.d_ph,     db.d_ob221, db.d_pandya, db.d_invp,   db.d_one,
+                           db.d_mirror, db.d_pphh64, db.d_pack,  db.d_c122w,  db.d_invp32, db.d_pphh_b3};
   const size_t invp_lds[2] = {db.invp_lds(false), db.invp_lds(true)};
-  int cnt[11] = {(int)db.wl.pphh.size(),   (int)db.wl.ph.size(),   (int)db.wl.ob221.size(),
+  int cnt[12] = {(int)db.wl.pphh.size(),   (int)db.wl.ph.size(),   (int)db.wl.ob221.size(),
                  (int)db.wl.pandya.size(), (int)db.wl.invp.size(),  (int)db.wl.one.size(),
                  (int)db.wl.mirror.size(), (int)db.wl.pphh64.size(), (int)db.wl.pack.size(),
-                 (int)db.wl.c122w.size(),  (int)db.wl.invp32.size()};
+                 (int)db.wl.c122w.size(),  (int)db.wl.invp32.size(), (int)db.wl.pphh_b3.size()};
   if (!ctx->use_graphs || ctx->profiling || ws)
     return run_commutator(ctx, pa, 1, items, cnt, mask, prec, db.h.maxn, db.h.nch, db.h.n1pairs,
                           db.h.c122_maxbin, invp_lds);
@@ -2252,6 +2264,8 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       bc.cnt[t] = (int)all[t].size();
       tot += all[t].size();
     }
+    bc.off[11] = bc.off[0];  // the pairs are small: one order of the 128x128 tiles for all precisions
+    bc.cnt[11] = bc.cnt[0];
     HIPCHK(c0, hipMalloc(&bc.d_items, sizeof(int4) * std::max<size_t>(tot, 1)));
     for (int t = 0; t < 11; ++t)
       if (!all[t].empty())
@@ -2263,8 +2277,8 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
   PairArg pa;
   std::memset(&pa.p0, 0, sizeof(pa.p0));
   pa.tab = bc.d_tab;
-  const int4 *items[11];
-  for (int t = 0; t < 11; ++t) items[t] = bc.d_items + bc.off[t];
+  const int4 *items[12];
+  for (int t = 0; t < 12; ++t) items[t] = bc.d_items + bc.off[t];
   // The batch runs on c0's stream.  Work queued on the other contexts' streams
   // (uploads, copies, axpy, generators of X_i / Y_i) finishes before it starts,
   // and their later work (downloads, norms of Z_i) waits for it to end.

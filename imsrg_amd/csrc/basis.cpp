@@ -736,7 +736,7 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
   wl = WorkLists();
   {
     // pp/hh tiles: 64x64 for channels with n <= t.pphh_small, 128x128 otherwise
-    std::vector<TileGroup> groups;
+    std::vector<TileGroup> groups, supers;
     for (int c = 0; c < nch; ++c) {
       const int nk = ch_n[c];
       if (nk == 0) continue;
@@ -748,21 +748,18 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
       }
       const int nt = (nk + kTileB - 1) / kTileB;
       const long kk = k_start[c + 1] - k_start[c];
-      if (t.pphh_order == 2) {
-        // square super-tiles of kSuper x kSuper tiles: their work-groups run
-        // together on one XCD and share the A and B row blocks in its L2
-        for (int rs = 0; rs < nt; rs += kSuper)
-          for (int ss = rs; ss < nt; ss += kSuper) {
-            TileGroup g;
-            for (int rb = rs; rb < std::min(rs + kSuper, nt); ++rb)
-              for (int sb = std::max(rb, ss); sb < std::min(ss + kSuper, nt); ++sb)
-                g.tiles.push_back(make_int4(0, c, rb, sb));
-            if (g.tiles.empty()) continue;
-            g.cost = (kk + 1) * (long)g.tiles.size();
-            groups.push_back(g);
-          }
-        continue;
-      }
+      // square super-tiles of kSuper x kSuper tiles: their work-groups run together on one
+      // XCD and share the A and B row blocks in its L2
+      for (int rs = 0; rs < nt; rs += kSuper)
+        for (int ss = rs; ss < nt; ss += kSuper) {
+          TileGroup g;
+          for (int rb = rs; rb < std::min(rs + kSuper, nt); ++rb)
+            for (int sb = std::max(rb, ss); sb < std::min(ss + kSuper, nt); ++sb)
+              g.tiles.push_back(make_int4(0, c, rb, sb));
+          if (g.tiles.empty()) continue;
+          g.cost = (kk + 1) * (long)g.tiles.size();
+          supers.push_back(g);
+        }
       for (int rb = 0; rb < nt; ++rb) {
         TileGroup g;
         for (int sb = rb; sb < nt; ++sb) g.tiles.push_back(make_int4(0, c, rb, sb));
@@ -780,7 +777,7 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
         for (int r = 0; r < nrp; r += 256) wl.pack.push_back(make_int4(0, c, o, r / 256));
     }
     if (t.pphh_order >= 1) {
-      wl.pphh = xcd_order(groups, kXcd);
+      wl.pphh = xcd_order(t.pphh_order == 2 ? supers : groups, kXcd);
     } else {
       std::vector<std::pair<long, int4>> ts;
       for (auto &g : groups)
@@ -790,6 +787,11 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
       });
       for (auto &x : ts) wl.pphh.push_back(x.second);
     }
+    // the bf16x3 GEMM reads its panels faster than memory delivers them: unless row-block
+    // groups are asked for it takes the super-tiles (emax = 8 402 -> 393 us, emax = 10
+    // 1806 -> 1764 us, emax = 12 with the kernel's phases 8.36 -> 8.24 ms; the FP64 GEMM
+    // is slower with them, emax = 10 2624 -> 2662 us: their last ones leave CUs idle)
+    wl.pphh_b3 = t.pphh_order == 1 ? wl.pphh : xcd_order(supers, kXcd);
   }
   for (int c = 0; c < nch; ++c) {
     const int nk = ch_n[c];
@@ -866,7 +868,7 @@ std::string DeviceBasis::build_lists(const Tuning &t) {
     return (int4 *)p;
   };
   d_pphh = up(wl.pphh); d_pphh64 = up(wl.pphh64); d_ph = up(wl.ph); d_pack = up(wl.pack);
-  d_pandya = up(wl.pandya); d_invp = up(wl.invp); d_invp32 = up(wl.invp32);
+  d_pandya = up(wl.pandya); d_invp = up(wl.invp); d_invp32 = up(wl.invp32); d_pphh_b3 = up(wl.pphh_b3);
   d_one = up(wl.one); d_mirror = up(wl.mirror); d_gen = up(wl.gen); d_ob221 = up(wl.ob221);
   d_c122w = up(wl.c122w);
   if (err.empty()) tune = t;

@@ -59,6 +59,7 @@ struct Tuning {
 // Work-item lists (int4: pair, a, b, c) for every kernel of one commutator.
 struct WorkLists {
   std::vector<int4> pphh;    // (pair, ch, rb, sb), rb <= sb, 128x128 tiles
+  std::vector<int4> pphh_b3; // the same tiles in the order of the bf16x3 GEMM
   std::vector<int4> pphh64;  // (pair, ch, rb, sb), rb <= sb, 64x64 tiles (channels n <= pphh_small)
   std::vector<int4> pack;    // (pair, ch, k octet, 256-row block): bf16x3 panels of the 128x128-tile channels
   std::vector<int4> ph;      // (pair, cc, rb, sb), rb <= sb, tiles of 128 (ph_big) or 64
@@ -82,7 +83,7 @@ struct DeviceBasis {
   Tuning tune;
   int4 *d_pphh = nullptr, *d_pphh64 = nullptr, *d_ph = nullptr, *d_pandya = nullptr, *d_pack = nullptr,
        *d_invp = nullptr, *d_one = nullptr, *d_mirror = nullptr, *d_gen = nullptr, *d_ob221 = nullptr,
-       *d_c122w = nullptr, *d_invp32 = nullptr;
+       *d_c122w = nullptr, *d_invp32 = nullptr, *d_pphh_b3 = nullptr;
   // host tables the work lists are built from
   std::vector<int> ch_n, k_start, cc_n, cc_nph, grp_start, grp_kets, gen_ok;
   std::vector<int> ch_kstart, c122_start;

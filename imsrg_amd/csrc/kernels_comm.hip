@@ -1080,16 +1080,31 @@ __global__ __launch_bounds__(256) void k_pack_pphh(PairArg pa, const int4 *items
   }
 }
 
-// Measured alternatives at emax = 10 (pp/hh phase with the packing, 740 us
-// for this kernel): register-staged copies two stages ahead 751 us; three LDS
-// stages with the copies' waits written by hand 790 us; two wave groups that
-// alternate between LDS reads and MFMA 800 us.  The kernel streams 4.0 GB of
-// panels per commutator through L2 into LDS, and that stream sets its time:
-// the copies alone take 510 us, 205 us when every tile re-reads data that
-// stays in L2.
+// The stream of panels through the L2 into LDS (4.0 GB per commutator at emax = 10) and the
+// matrix instructions take about as long as each other: alone, 494 us and 377 us at
+// emax = 10, 2.96 and 2.39 ms at emax = 12 (327 us and 1.94 ms for the stream with the tiles
+// in super-tile order).  One work-group of two waves per SIMD that waited for its copies,
+// read and computed stage by stage took 541 us and 3.49 ms, with the copies two stages ahead
+// 541 and 3.38, with the FP64 sums of a stage between the next one's matrix instructions
+// 530 and 3.40; with both, the waves in two groups a phase apart and the super-tiles 496 us
+// and 3.08 ms (the same phases with two LDS stages: 550 us and 3.55 ms).
+// Waits until at most N of this wave's copies into LDS are in flight.
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  __builtin_amdgcn_s_waitcnt(0x0F70 | N);  // expcnt and lgkmcnt untouched
+}
+// Work-group barrier that waits for this wave's LDS reads and writes but, unlike
+// __syncthreads(), not for its copies from memory into LDS.
+__device__ __forceinline__ void barrier_lds() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, const int4 *items) {
   constexpr int T = kTileB;
-  __shared__ __align__(16) StageB3 L0, L1;
+  __shared__ __align__(16) StageB3 L0, L1, L2;  // 3 x 48 KiB: one work-group per CU
   __shared__ signed char s_ph[2][T];  // unused in this mode (epilogue signature)
   const int4 it = items[blockIdx.x];
   if (it.y < 0) return;  // padding item of the XCD-balanced order
@@ -1131,56 +1146,94 @@ __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, co
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int b = 0; b < kGN; ++b) acc[a][b] = dbl4{0.0, 0.0, 0.0, 0.0};
-  // six bf16 products of a stage summed in FP32 (smallest first), then
-  // flushed into FP64 with the half's factor (1, or h for the second half)
-  auto compute = [&](const StageB3 &L, double fl) {
+  // A stage in two phases: its operands from LDS into registers, then six bf16 products
+  // summed in FP32 (smallest first) into t, while the previous stage's sums u go to the FP64
+  // accumulators with their half's factor (1, or h for the second half).  Waves 0..3, one per
+  // SIMD, are one phase ahead of waves 4..7: while one wave of a SIMD keeps the matrix unit
+  // busy, the other reads.
+  bf16x8 bfr[kGN][3], af[3][4];
+  auto read = [&](const StageB3 &L) {
     if (!wave_live) return;
     const int oc = lane >> 4, rl = lane & 15;
-    bf16x8 bfr[kGN][3];
 #pragma unroll
-    for (int pc = 0; pc < 3; ++pc)
+    for (int pc = 2; pc >= 0; --pc) {
 #pragma unroll
       for (int ni = 0; ni < kGN; ++ni) bfr[ni][pc] = L[1][pc][oc][wc + ni * 16 + rl];
-    flt4 t[4][kGN];
+#pragma unroll
+      for (int mi = 0; mi < 4; ++mi) af[pc][mi] = L[0][pc][oc][wr + mi * 16 + rl];
+    }
+  };
+  auto compute = [&](flt4 (&t)[4][kGN], const flt4 (&u)[4][kGN], double fl) {
+    if (!wave_live) return;
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
       for (int ni = 0; ni < kGN; ++ni) t[mi][ni] = flt4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int pa3 = 2; pa3 >= 0; --pa3) {
-      bf16x8 af[4];
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi) af[mi] = L[0][pa3][oc][wr + mi * 16 + rl];
+    for (int pa3 = 2; pa3 >= 0; --pa3)
 #pragma unroll
       for (int pb3 = 2 - pa3; pb3 >= 0; --pb3)
 #pragma unroll
         for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
           for (int ni = 0; ni < kGN; ++ni)
-            t[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ni][pb3], af[mi], t[mi][ni], 0, 0, 0);
-    }
+            t[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[ni][pb3], af[pa3][mi], t[mi][ni], 0, 0, 0);
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
       for (int ni = 0; ni < kGN; ++ni)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[mi][ni][q] += fl * (double)t[mi][ni][q];
+        for (int q = 0; q < 4; ++q) acc[mi][ni][q] += fl * (double)u[mi][ni][q];
+    // 48 matrix instructions with the 64 conversions and adds between them
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+    }
   };
   if (nst > 0) {  // a channel without pp or hh kets only writes zeros
+    flt4 t0[4][kGN], t1[4][kGN];
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < kGN; ++ni) t0[mi][ni] = t1[mi][ni] = flt4{0.f, 0.f, 0.f, 0.f};
+    auto factor = [&](int st) { return st >= nst1 ? h : 1.0; };
     issue(0, L0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    for (int st = 0; st < nst; st += 2) {
-      if (st + 1 < nst) issue(st + 1, L1);
-      compute(L0, st >= nst1 ? h : 1.0);
-      __builtin_amdgcn_s_waitcnt(0);  // this wave's copies of the next stage have landed
-      __syncthreads();
-      if (st + 1 >= nst) break;
-      if (st + 2 < nst) issue(st + 2, L0);
-      compute(L1, st + 1 >= nst1 ? h : 1.0);
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
+    issue(1, L1);  // nst is even
+    wait_copies<6>();
+    barrier_lds();
+    if (wv >= 4) barrier_lds();
+    // stage st in L.  When it starts, the copies of st have landed in every wave, and every
+    // wave has read st - 1, whose buffer Ln takes st + 2; past the end the last stage again,
+    // so that six copies are in flight always
+    auto stage = [&](int st, const StageB3 &L, StageB3 &Ln, flt4 (&t)[4][kGN], const flt4 (&u)[4][kGN]) {
+      issue(min(st + 2, nst - 1), Ln);
+      read(L);
+      wait_copies<6>();  // those of st + 1
+      barrier_lds();
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t, u, factor(st - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      barrier_lds();
+    };
+    for (int st = 0; st < nst; st += 6) {
+      stage(st, L0, L2, t0, t1);
+      stage(st + 1, L1, L0, t1, t0);
+      if (st + 2 >= nst) break;
+      stage(st + 2, L2, L1, t0, t1);
+      stage(st + 3, L0, L2, t1, t0);
+      if (st + 4 >= nst) break;
+      stage(st + 4, L1, L0, t0, t1);
+      stage(st + 5, L2, L1, t1, t0);
     }
+    if (wv < 4) barrier_lds();
+    wait_copies<0>();
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < kGN; ++ni)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[mi][ni][q] += h * (double)t1[mi][ni][q];
   }
   gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph);
 }

@@ -321,8 +321,9 @@ int imsrg_hip_set_graphs(imsrg_ctx *ctx, int on);
 typedef struct {
   int pphh_small_tile_max;  /* channels with n <= this use 64x64 pp/hh tiles, larger ones 128x128
                                (default 64) */
-  int pphh_order;           /* 0: pp/hh tiles by decreasing k-length; 1: row-block groups balanced over XCDs;
-                               2: 8x8-tile super-tiles balanced over XCDs (shared operand blocks in one L2) */
+  int pphh_order;           /* 0: pp/hh tiles by decreasing k-length (bf16 MFMA: as 2); 1: row-block groups
+                               balanced over XCDs; 2: 8x8-tile super-tiles balanced over XCDs (shared operand
+                               blocks in one L2) */
   int mixed_pphh_fp32;      /* IMSRG_PREC_MIXED: pp/hh GEMM on 2 = bf16 MFMA with three-way split
                                operands (default; channels on 64x64 tiles stay FP64), 1 = FP32 MFMA
                                on FP32-rounded operands, 0 = FP64 MFMA (IMSRG_PREC_SPLIT ignores both
@@ -333,8 +334,8 @@ typedef struct {
   int ph_tile_128;          /* 1: ph GEMM on 128x128 tiles, 0: on 64x64 tiles */
   int finish_order;         /* tile pairs of the last kernel (fold, comm122, mirror): 0 in channel and
                                row-block order, 1 cut into 8 runs of consecutive tiles, one per XCD */
-  int overlap_pphh;         /* pp/hh GEMM (then comm122) on a second stream of the context: 0 no (one
-                               stream); 1 forked before the first kernel, beside the one-body, Pandya,
+  int overlap_pphh;         /* pp/hh GEMM (then comm122, unless that GEMM is the longer part) on a second
+                               stream of the context: 0 no (one stream); 1 forked before the first kernel, beside the one-body, Pandya,
                                ph GEMM and inverse Pandya kernels; 2 forked after the ph GEMM, beside
                                the inverse Pandya kernel only */
   double us_per_commutator; /* autotune: measured time of the chosen setting (0 when set by hand) */
