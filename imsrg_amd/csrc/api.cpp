@@ -1376,20 +1376,28 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   const int prec_pphh = gemm_family(prec, tu.mixed_pphh);
   const int prec_ph = gemm_family(prec, tu.mixed_ph);
   hipStream_t s = ctx->stream;
+  // On small bases the first launch takes comm122's W and the 64x64 pp/hh tiles as well.
   // With overlap, the pp/hh GEMM and then (mostly) comm122's W run on the side stream
   // next to the first launch (zero-body, one-body, Pandya), the ph GEMM and the
   // inverse Pandya kernel (none of them touches the upper triangle of Z's
   // two-body blocks); the main stream waits for them before the last kernel,
   // which folds, applies W and mirrors.
-  const bool overlap = tu.overlap_pphh && (mask & MPPHH);
+  const int big = prec_pphh == kGemmB3 ? 11 : 0;  // the bf16x3 GEMM's order of the 128x128 tiles
+  const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
+  FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
+                mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big, items[7], items[9], mask & MPPHH ? cnt[7] : 0,
+                mask & M122 ? cnt[9] : 0};
+  const bool small = fi.blocks() <= (prec_pphh == 0 || prec_pphh == 2 ? kFrontSmallF64 : kFrontSmall);
+  if (!small) fi.n64 = fi.nc122 = 0;
+  const bool overlap = tu.overlap_pphh && (mask & MPPHH) && !(small && cnt[big] == 0);
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so
   // that the pp/hh GEMM shares the GPU with the inverse Pandya gather only
   const bool fork_late = overlap && tu.overlap_pphh == 2;
-  const int big = prec_pphh == kGemmB3 ? 11 : 0;  // the bf16x3 GEMM's order of the 128x128 tiles
   // comm122's W on the main stream, after the inverse Pandya kernel, where the bf16x3 GEMM
   // takes longer than the main stream's kernels: that GEMM leaves the memory idle.  emax = 10
   // (1539 tiles) 1801 -> 1759 us, emax = 12 (5387) 8.22 -> 8.08 ms; emax = 9 (700) 805 -> 812,
   // FP64 emax = 10 2630 -> 2638 us, where the FP64 GEMM's waves leave no room beside them.
+  const bool m122 = (mask & M122) && fi.nc122 == 0;  // comm122's W in a launch of its own
   const bool c122_main = overlap && prec_pphh == kGemmB3 && cnt[big] > 1024;
   // profiling: this commutator's phase events go to the next free set of the ring
   std::array<hipEvent_t, imsrg_ctx::kMarks> *set = nullptr;
@@ -1407,9 +1415,10 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   auto side_work = [&]() -> int {
     HIPCHK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork, 0));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[7], ctx->side));
-    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, ctx->side));
+    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7] - fi.n64, items[8], cnt[8], prec_pphh, maxn,
+                            ctx->side));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[8], ctx->side));
-    if ((mask & M122) && !c122_main) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
+    if (m122 && !c122_main) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
     if (set && !c122_main) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, hipEventRecord(ctx->join, ctx->side));
     return IMSRG_OK;
@@ -1418,17 +1427,14 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   HIPCHK(ctx, mark(0));
   if (overlap) {
   } else if (mask & MPPHH) {
-    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7], items[8], cnt[8], prec_pphh, maxn, s));
+    HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7] - fi.n64, items[8], cnt[8], prec_pphh, maxn, s));
   } else {
     HIPCHK(ctx, launch_zero_two(pa, items[6], cnt[6], s));
   }
   HIPCHK(ctx, mark(1));
-  if ((mask & M122) && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
+  if (m122 && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
   HIPCHK(ctx, mark(2));
-  const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
-  const FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
-                      mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big};
-  HIPCHK(ctx, launch_front(pa, fi, maxnch, s));
+  HIPCHK(ctx, launch_front(pa, fi, maxnch, maxbin, prec_pphh == 1, s));
   HIPCHK(ctx, mark(3));
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));
   if (fork_late) HIPCHK(ctx, hipEventRecord(ctx->fork, s));
@@ -1439,7 +1445,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   }
   if (c122_main) {
     HIPCHK(ctx, mark(9));
-    if (mask & M122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
+    if (m122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
     HIPCHK(ctx, mark(10));
   }
   if (overlap) {

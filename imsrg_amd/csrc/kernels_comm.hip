@@ -281,7 +281,7 @@ __device__ __forceinline__ void final_one(const PairPtrs &P, int blk) {
 // MIXED: operands rounded to FP32 in LDS, products on f32 16x16x4 MFMA, FP32
 // partial sums over kF32Flush k-steps added into the FP64 accumulators.
 template <int MODE, bool MIXED>
-__global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, int accumulate) {
+__device__ __forceinline__ void syr2k_tile(const PairArg &pa, const int4 &it) {
   constexpr int LD = kTile + 2;
   using ST = typename std::conditional<MIXED, float, double>::type;
   // the FP32-product ph GEMM keeps Zbar in FP32 (its inverse Pandya gather reads
@@ -289,7 +289,6 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
   using ZT = typename std::conditional<MIXED && MODE != 0, float, double>::type;
   __shared__ ST As[2][kTileK][LD];
   __shared__ ST Bs[2][kTileK][LD];
-  const int4 it = items[blockIdx.x];
   PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
   const double *Am, *Bm;
@@ -456,7 +455,7 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
           if (row < n && col < n && row <= col) {
             const double v = alpha * acc[mi][ni][q];
             double *dp = D + (long)col * n + row;
-            *dp = accumulate ? *dp + v : v;
+            *dp = v;
           }
         }
   } else {
@@ -491,6 +490,10 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items, in
       }
     }
   }
+}
+template <int MODE, bool MIXED>
+__global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items) {
+  syr2k_tile<MODE, MIXED>(pa, items[blockIdx.x]);
 }
 
 
@@ -1515,9 +1518,7 @@ __device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, 
 // order): zero-body channels, one-body pairs, comm221 partial sums, Pandya chunks.
 // Launched one after another they are a chain of four launches of mostly latency
 // before the ph GEMM can start (emax = 6: 6 + 18 + 15 + 15 us and the gaps).
-__global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  int b = blockIdx.x;
+__device__ __forceinline__ void front(const PairArg &pa, const FrontItems &f, int b, unsigned char *lds_raw) {
   if (b < f.nzeros) {
     front_zero(pa.get(b / f.nzero), b % f.nzero);
     return;
@@ -1536,6 +1537,10 @@ __global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
   }
   const int4 it = f.pandya[b - f.n221];
   front_pandya(pa.get(it.x), it, f.xbar_f32, lds_raw);
+}
+__global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  front(pa, f, blockIdx.x, lds_raw);
 }
 
 // AddInversePandyaTransformation (src/Commutator.cc:1501-1616), by bra.
@@ -1938,11 +1943,8 @@ inline size_t c122w_lds_bytes(int maxbin) {
   return 16 * std::max(full, 16 * k4) +  // both matrices of a whole bin, or of 16 columns of a larger one
          sizeof(int) * (size_t)maxbin;
 }
-__global__ __launch_bounds__(256, 4) void k_c122_w(PairArg pa, const int4 *items) {
-  extern __shared__ __align__(16) unsigned char lds_raw[];
+__device__ __forceinline__ void c122_w_tile(const PairPtrs &P, const int4 &it, unsigned char *lds_raw) {
   constexpr int KF = kC122MaxN / 4;  // A fragments (4 columns each) held at once
-  const int4 it = items[blockIdx.x];
-  PairPtrs P = pa.get(it.x);
   const BasisDev &B = *P.basis;
   const int ch = it.y, n = B.ch_n[ch];
   const int b0 = B.c122_boff[it.z], nc = B.c122_boff[it.z + 1] - b0;
@@ -2008,6 +2010,26 @@ __global__ __launch_bounds__(256, 4) void k_c122_w(PairArg pa, const int4 *items
       }
     }
   }
+}
+__global__ __launch_bounds__(256, 4) void k_c122_w(PairArg pa, const int4 *items) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int4 it = items[blockIdx.x];
+  c122_w_tile(pa.get(it.x), it, lds_raw);
+}
+
+// The first launch of small bases: their comm122 W items and 64x64 pp/hh tiles, which wait
+// for nothing either, beside the others.
+template <bool MIXED>
+__global__ __launch_bounds__(256, 4) void k_front_small(PairArg pa, FrontItems f) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  int b = blockIdx.x;
+  if (b < f.n64) return syr2k_tile<0, MIXED>(pa, f.pphh64[b]);
+  b -= f.n64;
+  if (b < f.nc122) {
+    const int4 it = f.c122[b];
+    return c122_w_tile(pa.get(it.x), it, lds_raw);
+  }
+  front(pa, f, b - f.nc122, lds_raw);
 }
 
 // 16-byte access to elements idx, idx + 1 of a channel block (8-byte aligned)
@@ -2162,8 +2184,17 @@ hipError_t launch_set_pairs(PairPtrs *tab, const PairOps &ops, hipStream_t s) {
 // faster (emax = 8 mixed 492 -> 473 us, emax = 6 mixed 159 -> 146 us).
 constexpr int kFrontSplit = 12288;
 
-hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipStream_t s) {
-  const size_t lds = sizeof(int4) * (size_t)std::max(maxnch, 1);  // the Pandya chunks' channel table
+hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int maxbin, bool mixed64, hipStream_t s) {
+  size_t lds = sizeof(int4) * (size_t)std::max(maxnch, 1);  // the Pandya chunks' channel table
+  if (f.n64 + f.nc122 > 0) {
+    if (f.nc122 > 0) lds = std::max(lds, c122w_lds_bytes(maxbin));
+    const dim3 grid(f.blocks());
+    if (mixed64)
+      hipLaunchKernelGGL(k_front_small<true>, grid, dim3(256), lds, s, pa, f);
+    else
+      hipLaunchKernelGGL(k_front_small<false>, grid, dim3(256), lds, s, pa, f);
+    return hipGetLastError();
+  }
   FrontItems part[2] = {f, f};
   if (f.npandya > kFrontSplit) {
     part[0].npandya = 0;
@@ -2171,10 +2202,8 @@ hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipS
   } else {
     part[1].nzeros = part[1].none = part[1].n221 = part[1].npandya = 0;
   }
-  for (const FrontItems &p : part) {
-    const int n = p.nzeros + p.none + p.n221 + p.npandya;
-    if (n > 0) hipLaunchKernelGGL(k_front, dim3(n), dim3(256), lds, s, pa, p);
-  }
+  for (const FrontItems &p : part)
+    if (p.blocks() > 0) hipLaunchKernelGGL(k_front, dim3(p.blocks()), dim3(256), lds, s, pa, p);
   return hipGetLastError();
 }
 hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const int4 *items64, int nitems64,
@@ -2194,9 +2223,9 @@ hipError_t launch_pphh(const PairArg &pa, const int4 *items, int nitems, const i
   }
   if (nitems64 > 0) {  // split and bf16x3 products take FP64 64x64 tiles
     if (precision == 1)
-      hipLaunchKernelGGL((k_syr2k<0, true>), dim3(nitems64), dim3(256), 0, s, pa, items64, 0);
+      hipLaunchKernelGGL((k_syr2k<0, true>), dim3(nitems64), dim3(256), 0, s, pa, items64);
     else
-      hipLaunchKernelGGL((k_syr2k<0, false>), dim3(nitems64), dim3(256), 0, s, pa, items64, 0);
+      hipLaunchKernelGGL((k_syr2k<0, false>), dim3(nitems64), dim3(256), 0, s, pa, items64);
   }
   return hipGetLastError();
 }
@@ -2215,11 +2244,11 @@ hipError_t launch_ph_gemm(const PairArg &pa, const int4 *items, int nitems, int 
     return hipGetLastError();
   }
   if (precision == 1) {
-    hipLaunchKernelGGL((k_syr2k<1, true>), dim3(nitems), dim3(256), 0, s, pa, items, 0);
-    hipLaunchKernelGGL((k_syr2k<2, true>), dim3(nitems), dim3(256), 0, s, pa, items, 0);
+    hipLaunchKernelGGL((k_syr2k<1, true>), dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL((k_syr2k<2, true>), dim3(nitems), dim3(256), 0, s, pa, items);
   } else {
-    hipLaunchKernelGGL((k_syr2k<1, false>), dim3(nitems), dim3(256), 0, s, pa, items, 0);
-    hipLaunchKernelGGL((k_syr2k<2, false>), dim3(nitems), dim3(256), 0, s, pa, items, 0);
+    hipLaunchKernelGGL((k_syr2k<1, false>), dim3(nitems), dim3(256), 0, s, pa, items);
+    hipLaunchKernelGGL((k_syr2k<2, false>), dim3(nitems), dim3(256), 0, s, pa, items);
   }
   return hipGetLastError();
 }

@@ -33,8 +33,20 @@ struct FrontItems {
   const int4 *one, *ob221, *pandya;
   int nzero, nzeros, none, n221, npandya;
   bool xbar_f32;  // Xbar and Ybar in FP32 (the ph GEMM on 128x128 tiles with FP32 products reads them so)
+  // small bases: the 64x64 pp/hh tiles and comm122's W items, in the same launch
+  const int4 *pphh64, *c122;
+  int n64, nc122;
+  int blocks() const { return n64 + nc122 + nzeros + none + n221 + npandya; }
 };
-hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, hipStream_t s);
+// mixed64: the pp/hh tiles with FP32 products
+hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int maxbin, bool mixed64, hipStream_t s);
+// Work-groups up to which the first launch takes those as well: one launch, and without
+// 128x128 pp/hh tiles no second stream, instead of three launches and four stream events,
+// which cost the smallest bases more than their work (emax = 2 FP64 49 -> 28 us, emax = 3
+// 50 -> 34, emax = 5 95 -> 90, mixed 76 -> 71 us).  Where they fill the chip they only hold up the main
+// stream: emax = 6 mixed 100 -> 105 us.  Beside an FP64 (or split) GEMM, which makes the side
+// stream the longer one, that comes later: emax = 6 155 -> 142 us, emax = 7 250 -> 254 us.
+constexpr int kFrontSmall = 3000, kFrontSmallF64 = 6000;
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
 // under bf16x3 products (kGemmB3) the pack items first write the operand panels
 // maxn: the largest channel dimension of the pairs (sizes the kernel's LDS index list)

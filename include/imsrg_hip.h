@@ -352,7 +352,8 @@ int imsrg_hip_autotune(imsrg_ctx *ctx, int precision, const char *cache_path, im
 
 /* Per-phase timing of commutators on ctx (microseconds, HIP events):
  * [2] comm122's W, [3] pp/hh GEMM, [4] first launch (Pandya gather with the
- * zero- and one-body terms beside it), [5] ph GEMM, [6] inverse Pandya, [7] last
+ * zero- and one-body terms beside it; on small bases comm122's W and the pp/hh blocks of
+ * small channels too), [5] ph GEMM, [6] inverse Pandya, [7] last
  * launch (fold of the inverse-Pandya terms, comm122, mirror, the sums of the
  * zero- and one-body parts); [0] and [1], once the zero- and one-body launches, are 0.  Enabled by imsrg_hip_set_profiling:
  * each commutator records HIP events on the stream its phases run on (the
