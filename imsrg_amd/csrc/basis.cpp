@@ -642,10 +642,13 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       const int g = bra_g[k];
       allquads = std::max(allquads, quads(hb.kp[k], hb.kq[k], g, bra_e[k], grp_start[g + 1] - grp_start[g]));
     }
+    const int quadcap = allquads / 2 + 64;  // few items have more, and their list takes LDS from all
+    // chunks of an item: of the FP32 elements that fit with 2 bytes per chunk, one more per block
+    const int chunkcap = std::max(2048, (int)((kInvpLds - InvpLds(nJ, nt, norb, ncls, quadcap, 2 * nt).M) /
+                                              (sizeof(float) + 2.0 / 64))) / 64 + 2 * nt + 1;
     for (int v = 0; v < 2; ++v) {
-      const double es = v ? sizeof(float) : sizeof(double);  // and 2 bytes per chunk, one chunk more per block
-      const long cap = std::max(2048L, (long)((kInvpLds - InvpLds(nJ, nt, norb, ncls, allquads, 2 * nt).M - es) /
-                                              (es + 2.0 / 64)));
+      const long cap = std::max(2048L, (long)((kInvpLds - InvpLds(nJ, nt, norb, ncls, quadcap, chunkcap).M) /
+                                              (v ? sizeof(float) : sizeof(double))) - 1);
       long maxel = 1;
       std::vector<TileGroup> groups;
       for (int j = 0; j < norb; ++j) {
@@ -674,19 +677,21 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
             }
             return tot;
           };
+          const int *gf = &grp_first[(size_t)g * (norb + 1)];
+          auto fits = [&](int k0, int k1) {
+            return need(k0, k1) <= cap && quads(i, j, g, std::max(gf[k0], bra_e[kb]), std::max(gf[k1], bra_e[kb])) <= quadcap;
+          };
           for (int k0 = i; k0 < norb;) {
             int k1 = norb;
-            long el = need(k0, k1);
-            if (el > cap) {  // the largest k1 that fits, at least k0 + 1
+            if (!fits(k0, k1)) {  // the largest k1 that does, at least k0 + 1
               int lo = k0 + 1, hi = norb - 1;
               while (lo < hi) {
                 const int mid = (lo + hi + 1) / 2;
-                if (need(k0, mid) <= cap) lo = mid; else hi = mid - 1;
+                if (fits(k0, mid)) lo = mid; else hi = mid - 1;
               }
               k1 = lo;
-              el = need(k0, k1);
             }
-            const int *gf = &grp_first[(size_t)g * (norb + 1)];
+            const long el = need(k0, k1);
             const int kets = gf[k1] - std::max(gf[k0], bra_e[kb]);
             if (kets > 0) {
               G.tiles.push_back(make_int4(0, i | j << 16, k0 | k1 << 16, std::max(gf[k0], bra_e[kb]) | g << 28));

@@ -180,7 +180,7 @@ struct PairArg {
 
 // LDS layout of the inverse Pandya kernel, in bytes
 struct InvpLds {
-  int set, q, z, cls, row, cf, pre, tab, blk, chunk, M;
+  int set, q, z, cls, row, cf, pre, tab, quad, chunk, M;
   __host__ __device__ InvpLds(int nJ, int nt, int norb, int ncls, int nquad, int nchunk) {
     set = 0;                       // int4[nt]: columns in [k0, k1), orbits < k0 of j's and of i's set
     q = set + 16 * nt;             // int4[2 nt]: offset, rows, columns, first entry of cc_cols of the blocks
@@ -190,8 +190,8 @@ struct InvpLds {
     cf = row + 8 * (nJ + 16);      // int[2 nt + 2]: first chunk of each block, then all elements
     pre = cf + 4 * (2 * nt + 2);   // int[ncls + 1]: first result quad of each class
     tab = (pre + 4 * (ncls + 1) + 15) & ~15;    // ushort2[(nt / 4 + 1) norb4]: column offset and row of (J', orbit)
-    blk = tab + (nt + 4) * ((norb + 3) & ~3);   // unsigned[nquad]: class << 20 | J quad << 15 | ket quad of the results
-    chunk = blk + 4 * nquad;       // ushort[nchunk]: block of each chunk
+    quad = tab + (nt + 4) * ((norb + 3) & ~3);  // unsigned[nquad]: class << 20 | J quad << 15 | ket quad
+    chunk = quad + 4 * nquad;      // ushort[nchunk]: block of each chunk
     M = (chunk + 2 * nchunk + 15) & ~15;
   }
 };

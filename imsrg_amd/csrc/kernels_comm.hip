@@ -1569,7 +1569,7 @@ __global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
 // A lane per ket that gathered its elements from memory (the kernel before this one) read
 // the lines again for each class with a ket in them, 3.4 GB at emax = 10 where 0.4 GB are
 // needed, and was bound by that: 594 us at emax = 10 FP64, 531 us with FP32 Zbar, 2310 us at
-// emax = 12 with FP32 Zbar.  Now 395, 342 and 1360 us; 0.6 GB read.  What bounds it now is
+// emax = 12 with FP32 Zbar.  Now 380, 319 and 1303 us; 0.6 GB read.  What bounds it now is
 // instruction issue and latency, in about equal parts of the tables, the copies and the
 // results: 24 waves per CU, 45% of the cycles with a vector instruction issued.  Tried:
 // 16x16x4 matrix instructions on blocks of 16 J x 16 kets (a class of a bra has 13 kets and
@@ -1607,12 +1607,12 @@ __global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *ite
   const int norb4 = (norb + 3) & ~3;  // entries of a table row
   const InvpLds L(nJ, nt, norb, ncls, B.invp_nquad, B.invp_nchunk);
   int4 *s_set = (int4 *)(lds_raw + L.set), *s_q = (int4 *)(lds_raw + L.q), *s_z = (int4 *)(lds_raw + L.z);
-  int4 *s_cls = (int4 *)(lds_raw + L.cls), *s_cls2 = s_cls + ncls;
+  int4 *s_cls = (int4 *)(lds_raw + L.cls), *s_sum = s_cls + ncls;
   long *s_row = (long *)(lds_raw + L.row);
   int *s_cf = (int *)(lds_raw + L.cf), *s_pre = (int *)(lds_raw + L.pre);
   unsigned *tabw = (unsigned *)(lds_raw + L.tab);
   const unsigned short *tab = (const unsigned short *)tabw;
-  unsigned *s_blk = (unsigned *)(lds_raw + L.blk);
+  unsigned *s_quad = (unsigned *)(lds_raw + L.quad);
   unsigned short *s_chunk = (unsigned short *)(lds_raw + L.chunk);
   TZ *M = (TZ *)(lds_raw + L.M);
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1668,10 +1668,9 @@ __global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *ite
       const int Dlo = max(abs(ji - jb), abs(jj - ja)) / 2, nD = min(min(ji + jb, jj + ja) / 2, nJp - 1) - Dlo + 1;
       const int Xlo = max(abs(jj - jb), abs(ji - ja)) / 2, nX = min(min(jj + jb, ji + ja) / 2, nJp - 1) - Xlo + 1;
       s_cls[c] = make_int4(B.cls_start[g * ncls + c] + lo, cnt, Jlo | (ja + jb) / 2 << 16, (max(nj, 0) + 3) >> 2);
-      // the two sums' rows of weights at J' = 0, first J', and steps of 4 J'
-      s_cls2[c] = make_int4((int)(sixjQ_index(d1, d2, ji, jj, 0, ja, jb, 0) / d2),
-                            (int)(sixjQ_index(d1, d2, jj, ji, 0, ja, jb, 0) / d2), Dlo | Xlo << 16,
-                            (max(max(nD, same ? 0 : nX), 0) + 3) >> 2);
+      // row of the weights at J' = 0 (from that of ja = jb = 1/2), first J' of the two sums, steps of 4 J'
+      s_sum[c] = make_int4(((ja >> 1) * d1 + (jb >> 1)) * d2, Dlo, Xlo,
+                           (max(max(nD, same ? 0 : nX), 0) + 3) >> 2);
     }
   }
   __syncthreads();
@@ -1729,18 +1728,19 @@ __global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *ite
   }
   for (int q = threadIdx.x; q < 2 * nt; q += kT)
     for (int c = s_cf[q]; c < s_cf[q + 1]; ++c) s_chunk[c] = (unsigned short)q;
+  // the result quads: class << 20 | J quad << 15 | ket quad
   for (int c = threadIdx.x; c < ncls; c += kT) {
-    const int njb = s_cls[c].w;
+    const int njq = s_cls[c].w;
     int jq = 0, kq = 0;
     for (int q = s_pre[c]; q < s_pre[c + 1]; ++q) {
-      s_blk[q] = c << 20 | jq << 15 | kq;
-      if (++jq == njb) {
+      s_quad[q] = c << 20 | jq << 15 | kq;
+      if (++jq == njq) {
         jq = 0;
         ++kq;
       }
     }
     if (s_pre[c] < nquad && s_pre[c + 1] == nquad)  // the last block's quads of no ket
-      for (int q = nquad; q < 4 * nblk; ++q) s_blk[q] = c << 20 | 0x7FFF;
+      for (int q = nquad; q < 4 * nblk; ++q) s_quad[q] = c << 20 | 0x7FFF;
   }
   if (threadIdx.x == 0) M[mz] = TZ(0);
   __syncthreads();
@@ -1782,41 +1782,44 @@ __global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *ite
   // formed: loaded where they are used they cost most of the time.
   const int rl = lane >> 4, ml = lane & 3;
   struct Blk {
-    int Jl, jh;        // the lane's J as a result, (ja + jb) / 2
+    int Jl, JA, jh;    // the lane's J as a result and as a row of the weights, (ja + jb) / 2
     int pd, px, ns;    // the lane's first J' in the two sums; steps of 4 J'
-    int cd, cx, JA;    // rows of weights at J' = 0, the lane's J as a row of the weights
+    int row;           // row of the weights at J' = 0
     bool active;
     int2 rec;
     int ik;
     double wd[kInvpW], wx[kInvpW];
   };
   // held in registers: the stores below could alias B
-  const IMSRG_G double *sixq = B.sixjQ;
+  const IMSRG_G double *wdir = B.sixjQ + sixjQ_index(d1, d2, ji, jj, 0, 1, 1, 0);
+  const IMSRG_G double *wexc = B.sixjQ + sixjQ_index(d1, d2, jj, ji, 0, 1, 1, 0);
   const IMSRG_G int2 *crec = B.cls_rec;
   const IMSRG_G int *ckm = B.cls_kmap;
   IMSRG_G char *Ztwo = (IMSRG_G char *)(P.Z + B.two_off);
+  auto weight = [&](const Blk &k, const IMSRG_G double *w, int Jp) -> double {
+    return ld_at<double>(w, 8u * ((k.row + min(Jp, nJp)) * d2 + k.JA));
+  };
   auto load = [&](int bk) -> Blk {
     Blk k;
-    const unsigned q = s_blk[4 * bk + ((lane >> 2) & 3)];
-    const int c = q >> 20;
-    const int4 c1 = s_cls[c], c2 = s_cls2[c];
-    const int J0 = (c1.z & 0xFFFF) + (q >> 15 & 31) * 4, p = (q & 0x7FFF) * 4 + ml;
+    const unsigned q = s_quad[4 * bk + ((lane >> 2) & 3)];
+    const int4 k4 = s_cls[q >> 20], c = s_sum[q >> 20];
+    const int J0 = (k4.z & 0xFFFF) + (q >> 15 & 31) * 4, p = (q & 0x7FFF) * 4 + ml;
+    k.active = p < k4.y;
+    const int pos = k4.x + (k.active ? p : 0);
     k.Jl = J0 + rl;
-    k.jh = c1.z >> 16;
-    k.active = p < c1.y;
-    const int pos = c1.x + (k.active ? p : 0);
-    k.rec = ld_at<int2>(crec, 8u * pos);
-    k.ik = ld_at<int>(ckm, (k.Jl * nk + pos) * 4u);
-    k.pd = (c2.z & 0xFFFF) + rl;
-    k.px = (c2.z >> 16) + rl;
-    k.ns = c2.w;
-    k.cd = c2.x;
-    k.cx = c2.y;
     k.JA = min(J0 + ml, d2 - 1);
+    k.jh = k4.z >> 16;
+    k.rec = ld_at<int2>(crec, 8u * pos);
+    k.ik = ld_at<int>(ckm, 4u * (k.Jl * nk + pos));
+    k.row = c.x;
+    k.pd = c.y + rl;
+    k.px = c.z + rl;
+    k.ns = c.w;
 #pragma unroll
-    for (int u = 0; u < kInvpW; ++u) {  // past the quad's last step: row 0
-      k.wd[u] = sixq[(long)(u < k.ns ? k.cd + min(k.pd + 4 * u, nJp) : 0) * d2 + k.JA];
-      k.wx[u] = sixq[(long)(u < k.ns ? k.cx + min(k.px + 4 * u, nJp) : 0) * d2 + k.JA];
+    for (int u = 0; u < kInvpW; ++u) {  // past the quad's last step: the first one's again
+      const int s4 = u < k.ns ? 4 * u : 0;
+      k.wd[u] = weight(k, wdir, k.pd + s4);
+      k.wx[u] = weight(k, wexc, k.px + s4);
     }
     return k;
   };
@@ -1845,8 +1848,7 @@ __global__ __launch_bounds__(kT, 6) void k_invpandya(PairArg pa, const int4 *ite
 #pragma unroll
     for (int u = 0; u < kInvpW; ++u)
       if (u < ns) step(u, k.wd[u], k.wx[u]);
-    for (int u = kInvpW; u < ns; ++u)
-      step(u, sixq[(long)(k.cd + min(k.pd + 4 * u, nJp)) * d2 + k.JA], sixq[(long)(k.cx + min(k.px + 4 * u, nJp)) * d2 + k.JA]);
+    for (int u = kInvpW; u < ns; ++u) step(u, weight(k, wdir, k.pd + 4 * u), weight(k, wexc, k.px + 4 * u));
     const bool odd = (k.jh - k.Jl) & 1;
     double f;
     if (same) {
