@@ -175,84 +175,120 @@ hipError_t launch_scale(double *y, double a, long n, hipStream_t s) {
 
 // One pass over an operator buffer x with the partial sums of its norm: OP 0 the sums
 // alone, OP 1 y += a x beside them (the BCH_Transform step, src/BCH.cc:176-191), OP 2
-// y = x (a copy).  Block b < nblk2 takes the b-th contiguous chunk of the two-body arena
-// and the channels it overlaps, each with its weight (2J+1)^2; the last block the
-// one-body part (weights 2 j_p + 1) and the words around the two parts.  Bound by HBM:
-// a block has four 16-byte loads per thread in flight (one 8-byte load each: the norm
-// 101 us for 293 MB at emax = 10, and a separate device copy about as long again).
+// y = x (a copy).  Block b < nblk2 takes the b-th contiguous chunk of the two-body arena,
+// each word with its channel's weight (2J+1)^2; blocks nblk2 .. nblk2 + nblk1 - 1 share the
+// one-body part (weights 2 j_p + 1), the first of them the words around the two parts.
+// Bound by HBM at large sizes: a block has four 16-byte loads per thread in flight (one
+// 8-byte load each: the norm 101 us for 293 MB at emax = 10, and a separate device copy about
+// as long again).  At small sizes by the longest chain of loads in a block: with one block
+// for the one-body part and the channels of a chunk one after the other, axpy and norm took
+// 37 us at emax = 7 (22 MB) and 27 us at emax = 6, now 16 and 9 us.
+constexpr int kNormCh = 640;  // channels whose offsets fit in the kernel's LDS list
 template <int OP>
 __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y, double a, const double *x,
-                                                   double *part, int nblk2) {
+                                                   double *part, int nblk2, int nblk1) {
   const BasisDev &B = *bd;
   __shared__ double red[4];
+  __shared__ long s_off[kNormCh];
   double acc = 0.0;
-  auto put = [&](long e, double v) {  // one word of y
-    if (OP == 1) {
-      double t = a * v;  // (a x) formed first, then added (Operator operator* then +=)
-      y[e] += t;
-    }
-    if (OP == 2) y[e] = v;
-  };
-  if ((int)blockIdx.x == nblk2) {
+  constexpr int U = 4;
+  if ((int)blockIdx.x >= nblk2) {
+    auto put = [&](long e, double v) {  // one word of y
+      if (OP == 1) {
+        double t = a * v;  // (a x) formed first, then added (Operator operator* then +=)
+        y[e] += t;
+      }
+      if (OP == 2) y[e] = v;
+    };
+    const int b1 = blockIdx.x - nblk2;
     const long n1 = (long)B.norb * B.norb;
     // the zero-body and padding words around the one-body block and after the two-body arena
     const long rg[3][2] = {{0, B.one_off}, {B.one_off + n1, B.two_off}, {B.two_off + B.tbsize, B.opsize}};
-    if (OP != 0)
+    if (OP != 0 && b1 == 0)
       for (int g = 0; g < 3; ++g)
         for (long e = rg[g][0] + threadIdx.x; e < rg[g][1]; e += blockDim.x) put(e, x[e]);
-    for (long e = threadIdx.x; e < n1; e += blockDim.x) {
-      const double v = x[B.one_off + e];
-      acc += v * v * B.w1norm[e];
-      put(B.one_off + e, v);
+    const double *x1 = x + B.one_off;
+    double *y1 = OP ? y + B.one_off : nullptr;
+    for (long q = (long)b1 * blockDim.x + threadIdx.x; q < n1; q += (long)U * nblk1 * blockDim.x) {
+      double v[U], w[U], o[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long e = min(q + (long)u * nblk1 * blockDim.x, n1 - 1);
+        v[u] = x1[e];
+        w[u] = B.w1norm[e];
+        if (OP == 1) o[u] = y1[e];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long e = q + (long)u * nblk1 * blockDim.x;
+        if (e >= n1) break;
+        acc += v[u] * v[u] * w[u];
+        if (OP == 1) {
+          double t = a * v[u];
+          y1[e] = o[u] + t;
+        }
+        if (OP == 2) y1[e] = v[u];
+      }
     }
   } else {
     const double *two = x + B.two_off;
     double *y2 = OP ? y + B.two_off : nullptr;
     const long tb = B.tbsize, chunk = (tb + nblk2 - 1) / nblk2;
     const long c0 = (long)blockIdx.x * chunk, c1 = min(c0 + chunk, tb);
-    int lo = 0, hi = B.nch - 1;  // last channel starting at or before c0
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (B.ch_off[mid] <= c0) lo = mid; else hi = mid - 1;
+    // the channels that the chunk overlaps: lo .. hi
+    const int nch = B.nch;
+    int lo = -1, hi = -1;
+    for (int c = 0; c < nch; c += blockDim.x) {
+      const int ch = c + threadIdx.x;
+      const long off = ch < nch ? B.ch_off[ch] : tb;
+      if (ch < min(nch, kNormCh)) s_off[ch] = off;
+      lo += __syncthreads_count(ch < nch && off <= c0);
+      hi += __syncthreads_count(ch < nch && off < c1);
     }
-    for (int ch = lo; ch < B.nch && B.ch_off[ch] < c1; ++ch) {
-      const long off = B.ch_off[ch], nn = (long)B.ch_n[ch] * B.ch_n[ch];
-      const long e0 = max(c0, off), e1 = min(c1, off + nn);
-      const double w = (double)((2 * (ch / 6) + 1) * (2 * (ch / 6) + 1));
-      double s = 0.0;
-      // pairs of words at even offsets (the arena is 64-byte aligned), clamped into
-      // [e0, e1): a pair across an end counts its inner word only
-      constexpr int U = 4;
-      for (long q = (e0 & ~1L) + 2 * (long)threadIdx.x; q < e1; q += 2 * U * (long)blockDim.x) {
-        double2 v[U], o[U];
+    auto weight = [](int ch) { return (double)((2 * (ch / 6) + 1) * (2 * (ch / 6) + 1)); };
+    auto offset = [&](int ch) -> long { return ch < kNormCh ? s_off[ch] : B.ch_off[ch]; };
+    const double wlo = weight(max(lo, 0));
+    // pairs of words at even offsets (the arena is 64-byte aligned), clamped into [c0, c1):
+    // a pair across an end counts its inner word only
+    for (long q = (c0 & ~1L) + 2 * (long)threadIdx.x; q < c1; q += 2 * U * (long)blockDim.x) {
+      double2 v[U], o[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const long e = min(q + 2 * u * (long)blockDim.x, (e1 - 1) & ~1L);
-          v[u] = *reinterpret_cast<const double2 *>(two + e);
-          if (OP == 1) o[u] = *reinterpret_cast<const double2 *>(y2 + e);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const long e = q + 2 * u * (long)blockDim.x;
-          const bool m0 = e < e1 && e >= e0, m1 = e + 1 < e1;
-          if (m0) s += v[u].x * v[u].x;
-          if (m1) s += v[u].y * v[u].y;
-          if (OP == 0) continue;
-          double2 r = v[u];
-          if (OP == 1) {
-            double t0 = a * v[u].x, t1 = a * v[u].y;
-            r.x = o[u].x + t0;
-            r.y = o[u].y + t1;
-          }
-          if (m0 && m1)
-            *reinterpret_cast<double2 *>(y2 + e) = r;
-          else if (m0)
-            y2[e] = r.x;
-          else if (m1)
-            y2[e + 1] = r.y;
-        }
+      for (int u = 0; u < U; ++u) {
+        const long e = min(q + 2 * u * (long)blockDim.x, (c1 - 1) & ~1L);
+        v[u] = *reinterpret_cast<const double2 *>(two + e);
+        if (OP == 1) o[u] = *reinterpret_cast<const double2 *>(y2 + e);
       }
-      acc += w * s;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long e = q + 2 * u * (long)blockDim.x;
+        const bool m0 = e < c1 && e >= c0, m1 = e + 1 < c1;
+        double w0 = wlo, w1 = wlo;
+        if (lo < hi) {  // the words' channels
+          int a0 = lo, a1 = hi;
+          while (a0 < a1) {
+            const int mid = (a0 + a1 + 1) >> 1;
+            if (offset(mid) <= max(e, c0)) a0 = mid; else a1 = mid - 1;
+          }
+          w0 = weight(a0);
+          while (a0 < hi && offset(a0 + 1) <= e + 1) ++a0;
+          w1 = weight(a0);
+        }
+        if (m0) acc += w0 * (v[u].x * v[u].x);
+        if (m1) acc += w1 * (v[u].y * v[u].y);
+        if (OP == 0) continue;
+        double2 r = v[u];
+        if (OP == 1) {
+          double t0 = a * v[u].x, t1 = a * v[u].y;
+          r.x = o[u].x + t0;
+          r.y = o[u].y + t1;
+        }
+        if (m0 && m1)
+          *reinterpret_cast<double2 *>(y2 + e) = r;
+        else if (m0)
+          y2[e] = r.x;
+        else if (m1)
+          y2[e + 1] = r.y;
+      }
     }
   }
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
@@ -264,20 +300,20 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
 // The norm's two sums into out[0..1]; with seq != 0, out is host memory, and seq goes
 // into *done after them, so that the host can read the sums without a copy and without
 // waiting for the stream.
-__global__ void k_norm_final(const double *part, int nblk2, double *out, unsigned long long *done,
-                             unsigned long long seq) {
-  __shared__ double red[256];
-  double acc = 0.0;
+__global__ __launch_bounds__(256) void k_norm_final(const double *part, int nblk2, int nblk1, double *out,
+                                                    unsigned long long *done, unsigned long long seq) {
+  __shared__ double red[4];
+  double acc = 0.0, one = (int)threadIdx.x < nblk1 ? part[nblk2 + threadIdx.x] : 0.0;
   for (int i = threadIdx.x; i < nblk2; i += blockDim.x) acc += part[i];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  for (int o = 32; o > 0; o >>= 1) {
+    acc += __shfl_down(acc, o, 64);
+    one += __shfl_down(one, o, 64);
   }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    out[0] = part[nblk2];
-    out[1] = red[0];
+    out[0] = one;  // nblk1 <= 64: the first wave's
+    out[1] = (red[0] + red[1]) + (red[2] + red[3]);
     if (seq) {
       __threadfence_system();
       __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -371,15 +407,16 @@ hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double
                        double *partials, int maxpart, double *out, unsigned long long *done, unsigned long long seq,
                        hipStream_t s) {
   // two-body chunks of at least 2048 words, so that small bases do not pay for idle blocks
-  const int nblk2 = (int)std::max<long>(1, std::min<long>(maxpart - 1, (bh.tbsize + 2047) / 2048));
-  const dim3 grid(nblk2 + 1), blk(256);
+  const int nblk1 = (int)std::max(1, std::min(32, bh.norb * bh.norb / 1024));
+  const int nblk2 = (int)std::max<long>(1, std::min<long>(maxpart - nblk1, (bh.tbsize + 2047) / 2048));
+  const dim3 grid(nblk2 + nblk1), blk(256);
   if (op == NormOp::kSum)
-    hipLaunchKernelGGL((k_norm_pass<0>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
+    hipLaunchKernelGGL((k_norm_pass<0>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
   else if (op == NormOp::kAxpy)
-    hipLaunchKernelGGL((k_norm_pass<1>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
+    hipLaunchKernelGGL((k_norm_pass<1>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
   else
-    hipLaunchKernelGGL((k_norm_pass<2>), grid, blk, 0, s, bd, y, a, x, partials, nblk2);
-  hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, out, done, seq);
+    hipLaunchKernelGGL((k_norm_pass<2>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
+  hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, nblk1, out, done, seq);
   return hipGetLastError();
 }
 
