@@ -611,9 +611,9 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
 
     // Items (pair, i | j << 16, k0 | k1 << 16, first ket | group << 28) of the bra (ij) and its
     // kets whose smaller orbit k is in [k0, k1), such that the elements of Zbar they need fit
-    // in LDS, kInvpLds bytes with the tables (a range of one orbit may exceed them).  All items of one j = bra's second orbit run on one XCD,
-    // by ascending i: the work-groups of bras (i, j), (i + 1, j), ... read neighbouring
-    // rows of the same columns of Zbar.
+    // in LDS, kInvpLds bytes or less with the tables (a range of one orbit may exceed them).  All
+    // items of one j = bra's second orbit run on one XCD, by ascending i: the work-groups of bras
+    // (i, j), (i + 1, j), ... read neighbouring rows of the same columns of Zbar.
     int maxquad = 0, maxchunk = 0;
     std::vector<int> bra_g(hb.nkets), bra_e(hb.nkets);
     for (int g = 0; g < 6; ++g)
@@ -646,9 +646,34 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
     // chunks of an item: of the FP32 elements that fit with 2 bytes per chunk, one more per block
     const int chunkcap = std::max(2048, (int)((kInvpLds - InvpLds(nJ, nt, norb, ncls, quadcap, 2 * nt).M) /
                                               (sizeof(float) + 2.0 / 64))) / 64 + 2 * nt + 1;
+    // the elements of the bra (ij) with k in [k0, k1): rows x >= k0 of the columns y in [k0, k1) and
+    // rows x in [k0, k1) of the columns y >= k1; sets of the other Tz (same) have none
+    auto elements = [&](int i, int j, int k0, int k1) {
+      const unsigned short *ci = &ccnt[(size_t)i * (norb + 1) * nt], *cj = &ccnt[(size_t)j * (norb + 1) * nt];
+      const bool same = hb.tz2[i] == hb.tz2[j];
+      const unsigned short *i0 = ci + (size_t)k0 * nt, *i1 = ci + (size_t)k1 * nt, *in = ci + (size_t)norb * nt;
+      const unsigned short *j0 = cj + (size_t)k0 * nt, *j1 = cj + (size_t)k1 * nt, *jn = cj + (size_t)norb * nt;
+      int tot = 0;
+      for (int t = 0; t < nt; ++t)
+        tot += (same && (t & 2)) ? 0 : (j1[t] - j0[t]) * (in[t] - i0[t]) + (jn[t] - j1[t]) * (i1[t] - i0[t]);
+      return (long)tot;
+    };
     for (int v = 0; v < 2; ++v) {
-      const long cap = std::max(2048L, (long)((kInvpLds - InvpLds(nJ, nt, norb, ncls, quadcap, chunkcap).M) /
-                                              (v ? sizeof(float) : sizeof(double))) - 1);
+      auto cap_of = [&](int lds) {
+        return std::max(2048L, (long)((lds - InvpLds(nJ, nt, norb, ncls, quadcap, chunkcap).M) /
+                                      (v ? sizeof(float) : sizeof(double))) - 1);
+      };
+      // the smallest LDS size at which four of five bras that fit as a whole at the largest still do
+      long cap = cap_of(kInvpLds);
+      std::vector<long> el(hb.nkets);
+      for (int k = 0; k < hb.nkets; ++k) el[k] = elements(hb.kp[k], hb.kq[k], hb.kp[k], norb);
+      auto whole = [&](long c) { return std::count_if(el.begin(), el.end(), [c](long e) { return e <= c; }); };
+      const long most = whole(cap);
+      for (int lds : kInvpLdsSmall)
+        if (5 * whole(cap_of(lds)) >= 4 * most) {
+          cap = cap_of(lds);
+          break;
+        }
       long maxel = 1;
       std::vector<TileGroup> groups;
       for (int j = 0; j < norb; ++j) {
@@ -657,16 +682,7 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
           const int kb = ket_index(norb, i, j), g = bra_g[kb];
           const unsigned short *ci = &ccnt[(size_t)i * (norb + 1) * nt], *cj = &ccnt[(size_t)j * (norb + 1) * nt];
           const bool same = hb.tz2[i] == hb.tz2[j];
-          // elements of the kets with k in [k0, k1): rows x >= k0 of the columns y in [k0, k1) and
-          // rows x in [k0, k1) of the columns y >= k1; sets of the other Tz (same) have none
-          auto need = [&](int k0, int k1) {
-            const unsigned short *i0 = ci + (size_t)k0 * nt, *i1 = ci + (size_t)k1 * nt, *in = ci + (size_t)norb * nt;
-            const unsigned short *j0 = cj + (size_t)k0 * nt, *j1 = cj + (size_t)k1 * nt, *jn = cj + (size_t)norb * nt;
-            int tot = 0;
-            for (int t = 0; t < nt; ++t)
-              tot += (same && (t & 2)) ? 0 : (j1[t] - j0[t]) * (in[t] - i0[t]) + (jn[t] - j1[t]) * (i1[t] - i0[t]);
-            return (long)tot;
-          };
+          auto need = [&](int k0, int k1) { return elements(i, j, k0, k1); };
           auto chunks = [&](int k0, int k1) {  // of 64 elements
             int tot = 0;
             for (int t = 0; t < nt; ++t) {

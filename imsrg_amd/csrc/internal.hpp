@@ -28,6 +28,11 @@ constexpr int kGC = kTileK / kGWaves;  // k columns each wave copies into LDS pe
 constexpr int kChunk = 256;       // elements per work item of the gather kernels
 constexpr int kLdsUnit = 1280;    // LDS allocation unit in bytes, 128 of them in a CU
 constexpr int kInvpLds = 42 * kLdsUnit;  // LDS of an inverse Pandya work-group: three in a CU
+// ... or of one of a small basis, six or five in a CU, with 256 threads instead of 512 (the
+// serial parts of more items run at once): FP64 emax = 6 33 -> 29 us, emax = 7 55 -> 46, emax = 8
+// 97 -> 92, FP32 Zbar emax = 7 53 -> 45, emax = 8 93 -> 83, emax = 9 171 -> 161.  Where many more bras
+// have to be taken in parts it is slower: FP64 emax = 9 184 -> 197, FP32 emax = 10 320 -> 338.
+constexpr int kInvpLdsSmall[] = {21 * kLdsUnit, 25 * kLdsUnit};
 constexpr int kC122MaxN = 64;     // columns of a comm122 bin formed at once (a larger bin takes one item per 16)
 constexpr int kC122MaxCols = 150; // largest bin (LDS: 1 KiB of coefficients per ket)
 constexpr int kC122Rows = 128;    // rows of one comm122 W item (256: 221 against 210 us at emax = 10)

@@ -498,8 +498,8 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items) {
 
 
 // ---------------------------------------------------------------------------
-// SYR2K on 128x128 output tiles: each of the 4 waves owns a 64x64 sub-tile
-// (4x4 MFMA blocks), so one LDS read feeds four MFMAs; k-stages of 16 are
+// SYR2K on 128x128 output tiles: each of the 8 waves owns a 64x32 sub-tile
+// (4x2 MFMA blocks), so one LDS read feeds two or four MFMAs; k-stages of 16 are
 // double-buffered in LDS and filled by direct global->LDS copies issued one
 // stage ahead.
 //   D(r,s) = alpha * cph(s) * sum_k w_k [ A(r,ka_k) B(s,kb_k) + h B(r,kb_k) A(s,ka_k) ],  r <= s
@@ -2258,10 +2258,10 @@ hipError_t launch_invpandya(const PairArg &pa, const int4 *items, int nitems, si
                             hipStream_t s) {
   if (nitems <= 0) return hipSuccess;
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  // 256 threads where seven and more work-groups fit in a CU: 512 take longer on small items
-  // (emax = 5, FP32 Zbar: 23.7 against 19.2 us) and less on large ones (emax = 10, FP64: 438
-  // against 529 us), of which few fit
-  const bool small = lds <= 18 * kLdsUnit;
+  // 256 threads where five and more work-groups fit in a CU: 512 take longer on small items
+  // (emax = 5, FP32 Zbar: 23.7 against 19.2 us, 48 pairs at emax 4-7 998 against 635 us) and less
+  // on large ones (emax = 10, FP64: 383 against 452 us), of which few fit
+  const bool small = lds <= kInvpLdsSmall[1];
   const dim3 grid(nitems), blk(small ? 256 : 512);
   if (zbar_f32 && small)
     hipLaunchKernelGGL((k_invpandya<float, 256>), grid, blk, lds, s, pa, items);

@@ -1,6 +1,6 @@
 """comm222_ph against the oracle where the inverse Pandya kernel's items change shape:
-bras whose elements of Zbar exceed one work-group's LDS (ranges of k), groups of many
-kets of one class, both work-group sizes, and a space without holes (Zbar = 0)."""
+bras whose elements of Zbar exceed one work-group's LDS (ranges of k; with any of its
+sizes), groups of many kets of one class, both work-group sizes, and a space without holes (Zbar = 0)."""
 import numpy as np
 import pytest
 
@@ -22,6 +22,8 @@ def ia():
     (2, [(0, 1), (1, 1), (1, 3)], [(0, 0, 1)]),
     (1, [(0, 1), (1, 3), (3, 7), (4, 7)], [(0, 1, 3), (0, 4, 7)]),
     (3, [(0, 1), (1, 1), (1, 3)], []),
+    (6, [(0, 1), (1, 1), (1, 3), (2, 3), (2, 5)], [(0, 0, 1), (0, 2, 5)]),
+    (8, [(0, 1), (1, 1), (1, 3), (2, 3), (2, 5)], [(0, 0, 1), (0, 2, 5)]),
     (12, [(0, 1), (1, 1), (1, 3), (2, 3), (2, 5)], [(0, 0, 1), (0, 2, 5)]),
 ])
 def test_ph_items(ia, nrad, lj, holes):
