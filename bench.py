@@ -29,6 +29,8 @@ PEAK_BF16_MFMA = 2.5e15    # FLOP/s, MI355X dense bf16 matrix
 B3_PRODUCTS = 6            # bf16 MFMA products per FP64 product in the bf16x3 kernels
 PEAK_HBM = 8.0e12          # B/s
 
+# zerobody and onebody are 0: their terms run in the first launch, beside the Pandya
+# gather (pandya_gather), and are summed in the last one (fold_mirror)
 PHASES = ["zerobody", "onebody", "comm122", "pphh_gemm", "pandya_gather", "ph_gemm", "inverse_pandya", "fold_mirror"]
 
 
@@ -37,7 +39,8 @@ def algorithmic_counts(ms):
     basis tables (src/ModelSpace.cc:1120-1201, src/TwoBodyChannel.cc:142-188):
       F_A = sum_ch 2 n^2 (n_pp + 2 n_hh + n_ph)   pp/hh GEMMs (src/Commutator.cc:1176-1183)
       F_C = sum_cc 8 c^2 n_ph,cc                   ph GEMM (src/Commutator.cc:1789)
-      B_I = z sum_cc 2 c^2 + 8 sum_ch n(n+1)/2     inverse Pandya: one read of Zbar over the
+      B_I = z sum_cc c(c+1) + 8 sum_ch n(n+1)/2    inverse Pandya: one read of the upper
+                                                   triangles of Zbar's head and tail over the
                                                    CC channels with ph kets (Zbar is zero in
                                                    the others), one store per upper Z element;
                                                    z = 8 for FP64 Zbar, 4 for the FP32 Zbar of
@@ -76,7 +79,7 @@ def algorithmic_counts(ms):
                 e[0] += 1
                 e[1] += ph
     FC = sum(8 * c * c * nph for c, nph in cc.values() if nph > 0)
-    zbar = sum(2 * c * c for c, nph in cc.values() if nph > 0)
+    zbar = sum(c * (c + 1) for c, nph in cc.values() if nph > 0)
     return FA, executed_A, FC, 8 * zbar + 8 * upper, 4 * zbar + 8 * upper
 
 
@@ -653,7 +656,7 @@ def main():
                 "executed_flops": execA}
     elif PHASES[dom] == "inverse_pandya":
         ach = BI / t_dom
-        kname = "k_invpandya<float>" if zbar32 else "k_invpandya<double>"
+        kname = "k_invpandya<float, 512>" if zbar32 else "k_invpandya<double, 512>"
         roof = {"kernel": kname, "bound": "hbm", "achieved": ach / 1e9, "peak": PEAK_HBM / 1e9,
                 "unit": "GB/s", "frac": ach / PEAK_HBM, "traffic": profiled_traffic(kname),
                 "algorithmic_bytes": BI}

@@ -1550,13 +1550,14 @@ __global__ __launch_bounds__(256, 7) void k_front(PairArg pa, FrontItems f) {
 // (i, x) of a column follow one another in x.  f(J) stands for the second sum where k = l
 // or i = j (1 - (-1)^{(jk+jl)/2 - J}, with (-1)^{(ji+jj+jk+jl)/2} for i = j).
 // One work-group per bra, or per range [k0, k1) of its kets' k where the bra's M exceeds
-// kInvpM bytes.  It
+// the LDS of a work-group.  It
 //  * lays out M in LDS by sets t = (J', parity and |tz| of (i, x)), each in two blocks: the
 //    columns y in [k0, k1) with the rows x >= k0, then the columns y >= k1 with the rows x in
 //    [k0, k1); and a table over (J', orbit) of the orbit's column offset and row;
 //  * copies M in chunks of 64 elements of one block, each read once;
-//  * takes the kets 16 at a time by class (ja <= jb, the unordered j of k and l): the class's
-//    weights W(J, J') times the gathered M(J', ket) on the FP64 matrix units, 16 J at once.
+//  * takes the kets by class (ja <= jb, the unordered j of k and l): the class's weights
+//    W(J, J') times the gathered M(J', ket) on the FP64 matrix units, four quads of 4 J x 4
+//    kets at once.
 //    A ket with jk > jl is its class's with both sums exchanged, which is the factor
 //    -(-1)^{(jk+jl)/2 - J} on the result.
 // sixjQ holds the weights (2J'+1) {...}, with zeros where the reference skips |6j| < 1e-8.
