@@ -1387,7 +1387,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
                 mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big, items[7], items[9], mask & MPPHH ? cnt[7] : 0,
                 mask & M122 ? cnt[9] : 0};
-  const bool small = fi.blocks() <= (prec_pphh == 0 || prec_pphh == 2 ? kFrontSmallF64 : kFrontSmall);
+  const bool small = fi.blocks() <= kFrontSmall;
   if (!small) fi.n64 = fi.nc122 = 0;
   const bool overlap = tu.overlap_pphh && (mask & MPPHH) && !(small && cnt[big] == 0);
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so

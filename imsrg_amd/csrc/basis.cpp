@@ -489,20 +489,26 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   ob221.clear();
   {
     int slot = 0;
+    std::vector<int> cj;
     for (size_t p = 0; p < pairs1.size(); ++p) {
       ob_start[p] = slot++;
       const int i = pairs1[p].x, j = pairs1[p].y;
+      const int first = (int)cj.size();
       for (int c = 0; c < norb; ++c) {
         if (!(std::fabs(hb.occ[c]) > 1e-9)) continue;
         const int Jmin = std::max(std::abs(hb.j2[c] - hb.j2[i]), std::abs(hb.j2[c] - hb.j2[j])) / 2;
         const int Jmax = (hb.j2[c] + std::min(hb.j2[i], hb.j2[j])) / 2;
-        for (int J = Jmin; J <= Jmax; ++J) ob221.push_back(make_int4(0, (int)p, (c << 8) | J, slot++));
+        for (int J = Jmin; J <= Jmax; ++J) cj.push_back((c << 8) | J);
       }
-      for (size_t q = 0; q < cpart.size(); q += 4)
+      const int last = (int)cj.size();
+      for (int e = first; e < last; e += 4)
+        ob221.push_back(make_int4(0, (int)p, (std::min(last - e, 4) - 1) << 28 | e, slot++));
+      for (size_t q = 0; q < cpart.size(); q += 16)
         ob221.push_back(make_int4(0, (int)p, (1 << 30) | (int)q, slot++));
     }
     ob_start[pairs1.size()] = slot;
     B.nobpart = slot;
+    B.ob_cj = dupload(*this, cj, err);
   }
   B.ncpart = (int)cpart.size();
   B.ob_start = dupload(*this, ob_start, err);

@@ -136,8 +136,9 @@ struct BasisDev {
   int invp_nquad, invp_nchunk;  // most result quads and 64-element chunks of an inverse Pandya item
   const IMSRG_G int2 *pairs1;   // one-body pairs (i<=j, same (l,j2,tz2) block)
   // partial sums of the one-body part: slots ob_start[p] .. ob_start[p+1]-1 of pair p
-  // (the first: comm111 + comm121, the others: comm221 items); cpart: orbits with 1 - n_c != 0
-  const IMSRG_G int *ob_start, *cpart;
+  // (the first: comm111 + comm121, the others: comm221 items); cpart: orbits with 1 - n_c != 0;
+  // ob_cj: c << 8 | J of each pair's orbits c with n_c != 0
+  const IMSRG_G int *ob_start, *cpart, *ob_cj;
   int nobpart, ncpart;
   int ndiag;  // kets summed over all channels (ch_kstart[nch])
   const IMSRG_G double *w1norm; // norb*norb one-body norm weights

@@ -217,28 +217,37 @@ __device__ __forceinline__ double m221_part(const BasisDev &B, const double *X2,
 }
 
 // comm221 one-body part in partial sums, one slot per item (it.w):
-//  kind 0 (n_c != 0): n_c M_pp for one (c, J), the block's lanes over the pp list;
-//  kind 1 (1 - n_c != 0): (1 - n_c) M_hh for 4 orbits c of the list cpart
-//  (one per wave), the wave's lanes over J and the hh lists.
+//  kind 0 (n_c != 0): n_c M_pp for 4 entries (c, J) of the list ob_cj (one per wave), the
+//  wave's lanes over the pp list;
+//  kind 1 (1 - n_c != 0): (1 - n_c) M_hh for 16 orbits c of the list cpart, 16 lanes on
+//  each, over J and the hh lists.
+// A work-group is a chain of index loads with little work behind it: kind 0 by the block
+// and kind 1 by the wave, with four times the work-groups, took 481 us in a batch of 48
+// pairs at emax 4-7 with the other work-groups before the Pandya chunks (now 232), and the
+// first launch 68 us at emax = 8 (58) and 550 at emax = 12 (505).
 __device__ __forceinline__ void front_221(const PairPtrs &P, const int4 &it) {
   const BasisDev &B = *P.basis;
   const int2 pr = B.pairs1[it.y];
   const int i = pr.x, j = pr.y;
   const double *X2 = P.X + B.two_off, *Y2 = P.Y + B.two_off;
   const double hZ = P.hZ;
+  const int lane = threadIdx.x & 63;
   double acc[1] = {0.0};
   if (!(it.z >> 30)) {
-    const int c = (it.z >> 8) & 0xffff, J = it.z & 0xff;
-    acc[0] = B.occ[c] * m221_part(B, X2, Y2, i, j, c, J, true, threadIdx.x, blockDim.x, hZ);
+    const int e = threadIdx.x >> 6;
+    if (e <= (it.z >> 28 & 3)) {
+      const int cj = B.ob_cj[(it.z & 0xfffffff) + e], c = cj >> 8, J = cj & 0xff;
+      acc[0] = B.occ[c] * m221_part(B, X2, Y2, i, j, c, J, true, lane, 64, hZ);
+    }
   } else {
-    const int q = (it.z & 0x3fffffff) + (threadIdx.x >> 6);
+    const int q = (it.z & 0x3fffffff) + (threadIdx.x >> 4);
     if (q < B.ncpart) {
-      const int c = B.cpart[q], lane = threadIdx.x & 63;
+      const int c = B.cpart[q];
       const int Jmin = max(abs(B.j2[c] - B.j2[i]), abs(B.j2[c] - B.j2[j])) / 2;
       const int Jmax = (B.j2[c] + min(B.j2[i], B.j2[j])) / 2;
       double m = 0.0;
-      // eight J at a time, eight lanes on each one's hh list (a few kets)
-      for (int J = Jmin + (lane >> 3); J <= Jmax; J += 8) m += m221_part(B, X2, Y2, i, j, c, J, false, lane & 7, 8, hZ);
+      // eight J at a time, two lanes on each one's hh list (a few kets)
+      for (int J = Jmin + (lane >> 1 & 7); J <= Jmax; J += 8) m += m221_part(B, X2, Y2, i, j, c, J, false, lane & 1, 2, hZ);
       acc[0] = (1.0 - B.occ[c]) * m;
     }
   }

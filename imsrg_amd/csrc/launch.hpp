@@ -43,10 +43,9 @@ hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int 
 // Work-groups up to which the first launch takes those as well: one launch, and without
 // 128x128 pp/hh tiles no second stream, instead of three launches and four stream events,
 // which cost the smallest bases more than their work (emax = 2 FP64 49 -> 28 us, emax = 3
-// 50 -> 34, emax = 5 95 -> 90, mixed 76 -> 71 us).  Where they fill the chip they only hold up the main
-// stream: emax = 6 mixed 100 -> 105 us.  Beside an FP64 (or split) GEMM, which makes the side
-// stream the longer one, that comes later: emax = 6 155 -> 142 us, emax = 7 250 -> 254 us.
-constexpr int kFrontSmall = 3000, kFrontSmallF64 = 6000;
+// 50 -> 34, emax = 5 90 -> 87, mixed 71 -> 68, emax = 6 147 -> 140 and 99 -> 93 us).  Where they fill
+// the chip they only hold up the main stream: emax = 7 235 -> 239 us, mixed 161 -> 174 us.
+constexpr int kFrontSmall = 3500;
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
 // under bf16x3 products (kGemmB3) the pack items first write the operand panels
 // maxn: the largest channel dimension of the pairs (sizes the kernel's LDS index list)
