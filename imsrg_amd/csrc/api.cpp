@@ -698,7 +698,7 @@ extern "C" int imsrg_hip_op_scale(imsrg_dop *op, double f) {
 }
 extern "C" int imsrg_hip_op_axpy(imsrg_dop *y, double a, const imsrg_dop *x) {
   if (!same_ctx(y, x)) return IMSRG_E_INVALID;
-  HIPCHK(y->ctx, launch_axpy(y->buf, a, x->buf, y->ctx->db.h.opsize, y->ctx->stream));
+  HIPCHK(y->ctx, launch_axpy(y->buf, y->buf, a, x->buf, y->ctx->db.h.opsize, y->ctx->stream));
   return IMSRG_OK;
 }
 extern "C" int imsrg_hip_op_zero(imsrg_dop *op) {
@@ -707,15 +707,15 @@ extern "C" int imsrg_hip_op_zero(imsrg_dop *op) {
   return IMSRG_OK;
 }
 
-// Queues the norm sums of op into host slot `slot` (and in the same pass, kAxpy: to +=
-// a op, kCopy: to = op).  norm_wait reads them: it watches the slot, so that no copy and
+// Queues the norm sums of op into host slot `slot` (and in the same pass, kAxpy: to =
+// base + a op).  norm_wait reads them: it watches the slot, so that no copy and
 // no stream wake-up follows the kernel, and asks the stream now and then, so that a
 // failed launch ends it.
 static int norm_launch(imsrg_ctx *ctx, int slot, const imsrg_dop *op, NormOp what = NormOp::kSum,
-                       imsrg_dop *to = nullptr, double a = 0.0) {
+                       imsrg_dop *to = nullptr, const imsrg_dop *base = nullptr, double a = 0.0) {
   imsrg_ctx::NormSlot &h = ctx->norm_host[slot];
-  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, what, to ? to->buf : nullptr, a, op->buf, ctx->partials, ctx->npart,
-                          h.sum, &h.done, ++ctx->norm_seq, ctx->stream));
+  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, what, to ? to->buf : nullptr, base ? base->buf : nullptr, a, op->buf,
+                          ctx->partials, ctx->npart, h.sum, &h.done, ++ctx->norm_seq, ctx->stream));
   return IMSRG_OK;
 }
 // seq: ctx->norm_seq right after the slot's norm_launch
@@ -737,17 +737,17 @@ static int norm_wait(imsrg_ctx *ctx, int slot, unsigned long long seq, double *n
     return fail(ctx, IMSRG_E_NONFINITE, "operator holds non-finite values");
   return IMSRG_OK;
 }
-// norm of op; with axpy_to, axpy_to += axpy_a * op in the same pass over op
+// norm of op; with axpy_to, axpy_to = base + axpy_a * op in the same pass over op (base may be axpy_to)
 static int op_norm(const imsrg_dop *op, double *n1, double *n2, double *n, imsrg_dop *axpy_to = nullptr,
-                   double axpy_a = 0.0) {
+                   const imsrg_dop *base = nullptr, double axpy_a = 0.0) {
   imsrg_ctx *ctx = op->ctx;
-  if (int rc = norm_launch(ctx, 0, op, axpy_to ? NormOp::kAxpy : NormOp::kSum, axpy_to, axpy_a)) return rc;
+  if (int rc = norm_launch(ctx, 0, op, axpy_to ? NormOp::kAxpy : NormOp::kSum, axpy_to, base, axpy_a)) return rc;
   return norm_wait(ctx, 0, ctx->norm_seq, n1, n2, n);
 }
-// norms of two operators, one wait for both; with copy_to, copy_to = x in the pass over x
-static int op_norms(const imsrg_dop *x, const imsrg_dop *y, double *nx, double *ny, imsrg_dop *copy_to = nullptr) {
+// norms of two operators, one wait for both
+static int op_norms(const imsrg_dop *x, const imsrg_dop *y, double *nx, double *ny) {
   imsrg_ctx *ctx = x->ctx;
-  if (int rc = norm_launch(ctx, 0, x, copy_to ? NormOp::kCopy : NormOp::kSum, copy_to)) return rc;
+  if (int rc = norm_launch(ctx, 0, x)) return rc;
   const unsigned long long sx = ctx->norm_seq;
   if (int rc = norm_launch(ctx, 1, y)) return rc;
   const unsigned long long sy = ctx->norm_seq;
@@ -770,8 +770,8 @@ extern "C" int imsrg_hip_op_normal_order(imsrg_dop *out, const imsrg_dop *op, in
     return fail(ctx, IMSRG_E_UNSUPPORTED, "normal ordering needs a Hermitian or anti-Hermitian operator");
   // the one-body sum runs only when the two-body norm exceeds 1e-7 (src/Operator.cc:493):
   // the norm stays on the device, where the kernel tests it
-  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, out != op ? NormOp::kCopy : NormOp::kSum, out->buf, 0.0, op->buf,
-                          ctx->partials, ctx->npart, ctx->norm_dev, nullptr, 0, ctx->stream));
+  HIPCHK(ctx, launch_norm(ctx->db.d, ctx->db.h, out != op ? NormOp::kCopy : NormOp::kSum, out->buf, nullptr, 0.0,
+                          op->buf, ctx->partials, ctx->npart, ctx->norm_dev, nullptr, 0, ctx->stream));
   out->herm = op->herm;
   HIPCHK(ctx, launch_normal_order(ctx->db.d, ctx->db.h, out->buf, sign, op->herm, ctx->norm_dev, ctx->stream));
   return IMSRG_OK;
@@ -1680,10 +1680,11 @@ static int bch_transform(imsrg_ctx *ctx, const imsrg_dop *Op, const imsrg_dop *O
   int rc;
   if ((rc = ensure_ops(ctx, ctx->tmp, 2))) return rc;
   double nx, ny;
-  if ((rc = op_norms(Op, Omega, &nx, &ny, Out != Op ? Out : nullptr))) return rc;  // Out = Op
-  Out->herm = Op->herm;
+  if ((rc = op_norms(Op, Omega, &nx, &ny))) return rc;  // Out stays as it is when one is not finite
   int nc = 0;
   bool converged = true;
+  // the first term's pass makes Out = Op + fact * nested, the later ones add to Out
+  const imsrg_dop *base = Op;
   if (nx > o.transform_thr) {
     converged = false;
     // Out changes only after the first commutator has read Op.  With graphs on a copy of
@@ -1703,8 +1704,10 @@ static int bch_transform(imsrg_ctx *ctx, const imsrg_dop *Op, const imsrg_dop *O
       nested = next;
       fact /= i;
       eps *= i + 1;
-      double nn;  // Out += fact * nested, and the norm of nested, in one pass
-      if ((rc = op_norm(nested, nullptr, nullptr, &nn, Out, fact))) return rc;
+      double nn;  // Out = base + fact * nested, and the norm of nested, in one pass
+      Out->herm = Op->herm;
+      if ((rc = op_norm(nested, nullptr, nullptr, &nn, Out, base, fact))) return rc;
+      base = Out;
       if ((o.mode == 0 && nn < eps) || (o.mode == 1 && nn < o.transform_thr)) {
         converged = true;
         break;
@@ -1712,7 +1715,7 @@ static int bch_transform(imsrg_ctx *ctx, const imsrg_dop *Op, const imsrg_dop *O
     }
   }
   if (ncomm) *ncomm = nc;
-  Out->herm = Op->herm;
+  if (base != Out && (rc = imsrg_hip_op_copy(Out, Op))) return rc;  // no term
   if (!converged) return fail(ctx, IMSRG_E_NOT_CONVERGED, "BCH_Transform did not converge within max_terms");
   return IMSRG_OK;
 }
@@ -1726,8 +1729,8 @@ static int bch_product(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y, i
   if ((rc = ensure_ops(ctx, ctx->tmp, 3))) return rc;
   if (Out == X || Out == Y) return fail(ctx, IMSRG_E_INVALID, "Out must not alias X or Y");
   double nx, ny;
-  if ((rc = op_norms(X, Y, &nx, &ny, Out))) return rc;  // Out = X
-  if ((rc = imsrg_hip_op_axpy(Out, 1.0, Y))) return rc;
+  if ((rc = op_norms(X, Y, &nx, &ny))) return rc;  // Out stays as it is when one is not finite
+  HIPCHK(ctx, launch_axpy(Out->buf, X->buf, 1.0, Y->buf, ctx->db.h.opsize, ctx->stream));  // Out = X + Y
   Out->herm = X->herm;
   imsrg_dop *nested = ctx->tmp[0], *next = ctx->tmp[1];
   int nc = 0;

@@ -146,10 +146,11 @@ hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, hipS
 }
 
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_axpy(double *y, double a, const double *x, long n) {
+// y = z + a x; z may be y
+__global__ __launch_bounds__(256) void k_axpy(double *y, const double *z, double a, const double *x, long n) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     double t = a * x[i];  // (a*x) formed first, then added (Operator operator* then +=)
-    y[i] += t;
+    y[i] = z[i] + t;
   }
 }
 __global__ __launch_bounds__(256) void k_scale(double *y, double a, long n) {
@@ -164,8 +165,8 @@ hipError_t launch_fill(double *y, double v, long n, hipStream_t s) {
   hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, y, v, n);
   return hipGetLastError();
 }
-hipError_t launch_axpy(double *y, double a, const double *x, long n, hipStream_t s) {
-  hipLaunchKernelGGL(k_axpy, dim3(grid_for(n)), dim3(256), 0, s, y, a, x, n);
+hipError_t launch_axpy(double *y, const double *z, double a, const double *x, long n, hipStream_t s) {
+  hipLaunchKernelGGL(k_axpy, dim3(grid_for(n)), dim3(256), 0, s, y, z, a, x, n);
   return hipGetLastError();
 }
 hipError_t launch_scale(double *y, double a, long n, hipStream_t s) {
@@ -174,8 +175,8 @@ hipError_t launch_scale(double *y, double a, long n, hipStream_t s) {
 }
 
 // One pass over an operator buffer x with the partial sums of its norm: OP 0 the sums
-// alone, OP 1 y += a x beside them (the BCH_Transform step, src/BCH.cc:176-191), OP 2
-// y = x (a copy).  Block b < nblk2 takes the b-th contiguous chunk of the two-body arena,
+// alone, OP 1 y = z + a x beside them (z is y, or Op at the first term: the BCH_Transform
+// step, src/BCH.cc:176-191), OP 2 y = x (a copy).  Block b < nblk2 takes the b-th contiguous chunk of the two-body arena,
 // each word with its channel's weight (2J+1)^2; blocks nblk2 .. nblk2 + nblk1 - 1 share the
 // one-body part (weights 2 j_p + 1), the first of them the words around the two parts.
 // Bound by HBM at large sizes: a block has four 16-byte loads per thread in flight (one
@@ -185,8 +186,8 @@ hipError_t launch_scale(double *y, double a, long n, hipStream_t s) {
 // 37 us at emax = 7 (22 MB) and 27 us at emax = 6, now 16 and 9 us.
 constexpr int kNormCh = 640;  // channels whose offsets fit in the kernel's LDS list
 template <int OP>
-__global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y, double a, const double *x,
-                                                   double *part, int nblk2, int nblk1) {
+__global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y, const double *z, double a,
+                                                   const double *x, double *part, int nblk2, int nblk1) {
   const BasisDev &B = *bd;
   __shared__ double red[4];
   __shared__ long s_off[kNormCh];
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
     auto put = [&](long e, double v) {  // one word of y
       if (OP == 1) {
         double t = a * v;  // (a x) formed first, then added (Operator operator* then +=)
-        y[e] += t;
+        y[e] = z[e] + t;
       }
       if (OP == 2) y[e] = v;
     };
@@ -209,6 +210,7 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
         for (long e = rg[g][0] + threadIdx.x; e < rg[g][1]; e += blockDim.x) put(e, x[e]);
     const double *x1 = x + B.one_off;
     double *y1 = OP ? y + B.one_off : nullptr;
+    const double *z1 = OP == 1 ? z + B.one_off : nullptr;
     for (long q = (long)b1 * blockDim.x + threadIdx.x; q < n1; q += (long)U * nblk1 * blockDim.x) {
       double v[U], w[U], o[U];
 #pragma unroll
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
         const long e = min(q + (long)u * nblk1 * blockDim.x, n1 - 1);
         v[u] = x1[e];
         w[u] = B.w1norm[e];
-        if (OP == 1) o[u] = y1[e];
+        if (OP == 1) o[u] = z1[e];
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -233,6 +235,7 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
   } else {
     const double *two = x + B.two_off;
     double *y2 = OP ? y + B.two_off : nullptr;
+    const double *z2 = OP == 1 ? z + B.two_off : nullptr;
     const long tb = B.tbsize, chunk = (tb + nblk2 - 1) / nblk2;
     const long c0 = (long)blockIdx.x * chunk, c1 = min(c0 + chunk, tb);
     // the channels that the chunk overlaps: lo .. hi
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(256) void k_norm_pass(const BasisDev *bd, double *y
       for (int u = 0; u < U; ++u) {
         const long e = min(q + 2 * u * (long)blockDim.x, (c1 - 1) & ~1L);
         v[u] = *reinterpret_cast<const double2 *>(two + e);
-        if (OP == 1) o[u] = *reinterpret_cast<const double2 *>(y2 + e);
+        if (OP == 1) o[u] = *reinterpret_cast<const double2 *>(z2 + e);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -403,19 +406,19 @@ hipError_t launch_normal_order(const BasisDev *bd, const BasisDev &bh, double *o
   return hipGetLastError();
 }
 
-hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, double a, const double *x,
-                       double *partials, int maxpart, double *out, unsigned long long *done, unsigned long long seq,
-                       hipStream_t s) {
+hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, const double *z, double a,
+                       const double *x, double *partials, int maxpart, double *out, unsigned long long *done,
+                       unsigned long long seq, hipStream_t s) {
   // two-body chunks of at least 2048 words, so that small bases do not pay for idle blocks
   const int nblk1 = (int)std::max(1, std::min(32, bh.norb * bh.norb / 1024));
   const int nblk2 = (int)std::max<long>(1, std::min<long>(maxpart - nblk1, (bh.tbsize + 2047) / 2048));
   const dim3 grid(nblk2 + nblk1), blk(256);
   if (op == NormOp::kSum)
-    hipLaunchKernelGGL((k_norm_pass<0>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
+    hipLaunchKernelGGL((k_norm_pass<0>), grid, blk, 0, s, bd, y, z, a, x, partials, nblk2, nblk1);
   else if (op == NormOp::kAxpy)
-    hipLaunchKernelGGL((k_norm_pass<1>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
+    hipLaunchKernelGGL((k_norm_pass<1>), grid, blk, 0, s, bd, y, z, a, x, partials, nblk2, nblk1);
   else
-    hipLaunchKernelGGL((k_norm_pass<2>), grid, blk, 0, s, bd, y, a, x, partials, nblk2, nblk1);
+    hipLaunchKernelGGL((k_norm_pass<2>), grid, blk, 0, s, bd, y, z, a, x, partials, nblk2, nblk1);
   hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, s, partials, nblk2, nblk1, out, done, seq);
   return hipGetLastError();
 }

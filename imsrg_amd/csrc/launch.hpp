@@ -68,7 +68,8 @@ hipError_t launch_c122_w(const PairArg &pa, const int4 *items, int nitems, int m
 hipError_t launch_zero_two(const PairArg &pa, const int4 *items, int nitems, hipStream_t s);
 
 // operator arithmetic
-hipError_t launch_axpy(double *y, double a, const double *x, long n, hipStream_t s);
+// y = z + a x; z may be y
+hipError_t launch_axpy(double *y, const double *z, double a, const double *x, long n, hipStream_t s);
 hipError_t launch_scale(double *y, double a, long n, hipStream_t s);
 hipError_t launch_fill(double *y, double v, long n, hipStream_t s);  // y[i] = v
 // Operator::DoNormalOrdering2 / UndoNormalOrdering of a scalar operator in place
@@ -78,12 +79,12 @@ hipError_t launch_fill(double *y, double v, long n, hipStream_t s);  // y[i] = v
 hipError_t launch_normal_order(const BasisDev *bd, const BasisDev &bh, double *op, int sign, int herm,
                                const double *n2sq, hipStream_t s);
 // sums of squares of an operator buffer x into out[0] (one-body) and out[1] (two-body,
-// weighted), and in the same pass kAxpy: y += a x, kCopy: y = x over the whole buffer;
+// weighted), and in the same pass kAxpy: y = z + a x (z may be y), kCopy: y = x over the whole buffer;
 // seq != 0: out and *done are host memory, *done = seq once out holds the sums
 enum class NormOp { kSum, kAxpy, kCopy };
-hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, double a, const double *x,
-                       double *partials, int maxpart, double *out, unsigned long long *done, unsigned long long seq,
-                       hipStream_t s);
+hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, const double *z, double a,
+                       const double *x, double *partials, int maxpart, double *out, unsigned long long *done,
+                       unsigned long long seq, hipStream_t s);
 // the basis-change matrices D of every channel (two-body layout, tbsize doubles) from
 // the one-body basis change C (norb x norb, column-major)
 // the Hartree-Fock monopoles W[q] = sum_J (2J+1) V~^J_{ia,jb} of quads[q] = (i, a, j, b)

@@ -235,6 +235,8 @@ int imsrg_hip_commutator_ss_dev_async(imsrg_ctx *ctx, const imsrg_dop *X, const 
  * other contexts' streams) race; calls ordered on one stream do not. */
 int imsrg_hip_commutator_ss_dev_noalloc(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y, imsrg_dop *Z,
                                         const imsrg_comm_opts *opts);
+/* Out may be Op; Out and its Hermiticity stay as they are when Op or Omega (X or Y) holds
+ * Inf or NaN (IMSRG_E_NONFINITE). */
 int imsrg_hip_bch_transform_dev(imsrg_ctx *ctx, const imsrg_dop *Op, const imsrg_dop *Omega, imsrg_dop *Out,
                                 const imsrg_bch_opts *opts, int *n_commutators);
 int imsrg_hip_bch_product_dev(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y, imsrg_dop *Out,
