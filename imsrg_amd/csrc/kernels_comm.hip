@@ -2021,6 +2021,25 @@ __device__ __forceinline__ void c122_w_tile(const PairPtrs &P, const int4 &it, u
         if (c < nn && r0 + m < n) blk_at(W, (unsigned)sq[n0 + c] * n + row) = acc[j][q];
       }
     }
+    // A row with an Inf or NaN in a column of the bin is not finite in all of its results, the
+    // first among them, through products with 0: such a row again from its partner entries
+    // alone, each lane the columns it has stored.
+    if (!__builtin_isfinite(acc[0][0]) && r0 + m < n) {
+      for (int c = kq; c < nn; c += 4) blk_at(W, (unsigned)sq[n0 + c] * n + row) = 0.0;
+      double w = 0.0;
+      int last = -1;  // entries of one column follow one another
+      for (int t = 0; t < ne; ++t) {
+        const int4 rec = B.c122_brec[eo + t];
+        const int c = (rec.y >> 16) - n0;
+        if (c < 0 || c >= nn || (c & 3) != kq) continue;
+        if (c != last) w = 0.0;
+        last = c;
+        const double f = __hiloint2double(rec.w, rec.z);
+        const unsigned e = (unsigned)sq[rec.y & 0xffff] * n + row;
+        w += blk_at(Y2, e) * (P.X[B.one_off + rec.x] * f) - blk_at(X2, e) * (P.Y[B.one_off + rec.x] * f);
+        blk_at(W, (unsigned)sq[n0 + c] * n + row) = w;
+      }
+    }
   }
 }
 __global__ __launch_bounds__(256, 4) void k_c122_w(PairArg pa, const int4 *items) {
