@@ -1495,7 +1495,7 @@ __device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, 
             const double w = u == 0 ? w01.x : u == 1 ? w01.y : u == 2 ? w23.x : w23.y;
             const bool ok = J >= jmin && J <= jmax && !(even & J) && fabs(w) >= 1e-8 && r != 0xffff && cl != 0xffff;
             wv[u] = ok ? (2 * J + 1) * w * sgn_parity(s0 + sj * J) : 0.0;
-            // an invalid term reads the operator's first element and is weighted by 0
+            // an invalid term reads the operator's first element and counts as 0
             const int4 ch = s_ch[ok ? 6 * J + g : 0];
             const long idx = ok ? (((long)ch.y << 32) | (unsigned)ch.x) + (long)(cl * ch.z + r) : 0;
             xv[u] = X2[idx];
@@ -1503,8 +1503,8 @@ __device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, 
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            xbar -= wv[u] * xv[u];
-            ybar -= wv[u] * yv[u];
+            xbar -= wv[u] * (wv[u] != 0.0 ? xv[u] : 0.0);
+            ybar -= wv[u] * (wv[u] != 0.0 ? yv[u] : 0.0);
           }
         }
       }
