@@ -571,7 +571,10 @@ __global__ __launch_bounds__(256) void k_xf_pass(const BasisDev *bd, XformDev X,
     double a[kXfMaxM / 4];
 #pragma unroll
     for (int k = 0; k < kXfMaxM / 4; ++k)
-      if (k < nks) a[k] = v[(long)ket[4 * k + (lane >> 4)] * n];
+      if (k < nks) {
+        const double x = v[(long)ket[4 * k + (lane >> 4)] * n];
+        a[k] = 4 * k + (lane >> 4) < m ? x : 0.0;  // past the group: 0 whatever the last ket holds
+      }
     const double f = herm != 0.0 ? herm : 1.0;
     const int to = SECOND ? X.g_kets[cs + min(row, n - 1)] : 0;  // the row's place in V'
     for (int c = 0; c < nc; ++c) {
