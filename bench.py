@@ -168,13 +168,15 @@ def workload_emax12(args, ia, np, emax=12):
         ia.Commutator.CommutatorScalarScalar(X, Y, precision=prec, out=Z)
         ms.synchronize()
         steps = max(3, min(args.steps, 5))
-        ms.set_profiling(True)
-        ms.phase_times()
         t0 = time.perf_counter()
         for _ in range(steps):
             ia.Commutator.CommutatorScalarScalar(X, Y, precision=prec, out=Z)
         ms.synchronize()
         t = time.perf_counter() - t0
+        ms.set_profiling(True)
+        ms.phase_times()
+        for _ in range(steps):
+            ia.Commutator.CommutatorScalarScalar(X, Y, precision=prec, out=Z)
         phase = np.array(ms.phase_times())
         ms.set_profiling(False)
         hosts[name] = Z.to_host()
@@ -564,20 +566,23 @@ def main():
     ms.synchronize()
 
     def timed(precision):
-        """warm-up, then the timed steps; the library records HIP events around
-        every phase of the timed steps on the stream that phase runs on, with no
+        """warm-up, then the timed steps, then as many profiled ones, which have a
+        launch per phase (a few more than a commutator has otherwise): the library
+        records HIP events around every phase on the stream that phase runs on, with no
         host synchronisation per step, and averages them afterwards; returns the
         rate, the per-phase averages (us) and the result on the host"""
         for _ in range(args.warmup):
             ia.Commutator.CommutatorScalarScalar(X, Y, precision=precision, out=Z)
         ms.synchronize()
-        ms.set_profiling(True)
-        ms.phase_times()  # nothing pending from earlier calls
         t0 = time.perf_counter()
         for _ in range(args.steps):
             ia.Commutator.CommutatorScalarScalar(X, Y, precision=precision, out=Z)
         ms.synchronize()
         t = time.perf_counter() - t0
+        ms.set_profiling(True)
+        ms.phase_times()  # nothing pending from earlier calls
+        for _ in range(args.steps):
+            ia.Commutator.CommutatorScalarScalar(X, Y, precision=precision, out=Z)
         phases = np.array(ms.phase_times())
         ms.set_profiling(False)
         return args.steps / t, t, phases, Z.to_host()

@@ -177,10 +177,10 @@ struct imsrg_ctx {
   std::string err;
   bool profiling = false;
   // phase events of profiled commutators: a ring of sets recorded without host
-  // synchronisation, read (and summed) by imsrg_hip_phase_times; marks 0..6 on
-  // the main stream, 7, 8, 9 around the pp/hh GEMM and comm122 on the side stream (9, 10
+  // synchronisation, read (and summed) by imsrg_hip_phase_times; marks 0..8 on
+  // the main stream, 9, 10, 11 around the pp/hh GEMM and comm122 on the side stream (11, 12
   // around comm122 on the main one)
-  static constexpr int kRing = 32, kMarks = 11;
+  static constexpr int kRing = 32, kMarks = 13;
   std::vector<std::array<hipEvent_t, kMarks>> ring;
   int ring_head = 0, ring_count = 0;
   int ring_side[kRing] = {};  // 1: the pp/hh GEMM and comm122 on the side stream, 2: comm122 on the main one
@@ -1339,17 +1339,17 @@ static int herm_rule(int hx, int hy) { return (hx == hy) ? -1 : 1; }  // src/Com
 // Sums the phase durations of the oldest recorded event set (waits for it).
 static int harvest_oldest(imsrg_ctx *ctx) {
   auto &set = ctx->ring[ctx->ring_head];
-  HIPCHK(ctx, hipEventSynchronize(set[6]));
-  // marks on the main stream: pp/hh, comm122, first launch (Pandya, zero- and
-  // one-body), ph GEMM, inverse Pandya, last launch; reported in the header's order
-  const int map[6] = {3, 2, 4, 5, 6, 7};
+  HIPCHK(ctx, hipEventSynchronize(set[8]));
+  // marks on the main stream: pp/hh, comm122, zero-body, one-body, Pandya, ph GEMM,
+  // inverse Pandya, last launch; reported in the header's order
+  const int map[8] = {3, 2, 0, 1, 4, 5, 6, 7};
   const int side = ctx->ring_side[ctx->ring_head];
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < 8; ++i) {
     float ms = 0.f;
     int a = i, b = i + 1;
-    if (side && i == 0) a = 7, b = 8;
-    if (side && i == 1) a = side == 2 ? 9 : 8, b = side == 2 ? 10 : 9;
-    if (side == 2 && i == 4) b = 9;
+    if (side && i == 0) a = 9, b = 10;
+    if (side && i == 1) a = side == 2 ? 11 : 10, b = side == 2 ? 12 : 11;
+    if (side == 2 && i == 6) b = 11;
     HIPCHK(ctx, hipEventElapsedTime(&ms, set[a], set[b]));
     ctx->phase_sum[map[i]] += ms * 1000.0;
   }
@@ -1387,7 +1387,8 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
                 mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big, items[7], items[9], mask & MPPHH ? cnt[7] : 0,
                 mask & M122 ? cnt[9] : 0};
-  const bool small = fi.blocks() <= kFrontSmall;
+  // a profiled commutator has a launch per phase instead, each between its events
+  const bool small = fi.blocks() <= kFrontSmall && !ctx->profiling;
   if (!small) fi.n64 = fi.nc122 = 0;
   const bool overlap = tu.overlap_pphh && (mask & MPPHH) && !(small && cnt[big] == 0);
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so
@@ -1414,12 +1415,12 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   // was empty (a nested commutator follows a norm that the host has waited for).
   auto side_work = [&]() -> int {
     HIPCHK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork, 0));
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[7], ctx->side));
+    if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7] - fi.n64, items[8], cnt[8], prec_pphh, maxn,
                             ctx->side));
-    if (set) HIPCHK(ctx, hipEventRecord((*set)[8], ctx->side));
+    if (set) HIPCHK(ctx, hipEventRecord((*set)[10], ctx->side));
     if (m122 && !c122_main) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, ctx->side));
-    if (set && !c122_main) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
+    if (set && !c122_main) HIPCHK(ctx, hipEventRecord((*set)[11], ctx->side));
     HIPCHK(ctx, hipEventRecord(ctx->join, ctx->side));
     return IMSRG_OK;
   };
@@ -1434,27 +1435,37 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   HIPCHK(ctx, mark(1));
   if (m122 && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
   HIPCHK(ctx, mark(2));
+  if (set) {
+    FrontItems zero = fi, one = fi;
+    zero.none = zero.n221 = zero.npandya = 0;
+    one.nzeros = one.npandya = 0;
+    fi.nzeros = fi.none = fi.n221 = 0;
+    HIPCHK(ctx, launch_front(pa, zero, maxnch, maxbin, false, s));
+    HIPCHK(ctx, mark(3));
+    HIPCHK(ctx, launch_front(pa, one, maxnch, maxbin, false, s));
+    HIPCHK(ctx, mark(4));
+  }
   HIPCHK(ctx, launch_front(pa, fi, maxnch, maxbin, prec_pphh == 1, s));
-  HIPCHK(ctx, mark(3));
+  HIPCHK(ctx, mark(5));
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));
   if (fork_late) HIPCHK(ctx, hipEventRecord(ctx->fork, s));
-  HIPCHK(ctx, mark(4));
+  HIPCHK(ctx, mark(6));
   if (mask & MPH) {
     const int f = prec_ph == 1 ? 10 : 4;  // FP32 Zbar: twice the elements per item
     HIPCHK(ctx, launch_invpandya(pa, items[f], cnt[f], invp_lds[prec_ph == 1], prec_ph == 1, s));
   }
   if (c122_main) {
-    HIPCHK(ctx, mark(9));
+    HIPCHK(ctx, mark(11));
     if (m122) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
-    HIPCHK(ctx, mark(10));
+    HIPCHK(ctx, mark(12));
   }
   if (overlap) {
     if (int rc = side_work()) return rc;
     HIPCHK(ctx, hipStreamWaitEvent(s, ctx->join, 0));
   }
-  HIPCHK(ctx, mark(5));
+  HIPCHK(ctx, mark(7));
   HIPCHK(ctx, launch_finish(pa, items[6], cnt[6], (mask & MPH) != 0, (mask & M122) != 0, npairs, maxn1pairs, s));
-  HIPCHK(ctx, mark(6));
+  HIPCHK(ctx, mark(8));
   if (set) ++ctx->ring_count;
   return IMSRG_OK;
 }

@@ -353,15 +353,15 @@ int imsrg_hip_set_tuning(imsrg_ctx *ctx, const imsrg_tuning *t);
 int imsrg_hip_autotune(imsrg_ctx *ctx, int precision, const char *cache_path, imsrg_tuning *out);
 
 /* Per-phase timing of commutators on ctx (microseconds, HIP events):
- * [2] comm122's W, [3] pp/hh GEMM, [4] first launch (Pandya gather with the
- * zero- and one-body terms beside it; on small bases comm122's W and the pp/hh blocks of
- * small channels too), [5] ph GEMM, [6] inverse Pandya, [7] last
- * launch (fold of the inverse-Pandya terms, comm122, mirror, the sums of the
- * zero- and one-body parts); [0] and [1], once the zero- and one-body launches, are 0.  Enabled by imsrg_hip_set_profiling:
- * each commutator records HIP events on the stream its phases run on (the
- * pp/hh GEMM's own stream when it overlaps the others) without a host
- * synchronisation; imsrg_hip_phase_times returns the average over the
- * commutators profiled since its previous call (0 if none) and resets it. */
+ * [0] zero-body, [1] one-body, [2] comm122's W, [3] pp/hh GEMM, [4] Pandya
+ * gather, [5] ph GEMM, [6] inverse Pandya, [7] last launch (fold of the
+ * inverse-Pandya terms, comm122, mirror, the sums of the zero- and one-body
+ * parts).  Enabled by imsrg_hip_set_profiling: a commutator then has a launch per
+ * phase, where others put [0], [1], [4] and on small bases [2] and the small
+ * channels' part of [3] into one launch, and records HIP events on the stream
+ * its phases run on (the pp/hh GEMM's own stream when it overlaps the others)
+ * without a host synchronisation; imsrg_hip_phase_times returns the average over
+ * the commutators profiled since its previous call (0 if none) and resets it. */
 int imsrg_hip_set_profiling(imsrg_ctx *ctx, int on);
 int imsrg_hip_phase_times(imsrg_ctx *ctx, double *us, int n);
 
