@@ -1386,7 +1386,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   const bool m221 = (mask & M221) != 0, mph = (mask & MPH) != 0;
   FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
                 mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big, items[7], items[9], mask & MPPHH ? cnt[7] : 0,
-                mask & M122 ? cnt[9] : 0};
+                mask & M122 ? cnt[9] : 0, false};
   // a profiled commutator has a launch per phase instead, each between its events
   const bool small = fi.blocks() <= kFrontSmall && !ctx->profiling;
   if (!small) fi.n64 = fi.nc122 = 0;
@@ -1394,6 +1394,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so
   // that the pp/hh GEMM shares the GPU with the inverse Pandya gather only
   const bool fork_late = overlap && tu.overlap_pphh == 2;
+  fi.split = overlap && !fork_late && npairs == 1 && prec_pphh != kGemmB3 && cnt[big] > kFrontSplit;
   // comm122's W on the main stream, after the inverse Pandya kernel, where the bf16x3 GEMM
   // takes longer than the main stream's kernels: that GEMM leaves the memory idle.  emax = 10
   // (1539 tiles) 1801 -> 1759 us, emax = 12 (5387) 8.22 -> 8.08 ms; emax = 9 (700) 805 -> 812,

@@ -2208,13 +2208,6 @@ hipError_t launch_set_pairs(PairPtrs *tab, const PairOps &ops, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Above this many Pandya chunks (about 7 residencies of the chip) they get a launch of
-// their own after the others: the one-body work-groups then run beside the pp/hh GEMM's
-// packing, and the chunks are not held up behind them (emax = 10 FP64 2.95 -> 2.91 ms,
-// mixed 2.18 -> 2.15 ms, emax = 12 mixed 10.36 -> 10.25 ms); below it one launch is
-// faster (emax = 8 mixed 492 -> 473 us, emax = 6 mixed 159 -> 146 us).
-constexpr int kFrontSplit = 12288;
-
 hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int maxbin, bool mixed64, hipStream_t s) {
   size_t lds = sizeof(int4) * (size_t)std::max(maxnch, 1);  // the Pandya chunks' channel table
   if (f.n64 + f.nc122 > 0) {
@@ -2227,7 +2220,7 @@ hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int 
     return hipGetLastError();
   }
   FrontItems part[2] = {f, f};
-  if (f.npandya > kFrontSplit) {
+  if (f.split) {
     part[0].npandya = 0;
     part[1].nzeros = part[1].none = part[1].n221 = 0;
   } else {

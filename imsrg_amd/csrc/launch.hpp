@@ -36,6 +36,7 @@ struct FrontItems {
   // small bases: the 64x64 pp/hh tiles and comm122's W items, in the same launch
   const int4 *pphh64, *c122;
   int n64, nc122;
+  bool split;  // the Pandya chunks in a launch of their own, after the others (kFrontSplit)
   int blocks() const { return n64 + nc122 + nzeros + none + n221 + npandya; }
 };
 // mixed64: the pp/hh tiles with FP32 products
@@ -46,6 +47,16 @@ hipError_t launch_front(const PairArg &pa, const FrontItems &f, int maxnch, int 
 // 50 -> 34, emax = 5 90 -> 87, mixed 71 -> 68, emax = 6 147 -> 140 and 99 -> 93 us).  Where they fill
 // the chip they only hold up the main stream: emax = 7 235 -> 239 us, mixed 161 -> 174 us.
 constexpr int kFrontSmall = 3500;
+// 128x128 pp/hh tiles (two for each CU) above which the first launch of one commutator is two,
+// the Pandya chunks after the others: the FP64, FP32 and split FP32 GEMMs beside it take all
+// registers of a CU then, and the two launches together wait less for them than one (FP64 emax =
+// 9, 747 tiles, O16 1088 -> 1085 us and Ca40 1399 -> 1379, emax = 10 O16 2616 -> 2590 and Ca40 3222 ->
+// 3190, emax = 12 14.45 -> 14.3 ms; FP32 emax = 9 927 -> 914, emax = 10 2196 -> 2145; split emax = 10
+// 4824 -> 4643).  Not so with fewer tiles (FP64 emax = 8, 393 tiles, O16 469 -> 485 us, Ca40 604 ->
+// 638; emax = 7 235 -> 258), beside the bf16x3 GEMM, one work-group per CU (mixed emax = 8 Ca40
+// 465 -> 477, emax = 10 O16 1728 -> 1761, Ca40 2200 -> 2202, emax = 12 8.24 -> 8.22 ms), and in
+// batches (FP64, 24 pairs at emax = 6 1501 -> 1515 us, 8 at emax = 8 3.43 -> 3.43 ms).
+constexpr int kFrontSplit = 512;
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
 // under bf16x3 products (kGemmB3) the pack items first write the operand panels
 // maxn: the largest channel dimension of the pairs (sizes the kernel's LDS index list)
