@@ -1396,9 +1396,13 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   const bool fork_late = overlap && tu.overlap_pphh == 2;
   fi.split = overlap && !fork_late && npairs == 1 && prec_pphh != kGemmB3 && cnt[big] > kFrontSplit;
   // comm122's W on the main stream, after the inverse Pandya kernel, where the bf16x3 GEMM
-  // takes longer than the main stream's kernels: that GEMM leaves the memory idle.  emax = 10
-  // (1539 tiles) 1801 -> 1759 us, emax = 12 (5387) 8.22 -> 8.08 ms; emax = 9 (700) 805 -> 812,
-  // FP64 emax = 10 2630 -> 2638 us, where the FP64 GEMM's waves leave no room beside them.
+  // has many tiles: with one work-group per CU it leaves room beside it, whichever stream is the
+  // longer one (with heavier references the main stream is).  emax = 10 (1539 tiles) O16 1823 ->
+  // 1763 us, Ne20 2064 -> 2016, Si28 2042 -> 1993, Ca40 2259 -> 2203, Ni56 2569 -> 2511; emax = 11
+  // and 12 the same within 1% (O16 8.23 -> 8.20 ms, Ca40 10.05 -> 10.07); batches of 24 pairs at
+  // emax = 6 1369 -> 1361, of 16 Ca40 at emax = 7 3097 -> 3077.  Fewer tiles: emax = 9 (747) O16
+  // 763 -> 773, Ca40 1025 -> 1026; FP64 emax = 10 2630 -> 2638 us, where the FP64 GEMM's waves
+  // leave no room beside them.
   const bool m122 = (mask & M122) && fi.nc122 == 0;  // comm122's W in a launch of its own
   const bool c122_main = overlap && prec_pphh == kGemmB3 && cnt[big] > 1024;
   // profiling: this commutator's phase events go to the next free set of the ring
