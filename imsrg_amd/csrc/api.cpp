@@ -311,8 +311,6 @@ static int ctx_init(imsrg_ctx *ctx, const imsrg_basis_desc *b, int device) {
   HIPCHK(ctx, hipMalloc(&ctx->Xt, sizeof(double) * (std::max<long>(B.xsize, 1) + 8)));
   HIPCHK(ctx, hipMalloc(&ctx->Yt, sizeof(double) * (std::max<long>(B.xsize, 1) + 8)));
   HIPCHK(ctx, hipMalloc(&ctx->Zbar, sizeof(double) * std::max<long>(B.zsize, 1)));
-  // cross-coupled channels without ph kets are never written and must read as 0
-  HIPCHK(ctx, hipMemset(ctx->Zbar, 0, sizeof(double) * std::max<long>(B.zsize, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->scratch, sizeof(double) * (B.nch + 8)));
   HIPCHK(ctx, hipMalloc(&ctx->obpart, sizeof(double) * std::max(B.nobpart, 1)));
   HIPCHK(ctx, hipMalloc(&ctx->diag, sizeof(double) * std::max(B.ndiag, 1)));
@@ -1577,11 +1575,9 @@ int imsrg::ctx_device(const imsrg_ctx *ctx) { return ctx ? ctx->device : -1; }
 int imsrg::ctx_fail(imsrg_ctx *ctx, int code, const char *msg) { return fail(ctx, code, msg); }
 
 // The allocation-free commutator: the context's own workspaces are replaced by
-// ones carved from ws.  Cross-coupled channels with no ph kets are never
-// written by the ph GEMM and must read as 0, so that part (all of Zbar) is
-// cleared by a fill kernel on every call: ws keeps the previous call's
-// contents, possibly of another basis.  Every other workspace is written
-// before it is read.
+// ones carved from ws, which keeps the previous call's contents, possibly of another
+// basis: every workspace is written before it is read (the inverse Pandya kernel takes
+// channels without ph kets, whose Zbar the ph GEMM does not write, as 0).
 int imsrg::commutator_in_workspace(imsrg_ctx *ctx, const imsrg_dop *X, const imsrg_dop *Y, imsrg_dop *Z,
                                    const imsrg_comm_opts *opts, double *ws, long cap) {
   if (!X || !Y || !Z) return IMSRG_E_INVALID;
@@ -1599,7 +1595,6 @@ int imsrg::commutator_in_workspace(imsrg_ctx *ctx, const imsrg_dop *X, const ims
   }
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const Workspace w = carve_workspace(B, ws);
-  HIPCHK(ctx, launch_fill(w.Zbar, 0.0, std::max<long>(B.zsize, 1), ctx->stream));
   return commutator_dev(ctx, X, Y, Z, mask, prec, &w);
 }
 
@@ -2224,7 +2219,6 @@ extern "C" int imsrg_hip_commutator_ss_batched(int npairs, imsrg_ctx *const *ctx
       wtot += workspace_doubles(ctxs[i]->db.h, true);
     }
     HIPCHK(c0, hipMalloc(&bc.work, sizeof(double) * std::max<long>(wtot, 1)));
-    HIPCHK(c0, hipMemset(bc.work, 0, sizeof(double) * std::max<long>(wtot, 1)));
     std::vector<PairPtrs> tab(npairs, PairPtrs{});
     for (int i = 0; i < npairs; ++i) {
       const BasisDev &B = ctxs[i]->db.h;
