@@ -182,12 +182,9 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   obstart[norb] = (int)oblist.size();
   B.obstart = dupload(*this, obstart, err); B.oblist = dupload(*this, oblist, err);
   B.kp = dupload(*this, hb.kp, err); B.kq = dupload(*this, hb.kq, err);
-  B.kmap = dupload(*this, hb.kmap, err); B.cmap = dupload(*this, hb.cmap, err);
+  B.kmap = dupload(*this, hb.kmap, err);
   {
     std::vector<int> cT((size_t)hb.nkets * (hb.jmax + 1));
-    for (int k = 0; k < hb.nkets; ++k)
-      for (int J = 0; J <= hb.jmax; ++J) cT[(size_t)J * hb.nkets + k] = hb.cmap[(size_t)k * (hb.jmax + 1) + J];
-    B.cmapT = dupload(*this, cT, err);
     for (int k = 0; k < hb.nkets; ++k)
       for (int J = 0; J <= hb.jmax; ++J) cT[(size_t)J * hb.nkets + k] = hb.kmap[(size_t)k * (hb.jmax + 1) + J];
     B.kmapT = dupload(*this, cT, err);
@@ -214,7 +211,7 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
     }
   }
   grp_start[6] = (int)grp_kets.size();
-  B.grp_start = dupload(*this, grp_start, err); B.grp_kets = dupload(*this, grp_kets, err);
+  B.grp_start = dupload(*this, grp_start, err);
   std::vector<int> grp_first((size_t)6 * (norb + 1));
   for (int g = 0; g < 6; ++g) {
     int e = grp_start[g];
@@ -419,11 +416,9 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   std::vector<signed char> cc_phi, cc_phph;
   std::vector<long> cc_xoff(nch + 1), cc_zoff(nch + 1);
   long xo = 0, zo = 0;
-  int maxcc = 0;
   for (int c = 0; c < nch; ++c) {
     const HostChannel &C = hb.cc[c];
     int nk = (int)C.kets.size();
-    maxcc = std::max(maxcc, nk);
     cc_n[c] = nk;
     cc_kstart[c] = (int)cc_kets.size();
     cc_phstart[c] = (int)cc_ph.size();
@@ -453,7 +448,6 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   cc_phstart[nch] = (int)cc_ph.size();
   cc_xoff[nch] = xo;
   cc_zoff[nch] = zo;
-  B.maxcc = maxcc;
   B.ccjmax_ph = -1;
   for (int c = 0; c < nch; ++c)
     if (cc_nph[c] > 0) B.ccjmax_ph = std::max(B.ccjmax_ph, c / 6);
@@ -741,8 +735,6 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   this->k_start = k_start;
   this->cc_n = cc_n;
   this->cc_nph = cc_nph;
-  this->grp_start = grp_start;
-  this->grp_kets = grp_kets;
   this->pairs1 = pairs1;
   gen_ok.assign(nch, 0);
   for (int c = 0; c < nch; ++c) gen_ok[c] = gcore_start[c + 1] > gcore_start[c] && gnc_start[c + 1] > gnc_start[c];

@@ -85,7 +85,7 @@ struct DeviceBasis {
        *d_invp = nullptr, *d_one = nullptr, *d_mirror = nullptr, *d_gen = nullptr, *d_ob221 = nullptr,
        *d_c122w = nullptr, *d_invp32 = nullptr, *d_pphh_b3 = nullptr;
   // host tables the work lists are built from
-  std::vector<int> ch_n, k_start, cc_n, cc_nph, grp_start, grp_kets, gen_ok;
+  std::vector<int> ch_n, k_start, cc_n, cc_nph, gen_ok;
   std::vector<int> ch_kstart, c122_start;
   std::vector<int2> pairs1;
   std::vector<int4> c122w_items;  // the W kernel's items (basis only, not tuned)

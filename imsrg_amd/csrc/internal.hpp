@@ -56,7 +56,6 @@ constexpr unsigned M110 = 1u << 0, M220 = 1u << 1, M111 = 1u << 2, M121 = 1u << 
 //  * cross-coupled channel uses the same formula with Tz = |tz_p - tz_q|/2
 //  * kmap[k*(jmax+1)+J]: local index of ket k in the standard channel of
 //    angular momentum J with the ket's parity and Tz, or -1
-//  * cmap[k*(jmax+1)+J]: same for the cross-coupled channel
 struct BasisDev {
   int norb, nkets, nch, jmax, d1, d2;
   int nholes, n1pairs;
@@ -64,7 +63,7 @@ struct BasisDev {
   long one_off;  // offset of the one-body block inside an operator buffer
   long two_off;  // offset of the two-body arena inside an operator buffer
   long opsize;   // doubles per operator buffer (including 8 doubles of zero slack at the end)
-  int maxn, maxcc, maxblk;
+  int maxn, maxblk;
   int ccjmax_ph;  // largest J of a CC channel with ph kets (-1: none); Zbar is zero above it
   const IMSRG_G int *j2, *l, *tz2, *cvq;
   const IMSRG_G int *orbcode;   // j2 | (l & 1) << 16 | (tz2 > 0) << 17, norb4 = norb rounded up to 4 entries
@@ -72,8 +71,7 @@ struct BasisDev {
   const IMSRG_G int *holes;
   const IMSRG_G int *obstart, *oblist;  // one-body block of each orbit
   const IMSRG_G int *kp, *kq;
-  const IMSRG_G int *kmap, *cmap;
-  const IMSRG_G int *cmapT;     // cmapT[J*nkets + k] = cmap[k*(jmax+1) + J]
+  const IMSRG_G int *kmap;
   const IMSRG_G int *kmapT;     // kmapT[J*nkets + k] = kmap[k*(jmax+1) + J]
   // the cross-coupled kets of one orbit o, by t = 4J + 2|tz_o - tz_x|/2 + parity for J <= ccjmax_ph
   // (ccnt = 4 (ccjmax_ph + 1) such sets), in the order of the other orbit x:
@@ -87,9 +85,9 @@ struct BasisDev {
   // for none; kmorb_nx: jmax + 1 rounded up to a multiple of 8
   const IMSRG_G unsigned short *kmorb;
   int kmorb_nx;
-  // kets of each (parity, Tz) group g = 2(Tz+1) + parity (the channels 6J + g),
-  // ascending global index: grp_kets[grp_start[g] .. grp_start[g+1])
-  const IMSRG_G int *grp_start, *grp_kets;
+  // kets of each (parity, Tz) group g = 2(Tz+1) + parity (the channels 6J + g), in ascending
+  // global index one group after another: group g's start at position grp_start[g]
+  const IMSRG_G int *grp_start;
   const IMSRG_G int *grp_first;  // grp_first[g*(norb+1) + k]: first ket of group g with an orbit p >= k
   // standard channels
   const IMSRG_G long *ch_off;

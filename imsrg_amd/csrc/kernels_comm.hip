@@ -1117,7 +1117,6 @@ __device__ __forceinline__ void barrier_lds() {
 __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, const int4 *items) {
   constexpr int T = kTileB;
   __shared__ __align__(16) StageB3 L0, L1, L2;  // 3 x 48 KiB: one work-group per CU
-  __shared__ signed char s_ph[2][T];  // unused in this mode (epilogue signature)
   const int4 it = items[blockIdx.x];
   if (it.y < 0) return;  // padding item of the XCD-balanced order
   PairPtrs P = pa.get(it.x);
@@ -1247,7 +1246,7 @@ __global__ __launch_bounds__(kGWaves * 64, 2) void k_pphh_big_b3p(PairArg pa, co
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[mi][ni][q] += h * (double)t1[mi][ni][q];
   }
-  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, s_ph);
+  gemm_epilogue<false, true>(acc, D, n, R0, S0, alpha, h, B.cc_run, nullptr);
 }
 
 __global__ __launch_bounds__(kGWaves * 64, 2) void k_ph_big_b3(PairArg pa, const int4 *items, int nitems) {
