@@ -474,9 +474,10 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   // comm221 one-body work (src/Commutator.cc:1246-1294) in partial sums: pair p
   // owns the slots ob_start[p] .. ob_start[p + 1] - 1 of the per-call buffer;
   // the first takes its comm111 + comm121 part, every item one more slot.
-  //  kind 0 (n_c != 0, M_pp over the long pp lists): one item per (c, J);
-  //  kind 1 (1 - n_c != 0, M_hh over the short hh lists): one item per 4 entries
-  //  of the list cpart of such orbits c (one wave each, all J)
+  //  kind 0 (n_c != 0, M_pp over the long pp lists): one item per 4 entries (c, J) of the
+  //  pair's part of ob_cj, (entries - 1) << 28 | first entry;
+  //  kind 1 (1 - n_c != 0, M_hh over the short hh lists): one item per 16 entries of the
+  //  list cpart of such orbits c (all J), 1 << 30 | first entry
   std::vector<int> ob_start(pairs1.size() + 1, 0), cpart;
   for (int c = 0; c < norb; ++c)
     if (std::fabs(1.0 - hb.occ[c]) > 1e-9) cpart.push_back(c);
@@ -513,10 +514,10 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
   {
     long tot = (long)B.d1 * B.d1 * B.d2 * B.d1 * B.d1 * B.d2;
     void *p = nullptr, *pQ = nullptr;
-    // the inverse Pandya copy: rows of up to 3 J' past the last
-    // 8 more: the Pandya kernel reads the J of one row in aligned groups of four pairs
+    // 8 more: the Pandya kernel reads the J of one row in aligned groups of four
     if (hipMalloc(&p, (tot + 8) * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(p);
+    // the inverse Pandya kernel reads rows of up to 3 J' past the last
     if (hipMalloc(&pQ, (tot + 4 * B.d2) * sizeof(double)) != hipSuccess) return "hipMalloc failed for the 6j table";
     allocs.push_back(pQ);
     if (hipMemset((double *)pQ + tot, 0, 4 * B.d2 * sizeof(double)) != hipSuccess)

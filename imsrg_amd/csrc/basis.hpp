@@ -67,7 +67,8 @@ struct WorkLists {
   std::vector<int4> invp;    // (pair, i | j << 16, k0 | k1 << 16, first ket | group << 28), FP64 Zbar; .y = -1: empty
   std::vector<int4> invp32;  // the same with FP32 Zbar, twice the elements per item
   std::vector<int4> one;     // (pair, i, j, index of the one-body pair)
-  std::vector<int4> ob221;   // (pair, one-body pair, kind/c/J, partial-sum slot) of the comm221 one-body part
+  std::vector<int4> ob221;   // (pair, one-body pair, kind 0: (entries - 1) << 28 | first entry of ob_cj,
+                             // kind 1: 1 << 30 | first entry of cpart, partial-sum slot): comm221 one-body part
   std::vector<int4> mirror;  // (pair, ch, rb, sb), rb < sb  and diagonal tiles; ch = -1: empty item
   std::vector<int4> gen;     // (pair, ch, 0, 0) channels with work for the generator
   std::vector<int4> c122w;   // (pair, ch, comm122 column bin, block of kC122Rows rows) of the W kernel

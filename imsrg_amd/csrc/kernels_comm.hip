@@ -525,9 +525,9 @@ __global__ __launch_bounds__(256) void k_syr2k(PairArg pa, const int4 *items) {
 // lower elements are (head) hZ-sign or (tail) phi_r phi_s times the upper ones, as the
 // reference's folds make them (src/Commutator.cc:1792-1805).  Without the others the ph
 // GEMM took 420 us at emax = 10 (FP64; 472 with them) and 335 us with FP32 products (355).
-// MIXED: operands rounded to FP32 when read from LDS, products on f32
-// 16x16x4 MFMA, FP32 partial sums over two stages (32 k) added into the FP64
-// accumulators.
+// MIXED (pp/hh, or with SPLIT; the ph GEMM with FP32 products is k_ph_big_f32): operands
+// rounded to FP32 when read from LDS, products on f32 16x16x4 MFMA, FP32 partial sums
+// over two stages (32 k) added into the FP64 accumulators.
 // SPLIT (with MIXED): each operand is split into two FP32 values, a = ah + al
 // with ah = fl32(a), al = fl32(a - ah), and a product takes three f32 MFMAs,
 // ah*bh + ah*bl + al*bh (the dropped al*bl is 2^-48 of it); the FP32 partial

@@ -8,7 +8,7 @@ namespace imsrg {
 
 // dense 6j table {jj1 jj2 J3; jj4 jj5 J6} (double-double Racah): `table` in the layout of
 // SixJCache_112112, `tableQ` in the sixjQ_index layout as the weights (2 J6 + 1) {6j},
-// 0 in place of |6j| < 1e-8 (padding entries are left untouched)
+// 0 in place of |6j| < 1e-8
 hipError_t launch_sixj_table(double *table, double *tableQ, int d1, int d2, hipStream_t s);
 
 // commutator phases; items are device arrays of int4 work items
@@ -96,17 +96,18 @@ enum class NormOp { kSum, kAxpy, kCopy };
 hipError_t launch_norm(const BasisDev *bd, const BasisDev &bh, NormOp op, double *y, const double *z, double a,
                        const double *x, double *partials, int maxpart, double *out, unsigned long long *done,
                        unsigned long long seq, hipStream_t s);
-// the basis-change matrices D of every channel (two-body layout, tbsize doubles) from
-// the one-body basis change C (norb x norb, column-major)
 // the Hartree-Fock monopoles W[q] = sum_J (2J+1) V~^J_{ia,jb} of quads[q] = (i, a, j, b)
 hipError_t launch_hf_mono(const BasisDev *bd, const double *op, const int4 *quads, int nq, double *W,
                           hipStream_t s);
-// block-sparse basis transformation (C block diagonal in (l, j2, tz2)): the D blocks
-// into Dg, T = V D (items (group, first row), R rows each), out two-body = D^T T (items
-// (channel, first column), kc columns each), out one-body = C^T O C (through one_tmp)
+// block-sparse basis transformation (C block diagonal in (l, j2, tz2)): the groups' D
+// fragments into Dg, then two passes over items (group, first row; kXfRows rows each; group
+// -1: none), T = (V D)^T and out two-body = D^T V D (herm 0: neither Hermitian nor
+// anti-Hermitian), and out one-body = C^T O C (through one_tmp)
 hipError_t launch_xform_blocks(const BasisDev *bd, const BasisDev &bh, const XformDev &X, const double *C,
                                const double *op, double *out, double *T, double *Dg, double *one_tmp,
                                const int2 *items, int nitems, int herm, hipStream_t s);
+// the basis-change matrices D of every channel (two-body layout, tbsize doubles) from
+// the one-body basis change C (norb x norb, column-major)
 hipError_t launch_hf_D(const BasisDev *bd, const BasisDev &bh, const double *C, double *D, hipStream_t s);
 hipError_t launch_fill_random(const BasisDev *bd, const BasisDev &bh, double *op, int herm,
                               unsigned long long seed, hipStream_t s);
