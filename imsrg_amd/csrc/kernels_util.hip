@@ -571,12 +571,10 @@ __global__ __launch_bounds__(256) void k_xf_pass(const BasisDev *bd, XformDev X,
     double a[kXfMaxM / 4];
 #pragma unroll
     for (int k = 0; k < kXfMaxM / 4; ++k)
-      if (k < nks) {
-        const double x = v[(long)ket[4 * k + (lane >> 4)] * n];
-        a[k] = 4 * k + (lane >> 4) < m ? x : 0.0;  // past the group: 0 whatever the last ket holds
-      }
+      if (k < nks) a[k] = v[(long)ket[4 * k + (lane >> 4)] * n];
     const double f = herm != 0.0 ? herm : 1.0;
     const int to = SECOND ? X.g_kets[cs + min(row, n - 1)] : 0;  // the row's place in V'
+    bool nan = false;
     for (int c = 0; c < nc; ++c) {
       xfd4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -596,7 +594,22 @@ __global__ __launch_bounds__(256) void k_xf_pass(const BasisDev *bd, XformDev X,
           if (col < m && rr < n) oc[(long)rr * n + s - cs + col] = acc[q];
         }
       }
+      if (c == 0) nan = __builtin_isnan((acc[0] + acc[1]) + (acc[2] + acc[3]));
     }
+    // The last fragment repeats the group's last ket against zeros of D, which makes NaN of an
+    // infinite one: such rows' results again, without them (the whole transformation at emax =
+    // 10 525 -> 532 us; with 0 in its place among the loads 552 to 632).
+    if ((m & 3) && __any(nan))
+      for (int col = lane >> 4; col < m; col += 4) {
+        double x = 0.0;
+        for (int k = 0; k < m; ++k)
+          x += v[(long)ket[k] * n] * lds[((col >> 4) * nks + (k >> 2)) * 64 + 16 * (k & 3) + (col & 15)];
+        if (__builtin_isfinite(x) || row >= n) continue;
+        if constexpr (SECOND)
+          oc[herm != 0.0 ? (long)ket[col] * n + to : (long)to * n + ket[col]] = f * x;
+        else
+          oc[(long)row * n + s - cs + col] = x;
+      }
   }
 }
 
