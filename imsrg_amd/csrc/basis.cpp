@@ -660,9 +660,10 @@ std::string DeviceBasis::upload(const HostBasis &hb, int emax6j) {
       return (long)tot;
     };
     for (int v = 0; v < 2; ++v) {
+      // (signed: the tables alone exceed the smaller sizes from emax = 13 on)
       auto cap_of = [&](int lds) {
-        return std::max(2048L, (long)((lds - InvpLds(nJ, nt, norb, ncls, quadcap, chunkcap).M) /
-                                      (v ? sizeof(float) : sizeof(double))) - 1);
+        return std::max(2048L, (lds - InvpLds(nJ, nt, norb, ncls, quadcap, chunkcap).M) /
+                                       (long)(v ? sizeof(float) : sizeof(double)) - 1);
       };
       // the smallest LDS size at which four of five bras that fit as a whole at the largest still do
       long cap = cap_of(kInvpLds);
