@@ -140,6 +140,7 @@ struct imsrg_ctx {
   hipEvent_t batch_ev = nullptr;
   // order imsrg_hip_commutator_ss_dev_async against the caller's stream
   hipEvent_t async_in = nullptr, async_out = nullptr;
+  hipEvent_t side_on = nullptr;  // the second stream has reached its work
   long long serial = 0;  // unique per context of the process (batch cache keys)
   HostBasis hb;
   DeviceBasis db;
@@ -297,6 +298,7 @@ static int ctx_init(imsrg_ctx *ctx, const imsrg_basis_desc *b, int device) {
   if (int rc = make_side_stream(ctx)) return rc;
   HIPCHK(ctx, hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming));
   HIPCHK(ctx, hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming));
+  HIPCHK(ctx, hipEventCreateWithFlags(&ctx->side_on, hipEventDisableTiming));
   HIPCHK(ctx, hipEventCreateWithFlags(&ctx->batch_ev, hipEventDisableTiming));
   HIPCHK(ctx, hipEventCreateWithFlags(&ctx->async_in, hipEventDisableTiming));
   HIPCHK(ctx, hipEventCreateWithFlags(&ctx->async_out, hipEventDisableTiming));
@@ -394,6 +396,7 @@ extern "C" int imsrg_hip_ctx_destroy(imsrg_ctx *ctx) {
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   if (ctx->fork) (void)hipEventDestroy(ctx->fork);
   if (ctx->join) (void)hipEventDestroy(ctx->join);
+  if (ctx->side_on) (void)hipEventDestroy(ctx->side_on);
   if (ctx->batch_ev) (void)hipEventDestroy(ctx->batch_ev);
   if (ctx->async_in) (void)hipEventDestroy(ctx->async_in);
   if (ctx->async_out) (void)hipEventDestroy(ctx->async_out);
@@ -1385,14 +1388,22 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   FrontItems fi{items[5], items[2], items[3], maxnch + 1, npairs * (maxnch + 1), cnt[5], m221 ? cnt[2] : 0,
                 mph ? cnt[3] : 0, prec_ph == 1 && tu.ph_big, items[7], items[9], mask & MPPHH ? cnt[7] : 0,
                 mask & M122 ? cnt[9] : 0, false};
+  // Split products cost three times the FP32 ones, so that with a light reference the pp/hh GEMM
+  // is the longer stream by far.  Its work-groups, one or two per CU, then have to be placed before
+  // the first launch fills the CUs (some had to wait for ph GEMM work-groups: emax = 7 He4
+  // 502 -> 386 us, emax = 8 862 -> 664, H 866 -> 667, O16 849 -> 745; not so with more ph work, emax =
+  // 8 Ca40, 32 Pandya chunks per tile, 1030 -> 1057).
+  const bool gemm_first = tu.overlap_pphh == 1 && (mask & MPPHH) && npairs == 1 && prec_pphh == 2 && cnt[big] >= 128 &&
+                          cnt[big] <= kFrontSplit && fi.npandya < 20 * cnt[big];
   // a profiled commutator has a launch per phase instead, each between its events
-  const bool small = fi.blocks() <= kFrontSmall && !ctx->profiling;
+  const bool small = fi.blocks() <= kFrontSmall && !ctx->profiling && !gemm_first;
   if (!small) fi.n64 = fi.nc122 = 0;
   const bool overlap = tu.overlap_pphh && (mask & MPPHH) && !(small && cnt[big] == 0);
   // overlap_pphh 1: fork before the first kernel; 2: fork after the ph GEMM, so
   // that the pp/hh GEMM shares the GPU with the inverse Pandya gather only
   const bool fork_late = overlap && tu.overlap_pphh == 2;
-  fi.split = overlap && !fork_late && npairs == 1 && prec_pphh != kGemmB3 && cnt[big] > kFrontSplit;
+  fi.split = overlap && !fork_late && npairs == 1 && prec_pphh != kGemmB3 &&
+             cnt[big] > (prec_pphh == 2 ? kFrontSplit / 2 : kFrontSplit);
   // comm122's W on the main stream, after the inverse Pandya kernel, where the bf16x3 GEMM
   // has many tiles: with one work-group per CU it leaves room beside it, whichever stream is the
   // longer one (with heavier references the main stream is).  emax = 10 (1539 tiles) O16 1823 ->
@@ -1418,6 +1429,7 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   // was empty (a nested commutator follows a norm that the host has waited for).
   auto side_work = [&]() -> int {
     HIPCHK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork, 0));
+    if (gemm_first) HIPCHK(ctx, hipEventRecord(ctx->side_on, ctx->side));
     if (set) HIPCHK(ctx, hipEventRecord((*set)[9], ctx->side));
     HIPCHK(ctx, launch_pphh(pa, items[big], cnt[big], items[7], cnt[7] - fi.n64, items[8], cnt[8], prec_pphh, maxn,
                             ctx->side));
@@ -1438,16 +1450,24 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
   HIPCHK(ctx, mark(1));
   if (m122 && !overlap) HIPCHK(ctx, launch_c122_w(pa, items[9], cnt[9], maxbin, s));
   HIPCHK(ctx, mark(2));
-  if (set) {
-    FrontItems zero = fi, one = fi;
-    zero.none = zero.n221 = zero.npandya = 0;
-    one.nzeros = one.npandya = 0;
-    fi.nzeros = fi.none = fi.n221 = 0;
-    HIPCHK(ctx, launch_front(pa, zero, maxnch, maxbin, false, s));
-    HIPCHK(ctx, mark(3));
-    HIPCHK(ctx, launch_front(pa, one, maxnch, maxbin, false, s));
-    HIPCHK(ctx, mark(4));
+  if (gemm_first) {
+    if (int rc = side_work()) return rc;
+    HIPCHK(ctx, hipStreamWaitEvent(s, ctx->side_on, 0));
   }
+  if (set || gemm_first) {  // the zero-body part (a few us) alone
+    FrontItems zero = fi;
+    zero.none = zero.n221 = zero.npandya = 0;
+    fi.nzeros = 0;
+    HIPCHK(ctx, launch_front(pa, zero, maxnch, maxbin, false, s));
+  }
+  HIPCHK(ctx, mark(3));
+  if (set) {
+    FrontItems one = fi;
+    one.npandya = 0;
+    fi.none = fi.n221 = 0;
+    HIPCHK(ctx, launch_front(pa, one, maxnch, maxbin, false, s));
+  }
+  HIPCHK(ctx, mark(4));
   HIPCHK(ctx, launch_front(pa, fi, maxnch, maxbin, prec_pphh == 1, s));
   HIPCHK(ctx, mark(5));
   if (mask & MPH) HIPCHK(ctx, launch_ph_gemm(pa, items[1], cnt[1], prec_ph, tu.ph_big != 0, s));
@@ -1463,7 +1483,8 @@ static int run_commutator(imsrg_ctx *ctx, const PairArg &pa, int npairs, const i
     HIPCHK(ctx, mark(12));
   }
   if (overlap) {
-    if (int rc = side_work()) return rc;
+    if (!gemm_first)
+      if (int rc = side_work()) return rc;
     HIPCHK(ctx, hipStreamWaitEvent(s, ctx->join, 0));
   }
   HIPCHK(ctx, mark(7));

@@ -55,7 +55,8 @@ constexpr int kFrontSmall = 3500;
 // 4824 -> 4643).  Not so with fewer tiles (FP64 emax = 8, 393 tiles, O16 469 -> 485 us, Ca40 604 ->
 // 638; emax = 7 235 -> 258), beside the bf16x3 GEMM, one work-group per CU (mixed emax = 8 Ca40
 // 465 -> 477, emax = 10 O16 1728 -> 1761, Ca40 2200 -> 2202, emax = 12 8.24 -> 8.22 ms), and in
-// batches (FP64, 24 pairs at emax = 6 1501 -> 1515 us, 8 at emax = 8 3.43 -> 3.43 ms).
+// batches (FP64, 24 pairs at emax = 6 1501 -> 1515 us, 8 at emax = 8 3.43 -> 3.43 ms).  Split products,
+// three times the FP32 work per tile: from half as many (emax = 8 Ca40 1032 -> 987 us).
 constexpr int kFrontSplit = 512;
 // pp/hh SYR2K: items on 128x128 tiles, items64 on 64x64 tiles (disjoint channels);
 // under bf16x3 products (kGemmB3) the pack items first write the operand panels
