@@ -1984,6 +1984,7 @@ __device__ __forceinline__ void c122_w_tile(const PairPtrs &P, const int4 &it, u
   double *W = P.c122w + off;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m = lane & 15, kq = lane >> 4;
+  bool bad = false;
   for (int r0 = R0 + 16 * wv; r0 < min(R0 + kC122Rows, n); r0 += 64) {
     const int row = min(r0 + m, n - 1);
     dbl4 acc[kC122MaxN / 16];
@@ -2020,24 +2021,27 @@ __device__ __forceinline__ void c122_w_tile(const PairPtrs &P, const int4 &it, u
         if (c < nn && r0 + m < n) blk_at(W, (unsigned)sq[n0 + c] * n + row) = acc[j][q];
       }
     }
-    // A row with an Inf or NaN in a column of the bin is not finite in all of its results, the
-    // first among them, through products with 0: such a row again from its partner entries
-    // alone, each lane the columns it has stored.
-    if (!__builtin_isfinite(acc[0][0]) && r0 + m < n) {
-      for (int c = kq; c < nn; c += 4) blk_at(W, (unsigned)sq[n0 + c] * n + row) = 0.0;
-      double w = 0.0;
-      int last = -1;  // entries of one column follow one another
-      for (int t = 0; t < ne; ++t) {
-        const int4 rec = B.c122_brec[eo + t];
-        const int c = (rec.y >> 16) - n0;
-        if (c < 0 || c >= nn || (c & 3) != kq) continue;
-        if (c != last) w = 0.0;
-        last = c;
-        const double f = __hiloint2double(rec.w, rec.z);
-        const unsigned e = (unsigned)sq[rec.y & 0xffff] * n + row;
-        w += blk_at(Y2, e) * (P.X[B.one_off + rec.x] * f) - blk_at(X2, e) * (P.Y[B.one_off + rec.x] * f);
-        blk_at(W, (unsigned)sq[n0 + c] * n + row) = w;
-      }
+    bad = bad || !__builtin_isfinite(acc[0][0]);
+  }
+  // A row with an Inf or NaN in a column of the bin is not finite in all of its results, the
+  // first among them, through products with 0: the wave's rows with such a result again from
+  // their partner entries alone, each lane the columns that it has stored.
+  if (!__any(bad)) return;
+  for (int row = R0 + 16 * wv + m; row < min(R0 + kC122Rows, n); row += 64) {
+    if (__builtin_isfinite(blk_at(W, (unsigned)sq[n0 + min(kq, nn - 1)] * n + row))) continue;
+    for (int c = kq; c < nn; c += 4) blk_at(W, (unsigned)sq[n0 + c] * n + row) = 0.0;
+    double w = 0.0;
+    int last = -1;  // entries of one column follow one another
+    for (int t = 0; t < ne; ++t) {
+      const int4 rec = B.c122_brec[eo + t];
+      const int c = (rec.y >> 16) - n0;
+      if (c < 0 || c >= nn || (c & 3) != kq) continue;
+      if (c != last) w = 0.0;
+      last = c;
+      const double f = __hiloint2double(rec.w, rec.z);
+      const unsigned e = (unsigned)sq[rec.y & 0xffff] * n + row;
+      w += blk_at(Y2, e) * (P.X[B.one_off + rec.x] * f) - blk_at(X2, e) * (P.Y[B.one_off + rec.x] * f);
+      blk_at(W, (unsigned)sq[n0 + c] * n + row) = w;
     }
   }
 }
