@@ -1494,16 +1494,16 @@ __device__ __forceinline__ void front_pandya(const PairPtrs &P, const int4 &it, 
             const double w = u == 0 ? w01.x : u == 1 ? w01.y : u == 2 ? w23.x : w23.y;
             const bool ok = J >= jmin && J <= jmax && !(even & J) && fabs(w) >= 1e-8 && r != 0xffff && cl != 0xffff;
             wv[u] = ok ? (2 * J + 1) * w * sgn_parity(s0 + sj * J) : 0.0;
-            // an invalid term reads the operator's first element and counts as 0
+            // an invalid term is 0 (its address that of the operator's first element)
             const int4 ch = s_ch[ok ? 6 * J + g : 0];
             const long idx = ok ? (((long)ch.y << 32) | (unsigned)ch.x) + (long)(cl * ch.z + r) : 0;
-            xv[u] = X2[idx];
-            yv[u] = Y2[idx];
+            xv[u] = ok ? X2[idx] : 0.0;
+            yv[u] = ok ? Y2[idx] : 0.0;
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            xbar -= wv[u] * (wv[u] != 0.0 ? xv[u] : 0.0);
-            ybar -= wv[u] * (wv[u] != 0.0 ? yv[u] : 0.0);
+            xbar -= wv[u] * xv[u];
+            ybar -= wv[u] * yv[u];
           }
         }
       }
